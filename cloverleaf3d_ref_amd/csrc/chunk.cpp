@@ -1265,7 +1265,6 @@ int clover_chunk_create_ex(const clover_deck *deck, int device, int flags, clove
         c->fast = !(flags & CLOVER_CHUNK_PER_CALL);
         c->store = (flags & CLOVER_CHUNK_FP32) ? ST_F32 : ST_F64;
         c->halo_check = (flags & CLOVER_CHUNK_HALO_CHECK) != 0;
-        c->shapes = default_shapes();
         c->dt_tile = -1;
         // the uniform mesh as initialise_chunk.f90:37-39 and
         // initialise_chunk_kernel.f90:151-178 compute it
@@ -1318,6 +1317,8 @@ int clover_chunk_create_ex(const clover_deck *deck, int device, int flags, clove
             t.h_cellz = h.cellz;
             hip_check(hipStreamSynchronize(c->st), "sync");  // host buffers die here
         }
+        std::vector<Lay> lays;
+        for (auto &t : c->tiles) lays.push_back(t.g);
         // more than one tile: the fused step as batched launches, if every
         // tile's calc_dt partials fit the partial buffer at the shortest
         // march chunk the tuner may pick
@@ -1329,6 +1330,8 @@ int clover_chunk_create_ex(const clover_deck *deck, int device, int flags, clove
                 tiles_table_init(c);
             }
         }
+        // a launch covers every tile where the stages are batched, else one
+        c->shapes = size_shapes(c->store, lays.data(), c->batched ? T : 1);
         // start.f90:58-129
         c->time = 0.0;
         c->step = 0;
@@ -1571,7 +1574,8 @@ int clover_chunk_get_shape(const clover_chunk *c, int kernel, int *planes, int *
     CLOVER_API_BEGIN
     if (!c || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = c->shapes.k[kernel].planes;
+    const Shape &sh = c->shapes.k[kernel];
+    *planes = sh.cap ? sh.cap : sh.planes;
     *xcd = c->shapes.k[kernel].xcd;
     *block_x = c->shapes.k[kernel].bx;
     CLOVER_API_END

@@ -11,6 +11,7 @@
 // captured once in a graph and replayed.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <tuple>
@@ -43,7 +44,7 @@ struct clover_ensemble {
     int step = 0;
     int advect_x = 1;
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // index: advect_x
-    Shapes shapes = default_shapes();              // launch shapes (autotuner)
+    Shapes shapes{};                               // launch shapes (size_shapes, autotuner)
 };
 
 namespace {
@@ -475,10 +476,14 @@ int clover_ensemble_create(const clover_deck *decks, int ndecks, int device, int
         }
         hip_check(hipMalloc(&e->dev, sizeof(DeckDev) * ndecks), "hipMalloc decks");
         hip_check(hipMemcpy(e->dev, e->host.data(), sizeof(DeckDev) * ndecks, hipMemcpyHostToDevice), "H2D decks");
+        std::vector<Lay> lays(ndecks);
+        for (int d = 0; d < ndecks; d++) lays[d] = e->host[d].g;
+        e->shapes = size_shapes(e->store, lays.data(), ndecks);
         prepare_grids(e);
         // calc_dt's partials: room for the visc/dt grid of every shape the
-        // autotuner tries (the most blocks at its fewest planes)
-        const BatchGrid &vg = grid(e, BK_VISC_DT, kTunePlanes[0]);
+        // autotuner tries and of the one the decks start with (the most
+        // blocks at the fewest planes)
+        const BatchGrid &vg = grid(e, BK_VISC_DT, std::min(kTunePlanes[0], shape(e, BK_VISC_DT).planes));
         const BatchGrid &sg = kgrid(e, BK_SUMMARY);
         hip_check(hipMalloc(&e->visc_partial, sizeof(double) * (vg.total + 1)), "hipMalloc");
         hip_check(hipMalloc(&e->sum_partial, sizeof(double) * 5 * (sg.total + 1)), "hipMalloc");
@@ -619,7 +624,8 @@ int clover_ensemble_get_shape(const clover_ensemble *e, int kernel, int *planes,
     CLOVER_API_BEGIN
     if (!e || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = e->shapes.k[kernel].planes;
+    const Shape &sh = e->shapes.k[kernel];
+    *planes = sh.cap ? sh.cap : sh.planes;
     *xcd = e->shapes.k[kernel].xcd;
     *block_x = e->shapes.k[kernel].bx;
     CLOVER_API_END
@@ -649,6 +655,7 @@ int clover_ensemble_set_shape(clover_ensemble *e, int kernel, int planes, int xc
     sh.planes = planes;
     sh.xcd = xcd;
     sh.wgs = workgroups;
+    sh.cap = 0;
     shapes_changed(e);
     CLOVER_API_END
 }

@@ -50,6 +50,8 @@ struct Shape {
     int bx;   // z marches: threads along x per workgroup (64, 128, 256 or 512; see block_of)
     int wgs;  // batched launches: 0 for one workgroup per tile, else this many
               // persistent workgroups walk the tile list (batch.h tile_walk)
+    int cap;  // 0, or the most planes size_shapes allows on any mesh: `planes`
+              // is then what it gave this one
 };
 
 // Workgroup of a z march for shape sh: bx threads along x and 256/bx rows
@@ -69,14 +71,9 @@ constexpr int kTuneCount = sizeof(kTunePlanes) / sizeof(kTunePlanes[0]);
 // (the tuner's candidates give 1, 2 and 4)
 __host__ __device__ inline int cell_x_rows(int planes) { return planes >= 64 ? planes / 32 : 1; }
 
-// 64 positions per workgroup of 64 x 4 (one row per wave for the x cell
-// sweep); the XCD order for the y/z momentum sweeps
-inline Shapes default_shapes()
-{
-    Shapes s;
-    for (int i = 0; i < SK_COUNT; i++) s.k[i] = Shape{i == SK_CELL_X ? 32 : 64, i == SK_MOM_Y || i == SK_MOM_Z, 64};
-    return s;
-}
+// The launch shapes of a mesh (or of the tiles or decks one launch covers)
+// before any tuning, chosen from its size (fast_kernels.hip)
+Shapes size_shapes(Store s, const Lay *lays, int n);
 
 inline size_t store_bytes(Store s) { return s == ST_F32 ? sizeof(float) : sizeof(double); }
 

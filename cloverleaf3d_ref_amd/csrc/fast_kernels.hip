@@ -19,6 +19,8 @@
 // plane that uses it.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "batch.h"
 #include "fast.h"
 #include "launch.h"
@@ -1176,6 +1178,81 @@ int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
     default: return 0;
     }
     return gx * gy * gz;
+}
+
+// Launch shapes by size.  A march of `planes` positions costs about
+// planes + 1 position times (the extra one is the prologue that reloads the
+// planes below its chunk); the GPU runs `slots` workgroups of a kernel at a
+// time (FP64 accel_pdv one per CU and its FP32 form two, the others about
+// five), so n workgroups take ceil(n / slots) rounds where they are few (under
+// kRounds; whole rounds, since all workgroups of one run alike) and
+// n / slots where they are many.  The rule takes the planes with the least
+// (planes + 1) * rounds, up to a cap per kernel above which large meshes lose
+// (512^3, FP64: pdv_predict 1.43 ms at 8 planes against 1.55 at 64, mom_x
+// 2.18 against 2.62, mom_y 2.39 at 32 against 2.79 at 8).  With 64 planes on
+// every mesh a 64^3 tile ran visc_dt in 16 workgroups, one per sixteen CUs.
+// Measured per launch, 64 planes -> the rule, FP64: 64^3 accel_pdv
+// 161 -> 14 us, mom_z 59 -> 17, visc_dt 71 -> 10; 131 x 75 x 93 accel_pdv
+// 226 -> 40, mom_x 94 -> 25; 256^3 mom_z 478 -> 350, accel_pdv 691 -> 605.  Over
+// 13 meshes from 16^3 to 512^3 and both forms the rule stays within 1-4 % (mean
+// per kernel) of the best of 13 plane counts.
+// The XCD order pays in accel_pdv and cell_x, and in FP32 mom_x, on meshes
+// that do not fit the L2s (512^3: FP64 accel_pdv 4.33 -> 4.17 ms, cell_x 1.75
+// -> 1.59, FP32 accel_pdv 2.58 -> 2.33); below kXcdCells it costs a
+// microsecond or two per launch.
+constexpr int kXcdCells = 4000000;
+constexpr double kRounds = 2.0;
+
+static int size_planes(BatchKernel k, Store s, const Lay *lays, int n, int slots, int cap)
+{
+    int best = 1;
+    double best_t = 0.0;
+    for (int p = 1; p <= cap; p++) {
+        long long wgs = 0;
+        for (int i = 0; i < n; i++) wgs += batch_blocks(k, lays[i], p, s);
+        double r = (double)wgs / slots;
+        if (r < kRounds) r = std::ceil(r);
+        const double t = (p + 1) * r;
+        if (p == 1 || t <= best_t) {
+            best = p;
+            best_t = t;
+        }
+    }
+    return best;
+}
+
+Shapes size_shapes(Store s, const Lay *lays, int n)
+{
+    constexpr int cus = 256;
+    const bool f32 = s == ST_F32;
+    long long cells = 0;
+    for (int i = 0; i < n; i++) {
+        const Lay &g = lays[i];
+        cells += (long long)(g.x_max - g.x_min + 1) * (g.y_max - g.y_min + 1) * (g.z_max - g.z_min + 1);
+    }
+    const int far = cells >= kXcdCells;
+    struct {
+        int shape;
+        BatchKernel k;
+        int cap, slots, xcd;
+    } const marches[] = {
+        {SK_VISC_DT, BK_VISC_DT, 16, 5 * cus, 0},
+        {SK_PDV_PREDICT, BK_PDV_PREDICT, 8, 5 * cus, 0},
+        {SK_ACCEL_PDV, BK_ACCEL_PDV, f32 ? 8 : 32, f32 ? 2 * cus : cus, far},
+        {SK_CELL_Y, BK_CELL_Y, 16, 5 * cus, 0},
+        {SK_CELL_Z, BK_CELL_Z, 16, 5 * cus, 0},
+        {SK_MOM_X, BK_MOM_X, 8, 5 * cus, f32 ? far : 0},
+        {SK_MOM_Y, BK_MOM_Y, 32, 5 * cus, 0},
+        {SK_MOM_Z, BK_MOM_Z, 32, 5 * cus, 0},
+    };
+    Shapes sh;
+    // the x cell sweep has no march: a row per wave, two in FP32 (launch.h
+    // cell_x_rows) where the mesh fills the GPU several times over
+    const int rows = f32 && far ? 64 : 32;
+    sh.k[SK_CELL_X] = Shape{rows, far, 64, 0, rows};
+    for (const auto &m : marches)
+        sh.k[m.shape] = Shape{size_planes(m.k, s, lays, n, m.slots, m.cap), m.xcd, 64, 0, m.cap};
+    return sh;
 }
 
 #define BLAUNCH(name, kern, block, ...)                                                                       \

@@ -290,6 +290,9 @@ int clover_chunk_kernel_times(clover_chunk *c, char *buf, int buflen);
  * of the visc/dt and PdV-predictor z marches (64, 128, 256 or 512 threads
  * along x, with 256/64, 256/128 or 1 rows; the other kernels' workgroups are
  * fixed, block_x 64).
+ * A chunk (and an ensemble) starts with shapes chosen from its size: `planes`
+ * is then the most positions its workgroups march over, and a mesh with few
+ * tiles takes fewer so that they fill the GPU.
  * A shape changes how the work is split, never a value.  Kernel indices: */
 #define CLOVER_SHAPE_VISC_DT 0
 #define CLOVER_SHAPE_PDV_PREDICT 1
