@@ -32,46 +32,6 @@ int64_t dense_elems(const Lay &g, int cls)
     return (int64_t)ex * ey * ez;
 }
 
-void upload_dense_any(const Lay &g, int cls, const void *host, void *dev, size_t es, hipStream_t st)
-{
-    int ex, ey, ez;
-    class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
-    if (class_is_1d(cls)) {
-        hip_check(hipMemcpyAsync(dev, host, es * ex, hipMemcpyHostToDevice, st), "upload 1-D");
-        return;
-    }
-    for (int l = 0; l < ez; l++)
-        hip_check(hipMemcpy2DAsync((char *)dev + es * (g.base + (size_t)g.plane * l), es * g.ld,
-                                   (const char *)host + es * ((size_t)ex * ey * l), es * ex, es * ex, ey,
-                                   hipMemcpyHostToDevice, st),
-                  "upload plane");
-}
-
-void download_dense_any(const Lay &g, int cls, const void *dev, void *host, size_t es, hipStream_t st)
-{
-    int ex, ey, ez;
-    class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
-    if (class_is_1d(cls)) {
-        hip_check(hipMemcpyAsync(host, dev, es * ex, hipMemcpyDeviceToHost, st), "download 1-D");
-        return;
-    }
-    for (int l = 0; l < ez; l++)
-        hip_check(hipMemcpy2DAsync((char *)host + es * ((size_t)ex * ey * l), es * ex,
-                                   (const char *)dev + es * (g.base + (size_t)g.plane * l), es * g.ld, es * ex, ey,
-                                   hipMemcpyDeviceToHost, st),
-                  "download plane");
-}
-
-void upload_dense(const Lay &g, int cls, const double *host, double *dev, hipStream_t st)
-{
-    upload_dense_any(g, cls, host, dev, sizeof(double), st);
-}
-
-void download_dense(const Lay &g, int cls, const double *dev, double *host, hipStream_t st)
-{
-    download_dense_any(g, cls, dev, host, sizeof(double), st);
-}
-
 namespace {
 
 struct Resident {
@@ -88,8 +48,26 @@ struct Ctx {
     double *partial = nullptr;  // reduction partials (device)
     double *scalar = nullptr;   // reduction results (device)
     double *h_scalar = nullptr; // pinned host mirror of `scalar`
+    Stage stage;                // field uploads and fetches
     std::unordered_map<const void *, Resident> map;
     std::mutex mu;
+
+    // device copy <- host array, and back (which waits for the stream)
+    void upload(const Resident &r, const double *host)
+    {
+        if (class_is_1d(r.cls))
+            hip_check(hipMemcpyAsync(r.dev, host, r.bytes, hipMemcpyHostToDevice, stream), "upload 1-D");
+        else
+            stage.upload(r.g, r.cls, host, r.dev, stream);
+    }
+    void download(const Resident &r, double *host)
+    {
+        if (class_is_1d(r.cls))
+            hip_check(hipMemcpyAsync(host, r.dev, r.bytes, hipMemcpyDeviceToHost, stream), "download 1-D");
+        else
+            stage.download(r.g, r.cls, r.dev, sizeof(double), host, stream);
+        hip_check(hipStreamSynchronize(stream), "sync");
+    }
 };
 
 Ctx &ctx()
@@ -141,7 +119,7 @@ double *res(void *h, int cls, const Lay &g)
     }
     hip_check(hipMalloc(&r.dev, r.bytes), "hipMalloc field");
     hip_check(hipMemsetAsync(r.dev, 0, r.bytes, c.stream), "hipMemset field");
-    upload_dense(g, cls, (const double *)h, r.dev, c.stream);
+    c.upload(r, (const double *)h);
     c.map.emplace(h, r);
     return r.dev;
 }
@@ -188,6 +166,7 @@ int clover_hip_finalize(void)
     hip_check(hipStreamSynchronize(c.stream), "sync");
     for (auto &kv : c.map) hip_check(hipFree(kv.second.dev), "hipFree");
     c.map.clear();
+    c.stage.release();
     hip_check(hipFree(c.partial), "hipFree");
     hip_check(hipFree(c.scalar), "hipFree");
     hip_check(hipHostFree(c.h_scalar), "hipHostFree");
@@ -212,8 +191,7 @@ int clover_hip_fetch(const void *host)
     std::lock_guard<std::mutex> lock(c.mu);
     auto it = c.map.find(host);
     if (it == c.map.end()) throw Error(E_ARG, "clover_hip_fetch: address not resident");
-    download_dense(it->second.g, it->second.cls, it->second.dev, (double *)host, c.stream);
-    hip_check(hipStreamSynchronize(c.stream), "sync");
+    c.download(it->second, (double *)host);
     CLOVER_API_END
 }
 
@@ -225,7 +203,7 @@ int clover_hip_push(const void *host)
     std::lock_guard<std::mutex> lock(c.mu);
     auto it = c.map.find(host);
     if (it == c.map.end()) throw Error(E_ARG, "clover_hip_push: address not resident");
-    upload_dense(it->second.g, it->second.cls, (const double *)host, it->second.dev, c.stream);
+    c.upload(it->second, (const double *)host);
     hip_check(hipStreamSynchronize(c.stream), "sync");
     CLOVER_API_END
 }

@@ -114,6 +114,7 @@ struct clover_chunk {
     double *partial;  // per tile: kMaxPartials * 5
     double *scalar;   // per tile: 8
     double *h_scalar; // pinned
+    Stage stage;      // field fetches
     double dt, dtold, time;
     int step;
     int advect_x;
@@ -1214,6 +1215,7 @@ static void destroy(clover_chunk *c)
 {
     if (!c) return;
     if (c->st) (void)hipStreamSynchronize(c->st);
+    c->stage.release();
     for (auto &t : c->tiles) {
         for (int a = 0; a < NUM_ARRAYS; a++)
             if (t.f[a]) (void)hipFree(t.f[a]);
@@ -1495,15 +1497,7 @@ int clover_chunk_fetch_field(clover_chunk *c, int t, int field, double *host)
     // the fused step forms soundspeed where it reads it instead of storing it
     if (field == F_SOUNDSPEED && c->fast) ideal_gas(c, false, true);
     Tile &tt = c->tiles[t];
-    if (c->store == ST_F64) {
-        download_dense(tt.g, class_of(field), tt.f[field], host, c->st);
-        hip_check(hipStreamSynchronize(c->st), "sync");
-    } else {
-        std::vector<float> f((size_t)dense_elems(tt.g, class_of(field)));
-        download_dense_any(tt.g, class_of(field), tt.f[field], f.data(), sizeof(float), c->st);
-        hip_check(hipStreamSynchronize(c->st), "sync");
-        for (size_t q = 0; q < f.size(); q++) host[q] = f[q];
-    }
+    c->stage.download(tt.g, class_of(field), tt.f[field], store_bytes(c->store), host, c->st);
     CLOVER_API_END
 }
 

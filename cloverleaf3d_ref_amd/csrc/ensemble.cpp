@@ -40,6 +40,7 @@ struct clover_ensemble {
     double *visc_partial = nullptr;
     double *sum_partial = nullptr;
     double *sums = nullptr;
+    Stage stage;  // field fetches
     double g_small = 0.0, g_big = 0.0;
     int step = 0;
     int advect_x = 1;
@@ -374,6 +375,7 @@ void destroy(clover_ensemble *e)
 {
     if (!e) return;
     if (e->st) (void)hipStreamSynchronize(e->st);
+    e->stage.release();
     for (auto &g : e->graph)
         if (g) (void)hipGraphExecDestroy(g);
     for (int *p : e->tables) (void)hipFree(p);
@@ -595,16 +597,7 @@ int clover_ensemble_fetch_field(clover_ensemble *e, int deck, int field, double 
     DeckDev D;
     hip_check(hipMemcpyAsync(&D, e->dev + deck, sizeof D, hipMemcpyDeviceToHost, e->st), "D2H");
     hip_check(hipStreamSynchronize(e->st), "sync");
-    const int cls = class_of(field);
-    if (e->store == ST_F64) {
-        download_dense(D.g, cls, (const double *)D.f[field], host, e->st);
-        hip_check(hipStreamSynchronize(e->st), "sync");
-    } else {
-        std::vector<float> fl((size_t)dense_elems(D.g, cls));
-        download_dense_any(D.g, cls, D.f[field], fl.data(), sizeof(float), e->st);
-        hip_check(hipStreamSynchronize(e->st), "sync");
-        for (size_t q = 0; q < fl.size(); q++) host[q] = fl[q];
-    }
+    e->stage.download(D.g, class_of(field), D.f[field], store_bytes(e->store), host, e->st);
     CLOVER_API_END
 }
 

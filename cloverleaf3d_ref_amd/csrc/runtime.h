@@ -47,13 +47,38 @@ inline void hip_check(hipError_t e, const char *what)
         return clover::E_ARG;                             \
     }
 
-// Copy a dense Fortran array of class `cls` (host) into / out of the device
-// layout g.  1-D classes are plain contiguous copies.
-void upload_dense(const Lay &g, int cls, const double *host, double *dev, hipStream_t st);
-void download_dense(const Lay &g, int cls, const double *dev, double *host, hipStream_t st);
-// the same for arrays of es-byte elements
-void upload_dense_any(const Lay &g, int cls, const void *host, void *dev, size_t es, hipStream_t st);
-void download_dense_any(const Lay &g, int cls, const void *dev, void *host, size_t es, hipStream_t st);
+// Moves 3-D fields between the device layout g and dense Fortran arrays of
+// class `cls` on the host, through two pinned buffers that its owner keeps
+// (at most kPieceElems doubles each; allocated on first use, freed by the
+// owner's release()).  Every piece is enqueued on the stream, after what is
+// there.
+class Stage {
+  public:
+    Stage() = default;
+    Stage(const Stage &) = delete;
+    Stage &operator=(const Stage &) = delete;
+    // dev holds es-byte elements (8 or 4); returns when host is filled
+    void download(const Lay &g, int cls, const void *dev, size_t es, double *host, hipStream_t st);
+    // returns when host has been read; the device copy follows on the stream
+    void upload(const Lay &g, int cls, const double *host, double *dev, hipStream_t st);
+    // waits for the kernels that use the buffers and frees them; not a
+    // destructor's work, since an owner of static lifetime may outlive the
+    // device runtime
+    void release();
+
+  private:
+    struct Buf {
+        double *host = nullptr, *dev = nullptr;  // one pinned allocation, seen from both sides
+        hipEvent_t done = nullptr;               // the kernel that uses it last
+        bool busy = false;
+    };
+    static constexpr int64_t kPieceElems = 512 * 1024;  // 4 MiB
+    void reserve(int64_t total);
+    void wait(Buf &b);
+    Buf buf_[2];
+    int64_t elems_ = 0;  // doubles per buffer
+    int next_ = 0;       // upload's next buffer
+};
 
 // element count of the dense host array of class cls
 int64_t dense_elems(const Lay &g, int cls);
