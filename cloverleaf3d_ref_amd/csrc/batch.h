@@ -45,8 +45,11 @@ enum BatchKernel : int {
     BK_CELL_X, BK_CELL_Y, BK_CELL_Z, BK_MOM_X, BK_MOM_Y, BK_MOM_Z, BK_COUNT
 };
 int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s);
-// reflective halo along `axis` for `nitems` (field, face) items
-int batch_blocks_reflect(const Lay &g, int axis, int depth, int nitems);
+// a reflective exchange of n3[axis] (field, face) items per axis, which
+// batch_reflect_faces counts (both faces of every flagged field; axes, null
+// for all: as for launch_update_halo_store)
+int batch_blocks_reflect(const Lay &g, int depth, const int *n3);
+void batch_reflect_faces(const int *fields, const int *axes, int *n3);
 
 // The tiles (workgroup-sized blocks of the decks' grids, numbered through
 // the prefix table) that this workgroup runs: t, t+step, ... below end.
@@ -109,17 +112,20 @@ hipError_t batch_advec_cell(Store s, const DeckDev *decks, int nd, const BatchGr
 // advec_mom sweep `dir`; new velocities into X_W5..X_W7
 hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
                            int sweep_number, const Shape &sh, hipStream_t st);
-// reflective halo of the flagged fields along one axis, both faces; axes
-// (null: all) as for launch_update_halo_store
-hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int axis, int depth,
-                         const int *fields, hipStream_t st, const int *axes = nullptr);
+// reflective halo of the flagged fields, every face; axes (null: all) as for
+// launch_update_halo_store
+hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int depth, const int *fields,
+                         hipStream_t st, const int *axes = nullptr);
 
 // The tiles of one chunk as a batch (chunk.cpp, more than one tile): one
 // launch per pass of update_halo over every tile.  An item is one (tile,
 // face, field): a copy from tile `nbr` (update_tile_halo_kernel.f90), or the
 // reflective halo of an external face (update_halo_kernel.f90, nbr = tile).
+// code and want are a reflection's boundary and refreshed faces (halo_once.h).
 struct TileHaloItem {
     int tile, nbr, field, hi, kind, ea, eb, poison;
+    unsigned code;
+    int want;
     double sgn;
 };
 // blocks one item needs along the face's two tangential axes for tile g
@@ -128,6 +134,12 @@ void tile_halo_blocks(const Lay &g, int axis, int depth, int &per_a, int &per_b)
 // (items: device array; per_a x per_b: the largest tile's blocks)
 hipError_t batch_tile_halo(Store s, bool copy, const DeckDev *tiles, const TileHaloItem *items, int nitems, int per_a,
                            int per_b, int axis, int depth, hipStream_t st);
+// the reflective halos of every axis in one launch, for tiles at least 3 cells
+// thick: n3[k] items of the k-th axis in y, x, z order (one list), with
+// blocks3[k] blocks each (the most that tile_once_blocks gives for one)
+int tile_once_blocks(const Lay &g, int axis, int depth);
+hipError_t batch_tile_reflect(Store s, const DeckDev *tiles, const TileHaloItem *items, const int *n3,
+                              const int *blocks3, int depth, hipStream_t st);
 // the item lists of one update_halo over the tiles: copy[pass] for the three
 // tile passes (y, x, z faces), refl[k][side] for the reflective faces of the
 // k-th axis in y, x, z order; nbr6: 6 neighbours per tile (from 1, -1

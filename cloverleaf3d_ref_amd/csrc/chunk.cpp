@@ -146,6 +146,8 @@ struct clover_chunk {
         TileHaloItem *dev;
         int n_copy[3], off_copy[3], pa_copy[3], pb_copy[3];
         int n_refl[3][2], off_refl[3][2], pa_refl[3], pb_refl[3];
+        int n_axis[3], once_blocks[3];
+        bool once;      // the reflective faces of every axis in one launch
         bool split[3];  // the faces of that reflective axis in two launches (a tile under 3 cells thick)
     };
     std::map<std::string, HaloTabs> halo_tabs;  // per update_halo signature
@@ -474,7 +476,10 @@ static void batched_update_halo(clover_chunk *c, const int *fields, int depth, c
             }
             tab.pa_copy[p] = pa;
             tab.pb_copy[p] = pb;
-            pa = pb = 1;
+        }
+        for (int p = 0; p < 3; p++) {
+            const int axis = axis_order[p];
+            int pa = 1, pb = 1;
             bool split = false;
             for (int sd = 0; sd < 2; sd++) {
                 tab.off_refl[p][sd] = (int)all.size();
@@ -492,8 +497,17 @@ static void batched_update_halo(clover_chunk *c, const int *fields, int depth, c
             }
             tab.pa_refl[p] = pa;
             tab.pb_refl[p] = pb;
+            tab.n_axis[p] = tab.n_refl[p][0] + tab.n_refl[p][1];
+            for (int sd = 0; sd < 2; sd++)
+                for (auto &x : refl[p][sd])
+                    tab.once_blocks[p] = std::max(tab.once_blocks[p], tile_once_blocks(lays[x.tile], axis, depth));
             tab.split[p] = split;
         }
+        // one launch for all three axes where every tile is thick enough (a
+        // thin one anywhere: its halo cells trace back to other halo cells)
+        tab.once = !poison;
+        for (auto &g : lays)
+            tab.once = tab.once && g.x_max - g.x_min >= 2 && g.y_max - g.y_min >= 2 && g.z_max - g.z_min >= 2;
         tab.dev = nullptr;
         if (!all.empty()) {
             tab.dev = reinterpret_cast<TileHaloItem *>(dev_alloc_bytes(c, sizeof(TileHaloItem) * all.size()));
@@ -514,6 +528,12 @@ static void batched_update_halo(clover_chunk *c, const int *fields, int depth, c
                       "tile halo");
     }
     Phase ph(c, P_SELF_HALO);
+    if (tab.once) {  // the axes' lists follow one another in the table
+        hip_check(batch_tile_reflect(c->store, c->tdev, tab.dev + tab.off_refl[0][0], tab.n_axis,
+                                     tab.once_blocks, depth, c->st),
+                  "update_halo");
+        return;
+    }
     for (int p = 0; p < 3; p++) {
         if (tab.split[p]) {
             for (int sd = 0; sd < 2; sd++)

@@ -36,7 +36,7 @@ struct clover_ensemble {
     char *arena = nullptr;
     long long bytes = 0;
     std::vector<int *> tables;  // device prefix tables
-    std::map<std::tuple<int, int, int>, BatchGrid> grids;
+    std::map<std::tuple<int, int, int, int, int>, BatchGrid> grids;
     double *visc_partial = nullptr;
     double *sum_partial = nullptr;
     double *sums = nullptr;
@@ -82,21 +82,34 @@ int shape_index(int bk)
 
 const Shape &shape(clover_ensemble *e, int bk) { return e->shapes.k[shape_index(bk)]; }
 
-// kind: 0..BK_COUNT-1 kernels (a: planes of the launch shape, b unused);
-// 100 + axis reflective halos (a: depth, b: items)
-const BatchGrid &grid(clover_ensemble *e, int kind, int a, int b = 0)
+// the prefix table of `key`, from `count` blocks per deck
+template <typename Count>
+const BatchGrid &table(clover_ensemble *e, const std::tuple<int, int, int, int, int> &key, const Count &count)
 {
-    auto key = std::make_tuple(kind, a, b);
     auto it = e->grids.find(key);
     if (it != e->grids.end()) return it->second;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hip_check(hipStreamIsCapturing(e->st, &cs), "capture status");
     if (cs != hipStreamCaptureStatusNone) throw Error(E_STATE, "ensemble: launch table missing during capture");
     std::vector<int> counts(e->nd);
-    for (int d = 0; d < e->nd; d++)
-        counts[d] = kind < 100 ? batch_blocks((BatchKernel)kind, e->host[d].g, a, e->store)
-                               : batch_blocks_reflect(e->host[d].g, kind - 100, a, b);
+    for (int d = 0; d < e->nd; d++) counts[d] = count(e->host[d].g);
     return e->grids[key] = make_grid(e, counts);
+}
+
+// batched kernel `kind` (BK_*) at `planes` of the launch shape
+const BatchGrid &grid(clover_ensemble *e, int kind, int planes)
+{
+    return table(e, std::make_tuple(kind, planes, 0, 0, 0),
+                 [&](const Lay &g) { return batch_blocks((BatchKernel)kind, g, planes, e->store); });
+}
+
+// a reflective exchange
+const BatchGrid &halo_grid(clover_ensemble *e, const int *fields, const int *axes, int depth)
+{
+    int n[3];
+    batch_reflect_faces(fields, axes, n);
+    return table(e, std::make_tuple(BK_COUNT, depth, n[0], n[1], n[2]),
+                 [&](const Lay &g) { return batch_blocks_reflect(g, depth, n); });
 }
 
 // a kernel's grid for its current launch shape
@@ -112,42 +125,18 @@ void set_fields(int *fields, std::initializer_list<int> ids)
     for (int id : ids) fields[id] = 1;
 }
 
-// update_halo for single-tile decks: the reflective boundary on every face,
-// y faces, then x, then z (as launch_update_halo orders them), reduced to
-// the halos the fused kernels read (fused_halo_plan, driver.h)
-int items_on_axis(const HaloPlan &p, int axis)
+// update_halo for single-tile decks: the reflective boundary of every face
+// (axes null), or reduced to the halos the fused kernels read
+void halo(clover_ensemble *e, const int *fields, int depth, const int *axes = nullptr)
 {
-    int n = 0;
-    for (int f = 0; f < NUM_FIELDS; f++) n += p.fields[f] == 1 && ((p.raxes[f] >> axis) & 1);
-    return 2 * n;  // both faces
-}
-
-// every flagged field on every axis (start.f90's exchange)
-void halo(clover_ensemble *e, const int *fields, int depth)
-{
-    int n = 0;
-    for (int f = 0; f < NUM_FIELDS; f++) n += fields[f] == 1;
-    static const int axis_order[3] = {1, 0, 2};
-    for (int ao = 0; ao < 3; ao++) {
-        const int axis = axis_order[ao];
-        hip_check(batch_reflect(e->store, e->dev, e->nd, grid(e, 100 + axis, depth, 2 * n), axis, depth, fields,
-                                e->st),
-                  "halo");
-    }
+    hip_check(batch_reflect(e->store, e->dev, e->nd, halo_grid(e, fields, axes, depth), depth, fields, e->st, axes),
+              "halo");
 }
 
 void halo(clover_ensemble *e, int which)
 {
-    const HaloPlan p = fused_halo_plan(which, e->advect_x != 0, AX_ALL);
-    static const int axis_order[3] = {1, 0, 2};
-    for (int ao = 0; ao < 3; ao++) {
-        const int axis = axis_order[ao];
-        const int n = items_on_axis(p, axis);
-        if (n == 0) continue;
-        hip_check(batch_reflect(e->store, e->dev, e->nd, grid(e, 100 + axis, p.depth, n), axis, p.depth, p.fields,
-                                e->st, p.raxes),
-                  "halo");
-    }
+    const HaloPlan p = fused_halo_plan(which, e->advect_x != 0, AX_ALL);  // driver.h
+    halo(e, p.fields, p.depth, p.raxes);
 }
 
 void ideal_gas(clover_ensemble *e)
@@ -232,10 +221,7 @@ void prepare_grids(clover_ensemble *e)
     for (int ax = 0; ax < 2; ax++)
         for (int which = FH_TIMESTEP; which <= FH_MOM3; which++) {
             const HaloPlan p = fused_halo_plan(which, ax != 0, AX_ALL);
-            for (int axis = 0; axis < 3; axis++) {
-                const int n = items_on_axis(p, axis);
-                if (n) grid(e, 100 + axis, p.depth, n);
-            }
+            halo_grid(e, p.fields, p.raxes, p.depth);
         }
 }
 

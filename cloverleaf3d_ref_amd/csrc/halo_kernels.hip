@@ -2,10 +2,12 @@
 // (update_halo_kernel.f90:115-1425) and the tile-to-tile copies
 // (update_tile_halo_kernel.f90:31-1993), table driven.
 //
-// One launch handles one axis (both faces when the tile is at least 3 cells
-// thick along it, else one face) for every flagged field: blockIdx.z picks
-// (field, face), threads cover the two tangential axes, each thread walks
-// the 1..depth halo layers.  Exact moves, no arithmetic.
+// A reflective exchange of a tile at least 3 cells thick along every axis is
+// one launch for every flagged field and face (halo_once.h).  A thinner tile
+// takes the reference's passes in order: inside one workgroup per field where
+// the faces are small, else a launch per axis (or face).  Threads cover a
+// face's two tangential axes, each the 1..depth halo layers.  Exact moves,
+// no arithmetic.
 //
 // The resident driver refreshes only the (field, axis) halos its kernels
 // read (the axis masks below); in its test mode the halos it skips are
@@ -13,14 +15,14 @@
 // would put there), so any read of a skipped halo changes interior results.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "batch.h"
 #include "fast.h"
+#include "halo_once.h"
 #include "kernels.h"
 
 namespace clover {
-
-// How a field sits on an axis (see the reflective formulas below).
-enum { K_CELL = 0, K_STAG = 1, K_FTAN = 2 };
 
 struct HaloDesc {
     unsigned char kind[3];   // per axis x, y, z
@@ -28,12 +30,8 @@ struct HaloDesc {
     unsigned char ext[6][2]; // per face L,R,B,T,K,F: +1 on the first/second tangential range
 };
 
-// Reflective halo, per field id (data.f90:55-74).  For a face normal to
-// axis a, for d = 1..depth:   halo(W) = sgn * f(R)   with
-//   CELL  low W=1-d R=d     high W=max+d   R=max+1-d   (cell-centred data)
-//   STAG  low W=1-d R=1+d   high W=max+1+d R=max+1-d   (vertex data, face data normal to a)
-//   FTAN  low W=1-d R=1+d   high W=max+d   R=max-d     (face data tangential to a)
-// and tangential ranges min-depth..max+depth (+ext).  Transcribed from
+// Reflective halo, per field id (data.f90:55-74), in the terms of
+// halo_once.h.  Transcribed from
 // update_halo_kernel.f90: cells 115-596, velocities 604-1004, vol/mass_flux_x
 // 1018-1142, _y 1156-1280, _z 1291-1417 (vol_flux_z's bottom face stops at
 // z_max+depth, mass_flux_z's at z_max+1+depth).
@@ -58,6 +56,17 @@ static const HaloDesc kHalo[NUM_FIELDS] = {
     {{2, 1, 2}, {0, 1, 0}, {{1, 0}, {1, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}}},  // mass_flux_y
     {{2, 2, 1}, {0, 0, 1}, {{0, 1}, {0, 1}, {0, 1}, {0, 1}, {0, 0}, {0, 0}}},  // mass_flux_z
 };
+
+// kHalo[f] in one word (halo_once.h)
+static HaloCode halo_code(int f)
+{
+    const HaloDesc &d = kHalo[f];
+    HaloCode h = 0;
+    for (int a = 0; a < 3; a++) h |= (unsigned)d.kind[a] << (2 * a) | (unsigned)d.neg[a] << (6 + a);
+    for (int face = 0; face < 6; face++)
+        for (int t = 0; t < 2; t++) h |= (unsigned)d.ext[face][t] << (9 + 2 * face + t);
+    return h;
+}
 
 // staggered (vertex-like) along x, y, z, per field id
 static const unsigned char kStag[NUM_FIELDS][3] = {
@@ -162,10 +171,185 @@ static hipError_t run_batch_reflect(Store s, const Lay &g, int axis, int depth, 
     return hipGetLastError();
 }
 
+// blocks one face along `axis` needs for its two tangential axes (the widest
+// class, depth 1 or 2)
+__host__ __device__ inline void dims_reflect(const Lay &g, int axis, int depth, int &ga, int &gb)
+{
+    const int mn[3] = {g.x_min, g.y_min, g.z_min};
+    const int mx[3] = {g.x_max, g.y_max, g.z_max};
+    const int ta = axis == 0 ? 1 : 0, tb = axis == 2 ? 1 : 2;
+    const int na = mx[ta] - mn[ta] + 2 + 2 * depth, nb = mx[tb] - mn[tb] + 2 + 2 * depth;
+    ga = (na + HX - 1) / HX;
+    gb = (nb + HY - 1) / HY;
+}
+
+// What one launch refreshes: per face its field's slot, axis and side, axis by
+// axis; per slot the array, its boundary and the faces it refreshes (a bit
+// each).
+struct OnceSet {
+    int n[3];  // faces per axis
+    int face[6 * NUM_FIELDS];
+    int slots;
+    struct {
+        void *arr;  // null in the batched launches, which take it from the deck
+        HaloCode code;
+        short want, field;
+    } f[NUM_FIELDS];
+};
+
+// the fields flagged in `fields`, on the external faces of `ext` and the axes
+// of `axes` (null: all)
+static OnceSet once_set(const int *fields, const int *axes, const int *ext, void *const *fp)
+{
+    OnceSet o{};
+    for (int f = 0; f < NUM_FIELDS; f++) {
+        if (fields[f] != 1 || (fp && !fp[f])) continue;
+        int want = 0;
+        for (int face = 0; face < 6; face++)
+            if (ext[face] && wanted(axes, f, face / 2)) want |= 1 << face;
+        if (!want) continue;
+        auto &q = o.f[o.slots++];
+        q.arr = fp ? fp[f] : nullptr;
+        q.code = halo_code(f);
+        q.want = (short)want;
+        q.field = (short)f;
+    }
+    int at = 0;
+    for (int face = 0; face < 6; face++)
+        for (int q = 0; q < o.slots; q++)
+            if ((o.f[q].want >> face) & 1) {
+                o.face[at++] = 8 * q + face;
+                o.n[face / 2]++;
+            }
+    return o;
+}
+
+// blocks of a one-pass launch per face along `axis`: a thread per pair of
+// tangential coordinates
+constexpr int kOnceThreads = 256;
+__host__ __device__ inline int once_blocks(const Lay &g, int axis, int depth)
+{
+    const int nx = g.x_max - g.x_min + 2 + 2 * depth, ny = g.y_max - g.y_min + 2 + 2 * depth,
+              nz = g.z_max - g.z_min + 2 + 2 * depth;
+    return ((axis == 0 ? ny : nx) * (axis == 2 ? ny : nz) + kOnceThreads - 1) / kOnceThreads;
+}
+
+static int once_blocks(const Lay &g, int depth, const int *n)
+{
+    int total = 0;
+    for (int axis = 0; axis < 3; axis++) total += n[axis] * once_blocks(g, axis, depth);
+    return total;
+}
+
+// this thread's cells of block b of a face
+template <typename S>
+__device__ inline void once_body(const Lay &g, int depth, HaloCode h, int want, S *dst, int face, int b)
+{
+    const int axis = face >> 1, xn = g.x_min - depth, yn = g.y_min - depth, zn = g.z_min - depth;
+    const unsigned nx = (unsigned)(g.x_max - xn + 2 + depth), ny = (unsigned)(g.y_max - yn + 2 + depth),
+                   na = axis == 0 ? ny : nx;
+    const unsigned c = (unsigned)b * kOnceThreads + threadIdx.x, row = c / na, a = c - row * na;
+    reflect_once(g, depth, h, want, dst, axis, face & 1, (axis == 0 ? yn : xn) + (int)a, (axis == 2 ? yn : zn) + (int)row);
+}
+
+// the face (an index of OnceSet::face) and its block that block b of the
+// launch runs
+__device__ inline int once_face(const Lay &g, int depth, const int *n, int &b)
+{
+    int first = 0;
+    for (int axis = 0; axis < 3; axis++) {
+        const int blocks = once_blocks(g, axis, depth);
+        if (b < n[axis] * blocks) {
+            const int i = (int)((unsigned)b / (unsigned)blocks);
+            b -= i * blocks;
+            return first + i;
+        }
+        b -= n[axis] * blocks;
+        first += n[axis];
+    }
+    return -1;
+}
+
+// Bound by its launch on small meshes and by the x faces' partial lines on
+// large ones (a line per row for two cells).  One launch instead of three per
+// exchange, 4.2 us instead of 11 at 64^3 (the FP64 step 168 -> 140 us) and 0.37
+// instead of 0.45 ms per step at 512^3; the batched form 118 -> 77 us per step
+// for 24 FP32 decks of 16^3 to 64^3.  Both layers of a pair of tangential
+// coordinates go to one thread: unrolled further (four cells, 18 KB of code run
+// once per wave) the launch took 18 us at 64^3, instruction fetch included.
+template <typename S>
+__global__ void __launch_bounds__(kOnceThreads) k_reflect_once(Lay g, int depth, OnceSet o)
+{
+    const int face = o.face[blockIdx.y], q = face >> 3;
+    if ((int)blockIdx.x >= once_blocks(g, (face & 7) >> 1, depth)) return;
+    once_body<S>(g, depth, o.f[q].code, o.f[q].want, static_cast<S *>(o.f[q].arr), face & 7, (int)blockIdx.x);
+}
+
+// The reference's passes in their order for one field per workgroup, a barrier
+// after each face: what a tile under 3 cells thick needs, where a depth-2
+// reflection reads the opposite face's halo.  10 x 2 x 2: 40 launches per
+// step -> 8, the step 218 -> 95 us.
+constexpr int kOrderedThreads = 1024;
+constexpr int kOrderedCells = 16 * kOrderedThreads;  // largest face, layers included: beyond it the launches win
+
+template <typename S>
+__global__ void __launch_bounds__(kOrderedThreads) k_reflect_ordered(Lay g, int depth, OnceSet o)
+{
+    const int q = (int)blockIdx.x;
+    S *dst = static_cast<S *>(o.f[q].arr);
+    const HaloCode h = o.f[q].code;
+    const int want = o.f[q].want;
+    for (int pass = 0; pass < 3; pass++) {
+        const int axis = pass == 0 ? 1 : pass == 1 ? 0 : 2;
+        const int ta0 = (axis == 0 ? g.y_min : g.x_min) - depth, ta1 = (axis == 0 ? g.y_max : g.x_max) + depth;
+        const int tb0 = (axis == 2 ? g.y_min : g.z_min) - depth, tb1 = (axis == 2 ? g.y_max : g.z_max) + depth;
+        const int mx = axis == 0 ? g.x_max : axis == 1 ? g.y_max : g.z_max, kind = halo_kind(h, axis);
+        for (int side = 0; side < 2; side++) {
+            const int face = 2 * axis + side;
+            if (!((want >> face) & 1)) continue;  // the same for the whole workgroup
+            const int na = ta1 - ta0 + 1 + halo_ext(h, face, 0), nb = tb1 - tb0 + 1 + halo_ext(h, face, 1);
+            for (int c = (int)threadIdx.x; c < na * nb * depth; c += kOrderedThreads) {
+                const int d = c % depth + 1, a = ta0 + c / depth % na, b = tb0 + c / depth / na;
+                const int w = !side ? 1 - d : mx + d + (kind == K_STAG);
+                const int r = !side ? (kind == K_CELL ? d : 1 + d) : kind == K_FTAN ? mx - d : mx + 1 - d;
+                const Cell3 cw = axis == 0 ? Cell3{w, a, b} : axis == 1 ? Cell3{a, w, b} : Cell3{a, b, w};
+                const Cell3 cr = axis == 0 ? Cell3{r, a, b} : axis == 1 ? Cell3{a, r, b} : Cell3{a, b, r};
+                dst[idx(g, cw)] = signed_of(dst[idx(g, cr)], halo_neg(h, axis));
+            }
+            __syncthreads();
+        }
+    }
+}
+
 hipError_t launch_update_halo_store(Store s, const Lay &g, void *const *fp, const int *fields, const int *ext,
                                     int depth, hipStream_t st, const int *axes, bool poison)
 {
-    // The reference's order per field is bottom, top, left, right, back,
+    if (depth < 1 || depth > 2) return hipErrorInvalidValue;  // two layers per thread
+    const int n[3] = {g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1};
+    const bool thin = n[0] < 3 || n[1] < 3 || n[2] < 3;
+    int face = 0;  // cells of the largest one
+    for (int a = 0; a < 3; a++) face = std::max(face, depth * (n[a] + 5) * (n[(a + 1) % 3] + 5));
+    if (!poison && (!thin || face <= kOrderedCells)) {
+        const OnceSet o = once_set(fields, axes, ext, fp);
+        if (!o.slots) return hipSuccess;
+        if (t_kernel_timer) t_kernel_timer->begin("k_reflect", st);
+        if (thin) {
+            const dim3 grid((unsigned)o.slots), blk(kOrderedThreads);
+            if (s == ST_F32) hipLaunchKernelGGL(k_reflect_ordered<float>, grid, blk, 0, st, g, depth, o);
+            else hipLaunchKernelGGL(k_reflect_ordered<double>, grid, blk, 0, st, g, depth, o);
+        } else {
+            int most = 0;
+            for (int a = 0; a < 3; a++)
+                if (o.n[a]) most = std::max(most, once_blocks(g, a, depth));
+            const dim3 grid((unsigned)most, (unsigned)(o.n[0] + o.n[1] + o.n[2])), blk(kOnceThreads);
+            if (s == ST_F32) hipLaunchKernelGGL(k_reflect_once<float>, grid, blk, 0, st, g, depth, o);
+            else hipLaunchKernelGGL(k_reflect_once<double>, grid, blk, 0, st, g, depth, o);
+        }
+        if (t_kernel_timer) t_kernel_timer->end(st);
+        return hipGetLastError();
+    }
+    // A large thin tile, or the halo check (whose poisoned faces no later
+    // pass may shadow).  The reference's order per field is bottom, top, left, right, back,
     // front; fields are independent arrays, so all fields' y faces go first,
     // then x, then z.  The two faces of one axis touch disjoint cells when the
     // tile is at least 3 cells thick along it and then share a launch.
@@ -294,74 +478,42 @@ hipError_t launch_tile_halo_store(Store s, int face, const Lay &g, void *const *
 }
 
 // ---------------------------------------------------------------------------
-// Batched reflective halo over many decks (batch.h): both faces of one axis
-// for the flagged fields; every deck is at least 3 cells thick along every
-// axis, so the two faces touch disjoint cells and share the launch.
-struct BItem {
-    int field, hi, kind, ea, eb;
-    double sgn;
-};
-struct BItems {
-    int n;
-    BItem it[kMaxItems];
-};
+// Batched reflective halo over many decks (batch.h): one launch for every
+// flagged field and face of every deck (each at least 3 cells thick along
+// every axis, all its faces external).
+static const int kAllFaces[6] = {1, 1, 1, 1, 1, 1};
 
-__host__ __device__ inline void dims_reflect(const Lay &g, int axis, int depth, int &ga, int &gb)
-{
-    const int mn[3] = {g.x_min, g.y_min, g.z_min};
-    const int mx[3] = {g.x_max, g.y_max, g.z_max};
-    const int ta = axis == 0 ? 1 : 0, tb = axis == 2 ? 1 : 2;
-    const int na = mx[ta] - mn[ta] + 2 + 2 * depth, nb = mx[tb] - mn[tb] + 2 + 2 * depth;
-    ga = (na + HX - 1) / HX;
-    gb = (nb + HY - 1) / HY;
-}
+int batch_blocks_reflect(const Lay &g, int depth, const int *n3) { return once_blocks(g, depth, n3); }
 
-int batch_blocks_reflect(const Lay &g, int axis, int depth, int nitems)
+void batch_reflect_faces(const int *fields, const int *axes, int *n3)
 {
-    int ga, gb;
-    dims_reflect(g, axis, depth, ga, gb);
-    return nitems * ga * gb;
+    const OnceSet o = once_set(fields, axes, kAllFaces, nullptr);
+    for (int a = 0; a < 3; a++) n3[a] = o.n[a];
 }
 
 template <typename S>
-__global__ void kb_reflect(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int axis,
-                           int depth, BItems items)
+__global__ void __launch_bounds__(kOnceThreads)
+kb_reflect(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int depth, OnceSet o)
 {
     const int d = deck_of(start, nd, (int)blockIdx.x);
     const DeckDev &D = decks[d];
-    int ga, gb;
-    dims_reflect(D.g, axis, depth, ga, gb);
-    const int lb = (int)blockIdx.x - start[d];
-    const int item = lb / (ga * gb), r = lb % (ga * gb);
-    const BItem &it = items.it[item];
-    reflect_body<S>(D.g, axis, depth, static_cast<S *>(D.f[it.field]), it.sgn, it.kind, it.hi, it.ea, it.eb, r % ga,
-                    r / ga, 0);
+    const Lay g = D.g;
+    int b = (int)blockIdx.x - start[d];
+    const int i = once_face(g, depth, o.n, b);
+    if (i < 0) return;
+    const int face = o.face[i], q = face >> 3;
+    once_body<S>(g, depth, o.f[q].code, o.f[q].want, static_cast<S *>(D.f[o.f[q].field]), face & 7, b);
 }
 
-hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int axis, int depth,
-                         const int *fields, hipStream_t st, const int *axes)
+hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int depth, const int *fields,
+                         hipStream_t st, const int *axes)
 {
-    if (depth < 1 || depth > 2) return hipErrorInvalidValue;  // reflect_body holds two depths
-    BItems b;
-    b.n = 0;
-    for (int side = 0; side < 2; side++) {
-        const int face = 2 * axis + side;
-        for (int f = 0; f < NUM_FIELDS; f++) {
-            if (fields[f] != 1 || !wanted(axes, f, axis)) continue;
-            const HaloDesc &h = kHalo[f];
-            BItem &it = b.it[b.n++];
-            it.field = f;
-            it.hi = side;
-            it.kind = h.kind[axis];
-            it.ea = h.ext[face][0];
-            it.eb = h.ext[face][1];
-            it.sgn = h.neg[axis] ? -1.0 : 1.0;
-        }
-    }
-    if (b.n == 0 || bg.total == 0) return hipSuccess;
+    if (depth < 1 || depth > 2) return hipErrorInvalidValue;  // two layers per thread
+    const OnceSet o = once_set(fields, axes, kAllFaces, nullptr);
+    if (!o.slots || bg.total == 0) return hipSuccess;
     if (t_kernel_timer) t_kernel_timer->begin("kb_reflect", st);
-    if (s == ST_F32) hipLaunchKernelGGL(kb_reflect<float>, dim3(bg.total), dim3(HX, HY), 0, st, decks, bg.start, nd, axis, depth, b);
-    else hipLaunchKernelGGL(kb_reflect<double>, dim3(bg.total), dim3(HX, HY), 0, st, decks, bg.start, nd, axis, depth, b);
+    if (s == ST_F32) hipLaunchKernelGGL(kb_reflect<float>, dim3(bg.total), dim3(kOnceThreads), 0, st, decks, bg.start, nd, depth, o);
+    else hipLaunchKernelGGL(kb_reflect<double>, dim3(bg.total), dim3(kOnceThreads), 0, st, decks, bg.start, nd, depth, o);
     if (t_kernel_timer) t_kernel_timer->end(st);
     return hipGetLastError();
 }
@@ -404,6 +556,52 @@ kb_tile_reflect(const DeckDev *__restrict__ tiles, const TileHaloItem *__restric
     const DeckDev &D = tiles[it.tile];
     reflect_body<S>(D.g, axis, depth, static_cast<S *>(D.f[it.field]), it.sgn, it.kind, it.hi, it.ea, it.eb, bx, by,
                     it.poison);
+}
+
+// the three passes' items in one launch (halo_once.h): the k-th axis in y, x,
+// z order has n[k] items of blocks[k] blocks each
+struct TileOnce {
+    int n[3], blocks[3];
+};
+
+template <typename S>
+__global__ void __launch_bounds__(kOnceThreads)
+kb_tile_reflect_once(const DeckDev *__restrict__ tiles, const TileHaloItem *__restrict__ items, int depth, TileOnce o)
+{
+    int b = (int)blockIdx.x, first = 0, p = 0;
+    while (p < 2 && b >= o.n[p] * o.blocks[p]) {
+        b -= o.n[p] * o.blocks[p];
+        first += o.n[p++];
+    }
+    const int i = (int)((unsigned)b / (unsigned)o.blocks[p]);
+    const TileHaloItem it = items[first + i];
+    const DeckDev &D = tiles[it.tile];
+    const int axis = p == 0 ? 1 : p == 1 ? 0 : 2;
+    const Lay g = D.g;
+    once_body<S>(g, depth, it.code, it.want, static_cast<S *>(D.f[it.field]), 2 * axis + it.hi,
+                             b - i * o.blocks[p]);
+}
+
+int tile_once_blocks(const Lay &g, int axis, int depth) { return once_blocks(g, axis, depth); }
+
+hipError_t batch_tile_reflect(Store s, const DeckDev *tiles, const TileHaloItem *items, const int *n3,
+                              const int *blocks3, int depth, hipStream_t st)
+{
+    if (depth < 1 || depth > 2) return hipErrorInvalidValue;  // two layers per thread
+    TileOnce o;
+    int blocks = 0;
+    for (int p = 0; p < 3; p++) {
+        o.n[p] = n3[p];
+        o.blocks[p] = blocks3[p];
+        blocks += n3[p] * blocks3[p];
+    }
+    if (blocks == 0) return hipSuccess;
+    if (t_kernel_timer) t_kernel_timer->begin("kb_tile_reflect", st);
+    const dim3 grid((unsigned)blocks), blk(kOnceThreads);
+    if (s == ST_F32) hipLaunchKernelGGL(kb_tile_reflect_once<float>, grid, blk, 0, st, tiles, items, depth, o);
+    else hipLaunchKernelGGL(kb_tile_reflect_once<double>, grid, blk, 0, st, tiles, items, depth, o);
+    if (t_kernel_timer) t_kernel_timer->end(st);
+    return hipGetLastError();
 }
 
 void tile_halo_blocks(const Lay &g, int axis, int depth, int &per_a, int &per_b)
@@ -488,6 +686,9 @@ void tile_halo_items(const int *nbr6, int ntiles, const Lay *lays, const int *fi
                     if (!want && !poison) continue;
                     const HaloDesc &h = kHalo[f];
                     TileHaloItem it{};
+                    it.code = halo_code(f);
+                    for (int q = 0; q < 6; q++)
+                        if (nbr6[6 * t + q] == -1 && wanted(raxes, f, q / 2)) it.want |= 1 << q;
                     it.tile = t;
                     it.nbr = t;
                     it.field = f;
