@@ -63,7 +63,9 @@ ARRAYS_PER_CELL = {
     # sweeps.  visc_dt reads rho0, p, u0, v0, w0 (it forms the soundspeed
     # from rho0 and p) and writes q; pdv_predict reads rho0, e0, q, u0, v0, w0
     # (it forms the level-0 pressure from rho0 and e0) and writes p.
-    # accel_pdv reads rho0, e0, p, q, u0, v0, w0 and writes u1, v1, w1, rho1, e1 and the three volume fluxes
+    # accel_pdv reads rho0, e0, p, q, u0, v0, w0 and writes u1, v1, w1, rho1, e1 and the three volume fluxes;
+    # lagrange is pdv_predict and accel_pdv in one (single tiles): the same less p and one read of the state
+    "k_fast_lagrange": 14,
     "k_fast_visc_dt": 6, "k_fast_pdv_predict": 7, "k_fast_accel_pdv": 15,
     "k_fast_cell_x": 7.5, "k_fast_cell_y": 7, "k_fast_cell_z": 7.5,
     "k_fast_mom_x": 9, "k_fast_mom_y": 9, "k_fast_mom_z": 9,
@@ -76,7 +78,7 @@ def kernel_domain_cells(name: str, n: int) -> int:
     if name in ("k_cell_vols", "k_mom_vols"):
         return (n + 4) ** 3
     if name in ("k_accelerate", "k_reset_field", "k_flux_calc", "k_mom_flux", "k_mom_update", "k_node_flux",
-                "k_node_mass", "k_fast_accel_pdv", "k_fast_mom_x", "k_fast_mom_y",
+                "k_node_mass", "k_fast_accel_pdv", "k_fast_lagrange", "k_fast_mom_x", "k_fast_mom_y",
                 "k_fast_mom_z"):
         return (n + 1) ** 3
     return n ** 3

@@ -409,7 +409,8 @@ static int shape_of(int bk)
     switch (bk) {
     case BK_VISC_DT: return SK_VISC_DT;
     case BK_PDV_PREDICT: return SK_PDV_PREDICT;
-    case BK_ACCEL_PDV: return SK_ACCEL_PDV;
+    case BK_ACCEL_PDV:
+    case BK_LAGRANGE: return SK_ACCEL_PDV;
     case BK_CELL_X: return SK_CELL_X;
     case BK_CELL_Y: return SK_CELL_Y;
     case BK_CELL_Z: return SK_CELL_Z;
@@ -957,6 +958,8 @@ static void visit_prepare(clover_chunk *c)
 }
 
 // ---------------------------------------------------------------- autotuner
+static bool lagrange_chunk(const clover_chunk *c);
+
 // Launches shaped kernel k over every tile with its current shape, writing
 // only the spare work arrays: pdv_predict updates pressure in place, so it
 // runs on a copy of pressure in work array 3 (the copy is made by the caller,
@@ -988,7 +991,11 @@ static void tune_launch(clover_chunk *c, int k)
                                         t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[F_YVEL0], t.f[F_ZVEL0], sh, c->st);
             break;
         case SK_ACCEL_PDV:
-            e = launch_fast_accel_pdv(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
+            e = lagrange_chunk(c) ?
+                launch_fast_lagrange(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
+                                     t.f[X_W2], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[X_W5], t.f[F_YVEL0], t.f[X_W6],
+                                     t.f[F_ZVEL0], t.f[X_W7], t.f[X_W3], t.f[X_W4], t.f[X_W3], sh, c->st) :
+                launch_fast_accel_pdv(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
                                       t.f[X_W2], t.f[F_PRESSURE], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[X_W5],
                                       t.f[F_YVEL0], t.f[X_W6], t.f[F_ZVEL0], t.f[X_W7], t.f[X_W3], t.f[X_W4],
                                       t.f[X_W3], sh, c->st);
@@ -1129,6 +1136,7 @@ static void autotune(clover_chunk *c, double *before, double *after)
     DeckDev *ttab = nullptr;
     if (c->batched) hip_check(hipMalloc(&ttab, sizeof(DeckDev) * c->tiles.size()), "hipMalloc");
     for (int k = 0; k < SK_COUNT; k++) {
+        if (k == SK_PDV_PREDICT && lagrange_chunk(c)) continue;  // not launched: accel_pdv's shape is the whole phase's
         if (ttab) {
             const std::vector<DeckDev> h = tune_table(c, k);
             hip_check(hipMemcpyAsync(ttab, h.data(), sizeof(DeckDev) * h.size(), hipMemcpyHostToDevice, c->st),
@@ -1162,10 +1170,27 @@ static void autotune(clover_chunk *c, double *before, double *after)
     if (after) *after = t1;
 }
 
+// the Lagrangian phase runs as one march (lagrange_kernels.hip): one mirrored tile
+static bool lagrange_chunk(const clover_chunk *c)
+{
+    return c->fast && c->tiles.size() == 1 && lagrange_tile(c->tiles[0].g);
+}
+
 static void do_step(clover_chunk *c)
 {
-    pdv(c, true);
-    if (c->fast) {
+    const bool lagrange = lagrange_chunk(c);
+    if (!lagrange) pdv(c, true);
+    if (lagrange) {
+        // the predictor (revert is a no-op: nothing of it is stored),
+        // accelerate, the corrector and flux_calc
+        Phase ph(c, P_ACCEL);
+        Tile &t = c->tiles[0];
+        hip_check(launch_fast_lagrange(c->store, t.g, c->geo, c->dt, t.f[F_DENSITY0], t.f[F_DENSITY1], t.f[F_ENERGY0],
+                                       t.f[F_ENERGY1], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[F_XVEL1], t.f[F_YVEL0],
+                                       t.f[F_YVEL1], t.f[F_ZVEL0], t.f[F_ZVEL1], t.f[F_VOL_FLUX_X],
+                                       t.f[F_VOL_FLUX_Y], t.f[F_VOL_FLUX_Z], c->shapes.k[SK_ACCEL_PDV], c->st),
+                  "PdV predict + accelerate + PdV correct + flux_calc");
+    } else if (c->fast) {
         // accelerate, the PdV corrector and flux_calc in one march
         Phase ph(c, P_ACCEL);
         if (c->batched) {

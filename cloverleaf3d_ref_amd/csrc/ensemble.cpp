@@ -63,13 +63,16 @@ BatchGrid make_grid(clover_ensemble *e, const std::vector<int> &counts)
     return BatchGrid{p, start[e->nd]};
 }
 
+// whether an ensemble runs a batched kernel: its decks take the Lagrangian
+// phase as one march, not as the predictor and accel_pdv
+bool runs(int bk) { return bk != BK_PDV_PREDICT && bk != BK_ACCEL_PDV; }
+
 // the launch shape a batched kernel takes (none: -1)
 int shape_index(int bk)
 {
     switch (bk) {
     case BK_VISC_DT: return SK_VISC_DT;
-    case BK_PDV_PREDICT: return SK_PDV_PREDICT;
-    case BK_ACCEL_PDV: return SK_ACCEL_PDV;
+    case BK_LAGRANGE: return SK_ACCEL_PDV;
     case BK_CELL_X: return SK_CELL_X;
     case BK_CELL_Y: return SK_CELL_Y;
     case BK_CELL_Z: return SK_CELL_Z;
@@ -186,12 +189,9 @@ void enqueue_step(clover_ensemble *e)
               "visc_dt");
     hip_check(batch_deck_dt(e->dev, e->nd, vg.start, e->visc_partial, e->g_big, e->st), "deck dt");
     halo(e, FH_VISCOSITY);
-    // PdV predictor (+ ideal_gas on the predicted state), pressure halo
-    hip_check(batch_pdv_predict(e->store, e->dev, e->nd, kgrid(e, BK_PDV_PREDICT), shape(e, BK_PDV_PREDICT), e->st),
-              "PdV predict");
-    halo(e, FH_PRESSURE);
-    hip_check(batch_accel_pdv(e->store, e->dev, e->nd, kgrid(e, BK_ACCEL_PDV), shape(e, BK_ACCEL_PDV), e->st),
-              "accelerate + PdV correct");
+    // every deck is one mirrored tile: its Lagrangian phase is one march
+    hip_check(batch_lagrange(e->store, e->dev, e->nd, kgrid(e, BK_LAGRANGE), shape(e, BK_LAGRANGE), e->st),
+              "PdV predict + accelerate + PdV correct + flux_calc");
     // advection.f90:26-181
     int dir = e->advect_x ? 1 : 3;
     halo(e, FH_CELL1);
@@ -216,7 +216,8 @@ void enqueue_step(clover_ensemble *e)
 // one allocates and copies, which a capture cannot contain)
 void prepare_grids(clover_ensemble *e)
 {
-    for (int k = 0; k < BK_COUNT; k++) kgrid(e, k);
+    for (int k = 0; k < BK_COUNT; k++)
+        if (runs(k)) kgrid(e, k);
     // the step's halo updates, for both sweep orders
     for (int ax = 0; ax < 2; ax++)
         for (int which = FH_TIMESTEP; which <= FH_MOM3; which++) {
@@ -229,9 +230,7 @@ void prepare_grids(clover_ensemble *e)
 // The batched twin of the single-deck tuner (chunk.cpp): each shaped kernel
 // runs over all decks with every candidate shape and the fastest is kept.
 // The kernels take their arrays from the deck table, so outputs are sent to
-// spare arrays by exchanging table slots around the timed launches (the
-// pressure pdv_predict updates in place becomes a spare array too; its
-// contents do not matter for timing).
+// spare arrays by exchanging table slots around the timed launches.
 SlotSwap tune_slots(int bk)
 {
     SlotSwap sw{};
@@ -242,8 +241,7 @@ SlotSwap tune_slots(int bk)
     };
     switch (bk) {
     case BK_VISC_DT: pair(F_VISCOSITY, X_W1); break;
-    case BK_PDV_PREDICT: pair(F_PRESSURE, X_W1); break;
-    case BK_ACCEL_PDV:  // 8 outputs, 5 spare arrays: the volume fluxes keep their slots
+    case BK_LAGRANGE:  // 8 outputs, 5 spare arrays: the volume fluxes keep their slots
         pair(F_DENSITY1, X_W1); pair(F_ENERGY1, X_W2);
         pair(F_XVEL1, X_W5); pair(F_YVEL1, X_W6); pair(F_ZVEL1, X_W7);
         break;
@@ -261,8 +259,7 @@ void tune_launch(clover_ensemble *e, int bk, const Shape &sh)
     hipError_t r = hipSuccess;
     switch (bk) {
     case BK_VISC_DT: r = batch_visc_dt(e->store, e->dev, e->nd, g, sh, e->g_small, e->visc_partial, e->st); break;
-    case BK_PDV_PREDICT: r = batch_pdv_predict(e->store, e->dev, e->nd, g, sh, e->st); break;
-    case BK_ACCEL_PDV: r = batch_accel_pdv(e->store, e->dev, e->nd, g, sh, e->st); break;
+    case BK_LAGRANGE: r = batch_lagrange(e->store, e->dev, e->nd, g, sh, e->st); break;
     case BK_CELL_X:
     case BK_CELL_Y:
     case BK_CELL_Z: {

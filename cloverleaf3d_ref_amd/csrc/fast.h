@@ -158,6 +158,17 @@ hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, double dt,
                                  void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,
                                  void *vol_flux_z, const Shape &sh, hipStream_t st);
 
+// Tiles whose Lagrangian phase (the PdV predictor with its ideal_gas,
+// accelerate, the corrector and flux_calc) runs as one march
+// (lagrange_kernels.hip): every face external and mirrored, so nothing is
+// exchanged within it.  Writes what launch_fast_accel_pdv writes; the predicted
+// pressure is not stored.
+inline bool lagrange_tile(const Lay &g) { return g.mirror == 63; }
+hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, double dt, const void *density0, void *density1,
+                                const void *energy0, void *energy1, const void *viscosity, const void *xvel0,
+                                void *xvel1, const void *yvel0, void *yvel1, const void *zvel0, void *zvel1,
+                                void *vol_flux_x, void *vol_flux_y, void *vol_flux_z, const Shape &sh, hipStream_t st);
+
 // one advec_cell sweep, fluxes and cell update in one kernel
 // (cell_kernels.hip): mass_flux_<dir> is written over the reference's face
 // range, the new density1/energy1 of interior cells go to rho_out/e_out.

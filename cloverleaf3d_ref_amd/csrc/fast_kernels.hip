@@ -1159,6 +1159,7 @@ kb_field_summary(const DeckDev *__restrict__ decks, const int *__restrict__ star
 
 int batch_blocks_mom(int dir, const Lay &g, int planes);
 int batch_blocks_cell(int dir, const Lay &g, int planes);
+int batch_blocks_lagrange(const Lay &g, int planes, Store s);
 
 int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
 {
@@ -1168,6 +1169,7 @@ int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
     case BK_VISC_DT:
     case BK_PDV_PREDICT: dims_cells(g, planes, s == ST_F32 ? 2 : 1, gx, gy, gz); break;
     case BK_ACCEL_PDV: dims_accel_pdv(g, planes, gx, gy, gz); break;
+    case BK_LAGRANGE: return batch_blocks_lagrange(g, planes, s);
     case BK_SUMMARY: dims_summary(g, gx, gy, gz); break;
     case BK_CELL_X: return batch_blocks_cell(1, g, planes);
     case BK_CELL_Y: return batch_blocks_cell(2, g, planes);
@@ -1203,7 +1205,7 @@ int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
 constexpr int kXcdCells = 4000000;
 constexpr double kRounds = 2.0;
 
-static int size_planes(BatchKernel k, Store s, const Lay *lays, int n, int slots, int cap)
+static int size_planes(BatchKernel k, Store s, const Lay *lays, int n, int slots, int cap, int extra = 1)
 {
     int best = 1;
     double best_t = 0.0;
@@ -1212,7 +1214,7 @@ static int size_planes(BatchKernel k, Store s, const Lay *lays, int n, int slots
         for (int i = 0; i < n; i++) wgs += batch_blocks(k, lays[i], p, s);
         double r = (double)wgs / slots;
         if (r < kRounds) r = std::ceil(r);
-        const double t = (p + 1) * r;
+        const double t = (p + extra) * r;
         if (p == 1 || t <= best_t) {
             best = p;
             best_t = t;
@@ -1231,6 +1233,8 @@ Shapes size_shapes(Store s, const Lay *lays, int n)
         cells += (long long)(g.x_max - g.x_min + 1) * (g.y_max - g.y_min + 1) * (g.z_max - g.z_min + 1);
     }
     const int far = cells >= kXcdCells;
+    bool lagrange = true;
+    for (int i = 0; i < n; i++) lagrange = lagrange && lagrange_tile(lays[i]);
     struct {
         int shape;
         BatchKernel k;
@@ -1252,6 +1256,15 @@ Shapes size_shapes(Store s, const Lay *lays, int n)
     sh.k[SK_CELL_X] = Shape{rows, far, 64, 0, rows};
     for (const auto &m : marches)
         sh.k[m.shape] = Shape{size_planes(m.k, s, lays, n, m.slots, m.cap), m.xcd, 64, 0, m.cap};
+    // accel_pdv's shape is the Lagrangian march's where that runs: three extra
+    // planes per chunk (two predicted below it, one accelerated above), one
+    // workgroup per CU in FP64, two in FP32.  64^3 FP64 22.5 us at the rule's 4
+    // planes (61.8 at 32), 131 x 75 x 93 41.6 at 12 (10 by the rule; 83.9 at 32),
+    // FP32 101 x 143 x 67 27.2 at 8; 512^3 FP32 2.10 ms at 8, 2.31 at 32.
+    if (lagrange) {
+        const int cap = f32 ? 8 : 32;
+        sh.k[SK_ACCEL_PDV] = Shape{size_planes(BK_LAGRANGE, s, lays, n, f32 ? 2 * cus : cus, cap, 3), far, 64, 0, cap};
+    }
     return sh;
 }
 

@@ -243,6 +243,27 @@ __device__ inline int cell_xm(const Lay &g, int j) { return cell_m(g, 0, j); }
 __device__ inline int node_xm(const Lay &g, int j) { return node_m(g, 0, j); }
 __device__ inline bool node_xsign(const Lay &g, int j) { return node_xm(g, j) != j; }
 
+// The value lane+1 (lane-1) of the wavefront holds, 0 in lane 63 (0): a shift
+// in the VALU (DPP wave_shl:1, wave_shr:1) instead of __shfl's trip through
+// LDS.  Every lane of the wavefront must be active.
+template <int CTRL, typename T>
+__device__ inline T lane_shift(T x)
+{
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+    } else {
+        const int2 v = __builtin_bit_cast(int2, x);
+        int2 r;
+        r.x = __builtin_amdgcn_update_dpp(0, v.x, CTRL, 0xf, 0xf, true);
+        r.y = __builtin_amdgcn_update_dpp(0, v.y, CTRL, 0xf, 0xf, true);
+        return __builtin_bit_cast(T, r);
+    }
+}
+template <typename T>
+__device__ inline T next_lane(T x) { return lane_shift<0x130>(x); }
+template <typename T>
+__device__ inline T prev_lane(T x) { return lane_shift<0x138>(x); }
+
 constexpr int RED_THREADS = 256;
 
 __device__ inline double wave_min(double v)
