@@ -7,8 +7,10 @@
 // workgroup finds its deck by binary search and runs the single-deck kernel
 // body on that deck's block.  Array pointers, dt and time are read from the
 // device-side deck table, so a whole step needs no host involvement and can
-// be captured in a graph; the level and sweep exchanges of the fast path are
-// done on the device by exchanging the table's pointers.
+// be captured in a graph.  The sweeps of a step exchange array roles: within
+// the step the host keeps the map (Slots) and each launch takes the slots it
+// reads and writes, and one kernel at the step's end (batch_move) brings the
+// table's pointers in line, for the level exchange too.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -30,6 +32,16 @@ struct DeckDev {
     double dtc_safe, dtu_safe, dtv_safe, dtw_safe, dtdiv_safe;
     int steps;  // timesteps taken (dt formed)
     int small;  // 0, or the step at which dt first fell below dtmin (timestep.f90:120-122)
+};
+
+// The table slot that holds each array at this point of the step (host side)
+struct Slots {
+    int s[NUM_ARRAYS];
+    Slots()
+    {
+        for (int a = 0; a < NUM_ARRAYS; a++) s[a] = a;
+    }
+    int operator[](int a) const { return s[a]; }
 };
 
 // A batched launch: total workgroups and the device prefix table (nd+1).
@@ -110,14 +122,14 @@ hipError_t batch_field_summary(Store s, const DeckDev *decks, int nd, const Batc
 // advec_cell sweep `dir`; new density1/energy1 into the arrays X_W1/X_W2,
 // and with gas (third sweep only) ideal_gas's pressure of them into pressure
 hipError_t batch_advec_cell(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
-                            int sweep_number, bool gas, const Shape &sh, hipStream_t st);
+                            int sweep_number, bool gas, const Slots &sl, const Shape &sh, hipStream_t st);
 // advec_mom sweep `dir`; new velocities into X_W5..X_W7
 hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
-                           int sweep_number, const Shape &sh, hipStream_t st);
+                           int sweep_number, const Slots &sl, const Shape &sh, hipStream_t st);
 // reflective halo of the flagged fields, every face; axes (null: all) as for
 // launch_update_halo_store
 hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int depth, const int *fields,
-                         hipStream_t st, const int *axes = nullptr);
+                         const Slots &sl, hipStream_t st, const int *axes = nullptr);
 
 // The tiles of one chunk as a batch (chunk.cpp, more than one tile): one
 // launch per pass of update_halo over every tile.  An item is one (tile,
@@ -164,13 +176,8 @@ hipError_t batch_deck_dt(DeckDev *decks, int nd, const int *visc_start, const do
                          hipStream_t st);
 // the five sums of each deck's summary partials, as the single-deck final pass
 hipError_t batch_deck_sum5(int nd, const int *sum_start, const double *partial, double *out, hipStream_t st);
-// exchange up to 5 pairs of array slots in every deck's table; add dt to
-// time when add_time
-struct SlotSwap {
-    int n;
-    int a[5], b[5];
-    int add_time;
-};
-hipError_t batch_swap(DeckDev *decks, int nd, const SlotSwap &sw, hipStream_t st);
+// gives every array its own slot again in every deck's table (slot a takes the
+// pointer slot sl[a] holds); adds dt to time when add_time
+hipError_t batch_move(DeckDev *decks, int nd, const Slots &sl, bool add_time, hipStream_t st);
 
 }  // namespace clover

@@ -372,7 +372,12 @@ hipError_t launch_fast_advec_cell(Store s, const Lay &g, const Geo &m, int advec
 }
 
 // ---------------------------------------------------------------------------
-// Batched over many decks (batch.h): new density1/energy1 go to X_W1/X_W2.
+// Batched over many decks (batch.h): new density1/energy1 go to X_W1/X_W2,
+// wherever those and density1/energy1 are at this point of the step.
+struct CellSlots {
+    int rho, e, rho_out, e_out;
+};
+
 __host__ __device__ inline void dims_cell(int dir, const Lay &g, int planes, int &gx, int &gy, int &gz)
 {
     const int nx = g.x_max - g.x_min + 1, ny = g.y_max - g.y_min + 1, nz = g.z_max - g.z_min + 1;
@@ -396,7 +401,7 @@ int batch_blocks_cell(int dir, const Lay &g, int planes)
 template <int DIR, typename S>
 __global__ void __launch_bounds__(64 * CROWS)
 kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int gas, int planes,
-        int xcd)
+        int xcd, CellSlots cs)
 {
     int hb, end, step;  // the tiles of this workgroup (persistent when the grid is short)
     tile_walk(start[nd], xcd, hb, end, step);
@@ -410,12 +415,12 @@ kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd
 #define CF(id) static_cast<const S *>(D.f[id])
 #define MF(id) static_cast<S *>(D.f[id])
         if constexpr (DIR == 1)
-            cell_x_body<S>(bk, D.g, D.m, mode, cell_x_rows(planes), CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z), CF(F_DENSITY1),
-                           CF(F_ENERGY1), MF(F_MASS_FLUX_X), MF(X_W1), MF(X_W2), gas ? MF(F_PRESSURE) : nullptr);
+            cell_x_body<S>(bk, D.g, D.m, mode, cell_x_rows(planes), CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z), CF(cs.rho),
+                           CF(cs.e), MF(F_MASS_FLUX_X), MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
         else
             cell_march_body<DIR, S>(bk, D.g, D.m, mode, CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z),
-                                    CF(F_DENSITY1), CF(F_ENERGY1), MF(DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z),
-                                    MF(X_W1), MF(X_W2), gas ? MF(F_PRESSURE) : nullptr);
+                                    CF(cs.rho), CF(cs.e), MF(DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z),
+                                    MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
 #undef CF
 #undef MF
         __syncthreads();  // the next tile reuses the workgroup's LDS
@@ -423,7 +428,7 @@ kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd
 }
 
 hipError_t batch_advec_cell(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
-                            int sweep_number, bool gas, const Shape &sh, hipStream_t st)
+                            int sweep_number, bool gas, const Slots &sl, const Shape &sh, hipStream_t st)
 {
     int mode = 0;
     if (dir == 1) mode = sweep_number == 1 ? 1 : sweep_number == 3 ? 2 : 0;
@@ -432,10 +437,11 @@ hipError_t batch_advec_cell(Store s, const DeckDev *decks, int nd, const BatchGr
     if (!mode) return hipErrorInvalidValue;
     if (bg.total == 0) return hipSuccess;
     const dim3 grid(batch_wgs(bg, sh)), blk(64, CROWS);
+    const CellSlots cs{sl[F_DENSITY1], sl[F_ENERGY1], sl[X_W1], sl[X_W2]};
     if (gas && sweep_number != 3) return hipErrorInvalidValue;
 #define L(D_, T_)                                                                                          \
     TIMED_LAUNCH("kb_cell", st, (kb_cell<D_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, gas ? 1 : 0,   \
-                 sh.planes, sh.xcd)
+                 sh.planes, sh.xcd, cs)
     if (s == ST_F32) {
         if (dir == 1) L(1, float); else if (dir == 2) L(2, float); else L(3, float);
     } else {

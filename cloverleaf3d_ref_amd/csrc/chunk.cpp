@@ -136,10 +136,11 @@ struct clover_chunk {
     // More than one tile with the fused kernels: each stage is one launch over
     // every tile (batch.h, the ensemble's batched kernels with the tiles as
     // decks) and each update_halo one launch per pass.  The tiles' arrays
-    // are read from a device table that every array exchange keeps in step
-    // with `tiles`.
+    // are read from a device table, which a step brings in line with `tiles`
+    // at its end (settle).
     bool batched;
     DeckDev *tdev;
+    Slots slots;  // where the table holds each array (its own slot between steps)
     std::map<std::pair<int, int>, BatchGrid> grids;  // (batched kernel, planes) -> prefix table
     std::vector<int *> tables;
     struct HaloTabs {
@@ -427,17 +428,19 @@ static const BatchGrid &kgrid(clover_chunk *c, int bk)
     return tgrid(c, bk, si < 0 ? 0 : c->shapes.k[si].planes);
 }
 
-// exchange array roles in every tile, on the host and in the device table
+// exchange array roles in every tile; settle brings the device table in line
 static void tswap(clover_chunk *c, std::initializer_list<std::pair<int, int>> pairs)
 {
-    SlotSwap sw{};
     for (auto &pr : pairs) {
         for (auto &t : c->tiles) std::swap(t.f[pr.first], t.f[pr.second]);
-        sw.a[sw.n] = pr.first;
-        sw.b[sw.n] = pr.second;
-        sw.n++;
+        std::swap(c->slots.s[pr.first], c->slots.s[pr.second]);
     }
-    if (c->batched) hip_check(batch_swap(c->tdev, (int)c->tiles.size(), sw, c->st), "swap");
+}
+
+static void settle(clover_chunk *c)
+{
+    hip_check(batch_move(c->tdev, (int)c->tiles.size(), c->slots, false, c->st), "slots");
+    c->slots = Slots();
 }
 
 // update_halo over the tiles in one launch per pass: the three tile passes,
@@ -449,6 +452,8 @@ static void batched_update_halo(clover_chunk *c, const int *fields, int depth, c
     key += std::string(1, (char)depth) + std::string(1, (char)poison);
     if (axes) key += std::string(reinterpret_cast<const char *>(axes), sizeof(int) * NUM_FIELDS);
     if (raxes) key += std::string(reinterpret_cast<const char *>(raxes), sizeof(int) * NUM_FIELDS);
+    // the items name table slots
+    key += std::string(reinterpret_cast<const char *>(c->slots.s), sizeof(int) * NUM_FIELDS);
     auto it = c->halo_tabs.find(key);
     if (it == c->halo_tabs.end()) {
         const int T = (int)c->tiles.size();
@@ -460,6 +465,11 @@ static void batched_update_halo(clover_chunk *c, const int *fields, int depth, c
         }
         std::vector<TileHaloItem> copy[3], refl[3][2];
         tile_halo_items(nbr.data(), T, lays.data(), fields, depth, axes, raxes ? raxes : axes, poison, copy, refl);
+        for (auto &l : copy)
+            for (auto &x : l) x.field = c->slots[x.field];
+        for (auto &l : refl)
+            for (auto &side : l)
+                for (auto &x : side) x.field = c->slots[x.field];
         clover_chunk::HaloTabs tab{};
         std::vector<TileHaloItem> all;
         static const int axis_order[3] = {1, 0, 2};
@@ -791,7 +801,7 @@ static void advec_cell(clover_chunk *c, int sweep, int dir)
     if (c->batched) {
         const int k = dir == 1 ? BK_CELL_X : dir == 2 ? BK_CELL_Y : BK_CELL_Z;
         hip_check(batch_advec_cell(c->store, c->tdev, (int)c->tiles.size(), kgrid(c, k), c->advect_x, dir, sweep,
-                                   sweep == 3, c->shapes.k[shape_of(k)], c->st),
+                                   sweep == 3, c->slots, c->shapes.k[shape_of(k)], c->st),
                   "advec_cell");
         if (sweep == 3) {
             c->gas_fresh = true;
@@ -835,7 +845,7 @@ static void advec_mom(clover_chunk *c, int sweep, int dir)
     if (c->batched) {
         const int k = dir == 1 ? BK_MOM_X : dir == 2 ? BK_MOM_Y : BK_MOM_Z;
         hip_check(batch_advec_mom(c->store, c->tdev, (int)c->tiles.size(), kgrid(c, k), c->advect_x, dir, sweep,
-                                  c->shapes.k[shape_of(k)], c->st),
+                                  c->slots, c->shapes.k[shape_of(k)], c->st),
                   "advec_mom");
         tswap(c, {{F_XVEL1, X_W5}, {F_YVEL1, X_W6}, {F_ZVEL1, X_W7}});
         return;
@@ -1052,12 +1062,12 @@ static void tune_launch_batched(clover_chunk *c, int k, DeckDev *ttab)
     case SK_CELL_Y:
     case SK_CELL_Z: {
         const int dir = k - SK_CELL_X + 1;
-        e = batch_advec_cell(c->store, ttab, T, g, 1, dir, dir == 2 ? 2 : 1, false, sh, c->st);
+        e = batch_advec_cell(c->store, ttab, T, g, 1, dir, dir == 2 ? 2 : 1, false, Slots(), sh, c->st);
         break;
     }
     default: {
         const int dir = k - SK_MOM_X + 1;
-        e = batch_advec_mom(c->store, ttab, T, g, 1, dir, dir == 2 ? 2 : 1, sh, c->st);
+        e = batch_advec_mom(c->store, ttab, T, g, 1, dir, dir == 2 ? 2 : 1, Slots(), sh, c->st);
         break;
     }
     }
@@ -1232,6 +1242,7 @@ static void do_step(clover_chunk *c)
         // in the device table, as the per-tile fused path below does
         tswap(c, {{F_DENSITY0, F_DENSITY1}, {F_ENERGY0, F_ENERGY1}, {F_XVEL0, F_XVEL1}, {F_YVEL0, F_YVEL1},
                   {F_ZVEL0, F_ZVEL1}});
+        settle(c);
     } else {
         Phase ph(c, P_RESET);
         for (auto &t : c->tiles) {

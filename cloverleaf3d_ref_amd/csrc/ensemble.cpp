@@ -44,6 +44,7 @@ struct clover_ensemble {
     double g_small = 0.0, g_big = 0.0;
     int step = 0;
     int advect_x = 1;
+    Slots slots;  // where the table holds each array (its own slot between steps)
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // index: advect_x
     Shapes shapes{};                               // launch shapes (size_shapes, autotuner)
 };
@@ -132,7 +133,8 @@ void set_fields(int *fields, std::initializer_list<int> ids)
 // (axes null), or reduced to the halos the fused kernels read
 void halo(clover_ensemble *e, const int *fields, int depth, const int *axes = nullptr)
 {
-    hip_check(batch_reflect(e->store, e->dev, e->nd, halo_grid(e, fields, axes, depth), depth, fields, e->st, axes),
+    hip_check(batch_reflect(e->store, e->dev, e->nd, halo_grid(e, fields, axes, depth), depth, fields, e->slots,
+                            e->st, axes),
               "halo");
 }
 
@@ -147,16 +149,16 @@ void ideal_gas(clover_ensemble *e)
     hip_check(batch_ideal_gas(e->store, e->dev, e->nd, kgrid(e, BK_IDEAL_GAS), e->st), "ideal_gas");
 }
 
-void swap(clover_ensemble *e, std::initializer_list<std::pair<int, int>> pairs, bool add_time)
+// arrays exchange roles; settle brings the device table in line
+void swap(clover_ensemble *e, std::initializer_list<std::pair<int, int>> pairs)
 {
-    SlotSwap sw{};
-    for (auto &p : pairs) {
-        sw.a[sw.n] = p.first;
-        sw.b[sw.n] = p.second;
-        sw.n++;
-    }
-    sw.add_time = add_time ? 1 : 0;
-    hip_check(batch_swap(e->dev, e->nd, sw, e->st), "swap");
+    for (auto &p : pairs) std::swap(e->slots.s[p.first], e->slots.s[p.second]);
+}
+
+void settle(clover_ensemble *e, bool add_time)
+{
+    hip_check(batch_move(e->dev, e->nd, e->slots, add_time, e->st), "slots");
+    e->slots = Slots();
 }
 
 void advec_cell(clover_ensemble *e, int sweep, int dir)
@@ -165,17 +167,18 @@ void advec_cell(clover_ensemble *e, int sweep, int dir)
     // the third sweep also writes ideal_gas of the new state: the next step's
     // (or a summary's) equation of state
     hip_check(batch_advec_cell(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, sweep == 3,
-                               shape(e, k), e->st),
+                               e->slots, shape(e, k), e->st),
               "advec_cell");
-    swap(e, {{F_DENSITY1, X_W1}, {F_ENERGY1, X_W2}}, false);
+    swap(e, {{F_DENSITY1, X_W1}, {F_ENERGY1, X_W2}});
 }
 
 void advec_mom(clover_ensemble *e, int sweep, int dir)
 {
     const BatchKernel k = dir == 1 ? BK_MOM_X : dir == 2 ? BK_MOM_Y : BK_MOM_Z;
-    hip_check(batch_advec_mom(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, shape(e, k), e->st),
+    hip_check(batch_advec_mom(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, e->slots, shape(e, k),
+                              e->st),
               "advec_mom");
-    swap(e, {{F_XVEL1, X_W5}, {F_YVEL1, X_W6}, {F_ZVEL1, X_W7}}, false);
+    swap(e, {{F_XVEL1, X_W5}, {F_YVEL1, X_W6}, {F_ZVEL1, X_W7}});
 }
 
 // hydro.f90:48-68 for every deck, device only
@@ -208,8 +211,8 @@ void enqueue_step(clover_ensemble *e)
     advec_mom(e, 3, dir);
     // reset_field as an exchange of levels, then time = time + dt
     swap(e, {{F_DENSITY0, F_DENSITY1}, {F_ENERGY0, F_ENERGY1}, {F_XVEL0, F_XVEL1}, {F_YVEL0, F_YVEL1},
-             {F_ZVEL0, F_ZVEL1}},
-         true);
+             {F_ZVEL0, F_ZVEL1}});
+    settle(e, true);
 }
 
 // every prefix table a step uses, built before any graph capture (building
@@ -231,14 +234,11 @@ void prepare_grids(clover_ensemble *e)
 // runs over all decks with every candidate shape and the fastest is kept.
 // The kernels take their arrays from the deck table, so outputs are sent to
 // spare arrays by exchanging table slots around the timed launches.
-SlotSwap tune_slots(int bk)
+// (pairs only: moving by the map twice restores the table)
+Slots tune_slots(int bk)
 {
-    SlotSwap sw{};
-    auto pair = [&](int a, int b) {
-        sw.a[sw.n] = a;
-        sw.b[sw.n] = b;
-        sw.n++;
-    };
+    Slots sw;
+    auto pair = [&](int a, int b) { std::swap(sw.s[a], sw.s[b]); };
     switch (bk) {
     case BK_VISC_DT: pair(F_VISCOSITY, X_W1); break;
     case BK_LAGRANGE:  // 8 outputs, 5 spare arrays: the volume fluxes keep their slots
@@ -264,12 +264,12 @@ void tune_launch(clover_ensemble *e, int bk, const Shape &sh)
     case BK_CELL_Y:
     case BK_CELL_Z: {
         const int dir = bk - BK_CELL_X + 1;
-        r = batch_advec_cell(e->store, e->dev, e->nd, g, 1, dir, dir == 2 ? 2 : 1, false, sh, e->st);
+        r = batch_advec_cell(e->store, e->dev, e->nd, g, 1, dir, dir == 2 ? 2 : 1, false, Slots(), sh, e->st);
         break;
     }
     default: {
         const int dir = bk - BK_MOM_X + 1;
-        r = batch_advec_mom(e->store, e->dev, e->nd, g, 1, dir, dir == 2 ? 2 : 1, sh, e->st);
+        r = batch_advec_mom(e->store, e->dev, e->nd, g, 1, dir, dir == 2 ? 2 : 1, Slots(), sh, e->st);
         break;
     }
     }
@@ -280,13 +280,13 @@ double tune_time(clover_ensemble *e, int bk, const Shape &sh, hipEvent_t a, hipE
 {
     const int reps = 3;
     grid(e, bk, sh.planes);  // any table allocation happens before the timing
-    const SlotSwap sw = tune_slots(bk);
-    if (sw.n) hip_check(batch_swap(e->dev, e->nd, sw, e->st), "swap");
+    const Slots sw = tune_slots(bk);
+    hip_check(batch_move(e->dev, e->nd, sw, false, e->st), "slots");
     tune_launch(e, bk, sh);
     hip_check(hipEventRecord(a, e->st), "event");
     for (int r = 0; r < reps; r++) tune_launch(e, bk, sh);
     hip_check(hipEventRecord(b, e->st), "event");
-    if (sw.n) hip_check(batch_swap(e->dev, e->nd, sw, e->st), "swap back");
+    hip_check(batch_move(e->dev, e->nd, sw, false, e->st), "slots back");
     hip_check(hipEventSynchronize(b), "event sync");
     float ms = 0;
     hip_check(hipEventElapsedTime(&ms, a, b), "event time");

@@ -122,22 +122,22 @@ hipError_t batch_set_dt(DeckDev *decks, int nd, double dt, hipStream_t st)
     return hipGetLastError();
 }
 
-__global__ void kb_swap(DeckDev *__restrict__ decks, int nd, SlotSwap sw)
+// one wave per deck, one lane per array
+static_assert(NUM_ARRAYS <= 64, "kb_move: one lane per array");
+__global__ void __launch_bounds__(64) kb_move(DeckDev *__restrict__ decks, Slots sl, int add_time)
 {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= nd) return;
-    DeckDev &D = decks[d];
-    for (int q = 0; q < sw.n; q++) {
-        void *t = D.f[sw.a[q]];
-        D.f[sw.a[q]] = D.f[sw.b[q]];
-        D.f[sw.b[q]] = t;
-    }
-    if (sw.add_time) D.time = D.time + D.dt;
+    DeckDev &D = decks[blockIdx.x];
+    const int a = (int)threadIdx.x;
+    void *p = nullptr;
+    if (a < NUM_ARRAYS) p = D.f[sl.s[a]];
+    __syncthreads();  // every pointer is read before any is written
+    if (a < NUM_ARRAYS) D.f[a] = p;
+    if (a == 0 && add_time) D.time = D.time + D.dt;
 }
 
-hipError_t batch_swap(DeckDev *decks, int nd, const SlotSwap &sw, hipStream_t st)
+hipError_t batch_move(DeckDev *decks, int nd, const Slots &sl, bool add_time, hipStream_t st)
 {
-    TIMED_LAUNCH("kb_swap", st, kb_swap, dim3((nd + 63) / 64), dim3(64), 0, st, decks, nd, sw);
+    TIMED_LAUNCH("kb_move", st, kb_move, dim3(nd), dim3(64), 0, st, decks, sl, add_time ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -506,10 +506,11 @@ kb_reflect(const DeckDev *__restrict__ decks, const int *__restrict__ start, int
 }
 
 hipError_t batch_reflect(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int depth, const int *fields,
-                         hipStream_t st, const int *axes)
+                         const Slots &sl, hipStream_t st, const int *axes)
 {
     if (depth < 1 || depth > 2) return hipErrorInvalidValue;  // two layers per thread
-    const OnceSet o = once_set(fields, axes, kAllFaces, nullptr);
+    OnceSet o = once_set(fields, axes, kAllFaces, nullptr);
+    for (int q = 0; q < o.slots; q++) o.f[q].field = (short)sl[o.f[q].field];
     if (!o.slots || bg.total == 0) return hipSuccess;
     if (t_kernel_timer) t_kernel_timer->begin("kb_reflect", st);
     if (s == ST_F32) hipLaunchKernelGGL(kb_reflect<float>, dim3(bg.total), dim3(kOnceThreads), 0, st, decks, bg.start, nd, depth, o);

@@ -664,7 +664,12 @@ hipError_t launch_fast_advec_mom(Store s, const Lay &g, const Geo &m, int advect
 }
 
 // ---------------------------------------------------------------------------
-// Batched over many decks (batch.h): the new velocities go to X_W5..X_W7.
+// Batched over many decks (batch.h): the new velocities go to X_W5..X_W7,
+// wherever those and the step's arrays are at this point of it.
+struct MomSlots {
+    int rho, in[3], out[3];
+};
+
 __host__ __device__ inline void dims_mom(int dir, const Lay &g, int planes, int &gx, int &gy, int &gz)
 {
     const int nxn = g.x_max - g.x_min + 2, nyn = g.y_max - g.y_min + 2, nzn = g.z_max - g.z_min + 2;  // nodes
@@ -687,7 +692,7 @@ int batch_blocks_mom(int dir, const Lay &g, int planes)
 
 template <int DIR, typename S>
 __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
-                                         int mode, int planes, int hb)
+                                         int mode, int planes, const MomSlots &ms, int hb)
 {
     const int d = deck_of(start, nd, hb);
     const DeckDev &D = decks[d];
@@ -696,16 +701,15 @@ __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, cons
     const int lb = hb - start[d];
     const Blk bk{lb % gx, (lb / gx) % gy, lb / (gx * gy), gx, gy, gz};
     Vel3<S> v;
-    v.in[0] = static_cast<const S *>(D.f[F_XVEL1]);
-    v.in[1] = static_cast<const S *>(D.f[F_YVEL1]);
-    v.in[2] = static_cast<const S *>(D.f[F_ZVEL1]);
-    v.out[0] = static_cast<S *>(D.f[X_W5]);
-    v.out[1] = static_cast<S *>(D.f[X_W6]);
-    v.out[2] = static_cast<S *>(D.f[X_W7]);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        v.in[c] = static_cast<const S *>(D.f[ms.in[c]]);
+        v.out[c] = static_cast<S *>(D.f[ms.out[c]]);
+    }
     const S *vfx = static_cast<const S *>(D.f[F_VOL_FLUX_X]);
     const S *vfy = static_cast<const S *>(D.f[F_VOL_FLUX_Y]);
     const S *vfz = static_cast<const S *>(D.f[F_VOL_FLUX_Z]);
-    const S *rho = static_cast<const S *>(D.f[F_DENSITY1]);
+    const S *rho = static_cast<const S *>(D.f[ms.rho]);
     if constexpr (DIR == 1)
         mom_x_body<S>(bk, D.g, D.m, mode, static_cast<const S *>(D.f[F_MASS_FLUX_X]), vfx, vfy, vfz, rho, v);
     else
@@ -720,18 +724,19 @@ template <int DIR, typename S>
 // 8 tiles 4.81 -> 4.35 ms with one value spilled.  With the tail form five
 // values spill (20 bytes per lane) and the launches still run 4.41 -> 4.16 ms.
 __global__ void __launch_bounds__(64 * mw_of(DIR), DIR != 1 && sizeof(S) == 8 ? 5 : 1)
-kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int planes, int xcd)
+kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int planes, int xcd,
+       MomSlots ms)
 {
     int hb, end, step;  // the tiles of this workgroup (persistent when the grid is short)
     tile_walk(start[nd], xcd, hb, end, step);
     for (; hb < end; hb += step) {
-        mom_tile<DIR, S>(decks, start, nd, mode, planes, hb);
+        mom_tile<DIR, S>(decks, start, nd, mode, planes, ms, hb);
         __syncthreads();  // the next tile reuses the workgroup's LDS
     }
 }
 
 hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
-                           int sweep_number, const Shape &sh, hipStream_t st)
+                           int sweep_number, const Slots &sl, const Shape &sh, hipStream_t st)
 {
     int mode = 0;
     if (sweep_number == 1 && dir == 1) mode = 1;
@@ -743,8 +748,9 @@ hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGri
     if (!mode || dir < 1 || dir > 3) return hipErrorInvalidValue;
     if (bg.total == 0) return hipSuccess;
     const dim3 grid(batch_wgs(bg, sh)), blk(64, mw_of(dir));
+    const MomSlots ms{sl[F_DENSITY1], {sl[F_XVEL1], sl[F_YVEL1], sl[F_ZVEL1]}, {sl[X_W5], sl[X_W6], sl[X_W7]}};
 #define L(D_, T_)                                                                                          \
-    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, sh.planes, sh.xcd)
+    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, sh.planes, sh.xcd, ms)
     if (s == ST_F32) {
         if (dir == 1) L(1, float); else if (dir == 2) L(2, float); else L(3, float);
     } else {
