@@ -44,11 +44,9 @@ __device__ inline Blk hw_blk()
 }
 
 // The hardware deals workgroups round-robin to the 8 XCDs, each with its own
-// L2.  hw_blk_xcd() hands XCD x the x-th contiguous eighth of the grid (x
-// fastest) instead, so tiles that share cache lines with their neighbours
-// along x and y run on the same XCD at about the same time.  It pays in the
-// y and z momentum sweeps and costs in the other kernels, which keep the
-// plain order.
+// L2.  hw_blk_xcd() hands each XCD contiguous blocks (x fastest) instead, so
+// that tiles that share cache lines with their neighbours along x and y run on
+// the same XCD at about the same time.
 constexpr int kXcds = 8;
 
 // the logical block that hardware block hw of n runs in the XCD-contiguous
@@ -60,11 +58,27 @@ __host__ __device__ inline int xcd_block(int hw, int n)
     return xcd < r ? xcd * (q + 1) + t : r * (q + 1) + (xcd - r) * q + t;
 }
 
+// The same layer by layer, for the marches: of each layer of n blocks (one chunk
+// of the march) XCD x takes the x-th contiguous eighth, so that all XCDs march
+// the same planes at the same time, each on a band of rows.  Blocks count from
+// hardware block `off`.
+__host__ __device__ inline int xcd_layer_block(int hw, int n, int off = 0)
+{
+    const int first = off + (hw - off) / n * n;  // the layer's first hardware block
+    const int xcd = hw % kXcds;
+    int at = 0;  // blocks of the layer that XCDs below xcd take
+    for (int x = 0; x < xcd; x++) {
+        const int o = (x + kXcds - first % kXcds) % kXcds;  // where XCD x's first block lies in the layer
+        at += o < n ? (n - 1 - o) / kXcds + 1 : 0;
+    }
+    return first - off + at + (hw - first) / kXcds;
+}
+
 __device__ inline Blk hw_blk_xcd()
 {
     const int gx = (int)gridDim.x, gy = (int)gridDim.y, gz = (int)gridDim.z;
     const int hw = (int)blockIdx.x + gx * ((int)blockIdx.y + gy * (int)blockIdx.z);
-    const int id = xcd_block(hw, gx * gy * gz);
+    const int id = xcd_layer_block(hw, gx * gy);
     return Blk{id % gx, (id / gx) % gy, id / (gx * gy), gx, gy, gz};
 }
 
