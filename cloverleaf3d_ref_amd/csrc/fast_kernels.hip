@@ -1198,10 +1198,11 @@ int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
 // 226 -> 40, mom_x 94 -> 25; 256^3 mom_z 478 -> 350, accel_pdv 691 -> 605.  Over
 // 13 meshes from 16^3 to 512^3 and both forms the rule stays within 1-4 % (mean
 // per kernel) of the best of 13 plane counts.
-// The XCD order pays in accel_pdv and cell_x, and in FP32 mom_x, on meshes
-// that do not fit the L2s (512^3: FP64 accel_pdv 4.33 -> 4.17 ms, cell_x 1.75
-// -> 1.59, FP32 accel_pdv 2.58 -> 2.33); below kXcdCells it costs a
-// microsecond or two per launch.
+// The XCD order pays in the Lagrangian marches, cell_x and mom_x on meshes
+// that do not fit the L2s (512^3: FP64 lagrange 4.15 -> 3.87 ms, cell_x 1.75 ->
+// 1.53, mom_x 2.10 -> 2.04, FP32 lagrange 2.41 -> 2.00, mom_x 1.27 -> 1.06); below
+// kXcdCells it costs a microsecond or two per launch.  In the y and z sweeps it
+// is within 2 % either way.
 constexpr int kXcdCells = 4000000;
 constexpr double kRounds = 2.0;
 
@@ -1245,9 +1246,9 @@ Shapes size_shapes(Store s, const Lay *lays, int n)
         {SK_ACCEL_PDV, BK_ACCEL_PDV, f32 ? 8 : 32, f32 ? 2 * cus : cus, far},
         {SK_CELL_Y, BK_CELL_Y, 16, 5 * cus, 0},
         {SK_CELL_Z, BK_CELL_Z, 16, 5 * cus, 0},
-        {SK_MOM_X, BK_MOM_X, 8, 5 * cus, f32 ? far : 0},
-        {SK_MOM_Y, BK_MOM_Y, 32, 5 * cus, 0},
-        {SK_MOM_Z, BK_MOM_Z, 32, 5 * cus, 0},
+        {SK_MOM_X, BK_MOM_X, 8, 5 * cus, far},
+        {SK_MOM_Y, BK_MOM_Y, 32, 4 * cus, 0},
+        {SK_MOM_Z, BK_MOM_Z, 32, 4 * cus, 0},
     };
     Shapes sh;
     // the x cell sweep has no march: a row per wave, two in FP32 (launch.h

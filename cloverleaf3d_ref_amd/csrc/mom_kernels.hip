@@ -30,6 +30,8 @@
 // 16 mass-flux reads per pair of node fluxes of a plain per-node kernel.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "batch.h"
 #include "fast.h"
 #include "launch.h"
@@ -211,8 +213,8 @@ __device__ inline float shfl_d(float x, int src) { return __shfl(x, src, 64); }
 
 // ---------------------------------------------------------------------------
 // y and z sweeps: lanes along x on 64 line-aligned columns, all of which
-// store; lane 0 also loads and publishes column j-1 (publish65), which the
-// first column's node needs.  (A 63-column layout with lane 0 as the j-1
+// store; lane 0 also loads and publishes column j-1, which the first column's
+// node needs.  (A 63-column layout with lane 0 as the j-1
 // halo read rows that straddle cache lines: measured at 512^3 the aligned
 // one runs FP32 mom_y 1.35 -> 1.28 ms and mom_z 1.33 -> 1.20 ms, FP64 the
 // same.)  Waves lie along the other axis; the workgroup marches along the
@@ -239,44 +241,15 @@ __device__ inline T march_node_mass(const Quad<T> &pm, const Quad<T> &p0)  // ce
     return (T)0.125 * (p0.w + p0.c + p0.xw + p0.x + pm.w + pm.c + pm.xw + pm.x);
 }
 
-// The march's x exchange with 64 owned lanes: slot s of a row holds column
-// j0-1+s, lane L publishes its own column at slot L+1 and lane 0 also the
-// column j0-1 at slot 0.
-template <typename T, int W>
-__device__ inline void publish65(T (*buf)[W][65], int lane, int w, T a, T p, T am, T pm)
-{
-    buf[0][w][lane + 1] = a;
-    buf[1][w][lane + 1] = p;
-    if (lane == 0) {
-        buf[0][w][0] = am;
-        buf[1][w][0] = pm;
-    }
-    __syncthreads();
-}
-
-template <typename T, int W>
-__device__ inline void gather65(T (*buf)[W][65], int lane, int w, T a, T p, Quad<T> &A, Quad<T> &P)
-{
-    const int wd = w > 0 ? w - 1 : 0;
-    A.c = a;
-    A.x = buf[0][w][lane];
-    A.w = buf[0][wd][lane + 1];
-    A.xw = buf[0][wd][lane];
-    P.c = p;
-    P.x = buf[1][w][lane];
-    P.w = buf[1][wd][lane + 1];
-    P.xw = buf[1][wd][lane];
-}
-
 // The last x tile of a sweep holds the node columns left over by the
 // 64-column tiles: one (x_max+1) on a mesh a multiple of 64 cells wide.  In
 // the lane-along-x layout its workgroups march every plane with one live
 // lane, and at 512^3 they held 1/9 of the launch's workgroup slots (the y and
 // z sweeps ran 8 % faster on 511^3, whose nodes fill 8 tiles).  In the FP64
-// form a tail of at most kTailCols columns is marched instead with lanes
-// along the wave axis: one wave per column and 63 rows (lane 0 is the halo
-// row), each lane loading both x neighbours itself and taking the row below
-// from lane-1, in the grid's first workgroups (mom_march).  Every value is
+// form a tail of one column (a mesh a multiple of 64 cells wide) is marched
+// instead with lanes along the wave axis: one wave per column and 63 rows (lane
+// 0 is the halo row), each lane loading both x neighbours itself and taking the
+// row below from lane-1, in the grid's first workgroups (mom_march).  Every value is
 // formed by the same expressions from the same operands as in the 64-column
 // layout.  Measured at 512^3 FP64: mom_y 2.38 -> 2.32 ms, mom_z 2.26 -> 2.22
 // ms; 640^3 as 8 tiles (320^3 tiles, one tail column in six tiles): the
@@ -284,7 +257,7 @@ __device__ inline void gather65(T (*buf)[W][65], int lane, int w, T a, T p, Quad
 // 64-column layout: there the tail's loads (a line per lane, 4 bytes used)
 // cost more than the slots save (mom_y 1.29 -> 1.35 ms, mom_z 1.20 -> 1.25
 // ms, batched 2.29 -> 2.64 ms).
-constexpr int kTailCols = 4;
+constexpr int kTailCols = 1;  // 4 columns at 131x75x93 ran mom_y 28.0 -> 33.7 us, mom_z 29.2 -> 36.0
 static_assert(kTailCols <= mw_of(2) && kTailCols <= mw_of(3), "the tail's waves fit in the tile's workgroups");
 
 __host__ __device__ inline int mom_tail_cols(const Lay &g, int gx)
@@ -317,14 +290,12 @@ __device__ inline TailSplit mom_tail_split(const Lay &g, const Blk &bk, int tw)
     return t;
 }
 
-// TAN: vol_flux_y/z and the sweep's mass flux (y or z) read at the
-// mirrored column on mirrored x faces (tan_xm); the single-tile FP32 chunk
-// only, whose exchanges leave those x halos out (fused_halo_plan)
-template <int DIR, typename S, bool TAIL, bool TAN = false>
-__device__ __forceinline__ void mom_march_body(const Blk &bk, S (*xbuf)[2][mw_of(DIR)][65], TailSplit ts, Lay g,
-                                               Geo geo, int mode, const S *__restrict__ mf,
-                                               const S *__restrict__ vfx, const S *__restrict__ vfy,
-                                               const S *__restrict__ vfz, const S *__restrict__ density1, Vel3<S> v)
+// The tail: one wave's columns, a lane per row (no barrier on this path)
+template <int DIR, typename S>
+__device__ __forceinline__ void mom_tail_body(const Blk &bk, TailSplit ts, Lay g, Geo geo, int mode,
+                                              const S *__restrict__ mf, const S *__restrict__ vfx,
+                                              const S *__restrict__ vfy, const S *__restrict__ vfz,
+                                              const S *__restrict__ density1, Vel3<S> v)
 {
     using T = S;  // arithmetic type of the form
     constexpr int MW = mw_of(DIR);
@@ -336,55 +307,42 @@ __device__ __forceinline__ void mom_march_body(const Blk &bk, S (*xbuf)[2][mw_of
     const Recip rd = DIR == 3 ? geo.rz : geo.ry;
     const T V0 = (T)geo.vol;
 
-    int j, wp, m0, m1;
+    int m0, m1;
     chunk_range(bk, mmin, mmax + 1, m0, m1);
-    if constexpr (TAIL) {
-        // wave item: piece fastest, then row group (rows wmin..wmax+1 store), then column
-        const int item = bk.y * MW + w;
-        if (item >= ts.tw * ts.nrg * ts.nsub) return;  // this wave: no barrier on this path
-        const int sub = item % ts.nsub, rest = item / ts.nsub;
-        j = g.x_min + 64 * (bk.gx - 1) + rest / ts.nrg;
-        wp = wmin - 1 + (rest % ts.nrg) * 63 + lane;
-        const int len = (m1 - m0 + 1 + ts.nsub - 1) / ts.nsub;
-        m0 += sub * len;
-        m1 = min(m0 + len - 1, m1);
-    } else {
-        j = g.x_min + bk.x * 64 + lane;
-        wp = wmin - 1 + bk.y * (MW - 1) + w;
-    }
-    if (m0 > m1) return;  // the whole workgroup (the tail form: the wave), before any barrier
+    // wave item: piece fastest, then row group (rows wmin..wmax+1 store), then column
+    const int item = bk.y * MW + w;
+    if (item >= ts.tw * ts.nrg * ts.nsub) return;
+    const int sub = item % ts.nsub, rest = item / ts.nsub;
+    const int j = g.x_min + 64 * (bk.gx - 1) + rest / ts.nrg;
+    const int wp = wmin - 1 + (rest % ts.nrg) * 63 + lane;
+    const int len = (m1 - m0 + 1 + ts.nsub - 1) / ts.nsub;
+    m0 += sub * len;
+    m1 = min(m0 + len - 1, m1);
+    if (m0 > m1) return;
     // j >= x_min-1 and wp >= wmin-1 always; upper limits of the arrays read:
     // cells and the sweep's mass flux end at +2 across the sweep, vertices at +3
     const bool ok_cell = j <= g.x_max + 2 && wp <= wmax + 2;
-    // column j-1: loaded by lane 0 only in the 64-column layout (lane L-1 holds it for lane L)
-    const bool ok_cm = (TAIL || lane == 0) && j - 1 <= g.x_max + 2 && wp <= wmax + 2;
-    const bool store = (TAIL ? lane : w) >= 1 && j <= g.x_max + 1 && wp <= wmax + 1;
+    const bool ok_cm = j - 1 <= g.x_max + 2 && wp <= wmax + 2;
+    const bool store = lane >= 1 && j <= g.x_max + 1 && wp <= wmax + 1;
     const int i0 = DIR == 3 ? idx(g, j, wp, mmin) : idx(g, j, mmin, wp);  // offset at march position mmin
 #define OFF(q) (i0 + ((q) - mmin) * sM)
 
     const int dxc = cell_xm(g, j) - j;  // a mirrored x face: the interior cell its halo copies
     const int dxm = cell_xm(g, j - 1) - (j - 1);
-    const int dxt = TAN ? tan_xm(g, j) - j : 0, dxtm = TAN ? tan_xm(g, j - 1) - (j - 1) : 0;  // vol_flux_y/z
-    int b = 0;
+    const int dxt = tan_xm(g, j) - j, dxtm = tan_xm(g, j - 1) - (j - 1);  // vol_flux_y/z, the sweep's mass flux
     // the quads of a plane: columns j-1, j of rows wp-1, wp (Quad x, c, xw, w)
     auto xchg = [&](T a, T p, T am, T pm, Quad<T> &F, Quad<T> &P) {
-        if constexpr (TAIL) {
-            const int src = lane > 0 ? lane - 1 : 0;  // lane 0 (the halo row) stores nothing
-            F.c = a;
-            F.x = am;
-            F.w = shfl_d(a, src);
-            F.xw = shfl_d(am, src);
-            P.c = p;
-            P.x = pm;
-            P.w = shfl_d(p, src);
-            P.xw = shfl_d(pm, src);
-        } else {
-            publish65(xbuf[b], lane, w, a, p, am, pm);
-            gather65(xbuf[b], lane, w, a, p, F, P);
-            b ^= 1;
-        }
+        const int src = lane > 0 ? lane - 1 : 0;  // lane 0 (the halo row) stores nothing
+        F.c = a;
+        F.x = am;
+        F.w = shfl_d(a, src);
+        F.xw = shfl_d(am, src);
+        P.c = p;
+        P.x = pm;
+        P.w = shfl_d(p, src);
+        P.xw = shfl_d(pm, src);
     };
-    auto plane = [&](int q, Quad<T> &F, Quad<T> &P, int &b) {
+    auto plane = [&](int q, Quad<T> &F, Quad<T> &P) {
         const int i = OFF(q);
         const T a = ok_cell ? (T)mf[i + dxt] : (T)0;  // q <= mmax+3: inside the sweep's face extent
         const T p = (ok_cell && q <= mmax + 2)
@@ -400,15 +358,15 @@ __device__ __forceinline__ void mom_march_body(const Blk &bk, S (*xbuf)[2][mw_of
 
     Quad<T> Fa, Pa, Fb, Pb;
     // prologue: nf(m0-2..m0), node masses at m0-1, m0, m0+1, velocities m0-2..m0+1
-    plane(m0 - 2, Fa, Pa, b);
-    plane(m0 - 1, Fb, Pb, b);
+    plane(m0 - 2, Fa, Pa);
+    plane(m0 - 1, Fb, Pb);
     const T nf_m2 = march_node_flux<DIR, T>(Fa, Fb);
     const T mp_m1 = march_node_mass<DIR, T>(Pa, Pb);
-    plane(m0, Fa, Pa, b);
+    plane(m0, Fa, Pa);
     T nf_lo = march_node_flux<DIR, T>(Fb, Fa);  // nf(m-1)
     T mp0 = march_node_mass<DIR, T>(Pb, Pa);    // mp(m)
     const T mq_m1 = mp_m1 - nf_m2 + nf_lo;
-    plane(m0 + 1, Fb, Pb, b);
+    plane(m0 + 1, Fb, Pb);
     T nf0 = march_node_flux<DIR, T>(Fa, Fb);     // nf(m)
     T mp1 = march_node_mass<DIR, T>(Pa, Pb);     // mp(m+1)
     T mq0 = mp0 - nf_lo + nf0;                // mq(m)
@@ -468,43 +426,311 @@ __device__ __forceinline__ void mom_march_body(const Blk &bk, S (*xbuf)[2][mw_of
 #undef OFF
 }
 
+// A row of an array at a lane's byte offset: with the row's address scalar, the
+// access takes it and a 32-bit offset, and no vector address arithmetic.
+template <typename S>
+__device__ inline S ld(const S *__restrict__ row, unsigned off)
+{
+    return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(row) + off);
+}
+
+// sign-bit mask of x in the high word of its type
+__device__ inline unsigned sign_of(double x) { return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) & 0x80000000u; }
+__device__ inline unsigned sign_of(float x) { return __builtin_bit_cast(unsigned, x) & 0x80000000u; }
+__device__ inline double flip_sign(double x, unsigned m)
+{
+    return __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, x) ^ ((unsigned long long)m << 32));
+}
+__device__ inline float flip_sign(float x, unsigned m) { return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) ^ m); }
+
+// mom_face_flux from the velocity differences d0 = v0 - vm1, d1 = vp1 - v0,
+// d2 = vp2 - vp1, which successive faces share: for nf < 0 the reference's
+// differences are -d2 and -d1, exactly, and only their product, magnitudes and
+// the sign of the second count.  `wind` becomes a flip of the sign bit (sgn:
+// the sign bit where nf < 0).
+template <typename T>
+__device__ inline T mom_flux_of(T nf, bool neg, unsigned sgn, T one_m, T two_m, T one_p, T d, const Recip &rd,
+                                const Recip &r6, T v0, T vp1, T d0, T d1, T d2)
+{
+    const T du = neg ? d2 : d0;
+    const T donor = neg ? vp1 : v0;
+    const T auw = fabs(du), adw = fabs(d1);
+    const T lim = tmin(tmin(by_const<T>(d * (by_const<T>(two_m * adw, rd) + by_const<T>(one_p * auw, rd)), r6), auw), adw);
+    const T limiter = du * d1 > (T)0 ? flip_sign(lim, sign_of(d1) ^ sgn) : (T)0;
+    return (donor + one_m * limiter) * nf;
+}
+
+// The 64-column layout of the y and z sweeps.  mom_march_body's expressions
+// (MODE: the sweep's post_vol, mom_post_vol), with the work per plane cut to
+// what they need, since at 344 (FP64) and 253 (FP32) VALU instructions per wave
+// and plane the sweeps ran at or near the VALU's rate:
+//   * row addresses are scalar (the wave's row and the plane), a lane adds a
+//     byte offset; lanes and planes outside the arrays read clamped ones;
+//   * the march is unrolled by four, so the window of velocities, their
+//     differences and the planes' quads stay in their registers;
+//   * the halo row (wave 0) only loads and publishes;
+//   * the prologue's planes are loaded two at a time and exchanged past one
+//     barrier.
+// Now 205 and 107 instructions.  The old form against this one, best shapes, one
+// machine: 512^3 FP64 mom_y 2.37 -> 2.30 ms, mom_z 2.16 -> 2.15, FP32 1.24 -> 1.17
+// and 1.12 -> 1.06; 256^3 FP64 0.362 -> 0.328 and 0.338 -> 0.313; 131x75x93 38.6 ->
+// 28.0 and 41.8 -> 29.2 us (with the tail rule below); 64^3 18.5 -> 17.0 and
+// 17.7 -> 16.9; FP32 101x143x67 20.7 -> 17.5 and 20.1 -> 16.8; 320^3 as 8 tiles,
+// the three batched launches 2.13 -> 2.00 ms.  8-wave workgroups (fewer halo rows)
+// were within 1.5 % at 512^3 and 12-25 % slower at 64^3 to 131x75x93.
+template <int DIR, int MODE, typename S>
+__device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(DIR)][65], Lay g, Geo geo,
+                                              const S *__restrict__ mf, const S *__restrict__ vfx,
+                                              const S *__restrict__ vfy, const S *__restrict__ vfz,
+                                              const S *__restrict__ density1, Vel3<S> v)
+{
+    using T = S;  // arithmetic type of the form
+    constexpr int MW = mw_of(DIR);
+    const int lane = (int)threadIdx.x, w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int wmin = DIR == 3 ? g.y_min : g.z_min, wmax = DIR == 3 ? g.y_max : g.z_max;
+    const int mmin = DIR == 3 ? g.z_min : g.y_min, mmax = DIR == 3 ? g.z_max : g.y_max;
+    const T d = (T)(DIR == 3 ? geo.dz : geo.dy);
+    const Recip rd = DIR == 3 ? geo.rz : geo.ry;
+    const T V0 = (T)geo.vol;
+    int m0, m1;
+    chunk_range(bk, mmin, mmax + 1, m0, m1);
+    if (m0 > m1) return;  // the whole workgroup, before any barrier
+    const int j = g.x_min + bk.x * 64 + lane;
+    const int wp = wmin - 1 + bk.y * (MW - 1) + w;
+    const bool row = w >= 1 && wp <= wmax + 1;  // an owned row (uniform)
+    const bool store = j <= g.x_max + 1;
+    // cells and the sweep's mass flux end at +2 across the sweep
+    const int jr = min(j, g.x_max + 2), wr = min(wp, wmax + 2);
+    // byte offsets from column x_min-2: the lane's column, density's and the
+    // tangential fluxes' on a mirrored x face; lane 0's column j-1 likewise
+    auto off = [&](int col) { return (unsigned)(col - g.x_min + 2) * (unsigned)sizeof(S); };
+    unsigned oj = off(jr), orho = off(cell_xm(g, jr)), ot = off(tan_xm(g, jr));
+    const int jm = min(j - 1, g.x_max + 2);
+    unsigned ojm = off(jm), orhom = off(cell_xm(g, jm)), otm = off(tan_xm(g, jm));
+    // the wave's row at march position q (elements)
+    auto at = [&](int q) { return (int64_t)(DIR == 3 ? idx(g, g.x_min - 2, wr, q) : idx(g, g.x_min - 2, q, wr)); };
+    const int up = DIR == 3 ? g.ld : g.plane;  // to the next row across the sweep
+
+    // the values of a plane: the sweep's mass flux, density and the volume
+    // fluxes of post_vol (as stored, so that their loads can stay in flight), of
+    // column j and, in lane 0, of j-1
+    constexpr int NF = MODE == 2 ? 4 : MODE == 6 ? 0 : 2;
+    struct Col {
+        S a, rho, f[NF > 0 ? NF : 1];
+    };
+    struct Pl {
+        Col c, m;
+    };
+    auto load_col = [&](Col &x, int64_t r, int64_t rc, unsigned o, unsigned orh, unsigned otan) {
+        x.a = ld(mf + r, otan);
+        x.rho = ld(density1 + rc, orh);
+        if constexpr (MODE == 2 || MODE == 4) {
+            x.f[0] = ld(vfx + rc + 1, o);
+            x.f[1] = ld(vfx + rc, o);
+        }
+        if constexpr (MODE == 2) {
+            x.f[2] = ld(vfy + rc + up, otan);
+            x.f[3] = ld(vfy + rc, otan);
+        }
+        if constexpr (MODE == 3) {
+            x.f[0] = ld(vfz + rc + up, otan);
+            x.f[1] = ld(vfz + rc, otan);
+        }
+    };
+    auto load = [&](int q, Pl &x) {
+        const int64_t r = at(q), rc = at(min(q, mmax + 2));  // mass fluxes end at mmax+3, cells at mmax+2
+        load_col(x.c, r, rc, oj, orho, ot);
+        if (lane == 0) load_col(x.m, r, rc, ojm, orhom, otm);
+    };
+    auto cell_mass = [&](const Col &x) -> T {  // mom_post_vol's expressions
+        if constexpr (NF == 4) return x.rho * (V0 + x.f[0] - x.f[1] + x.f[2] - x.f[3]);
+        else if constexpr (NF == 2) return x.rho * (V0 + x.f[0] - x.f[1]);
+        else return x.rho * V0;
+    };
+    // publishes the plane's mass flux and cell mass; returns the cell mass of column j
+    auto publish = [&](int b, const Pl &x) {
+        const T p = cell_mass(x.c);
+        xbuf[b][0][w][lane + 1] = x.c.a;
+        xbuf[b][1][w][lane + 1] = p;
+        if (lane == 0) {
+            xbuf[b][0][w][0] = x.m.a;
+            xbuf[b][1][w][0] = cell_mass(x.m);
+        }
+        return p;
+    };
+    auto gather = [&](int b, T a, T p, Quad<T> &F, Quad<T> &P) {
+        F = Quad<T>{a, xbuf[b][0][w][lane], xbuf[b][0][w - 1][lane + 1], xbuf[b][0][w - 1][lane]};
+        P = Quad<T>{p, xbuf[b][1][w][lane], xbuf[b][1][w - 1][lane + 1], xbuf[b][1][w - 1][lane]};
+    };
+    auto vel_at = [&](int c, int q) { return ld(v.in[c] + at(q), oj); };
+
+    // waves without an owned row only load and publish; the barriers are the
+    // same in number: two, then one per position
+    if (!row) {
+        for (int q = 0; q < 4; q++) {
+            Pl x;
+            load(m0 - 2 + q, x);
+            publish(q, x);
+        }
+        __syncthreads();
+        __syncthreads();
+        for (int m = m0; m <= m1; m++) {
+            Pl x;
+            load(m + 2, x);
+            publish((m - m0) & 1, x);
+            __syncthreads();
+        }
+        return;
+    }
+
+    // by position mod 4 (quads mod 2): velocities, differences vel(q) = v(q+1)
+    // - v(q), node flux, node masses; the momentum flux through the face below
+    Quad<T> F[2], P[2];
+    T vel[4][3], dv[4][3], nf[4], mp[4], mq[4], flo[3];
+    {
+        // two planes at a time: all four would take the kernel's registers past the march's own
+        T a[4], p[4];
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+            Pl x, y;
+            load(m0 - 2 + q, x);
+            load(m0 - 1 + q, y);
+            a[q] = x.c.a;
+            p[q] = publish(q, x);
+            a[q + 1] = y.c.a;
+            p[q + 1] = publish(q + 1, y);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            vel[2][c] = vel_at(c, m0 - 2);
+            vel[3][c] = vel_at(c, m0 - 1);
+            vel[0][c] = vel_at(c, m0);
+            vel[1][c] = vel_at(c, m0 + 1);
+        }
+        __syncthreads();
+        gather(0, a[0], p[0], F[0], P[0]);
+        gather(1, a[1], p[1], F[1], P[1]);
+        const T nf_m2 = march_node_flux<DIR, T>(F[0], F[1]);
+        const T mp_m1 = march_node_mass<DIR, T>(P[0], P[1]);
+        gather(2, a[2], p[2], F[0], P[0]);
+        nf[3] = march_node_flux<DIR, T>(F[1], F[0]);
+        mp[0] = march_node_mass<DIR, T>(P[1], P[0]);
+        const T mq_m1 = mp_m1 - nf_m2 + nf[3];
+        gather(3, a[3], p[3], F[1], P[1]);
+        nf[0] = march_node_flux<DIR, T>(F[0], F[1]);
+        mp[1] = march_node_mass<DIR, T>(P[0], P[1]);
+        mq[0] = mp[0] - nf[3] + nf[0];
+        const T sig = face_sigma(nf[3], mq_m1, mq[0]);
+        const bool neg = nf[3] < (T)0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            dv[2][c] = vel[3][c] - vel[2][c];
+            dv[3][c] = vel[0][c] - vel[3][c];
+            dv[0][c] = vel[1][c] - vel[0][c];
+            flo[c] = mom_flux_of<T>(nf[3], neg, neg ? 0x80000000u : 0u, (T)1 - sig, (T)2 - sig, (T)1 + sig, d, rd,
+                                    geo.r6, vel[3][c], vel[0][c], dv[2][c], dv[3][c], dv[0][c]);
+        }
+        __syncthreads();  // slots 0 and 1 are read before the march rewrites them
+    }
+
+    // a plane's loads go out before the barrier of the plane before (AHEAD: up
+    // to 124 VGPRs in FP64, four waves per SIMD either way; 512^3 mom_y 2.39 ->
+    // 2.30 ms FP64, FP32 mom_z 1.04 -> 0.98), except where four volume fluxes
+    // would spill: FP64 mode 2, at the top of its own step (mom_z over both of its
+    // modes 2.15 ms that way, 2.26 with 20 values spilled)
+    constexpr bool AHEAD = sizeof(S) == 4 || MODE != 2;
+    Pl nx;
+    auto load_ahead = [&](int q, T(&vq)[3]) {
+        load(q, nx);
+#pragma unroll
+        for (int c = 0; c < 3; c++) vq[c] = vel_at(c, q);
+    };
+    if (AHEAD) load_ahead(m0 + 2, vel[2]);
+    auto step = [&](auto ic, int m) {
+        constexpr int i = decltype(ic)::value, i1 = (i + 1) & 3, i2 = (i + 2) & 3, im = (i + 3) & 3, e = i & 1;
+        // keeps the compiler from hoisting array + offset into vector registers
+        asm volatile("" : "+v"(oj), "+v"(orho), "+v"(ot), "+v"(ojm), "+v"(orhom), "+v"(otm));
+        if (!AHEAD) load_ahead(m + 2, vel[i2]);
+        const T a = nx.c.a, p = publish(e, nx);
+        if (AHEAD && m < m1) load_ahead(m + 3, vel[im]);  // vel(m-1) is done with
+        __syncthreads();
+        // F[1-e], P[1-e] hold plane m+1
+        gather(e, a, p, F[e], P[e]);
+        nf[i1] = march_node_flux<DIR, T>(F[1 - e], F[e]);  // nf(m+1)
+        mp[i2] = march_node_mass<DIR, T>(P[1 - e], P[e]);  // mp(m+2), not used at mmax+3
+        mq[i1] = mp[i1] - nf[i] + nf[i1];
+        const T sig = face_sigma(nf[i], mq[i], mq[i1]);
+        const bool neg = nf[i] < (T)0;
+        const unsigned sgn = neg ? 0x80000000u : 0u;
+        const T one_m = (T)1 - sig, two_m = (T)2 - sig, one_p = (T)1 + sig;
+        const int64_t r = at(m);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            dv[i1][c] = vel[i2][c] - vel[i1][c];
+            const T fhi = mom_flux_of<T>(nf[i], neg, sgn, one_m, two_m, one_p, d, rd, geo.r6, vel[i][c], vel[i1][c],
+                                         dv[im][c], dv[i][c], dv[i1][c]);  // F(m)
+            const T out = quo(vel[i][c] * mq[i] + flo[c] - fhi, mp[i]);
+            if (store) *reinterpret_cast<S *>(reinterpret_cast<char *>(v.out[c] + r) + oj) = out;
+            flo[c] = fhi;
+        }
+    };
+    for (int m = m0;;) {
+        step(std::integral_constant<int, 0>{}, m);
+        if (++m > m1) break;
+        step(std::integral_constant<int, 1>{}, m);
+        if (++m > m1) break;
+        step(std::integral_constant<int, 2>{}, m);
+        if (++m > m1) break;
+        step(std::integral_constant<int, 3>{}, m);
+        if (++m > m1) break;
+    }
+}
+
 // One workgroup of a y or z sweep.  With a narrow tail the grid's first
 // workgroups (in launch order) march the tail, TailSplit::tb per chunk: its
 // marches take longest per plane (each load touches a line per lane), and
 // dispatched last they ran past the rest of the launch.  The 64-column
 // tiles follow in the grid's order with gx-1 tiles to a row, and the
 // workgroups left over exit at once.
-template <int DIR, typename S, bool TAN = false>
-__device__ __forceinline__ void mom_march(const Blk &bk, Lay g, Geo geo, int mode, const S *__restrict__ mf,
-                                          const S *__restrict__ vfx, const S *__restrict__ vfy,
-                                          const S *__restrict__ vfz, const S *__restrict__ density1, Vel3<S> v)
+// lin: the workgroup's place in launch order on a gx x gy x gz grid; xcd: the
+// XCD order (launch.h xcd_layer_block, single-tile launches) for the 64-column
+// tiles.
+template <int DIR, int MODE, typename S>
+__device__ __forceinline__ void mom_march(int lin, int gx, int gy, int gz, int xcd, Lay g, Geo geo,
+                                          const S *__restrict__ mf, const S *__restrict__ vfx,
+                                          const S *__restrict__ vfy, const S *__restrict__ vfz,
+                                          const S *__restrict__ density1, Vel3<S> v)
 {
-    __shared__ S xbuf[2][2][mw_of(DIR)][65];
-    const int tw = sizeof(S) == 8 ? mom_tail_cols(g, bk.gx) : 0;  // the FP64 form only (mom_tail_cols)
-    if (!tw) {
-        mom_march_body<DIR, S, false, TAN>(bk, xbuf, TailSplit{}, g, geo, mode, mf, vfx, vfy, vfz, density1, v);
-        return;
+    __shared__ S xbuf[4][2][mw_of(DIR)][65];
+    int off = 0;
+    if constexpr (sizeof(S) == 8) {  // the tail form: FP64 only (mom_tail_cols)
+        const int tw = mom_tail_cols(g, gx);
+        if (tw) {
+            const TailSplit ts = mom_tail_split<DIR>(g, Blk{0, 0, 0, gx, gy, gz}, tw);
+            if (lin < ts.tb * gz) {
+                mom_tail_body<DIR, S>(Blk{gx - 1, lin % ts.tb, lin / ts.tb, gx, gy, gz}, ts, g, geo, MODE, mf, vfx,
+                                      vfy, vfz, density1, v);
+                return;
+            }
+            off = ts.tb * gz;
+            gx -= 1;  // the 64-column tiles
+            if (lin - off >= gx * gy * gz) return;
+        }
     }
-    const TailSplit ts = mom_tail_split<DIR>(g, bk, tw);
-    int lin = bk.x + bk.gx * (bk.y + bk.gy * bk.z);
-    if (lin < ts.tb * bk.gz) {
-        mom_march_body<DIR, S, true, TAN>(Blk{bk.gx - 1, lin % ts.tb, lin / ts.tb, bk.gx, bk.gy, bk.gz}, xbuf, ts, g,
-                                     geo, mode, mf, vfx, vfy, vfz, density1, v);
-        return;
-    }
-    lin -= ts.tb * bk.gz;
-    const int mx = bk.gx - 1;  // 64-column tiles
-    if (lin >= mx * bk.gy * bk.gz) return;
-    mom_march_body<DIR, S, false, TAN>(Blk{lin % mx, (lin / mx) % bk.gy, lin / (mx * bk.gy), bk.gx, bk.gy, bk.gz}, xbuf,
-                                  TailSplit{}, g, geo, mode, mf, vfx, vfy, vfz, density1, v);
+    const int id = xcd ? xcd_layer_block(lin, gx * gy, off) : lin - off;
+    mom_cols_body<DIR, MODE, S>(Blk{id % gx, (id / gx) % gy, id / (gx * gy), gx, gy, gz}, xbuf, g, geo, mf, vfx, vfy,
+                                vfz, density1, v);
 }
 
-template <int DIR, typename S>
-__global__ void __launch_bounds__(64 * mw_of(DIR)) k_fast_mom_march(int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
+template <int DIR, int MODE, typename S>
+__global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fast_mom_march(int xcd, Lay g, Geo geo, const S *__restrict__ mf, const S *__restrict__ vfx,
                  const S *__restrict__ vfy, const S *__restrict__ vfz,
                  const S *__restrict__ density1, Vel3<S> v)
 {
-    mom_march<DIR, S, sizeof(S) == 4>(hw_blk(xcd), g, geo, mode, mf, vfx, vfy, vfz, density1, v);
+    const int gx = (int)gridDim.x, gy = (int)gridDim.y, gz = (int)gridDim.z;
+    mom_march<DIR, MODE, S>((int)blockIdx.x + gx * ((int)blockIdx.y + gy * (int)blockIdx.z), gx, gy, gz, xcd, g, geo,
+                            mf, vfx, vfy, vfz, density1, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -513,7 +739,7 @@ __global__ void __launch_bounds__(64 * mw_of(DIR)) k_fast_mom_march(int xcd, Lay
 //   nf(j)  = 0.125*(f(0,-1,0)+f(0,0,0)+f(1,-1,0)+f(1,0,0)+f(0,-1,-1)+f(0,0,-1)+f(1,-1,-1)+f(1,0,-1))
 //   mp(j)  = cells (0,-1,0),(0,0,0),(-1,-1,0),(-1,0,0),(0,-1,-1),(0,0,-1),(-1,-1,-1),(-1,0,-1)
 
-template <typename S, bool TAN = false>  // TAN: as in mom_march_body
+template <typename S>
 __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
              const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1,
              Vel3<S> v)
@@ -540,7 +766,7 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mo
 #define OFF(q) (i0 + ((q) - g.z_min) * g.plane)
     // a mirrored x face: the interior cell and node its halos copy, and the
     // sign flip of the x velocity there
-    const int dxc = cell_xm(g, j) - j, dxn = node_xm(g, j) - j, dxt = TAN ? tan_xm(g, j) - j : 0;
+    const int dxc = cell_xm(g, j) - j, dxn = node_xm(g, j) - j, dxt = tan_xm(g, j) - j;
     const bool xneg = node_xsign(g, j);
 
     auto plane = [&](int q, Quad<T> &F, Quad<T> &P, int &b) {
@@ -603,11 +829,21 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mo
 }
 
 template <typename S>
-__global__ void __launch_bounds__(64 * mw_of(1)) k_fast_mom_x(int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
+__global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1) k_fast_mom_x(int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
              const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1,
              Vel3<S> v)
 {
-    mom_x_body<S, sizeof(S) == 4>(hw_blk(xcd), g, geo, mode, mf, vfx, vfy, vfz, density1, v);
+    mom_x_body<S>(hw_blk(xcd), g, geo, mode, mf, vfx, vfy, vfz, density1, v);
+}
+
+// mom_post_vol's mode of a sweep of advection.f90 (x and z in sweeps 1 and 3,
+// y in sweep 2); 0: no such sweep
+static int mom_mode(int advect_x, int sweep_number, int direction)
+{
+    if (direction == 1) return sweep_number == 1 ? 1 : sweep_number == 3 ? 5 : 0;
+    if (direction == 2) return sweep_number != 2 ? 0 : advect_x ? 3 : 4;
+    if (direction == 3) return sweep_number == 1 ? 2 : sweep_number == 3 ? 6 : 0;
+    return 0;
 }
 
 template <typename S>
@@ -630,12 +866,14 @@ static hipError_t fast_advec_mom_t(const Lay &g, const Geo &m, int mode, int dir
                      vol_flux_y, vol_flux_z, density1, v);
     } else if (direction == 2) {
         const dim3 grid((nxn + 63) / 64, (nzn + MW - 2) / (MW - 1), nchunks(nyn, sh.planes));
-        TIMED_LAUNCH("k_fast_mom_y", st, (k_fast_mom_march<2, S>), grid, blk, 0, st, sh.xcd, g, m, mode, mass_flux_y,
-                     vol_flux_x, vol_flux_y, vol_flux_z, density1, v);
+        const auto kern = mode == 3 ? k_fast_mom_march<2, 3, S> : k_fast_mom_march<2, 4, S>;
+        TIMED_LAUNCH("k_fast_mom_y", st, kern, grid, blk, 0, st, sh.xcd, g, m, mass_flux_y, vol_flux_x, vol_flux_y,
+                     vol_flux_z, density1, v);
     } else {
         const dim3 grid((nxn + 63) / 64, (nyn + MW - 2) / (MW - 1), nchunks(nzn, sh.planes));
-        TIMED_LAUNCH("k_fast_mom_z", st, (k_fast_mom_march<3, S>), grid, blk, 0, st, sh.xcd, g, m, mode, mass_flux_z,
-                     vol_flux_x, vol_flux_y, vol_flux_z, density1, v);
+        const auto kern = mode == 2 ? k_fast_mom_march<3, 2, S> : k_fast_mom_march<3, 6, S>;
+        TIMED_LAUNCH("k_fast_mom_z", st, kern, grid, blk, 0, st, sh.xcd, g, m, mass_flux_z, vol_flux_x, vol_flux_y,
+                     vol_flux_z, density1, v);
     }
     return hipGetLastError();
 }
@@ -646,14 +884,8 @@ hipError_t launch_fast_advec_mom(Store s, const Lay &g, const Geo &m, int advect
                                  const void *vol_flux_z, const void *density1, const void *const *vel_in,
                                  void *const *vel_out, const Shape &sh, hipStream_t st)
 {
-    int mode = 0;
-    if (sweep_number == 1 && direction == 1) mode = 1;
-    else if (sweep_number == 1 && direction == 3) mode = 2;
-    else if (sweep_number == 2 && advect_x) mode = 3;
-    else if (sweep_number == 2 && !advect_x) mode = 4;
-    else if (sweep_number == 3 && direction == 1) mode = 5;
-    else if (sweep_number == 3 && direction == 3) mode = 6;
-    if (!mode || direction < 1 || direction > 3) return hipErrorInvalidValue;
+    const int mode = mom_mode(advect_x, sweep_number, direction);
+    if (!mode) return hipErrorInvalidValue;  // the resident driver issues only the reference's sweeps
 #define CALL(T)                                                                                                 \
     fast_advec_mom_t<T>(g, m, mode, direction, static_cast<const T *>(mass_flux_x),                             \
                         static_cast<const T *>(vol_flux_x), static_cast<const T *>(mass_flux_y),                \
@@ -690,7 +922,7 @@ int batch_blocks_mom(int dir, const Lay &g, int planes)
     return gx * gy * gz;
 }
 
-template <int DIR, typename S>
+template <int DIR, int MODE, typename S>  // MODE: 0 for the x sweep, which takes `mode`
 __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
                                          int mode, int planes, const MomSlots &ms, int hb)
 {
@@ -713,24 +945,22 @@ __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, cons
     if constexpr (DIR == 1)
         mom_x_body<S>(bk, D.g, D.m, mode, static_cast<const S *>(D.f[F_MASS_FLUX_X]), vfx, vfy, vfz, rho, v);
     else
-        mom_march<DIR, S>(bk, D.g, D.m, mode,
-                               static_cast<const S *>(D.f[DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z]), vfx, vfy,
-                               vfz, rho, v);
+        mom_march<DIR, MODE, S>(lb, gx, gy, gz, 0, D.g, D.m,
+                                static_cast<const S *>(D.f[DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z]), vfx, vfy, vfz,
+                                rho, v);
 }
 
-template <int DIR, typename S>
-// The FP64 y/z sweeps held to five waves per SIMD (96 VGPRs; the tile walk
-// takes them to 101, four waves): the batched momentum launches of 640^3 as
-// 8 tiles 4.81 -> 4.35 ms with one value spilled.  With the tail form five
-// values spill (20 bytes per lane) and the launches still run 4.41 -> 4.16 ms.
-__global__ void __launch_bounds__(64 * mw_of(DIR), DIR != 1 && sizeof(S) == 8 ? 5 : 1)
+template <int DIR, int MODE, typename S>
+// The FP64 y/z sweeps held to four waves per SIMD (128 VGPRs): at five they
+// spill 18-34 values and the launches of 320^3 as 8 tiles ran 2.00 -> 2.42 ms.
+__global__ void __launch_bounds__(64 * mw_of(DIR), DIR != 1 && sizeof(S) == 8 ? 4 : 1)
 kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int planes, int xcd,
        MomSlots ms)
 {
     int hb, end, step;  // the tiles of this workgroup (persistent when the grid is short)
     tile_walk(start[nd], xcd, hb, end, step);
     for (; hb < end; hb += step) {
-        mom_tile<DIR, S>(decks, start, nd, mode, planes, ms, hb);
+        mom_tile<DIR, MODE, S>(decks, start, nd, mode, planes, ms, hb);
         __syncthreads();  // the next tile reuses the workgroup's LDS
     }
 }
@@ -738,24 +968,25 @@ kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
 hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, int advect_x, int dir,
                            int sweep_number, const Slots &sl, const Shape &sh, hipStream_t st)
 {
-    int mode = 0;
-    if (sweep_number == 1 && dir == 1) mode = 1;
-    else if (sweep_number == 1 && dir == 3) mode = 2;
-    else if (sweep_number == 2 && advect_x) mode = 3;
-    else if (sweep_number == 2 && !advect_x) mode = 4;
-    else if (sweep_number == 3 && dir == 1) mode = 5;
-    else if (sweep_number == 3 && dir == 3) mode = 6;
-    if (!mode || dir < 1 || dir > 3) return hipErrorInvalidValue;
+    const int mode = mom_mode(advect_x, sweep_number, dir);
+    if (!mode) return hipErrorInvalidValue;
     if (bg.total == 0) return hipSuccess;
     const dim3 grid(batch_wgs(bg, sh)), blk(64, mw_of(dir));
     const MomSlots ms{sl[F_DENSITY1], {sl[F_XVEL1], sl[F_YVEL1], sl[F_ZVEL1]}, {sl[X_W5], sl[X_W6], sl[X_W7]}};
-#define L(D_, T_)                                                                                          \
-    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, sh.planes, sh.xcd, ms)
+#define L(D_, M_, T_)                                                                                        \
+    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, M_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, sh.planes, sh.xcd, ms)
+#define LM(T_)                                                                                               \
+    if (dir == 1) L(1, 0, T_);                                                                               \
+    else if (mode == 3) L(2, 3, T_);                                                                         \
+    else if (mode == 4) L(2, 4, T_);                                                                         \
+    else if (mode == 2) L(3, 2, T_);                                                                         \
+    else L(3, 6, T_)
     if (s == ST_F32) {
-        if (dir == 1) L(1, float); else if (dir == 2) L(2, float); else L(3, float);
+        LM(float);
     } else {
-        if (dir == 1) L(1, double); else if (dir == 2) L(2, double); else L(3, double);
+        LM(double);
     }
+#undef LM
 #undef L
     return hipGetLastError();
 }
