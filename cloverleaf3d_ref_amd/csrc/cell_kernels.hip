@@ -177,11 +177,12 @@ __device__ __forceinline__ void cell_x_body(const Blk &bk, Lay g, Geo m, int mod
 }
 
 template <typename S>
-__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
+__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const double *__restrict__ dt, int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
               const S *__restrict__ vfz, const S *__restrict__ density1,
               const S *__restrict__ energy1, S *__restrict__ mass_flux_x, S *__restrict__ rho_out,
               S *__restrict__ e_out, S *__restrict__ p_out, int rows)
 {
+    if (*dt < 0.0) return;  // a small step (launch_dt_final)
     cell_x_body<S>(hw_blk(xcd), g, m, mode, rows, vfx, vfy, vfz, density1, energy1, mass_flux_x, rho_out, e_out,
                    p_out);
 }
@@ -315,17 +316,18 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, int
 }
 
 template <int DIR, typename S>
-__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
+__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
+    if (*dt < 0.0) return;
     cell_march_body<DIR, S>(hw_blk(xcd), g, m, mode, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
                             p_out);
 }
 
 template <typename S>
-static hipError_t fast_advec_cell_t(const Lay &g, const Geo &m, int mode, int dir, const S *density1,
+static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m, int mode, int dir, const S *density1,
                                     const S *energy1, S *mass_flux_x, const S *vol_flux_x, S *mass_flux_y,
                                     const S *vol_flux_y, S *mass_flux_z, const S *vol_flux_z, S *rho_out, S *e_out,
                                     S *p_out, const Shape &sh, hipStream_t st)
@@ -335,21 +337,21 @@ static hipError_t fast_advec_cell_t(const Lay &g, const Geo &m, int mode, int di
     if (dir == 1) {
         const int rows = cell_x_rows(sh.planes);
         const dim3 grid((nx + 2 + 59) / 60, ((ny * nz + rows - 1) / rows + CROWS - 1) / CROWS, 1);
-        TIMED_LAUNCH("k_fast_cell_x", st, k_fast_cell_x<S>, grid, blk, 0, st, sh.xcd, g, m, mode, vol_flux_x, vol_flux_y,
+        TIMED_LAUNCH("k_fast_cell_x", st, k_fast_cell_x<S>, grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x, vol_flux_y,
                      vol_flux_z, density1, energy1, mass_flux_x, rho_out, e_out, p_out, rows);
     } else if (dir == 2) {
         const dim3 grid((nx + 63) / 64, (nz + 2 + CROWS - 1) / CROWS, nchunks(ny + 2, sh.planes));
-        TIMED_LAUNCH("k_fast_cell_y", st, (k_fast_cell_march<2, S>), grid, blk, 0, st, sh.xcd, g, m, mode, vol_flux_x,
+        TIMED_LAUNCH("k_fast_cell_y", st, (k_fast_cell_march<2, S>), grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x,
                      vol_flux_y, vol_flux_z, density1, energy1, mass_flux_y, rho_out, e_out, p_out);
     } else {
         const dim3 grid((nx + 63) / 64, (ny + CROWS - 1) / CROWS, nchunks(nz + 2, sh.planes));
-        TIMED_LAUNCH("k_fast_cell_z", st, (k_fast_cell_march<3, S>), grid, blk, 0, st, sh.xcd, g, m, mode, vol_flux_x,
+        TIMED_LAUNCH("k_fast_cell_z", st, (k_fast_cell_march<3, S>), grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x,
                      vol_flux_y, vol_flux_z, density1, energy1, mass_flux_z, rho_out, e_out, p_out);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_fast_advec_cell(Store s, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
+hipError_t launch_fast_advec_cell(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
                                   const void *density1, const void *energy1, void *mass_flux_x,
                                   const void *vol_flux_x, void *mass_flux_y, const void *vol_flux_y,
                                   void *mass_flux_z, const void *vol_flux_z, void *rho_out, void *e_out,
@@ -362,7 +364,7 @@ hipError_t launch_fast_advec_cell(Store s, const Lay &g, const Geo &m, int advec
     if (!mode) return hipErrorInvalidValue;  // the resident driver issues only the reference's sweeps
     if (pressure && sweep_number != 3) return hipErrorInvalidValue;  // only the last sweep's state is final
 #define CALL(T)                                                                                                 \
-    fast_advec_cell_t<T>(g, m, mode, dir, static_cast<const T *>(density1), static_cast<const T *>(energy1),     \
+    fast_advec_cell_t<T>(dt, g, m, mode, dir, static_cast<const T *>(density1), static_cast<const T *>(energy1),     \
                          static_cast<T *>(mass_flux_x), static_cast<const T *>(vol_flux_x),                      \
                          static_cast<T *>(mass_flux_y), static_cast<const T *>(vol_flux_y),                      \
                          static_cast<T *>(mass_flux_z), static_cast<const T *>(vol_flux_z),                      \

@@ -114,6 +114,8 @@ struct clover_chunk {
     double *partial;  // per tile: kMaxPartials * 5
     double *scalar;   // per tile: 8
     double *h_scalar; // pinned
+    DtSlot *dt_slot;  // pinned: a pipelined step's dt (ahead)
+    unsigned long long dt_seq;
     Stage stage;      // field fetches
     double dt, dtold, time;
     int step;
@@ -656,13 +658,66 @@ static void ideal_gas(clover_chunk *c, bool predict, bool need_sound = false)
     }
 }
 
-// timestep.f90:28-128.  Returns 1 on a small time step.
+// the step's dt on the device (fused kernels: launch_dt_final's, else uploaded)
+static double *dt_dev(clover_chunk *c) { return c->scalar + 6; }
+
+static void put_dt(clover_chunk *c, double dt)
+{
+    c->h_scalar[6] = dt;
+    hip_check(hipMemcpyAsync(dt_dev(c), c->h_scalar + 6, sizeof(double), hipMemcpyHostToDevice, c->st), "dt");
+    hip_check(hipStreamSynchronize(c->st), "sync");
+}
+
+// A single tile's fused step is enqueued whole before the host learns its dt:
+// the kernels take it from device memory, and the host meets it while they
+// run.  Waiting first left the GPU idle for the copy, the wake-up and the next
+// launch on every step (10x2x2 98 -> 80 us per step, FP32 101x143x67 155 -> 148,
+// 64^3 FP64 140 -> 136).
+static bool ahead(const clover_chunk *c) { return c->fast && c->tiles.size() == 1; }
+
+// waits for the dt of step dt_seq, which the stream's kernels are bound to
+// deliver: if the stream ends or fails without it, so does the wait
+static double wait_dt(clover_chunk *c)
+{
+    for (long spins = 0;; spins++) {
+        if (__atomic_load_n(&c->dt_slot->seq, __ATOMIC_ACQUIRE) == c->dt_seq) return c->dt_slot->dtlp;
+        if (spins % 100000 == 99999) {
+            const hipError_t e = hipStreamQuery(c->st);
+            if (e == hipErrorNotReady) continue;
+            hip_check(e, "timestep");
+            if (__atomic_load_n(&c->dt_slot->seq, __ATOMIC_ACQUIRE) == c->dt_seq) return c->dt_slot->dtlp;
+            throw Error(E_HIP, "timestep: the stream ended without a dt");
+        }
+    }
+}
+
+// timestep.f90:93-126 from the tiles' minima.  Returns 1 on a small time step.
+static int take_dt(clover_chunk *c, const double *dtlp, int stride)
+{
+    const clover_deck &d = c->deck;
+    c->dt = c->g_big;
+    // timestep.f90:93-100: the minimum over tiles, ties to the last tile
+    for (int ti = 0; ti < (int)c->tiles.size(); ti++)
+        if (dtlp[stride * ti] <= c->dt) {
+            c->dt = dtlp[stride * ti];
+            c->dt_tile = ti;
+        }
+    double m = c->dt;
+    if (c->dtold * d.dtrise < m) m = c->dtold * d.dtrise;
+    if (d.dtmax < m) m = d.dtmax;
+    c->dt = m;
+    if (c->dt < d.dtmin) return 1;
+    c->dtold = c->dt;
+    return 0;
+}
+
+// timestep.f90:28-128; returns 1 on a small time step.  With ahead() the dt is
+// only enqueued, and the caller takes it (finish_step).
 static int timestep(clover_chunk *c)
 {
     int fields[NUM_FIELDS];
     const clover_deck &d = c->deck;
     const int T = (int)c->tiles.size();
-    c->dt = c->g_big;
     ideal_gas(c, false);
     if (c->fast) {
         fused_halo(c, FH_TIMESTEP);
@@ -692,6 +747,12 @@ static int timestep(clover_chunk *c)
                                           c->partial + (size_t)ti * kMaxPartials * 5, &nparts[ti % 64],
                                           c->shapes.k[SK_VISC_DT], c->st),
                       "visc_dt");
+            if (ahead(c)) {
+                hip_check(launch_dt_final(c->partial, nparts[0], c->g_big, c->dtold * d.dtrise, d.dtmax, d.dtmin,
+                                          dt_dev(c), c->dt_slot, ++c->dt_seq, c->st),
+                          "calc_dt min");
+                continue;
+            }
             hip_check(launch_min_final(c->partial + (size_t)ti * kMaxPartials * 5, nparts[ti % 64], c->g_big,
                                        c->scalar + 8 * ti, c->st),
                       "calc_dt min");
@@ -710,6 +771,7 @@ static int timestep(clover_chunk *c)
         set_fields(fields, {F_VISCOSITY});
         update_halo(c, fields, 1);
     }
+    if (ahead(c)) return 0;
     {
         Phase ph(c, P_TIMESTEP);
         if (!c->fast) {
@@ -729,22 +791,10 @@ static int timestep(clover_chunk *c)
         hip_check(hipMemcpyAsync(c->h_scalar, c->scalar, sizeof(double) * 8 * T, hipMemcpyDeviceToHost, c->st),
                   "dt D2H");
         hip_check(hipStreamSynchronize(c->st), "sync");
-        // timestep.f90:93-100: the minimum over tiles, ties to the last tile
-        for (int ti = 0; ti < T; ti++) {
-            const double dtlp = c->h_scalar[8 * ti];
-            if (dtlp <= c->dt) {
-                c->dt = dtlp;
-                c->dt_tile = ti;
-            }
-        }
     }
-    double m = c->dt;
-    if (c->dtold * d.dtrise < m) m = c->dtold * d.dtrise;
-    if (d.dtmax < m) m = d.dtmax;
-    c->dt = m;
-    if (c->dt < d.dtmin) return 1;
-    c->dtold = c->dt;
+    if (take_dt(c, c->h_scalar, 8)) return 1;
     if (c->batched) hip_check(batch_set_dt(c->tdev, T, c->dt, c->st), "set dt");
+    else if (c->fast) put_dt(c, c->dt);
     return 0;
 }
 
@@ -761,7 +811,7 @@ static void pdv(clover_chunk *c, bool predict)
                           "PdV predict");
             } else {
                 for (auto &t : c->tiles)
-                    hip_check(launch_fast_pdv_predict(c->store, t.g, c->geo, c->dt, t.f[F_DENSITY0],
+                    hip_check(launch_fast_pdv_predict(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0],
                                                       t.f[F_ENERGY0], t.f[F_PRESSURE], t.f[F_VISCOSITY],
                                                       t.f[F_XVEL0], t.f[F_YVEL0], t.f[F_ZVEL0],
                                                       c->shapes.k[SK_PDV_PREDICT], c->st),
@@ -815,7 +865,7 @@ static void advec_cell(clover_chunk *c, int sweep, int dir)
             // advec_cell sweep refreshes the halos before anything reads them)
             // the third sweep also writes the next step's ideal_gas pressure
             const bool last = sweep == 3;
-            hip_check(launch_fast_advec_cell(c->store, t.g, c->geo, c->advect_x, dir, sweep, t.f[F_DENSITY1], t.f[F_ENERGY1],
+            hip_check(launch_fast_advec_cell(c->store, dt_dev(c), t.g, c->geo, c->advect_x, dir, sweep, t.f[F_DENSITY1], t.f[F_ENERGY1],
                                              t.f[F_MASS_FLUX_X], t.f[F_VOL_FLUX_X], t.f[F_MASS_FLUX_Y],
                                              t.f[F_VOL_FLUX_Y], t.f[F_MASS_FLUX_Z], t.f[F_VOL_FLUX_Z], t.f[X_W1],
                                              t.f[X_W2], last ? t.f[F_PRESSURE] : nullptr,
@@ -856,7 +906,7 @@ static void advec_mom(clover_chunk *c, int sweep, int dir)
             // refreshed by the next update_halo before anything reads them)
             const void *vin[3] = {t.f[F_XVEL1], t.f[F_YVEL1], t.f[F_ZVEL1]};
             void *vout[3] = {t.f[X_W5], t.f[X_W6], t.f[X_W7]};
-            hip_check(launch_fast_advec_mom(c->store, t.g, c->geo, c->advect_x, sweep, dir, t.f[F_MASS_FLUX_X],
+            hip_check(launch_fast_advec_mom(c->store, dt_dev(c), t.g, c->geo, c->advect_x, sweep, dir, t.f[F_MASS_FLUX_X],
                                             t.f[F_VOL_FLUX_X], t.f[F_MASS_FLUX_Y], t.f[F_VOL_FLUX_Y],
                                             t.f[F_MASS_FLUX_Z], t.f[F_VOL_FLUX_Z], t.f[F_DENSITY1], vin, vout,
                                             c->shapes.k[SK_MOM_X + dir - 1], c->st),
@@ -995,15 +1045,15 @@ static void tune_launch(clover_chunk *c, int k)
             break;
         }
         case SK_PDV_PREDICT:
-            e = launch_fast_pdv_predict(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[F_ENERGY0], t.f[X_W3],
+            e = launch_fast_pdv_predict(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0], t.f[F_ENERGY0], t.f[X_W3],
                                         t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[F_YVEL0], t.f[F_ZVEL0], sh, c->st);
             break;
         case SK_ACCEL_PDV:
             e = lagrange_chunk(c) ?
-                launch_fast_lagrange(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
+                launch_fast_lagrange(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
                                      t.f[X_W2], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[X_W5], t.f[F_YVEL0], t.f[X_W6],
                                      t.f[F_ZVEL0], t.f[X_W7], t.f[X_W3], t.f[X_W4], t.f[X_W3], sh, c->st) :
-                launch_fast_accel_pdv(c->store, t.g, c->geo, c->dtold, t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
+                launch_fast_accel_pdv(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0], t.f[X_W1], t.f[F_ENERGY0],
                                       t.f[X_W2], t.f[F_PRESSURE], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[X_W5],
                                       t.f[F_YVEL0], t.f[X_W6], t.f[F_ZVEL0], t.f[X_W7], t.f[X_W3], t.f[X_W4],
                                       t.f[X_W3], sh, c->st);
@@ -1012,7 +1062,7 @@ static void tune_launch(clover_chunk *c, int k)
         case SK_CELL_Y:
         case SK_CELL_Z: {
             const int dir = k - SK_CELL_X + 1, sweep = dir == 2 ? 2 : 1;
-            e = launch_fast_advec_cell(c->store, t.g, c->geo, 1, dir, sweep, t.f[F_DENSITY1], t.f[F_ENERGY1],
+            e = launch_fast_advec_cell(c->store, dt_dev(c), t.g, c->geo, 1, dir, sweep, t.f[F_DENSITY1], t.f[F_ENERGY1],
                                        t.f[X_W3], t.f[F_VOL_FLUX_X], t.f[X_W3], t.f[F_VOL_FLUX_Y], t.f[X_W3],
                                        t.f[F_VOL_FLUX_Z], t.f[X_W1], t.f[X_W2], nullptr, sh, c->st);
             break;
@@ -1021,7 +1071,7 @@ static void tune_launch(clover_chunk *c, int k)
             const int dir = k - SK_MOM_X + 1, sweep = dir == 2 ? 2 : 1;
             const void *vin[3] = {t.f[F_XVEL1], t.f[F_YVEL1], t.f[F_ZVEL1]};
             void *vout[3] = {t.f[X_W5], t.f[X_W6], t.f[X_W7]};
-            e = launch_fast_advec_mom(c->store, t.g, c->geo, 1, sweep, dir, t.f[F_MASS_FLUX_X], t.f[F_VOL_FLUX_X],
+            e = launch_fast_advec_mom(c->store, dt_dev(c), t.g, c->geo, 1, sweep, dir, t.f[F_MASS_FLUX_X], t.f[F_VOL_FLUX_X],
                                       t.f[F_MASS_FLUX_Y], t.f[F_VOL_FLUX_Y], t.f[F_MASS_FLUX_Z], t.f[F_VOL_FLUX_Z],
                                       t.f[F_DENSITY1], vin, vout, sh, c->st);
             break;
@@ -1193,7 +1243,7 @@ static void do_step(clover_chunk *c)
         // accelerate, the corrector and flux_calc
         Phase ph(c, P_ACCEL);
         Tile &t = c->tiles[0];
-        hip_check(launch_fast_lagrange(c->store, t.g, c->geo, c->dt, t.f[F_DENSITY0], t.f[F_DENSITY1], t.f[F_ENERGY0],
+        hip_check(launch_fast_lagrange(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0], t.f[F_DENSITY1], t.f[F_ENERGY0],
                                        t.f[F_ENERGY1], t.f[F_VISCOSITY], t.f[F_XVEL0], t.f[F_XVEL1], t.f[F_YVEL0],
                                        t.f[F_YVEL1], t.f[F_ZVEL0], t.f[F_ZVEL1], t.f[F_VOL_FLUX_X],
                                        t.f[F_VOL_FLUX_Y], t.f[F_VOL_FLUX_Z], c->shapes.k[SK_ACCEL_PDV], c->st),
@@ -1207,7 +1257,7 @@ static void do_step(clover_chunk *c)
                       "accelerate + PdV correct + flux_calc");
         } else {
             for (auto &t : c->tiles)
-                hip_check(launch_fast_accel_pdv(c->store, t.g, c->geo, c->dt, t.f[F_DENSITY0], t.f[F_DENSITY1],
+                hip_check(launch_fast_accel_pdv(c->store, t.g, c->geo, dt_dev(c), t.f[F_DENSITY0], t.f[F_DENSITY1],
                                                 t.f[F_ENERGY0], t.f[F_ENERGY1], t.f[F_PRESSURE], t.f[F_VISCOSITY],
                                                 t.f[F_XVEL0], t.f[F_XVEL1], t.f[F_YVEL0], t.f[F_YVEL1],
                                                 t.f[F_ZVEL0], t.f[F_ZVEL1], t.f[F_VOL_FLUX_X], t.f[F_VOL_FLUX_Y],
@@ -1262,7 +1312,38 @@ static void do_step(clover_chunk *c)
         }
     }
     c->advect_x = !c->advect_x;
+}
+
+// hydro.f90:48-68: one step.  Returns 1 on a small time step, which leaves the
+// level-0 state as it was.
+static int hydro_step(clover_chunk *c)
+{
+    c->step = c->step + 1;
+    if (!ahead(c)) {
+        if (timestep(c)) return 1;
+        do_step(c);
+    } else {
+        // what a step that turns out small gives back: the roles its sweeps
+        // exchanged (its kernels do nothing then)
+        Tile &t = c->tiles[0];
+        double *f[NUM_ARRAYS];
+        std::copy(t.f, t.f + NUM_ARRAYS, f);
+        const int advect_x = c->advect_x;
+        timestep(c);
+        const bool gas_fresh = c->gas_fresh, sound_fresh = c->sound_fresh;
+        do_step(c);
+        const double dtlp = wait_dt(c);
+        if (take_dt(c, &dtlp, 0)) {
+            std::copy(f, f + NUM_ARRAYS, t.f);
+            c->advect_x = advect_x;
+            c->gas_fresh = gas_fresh;
+            c->sound_fresh = sound_fresh;
+            put_dt(c, c->dtold);
+            return 1;
+        }
+    }
     c->time = c->time + c->dt;
+    return 0;
 }
 
 static void destroy(clover_chunk *c)
@@ -1284,6 +1365,7 @@ static void destroy(clover_chunk *c)
     if (c->partial) (void)hipFree(c->partial);
     if (c->scalar) (void)hipFree(c->scalar);
     if (c->h_scalar) (void)hipHostFree(c->h_scalar);
+    if (c->dt_slot) (void)hipHostFree(c->dt_slot);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     delete c->ktimer;
@@ -1337,6 +1419,9 @@ int clover_chunk_create_ex(const clover_deck *deck, int device, int flags, clove
         c->partial = dev_alloc(c, (size_t)T * kMaxPartials * 5);
         c->scalar = dev_alloc(c, (size_t)T * 8);
         hip_check(hipHostMalloc(&c->h_scalar, sizeof(double) * 8 * T, hipHostMallocDefault), "hipHostMalloc");
+        hip_check(hipHostMalloc(&c->dt_slot, sizeof(DtSlot), hipHostMallocCoherent), "hipHostMalloc");
+        c->dt_slot->seq = c->dt_seq = 0;
+        put_dt(c, d.dtinit);
         bool thin = false;
         for (auto &t : c->tiles) thin = thin || t.nx < 3 || t.ny < 3 || t.nz < 3;
         for (auto &t : c->tiles) {
@@ -1424,14 +1509,12 @@ int clover_chunk_step(clover_chunk *c, double *dt)
     CLOVER_API_BEGIN
     if (!c) throw Error(E_ARG, "null chunk");
     KTIMER_SCOPE(c);
-    c->step = c->step + 1;
-    if (timestep(c)) {
-        if (dt) *dt = c->dt;
+    const int small = hydro_step(c);
+    if (dt) *dt = c->dt;
+    if (small) {
         set_last_error("timestep: small timestep");
         return 1;
     }
-    do_step(c);
-    if (dt) *dt = c->dt;
     CLOVER_API_END
 }
 
@@ -1475,13 +1558,11 @@ int clover_chunk_run(clover_chunk *c, int max_steps, clover_summary *rows, int m
         n++;
     };
     for (int it = 0; it < max_steps; it++) {
-        c->step = c->step + 1;
-        if (timestep(c)) {
+        if (hydro_step(c)) {
             if (nrows) *nrows = n < max_rows ? n : max_rows;
             set_last_error("timestep: small timestep");
             return 1;
         }
-        do_step(c);
         if (d.summary_frequency != 0 && c->step % d.summary_frequency == 0) summary_row();
         if (c->time + c->g_small > d.end_time || c->step >= d.end_step) {
             summary_row();

@@ -537,11 +537,13 @@ __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo 
 }
 
 template <typename S>
-__global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, Geo m, double dt, const S *__restrict__ density0, const S *__restrict__ energy0,
+__global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, const S *__restrict__ energy0,
                    S *__restrict__ pressure, const S *__restrict__ viscosity,
                    const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                    const S *__restrict__ zvel0)
 {
+    const double dt = *dtp;
+    if (dt < 0.0) return;
     if constexpr (sizeof(S) == 4)
         pdv_predict_pair_body(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
     else
@@ -549,7 +551,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, 
 }
 
 template <typename S>
-static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, double dt, const S *density0,
+static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, const double *dt, const S *density0,
                                    const S *energy0, S *pressure, const S *viscosity,
                                    const S *xvel0, const S *yvel0, const S *zvel0, const Shape &sh, hipStream_t st)
 {
@@ -921,19 +923,21 @@ __device__ __forceinline__ void accel_pdv_body(const Blk &bk, Lay g, Geo m, doub
 
 template <typename S>
 __global__ void __launch_bounds__(64 * AW, sizeof(S) == 4 ? 6 : 1)
-    k_fast_accel_pdv(int xcd, Lay g, Geo m, double dt, const S *__restrict__ density0, S *__restrict__ density1,
+    k_fast_accel_pdv(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
                      const S *__restrict__ energy0, S *__restrict__ energy1, const S *__restrict__ pressure,
                      const S *__restrict__ viscosity, const S *__restrict__ xvel0, S *__restrict__ xvel1,
                      const S *__restrict__ yvel0, S *__restrict__ yvel1, const S *__restrict__ zvel0,
                      S *__restrict__ zvel1, S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y,
                      S *__restrict__ vol_flux_z)
 {
+    const double dt = *dtp;
+    if (dt < 0.0) return;
     accel_pdv_body<S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, pressure, viscosity, xvel0, xvel1,
                       yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
 }
 
 template <typename S>
-static hipError_t fast_accel_pdv_t(const Lay &g, const Geo &m, double dt, const S *density0, S *density1,
+static hipError_t fast_accel_pdv_t(const Lay &g, const Geo &m, const double *dt, const S *density0, S *density1,
                                    const S *energy0, S *energy1, const S *pressure, const S *viscosity,
                                    const S *xvel0, S *xvel1, const S *yvel0, S *yvel1, const S *zvel0, S *zvel1,
                                    S *vol_flux_x, S *vol_flux_y, S *vol_flux_z, const Shape &sh, hipStream_t st)
@@ -973,7 +977,7 @@ hipError_t launch_fast_visc_dt(Store s, const Lay &g, const Geo &m, double dtc_s
 #undef CALL
 }
 
-hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, double dt, const void *density0,
+hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
                                    const void *energy0, void *pressure, const void *viscosity, const void *xvel0,
                                    const void *yvel0, const void *zvel0, const Shape &sh, hipStream_t st)
 {
@@ -984,7 +988,7 @@ hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, double d
 #undef CALL
 }
 
-hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, double dt, const void *density0,
+hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
                                  void *density1, const void *energy0, void *energy1, const void *pressure,
                                  const void *viscosity, const void *xvel0, void *xvel1, const void *yvel0,
                                  void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,

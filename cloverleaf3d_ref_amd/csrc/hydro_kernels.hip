@@ -224,8 +224,7 @@ hipError_t launch_calc_dt_cells(const Lay &g, double dtc_safe, double dtu_safe, 
 // loads are in flight at a time.  The minimum does not depend on the order.
 constexpr int MIN_THREADS = 1024;
 
-__global__ void __launch_bounds__(MIN_THREADS) k_min_final(const double *__restrict__ partial, int n, double seed,
-                                                           double *__restrict__ out)
+__device__ inline double min_of_partials(const double *__restrict__ partial, int n, double seed)
 {
     double m0 = seed, m1 = seed, m2 = seed, m3 = seed;
     int c = threadIdx.x;
@@ -243,11 +242,39 @@ __global__ void __launch_bounds__(MIN_THREADS) k_min_final(const double *__restr
     m = wave_min(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double b = red[0];
-        for (int w = 1; w < MIN_THREADS / 64; w++) b = dmin(b, red[w]);
-        *out = b;
-    }
+    double b = red[0];
+    for (int w = 1; w < MIN_THREADS / 64; w++) b = dmin(b, red[w]);
+    return b;
+}
+
+__global__ void __launch_bounds__(MIN_THREADS) k_min_final(const double *__restrict__ partial, int n, double seed,
+                                                           double *__restrict__ out)
+{
+    const double b = min_of_partials(partial, n, seed);
+    if (threadIdx.x == 0) *out = b;
+}
+
+__global__ void __launch_bounds__(MIN_THREADS) k_dt_final(const double *__restrict__ partial, int n, double g_big,
+                                                          double dt_rise, double dtmax, double dtmin,
+                                                          double *__restrict__ dt, DtSlot *host, unsigned long long seq)
+{
+    const double b = min_of_partials(partial, n, g_big);
+    if (threadIdx.x) return;
+    double m = g_big;
+    if (b <= m) m = b;
+    if (dt_rise < m) m = dt_rise;
+    if (dtmax < m) m = dtmax;
+    *dt = m < dtmin ? -1.0 : m;
+    host->dtlp = b;
+    __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_dt_final(const double *partial, int n, double g_big, double dt_rise, double dtmax, double dtmin,
+                           double *dt, DtSlot *host, unsigned long long seq, hipStream_t st)
+{
+    TIMED_LAUNCH("k_dt_final", st, k_dt_final, dim3(1), dim3(MIN_THREADS), 0, st, partial, n, g_big, dt_rise, dtmax,
+                 dtmin, dt, host, seq);
+    return hipGetLastError();
 }
 
 hipError_t launch_min_final(const double *partial, int n, double seed, double *out, hipStream_t st)

@@ -36,6 +36,19 @@ hipError_t launch_calc_dt_cells(const Lay &g, double dtc_safe, double dtu_safe, 
 // min over partial[0..n) seeded with `seed`, into *out (device scalar)
 hipError_t launch_min_final(const double *partial, int n, double seed, double *out, hipStream_t st);
 
+// Where a resident step's calc_dt minimum reaches the host: pinned memory that
+// the GPU writes, seq last
+struct DtSlot {
+    double dtlp;
+    unsigned long long seq;
+};
+// timestep.f90:86-126 for one tile on the device: the minimum of the partials
+// (seeded with g_big) goes to `host` (tagged seq) and the step's dt, min(dtlp,
+// dt_rise, dtmax), to *dt; -1 there when it lies below dtmin, which the step's
+// first kernel takes as nothing to do
+hipError_t launch_dt_final(const double *partial, int n, double g_big, double dt_rise, double dtmax, double dtmin,
+                           double *dt, DtSlot *host, unsigned long long seq, hipStream_t st);
+
 hipError_t launch_pdv(int predict, const Lay &g, double dt, const double *xarea, const double *yarea,
                       const double *zarea, const double *volume, const double *density0, double *density1,
                       const double *energy0, double *energy1, const double *pressure, const double *viscosity,

@@ -724,10 +724,11 @@ __device__ __forceinline__ void mom_march(int lin, int gx, int gy, int gz, int x
 }
 
 template <int DIR, int MODE, typename S>
-__global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fast_mom_march(int xcd, Lay g, Geo geo, const S *__restrict__ mf, const S *__restrict__ vfx,
+__global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fast_mom_march(const double *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf, const S *__restrict__ vfx,
                  const S *__restrict__ vfy, const S *__restrict__ vfz,
                  const S *__restrict__ density1, Vel3<S> v)
 {
+    if (*dt < 0.0) return;  // a small step (launch_dt_final)
     const int gx = (int)gridDim.x, gy = (int)gridDim.y, gz = (int)gridDim.z;
     mom_march<DIR, MODE, S>((int)blockIdx.x + gx * ((int)blockIdx.y + gy * (int)blockIdx.z), gx, gy, gz, xcd, g, geo,
                             mf, vfx, vfy, vfz, density1, v);
@@ -829,10 +830,11 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mo
 }
 
 template <typename S>
-__global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1) k_fast_mom_x(int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
+__global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1) k_fast_mom_x(const double *__restrict__ dt, int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
              const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1,
              Vel3<S> v)
 {
+    if (*dt < 0.0) return;
     mom_x_body<S>(hw_blk(xcd), g, geo, mode, mf, vfx, vfy, vfz, density1, v);
 }
 
@@ -847,7 +849,7 @@ static int mom_mode(int advect_x, int sweep_number, int direction)
 }
 
 template <typename S>
-static hipError_t fast_advec_mom_t(const Lay &g, const Geo &m, int mode, int direction, const S *mass_flux_x,
+static hipError_t fast_advec_mom_t(const double *dt, const Lay &g, const Geo &m, int mode, int direction, const S *mass_flux_x,
                                    const S *vol_flux_x, const S *mass_flux_y, const S *vol_flux_y,
                                    const S *mass_flux_z, const S *vol_flux_z, const S *density1,
                                    const void *const *vel_in, void *const *vel_out, const Shape &sh, hipStream_t st)
@@ -862,23 +864,23 @@ static hipError_t fast_advec_mom_t(const Lay &g, const Geo &m, int mode, int dir
     const dim3 blk(64, MW, 1);
     if (direction == 1) {
         const dim3 grid((nxn + 59) / 60, (nyn + MW - 2) / (MW - 1), nchunks(nzn, sh.planes));
-        TIMED_LAUNCH("k_fast_mom_x", st, k_fast_mom_x<S>, grid, blk, 0, st, sh.xcd, g, m, mode, mass_flux_x, vol_flux_x,
+        TIMED_LAUNCH("k_fast_mom_x", st, k_fast_mom_x<S>, grid, blk, 0, st, dt, sh.xcd, g, m, mode, mass_flux_x, vol_flux_x,
                      vol_flux_y, vol_flux_z, density1, v);
     } else if (direction == 2) {
         const dim3 grid((nxn + 63) / 64, (nzn + MW - 2) / (MW - 1), nchunks(nyn, sh.planes));
         const auto kern = mode == 3 ? k_fast_mom_march<2, 3, S> : k_fast_mom_march<2, 4, S>;
-        TIMED_LAUNCH("k_fast_mom_y", st, kern, grid, blk, 0, st, sh.xcd, g, m, mass_flux_y, vol_flux_x, vol_flux_y,
+        TIMED_LAUNCH("k_fast_mom_y", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, mass_flux_y, vol_flux_x, vol_flux_y,
                      vol_flux_z, density1, v);
     } else {
         const dim3 grid((nxn + 63) / 64, (nyn + MW - 2) / (MW - 1), nchunks(nzn, sh.planes));
         const auto kern = mode == 2 ? k_fast_mom_march<3, 2, S> : k_fast_mom_march<3, 6, S>;
-        TIMED_LAUNCH("k_fast_mom_z", st, kern, grid, blk, 0, st, sh.xcd, g, m, mass_flux_z, vol_flux_x, vol_flux_y,
+        TIMED_LAUNCH("k_fast_mom_z", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, mass_flux_z, vol_flux_x, vol_flux_y,
                      vol_flux_z, density1, v);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_fast_advec_mom(Store s, const Lay &g, const Geo &m, int advect_x, int sweep_number,
+hipError_t launch_fast_advec_mom(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int sweep_number,
                                  int direction, const void *mass_flux_x, const void *vol_flux_x,
                                  const void *mass_flux_y, const void *vol_flux_y, const void *mass_flux_z,
                                  const void *vol_flux_z, const void *density1, const void *const *vel_in,
@@ -887,7 +889,7 @@ hipError_t launch_fast_advec_mom(Store s, const Lay &g, const Geo &m, int advect
     const int mode = mom_mode(advect_x, sweep_number, direction);
     if (!mode) return hipErrorInvalidValue;  // the resident driver issues only the reference's sweeps
 #define CALL(T)                                                                                                 \
-    fast_advec_mom_t<T>(g, m, mode, direction, static_cast<const T *>(mass_flux_x),                             \
+    fast_advec_mom_t<T>(dt, g, m, mode, direction, static_cast<const T *>(mass_flux_x),                             \
                         static_cast<const T *>(vol_flux_x), static_cast<const T *>(mass_flux_y),                \
                         static_cast<const T *>(vol_flux_y), static_cast<const T *>(mass_flux_z),                \
                         static_cast<const T *>(vol_flux_z), static_cast<const T *>(density1), vel_in, vel_out, sh, st)
