@@ -31,24 +31,9 @@ namespace clover {
 
 constexpr int CROWS = 4;   // rows (or columns) per workgroup
 
-// pre_vol (advec_cell_kernel.f90:97-116, 193-210, 289-306) for `mode`:
+// pre_vol (advec_cell_kernel.f90:97-116, 193-210, 289-306) has a `mode`:
 // 1 x sweep 1, 2 x sweep 3, 3 y sweep with advect_x, 4 y without,
 // 5 z sweep 1, 6 z sweep 3
-template <typename S>
-__device__ inline double cell_pre_vol(int mode, const Lay &g, int i, double V0, const S *__restrict__ vfx,
-                                      const S *__restrict__ vfy, const S *__restrict__ vfz)
-{
-#define D(x) ((double)(x))
-    switch (mode) {
-    case 1:
-    case 5: return V0 + (D(vfx[i + 1]) - D(vfx[i]) + D(vfy[i + g.ld]) - D(vfy[i]) + D(vfz[i + g.plane]) - D(vfz[i]));
-    case 2: return V0 + D(vfx[i + 1]) - D(vfx[i]);
-    case 3: return V0 + D(vfy[i + g.ld]) - D(vfy[i]) + D(vfz[i + g.plane]) - D(vfz[i]);
-    case 4: return V0 + D(vfy[i + g.ld]) - D(vfy[i]) + D(vfx[i + 1]) - D(vfx[i]);
-    default: return V0 + D(vfz[i + g.plane]) - D(vfz[i]);
-    }
-#undef D
-}
 
 template <typename T>
 __device__ inline T cell_limiter(T sigma, T sigma3, T sigma4, T diffuw, T diffdw)
@@ -187,59 +172,25 @@ __global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const double *__rest
                    p_out);
 }
 
-// The volume fluxes pre_vol reads for the y and z sweeps (modes 3-6), kept
-// raw so a face's loads can be issued a step ahead of their use.
-template <typename S>
-struct PreRaw {
-    S a, b, c, d, e, f;  // storage type: converted where used, so the loads stay in flight
-};
-
-template <typename S>
-__device__ inline PreRaw<S> load_pre_raw(int mode, const Lay &g, int i, const S *__restrict__ vfx,
-                                         const S *__restrict__ vfy, const S *__restrict__ vfz)
-{
-    PreRaw<S> r{0, 0, 0, 0, 0, 0};
-    switch (mode) {
-    case 3: r.a = vfy[i + g.ld]; r.b = vfy[i]; r.c = vfz[i + g.plane]; r.d = vfz[i]; break;
-    case 4: r.a = vfy[i + g.ld]; r.b = vfy[i]; r.c = vfx[i + 1]; r.d = vfx[i]; break;
-    case 5:
-        r.a = vfx[i + 1]; r.b = vfx[i]; r.c = vfy[i + g.ld]; r.d = vfy[i]; r.e = vfz[i + g.plane]; r.f = vfz[i];
-        break;
-    default: r.a = vfz[i + g.plane]; r.b = vfz[i]; break;
-    }
-    return r;
-}
-
-// cell_pre_vol's expressions for modes 3-6 on the raw values
-template <typename S>
-__device__ inline double pre_of_raw(int mode, double V0, const PreRaw<S> &r)
-{
-    const double a = r.a, b = r.b, c = r.c, d = r.d, e = r.e, f = r.f;
-    switch (mode) {
-    case 3:
-    case 4: return V0 + a - b + c - d;
-    case 5: return V0 + (a - b + c - d + e - f);
-    default: return V0 + a - b;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // y and z sweeps: lanes along x (interior j), threadIdx.y along the cross
 // axis, march along the sweep axis over faces [smin, smax+2] in chunks.
 // Faces of the y sweep run over l in [z_min, z_max+2] (advec_cell_kernel.f90:
-// 215-217); the cells updated are interior.
-template <int DIR, typename S>
-__device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
+// 215-217); the cells updated are interior.  MODE: pre_vol's,
+// 3-6.  Row addresses are scalar (the wave's cross row and the face), a
+// lane adds a byte offset; density and energy across a mirrored face are read
+// at the interior cell.
+template <int DIR, int MODE, typename S>
+__device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
     const int j = g.x_min + (int)(bk.x * 64 + threadIdx.x);
-    const int cr = (DIR == 3 ? g.y_min : g.z_min) + (int)(bk.y * CROWS + threadIdx.y);
+    const int cr = (DIR == 3 ? g.y_min : g.z_min) + bk.y * CROWS + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int crmax = DIR == 3 ? g.y_max : g.z_max + 2;  // last cross position with faces
     if (j > g.x_max || cr > crmax) return;                 // no cross-lane traffic in this kernel
     const bool cross_in = DIR == 3 || cr <= g.z_max;       // updates only on interior cells
-    const int s = DIR == 3 ? g.plane : g.ld;
     const int smin = DIR == 3 ? g.z_min : g.y_min, smax = DIR == 3 ? g.z_max : g.y_max;
     using T = S;  // arithmetic type of the fluxes
     const T vd = (T)(DIR == 3 ? m.dz : m.dy);
@@ -247,43 +198,76 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, int
     int f0, f1;
     chunk_range(bk, smin, smax + 2, f0, f1);
     if (f0 > f1) return;
-    const int ib = DIR == 3 ? idx(g, j, cr, smin) : idx(g, j, smin, cr);  // offset at sweep position smin
-#define OFF(q) (ib + ((q) - smin) * s)
-    auto pre = [&](int q) { return cell_pre_vol(mode, g, OFF(q), m.vol, vfx, vfy, vfz); };
+    unsigned oj = (unsigned)(j - g.x_min) * (unsigned)sizeof(S);
+    auto row = [&](int q) { return (int64_t)(DIR == 3 ? idx(g, g.x_min, cr, q) : idx(g, g.x_min, q, cr)); };
+    const int crc = DIR == 3 ? cr : cell_m(g, 2, cr);
+    auto cell = [&](const S *__restrict__ p, int q) -> S {  // density or energy
+        const int qc = cell_m(g, DIR - 1, q);
+        return at(p + (int64_t)(DIR == 3 ? idx(g, g.x_min, crc, qc) : idx(g, g.x_min, qc, crc)), oj);
+    };
+    // pre_vol's volume fluxes of the cell at q, raw (converted where used, so
+    // that a face's loads can be issued a step ahead of their use)
+    struct Pre {
+        S v[MODE == 5 ? 6 : MODE == 6 ? 2 : 4];
+    };
+    auto load_pre = [&](int q) {
+        const int64_t r = row(q);
+        Pre x;
+        int n = 0;
+        auto pair = [&](const S *__restrict__ p, int up) {
+            x.v[n++] = at(p + r + up, oj);
+            x.v[n++] = at(p + r, oj);
+        };
+        if constexpr (MODE == 5) pair(vfx, 1);
+        if constexpr (MODE == 5 || MODE == 3 || MODE == 4) pair(vfy, g.ld);
+        if constexpr (MODE == 4) pair(vfx, 1);
+        if constexpr (MODE != 4) pair(vfz, g.plane);
+        return x;
+    };
+    // its expressions
+    auto pre_of = [&](const Pre &x) -> double {
+#define D(i) ((double)x.v[i])
+        if constexpr (MODE == 5) return m.vol + (D(0) - D(1) + D(2) - D(3) + D(4) - D(5));
+        else if constexpr (MODE == 6) return m.vol + D(0) - D(1);
+        else return m.vol + D(0) - D(1) + D(2) - D(3);
+#undef D
+    };
 
     // window of old values at f-2, f-1, f, f+1 and pre_vol at f-1, f
-    T r_m2 = density1[OFF(f0 - 2)], r_m1 = density1[OFF(f0 - 1)], r_0 = density1[OFF(f0)];
-    T e_m2 = energy1[OFF(f0 - 2)], e_m1 = energy1[OFF(f0 - 1)], e_0 = energy1[OFF(f0)];
-    double pv_m1 = pre(f0 - 1);
+    T r_m2 = cell(density1, f0 - 2), r_m1 = cell(density1, f0 - 1), r_0 = cell(density1, f0);
+    T e_m2 = cell(energy1, f0 - 2), e_m1 = cell(energy1, f0 - 1), e_0 = cell(energy1, f0);
+    const Pre pr_m1 = load_pre(f0 - 1);
+    // face f0's loads; each step issues the next face's before its arithmetic
+    S vf_n = at(vfs + row(f0), oj);
+    Pre pr_n = load_pre(f0);
+    S r_n = (S)0, e_n = (S)0;  // upwind for vf <= 0 is min(f+1, smax+2)
+    if (f0 + 1 <= smax + 2) {
+        r_n = cell(density1, f0 + 1);
+        e_n = cell(energy1, f0 + 1);
+    }
+    double pv_m1 = pre_of(pr_m1);
     // flux of face f0-1, needed when cell f0-1 is updated here (f0 > smin)
     T mf_lo = 0, ef_lo = 0, vf_lo = 0;
     if (f0 > smin) {
-        vf_lo = vfs[OFF(f0 - 1)];
-        const T r_m3 = density1[OFF(f0 - 3)], e_m3 = energy1[OFF(f0 - 3)];
+        vf_lo = at(vfs + row(f0 - 1), oj);
+        const T r_m3 = cell(density1, f0 - 3), e_m3 = cell(energy1, f0 - 3);
+        const double pv_m2 = pre_of(load_pre(f0 - 2));
         if (vf_lo > (T)0)
-            cell_face_flux(vf_lo, (T)pre(f0 - 2), vd, r_m3, r_m2, r_m1, e_m3, e_m2, e_m1, mf_lo, ef_lo);
+            cell_face_flux(vf_lo, (T)pv_m2, vd, r_m3, r_m2, r_m1, e_m3, e_m2, e_m1, mf_lo, ef_lo);
         else
             cell_face_flux(vf_lo, (T)pv_m1, vd, r_0, r_m1, r_m2, e_0, e_m1, e_m2, mf_lo, ef_lo);  // f0 <= smax+1
     }
-    // face f0's loads; each step issues the next face's before its arithmetic
-    S vf_n = vfs[OFF(f0)];
-    PreRaw<S> pr_n = load_pre_raw(mode, g, OFF(f0), vfx, vfy, vfz);
-    S r_n = (S)0, e_n = (S)0;  // upwind for vf <= 0 is min(f+1, smax+2)
-    if (f0 + 1 <= smax + 2) {
-        r_n = density1[OFF(f0 + 1)];
-        e_n = energy1[OFF(f0 + 1)];
-    }
     for (int f = f0; f <= f1; f++) {
-        const int i = OFF(f);
+        asm volatile("" : "+v"(oj));  // no array + offset hoisted into vector registers
         const T vf = vf_n;
-        const double pv_0 = pre_of_raw(mode, m.vol, pr_n);
+        const double pv_0 = pre_of(pr_n);
         const T r_p1 = f + 1 <= smax + 2 ? r_n : r_0, e_p1 = f + 1 <= smax + 2 ? e_n : e_0;
         if (f < f1) {
-            vf_n = vfs[OFF(f + 1)];
-            pr_n = load_pre_raw(mode, g, OFF(f + 1), vfx, vfy, vfz);
+            vf_n = at(vfs + row(f + 1), oj);
+            pr_n = load_pre(f + 1);
             if (f + 2 <= smax + 2) {
-                r_n = density1[OFF(f + 2)];
-                e_n = energy1[OFF(f + 2)];
+                r_n = cell(density1, f + 2);
+                e_n = cell(energy1, f + 2);
             }
         }
         T mf, ef;
@@ -291,15 +275,16 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, int
             cell_face_flux(vf, (T)pv_m1, vd, r_m2, r_m1, r_0, e_m2, e_m1, e_0, mf, ef);
         else
             cell_face_flux(vf, (T)pv_0, vd, r_p1, r_0, r_m1, e_p1, e_0, e_m1, mf, ef);
-        mass_flux[i] = mf;
+        at(mass_flux + row(f), oj) = mf;
         const int c = f - 1;  // cell between faces f-1 and f
         if (cross_in && c >= smin && c <= smax) {
             double rn, en;
             cell_update(r_m1, e_m1, pv_m1, mf_lo, mf, ef_lo, ef, vf_lo, vf, rn, en);
             const S rs = (S)rn, es = (S)en;
-            rho_out[OFF(c)] = rs;
-            e_out[OFF(c)] = es;
-            if (p_out) p_out[OFF(c)] = pressure_of<S>(rs, es);
+            const int64_t rc = row(c);
+            at(rho_out + rc, oj) = rs;
+            at(e_out + rc, oj) = es;
+            if (p_out) at(p_out + rc, oj) = pressure_of<S>(rs, es);
         }
         mf_lo = mf;
         ef_lo = ef;
@@ -312,18 +297,17 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, int
         e_0 = e_p1;
         pv_m1 = pv_0;
     }
-#undef OFF
 }
 
-template <int DIR, typename S>
-__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
+template <int DIR, int MODE, typename S>
+__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
     if (*dt < 0.0) return;
-    cell_march_body<DIR, S>(hw_blk(xcd), g, m, mode, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
-                            p_out);
+    cell_march_body<DIR, MODE, S>(hw_blk(xcd), g, m, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
+                                  p_out);
 }
 
 template <typename S>
@@ -341,12 +325,12 @@ static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m
                      vol_flux_z, density1, energy1, mass_flux_x, rho_out, e_out, p_out, rows);
     } else if (dir == 2) {
         const dim3 grid((nx + 63) / 64, (nz + 2 + CROWS - 1) / CROWS, nchunks(ny + 2, sh.planes));
-        TIMED_LAUNCH("k_fast_cell_y", st, (k_fast_cell_march<2, S>), grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x,
-                     vol_flux_y, vol_flux_z, density1, energy1, mass_flux_y, rho_out, e_out, p_out);
+        const auto kern = mode == 3 ? k_fast_cell_march<2, 3, S> : k_fast_cell_march<2, 4, S>;
+        TIMED_LAUNCH("k_fast_cell_y", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_y, rho_out, e_out, p_out);
     } else {
         const dim3 grid((nx + 63) / 64, (ny + CROWS - 1) / CROWS, nchunks(nz + 2, sh.planes));
-        TIMED_LAUNCH("k_fast_cell_z", st, (k_fast_cell_march<3, S>), grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x,
-                     vol_flux_y, vol_flux_z, density1, energy1, mass_flux_z, rho_out, e_out, p_out);
+        const auto kern = mode == 5 ? k_fast_cell_march<3, 5, S> : k_fast_cell_march<3, 6, S>;
+        TIMED_LAUNCH("k_fast_cell_z", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_z, rho_out, e_out, p_out);
     }
     return hipGetLastError();
 }
@@ -400,7 +384,7 @@ int batch_blocks_cell(int dir, const Lay &g, int planes)
     return gx * gy * gz;
 }
 
-template <int DIR, typename S>
+template <int DIR, int MODE, typename S>  // MODE: 0 for the x sweep, which takes `mode`
 __global__ void __launch_bounds__(64 * CROWS)
 kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int gas, int planes,
         int xcd, CellSlots cs)
@@ -420,7 +404,7 @@ kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd
             cell_x_body<S>(bk, D.g, D.m, mode, cell_x_rows(planes), CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z), CF(cs.rho),
                            CF(cs.e), MF(F_MASS_FLUX_X), MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
         else
-            cell_march_body<DIR, S>(bk, D.g, D.m, mode, CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z),
+            cell_march_body<DIR, MODE, S>(bk, D.g, D.m, CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z),
                                     CF(cs.rho), CF(cs.e), MF(DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z),
                                     MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
 #undef CF
@@ -441,14 +425,21 @@ hipError_t batch_advec_cell(Store s, const DeckDev *decks, int nd, const BatchGr
     const dim3 grid(batch_wgs(bg, sh)), blk(64, CROWS);
     const CellSlots cs{sl[F_DENSITY1], sl[F_ENERGY1], sl[X_W1], sl[X_W2]};
     if (gas && sweep_number != 3) return hipErrorInvalidValue;
-#define L(D_, T_)                                                                                          \
-    TIMED_LAUNCH("kb_cell", st, (kb_cell<D_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, gas ? 1 : 0,   \
+#define L(D_, M_, T_)                                                                                         \
+    TIMED_LAUNCH("kb_cell", st, (kb_cell<D_, M_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, gas ? 1 : 0, \
                  sh.planes, sh.xcd, cs)
+#define LM(T_)                                                                                                \
+    if (dir == 1) L(1, 0, T_);                                                                                \
+    else if (mode == 3) L(2, 3, T_);                                                                          \
+    else if (mode == 4) L(2, 4, T_);                                                                          \
+    else if (mode == 5) L(3, 5, T_);                                                                          \
+    else L(3, 6, T_)
     if (s == ST_F32) {
-        if (dir == 1) L(1, float); else if (dir == 2) L(2, float); else L(3, float);
+        LM(float);
     } else {
-        if (dir == 1) L(1, double); else if (dir == 2) L(2, double); else L(3, double);
+        LM(double);
     }
+#undef LM
 #undef L
     return hipGetLastError();
 }

@@ -93,13 +93,10 @@ void host_init(const clover_deck &d, const Tile &t, HostInit &h, bool fields = t
 //   halo (the value the reflection would write there, sign flip included),
 //   so those fields' reflections on those axes are left out of every
 //   exchange (raxes; the tile copies of internal faces stay, axes):
-//   visc_dt and accel_pdv mirror every axis (level-0 fields, viscosity,
-//   pressure), the advection sweeps the x axis (level-1 fields; along y
-//   and z the address arithmetic cost them more than the exchanges).  The
-//   face fields keep their exchanges, except vol_flux_y/z and mass_flux_y/z
-//   across x (launch.h tan_xm): some of their corner halos hold reflections of
-//   values the other passes had not yet refreshed, which only the exchange
-//   itself reproduces.
+//   every axis.  The face fields keep their exchanges, except vol_flux_y/z and
+//   mass_flux_y/z across x (launch.h tan_xm): some of their corner halos hold
+//   reflections of values the other passes had not yet refreshed, which only
+//   the exchange itself reproduces.
 enum FusedHalo : int { FH_TIMESTEP, FH_VISCOSITY, FH_PRESSURE, FH_CELL1, FH_MOM1, FH_CELL2, FH_MOM2, FH_MOM3 };
 
 enum : int { AX_X = 1, AX_Y = 2, AX_Z = 4, AX_ALL = 7 };
@@ -147,9 +144,8 @@ inline int mirror_axes(const Lay &g)
     return ((g.mirror & 3) == 3 ? AX_X : 0) | ((g.mirror & 12) == 12 ? AX_Y : 0) | ((g.mirror & 48) == 48 ? AX_Z : 0);
 }
 
-// mirror_axes: the axes whose faces the fused kernels mirror: their level-0
-// fields everywhere, level-1 ones and, by launch.h tan_xm, vol_flux_y/z and
-// mass_flux_y/z across x
+// mirror_axes: the axes whose faces the fused kernels mirror for cell and vertex
+// fields, and across x, by launch.h tan_xm, for vol_flux_y/z and mass_flux_y/z
 inline HaloPlan fused_halo_plan(int which, bool advect_x, int mirror_axes = 0)
 {
     HaloPlan p{};
@@ -200,9 +196,9 @@ inline HaloPlan fused_halo_plan(int which, bool advect_x, int mirror_axes = 0)
     default: mom(s3); break;
     }
     for (int f = 0; f < NUM_FIELDS; f++) p.raxes[f] = p.axes[f];
-    for (int f : {F_DENSITY0, F_ENERGY0, F_PRESSURE, F_VISCOSITY, F_SOUNDSPEED, F_XVEL0, F_YVEL0, F_ZVEL0})
+    for (int f : {F_DENSITY0, F_ENERGY0, F_PRESSURE, F_VISCOSITY, F_SOUNDSPEED, F_XVEL0, F_YVEL0, F_ZVEL0, F_DENSITY1,
+                  F_ENERGY1, F_XVEL1, F_YVEL1, F_ZVEL1})
         p.raxes[f] &= ~mirror_axes;
-    for (int f : {F_DENSITY1, F_ENERGY1, F_XVEL1, F_YVEL1, F_ZVEL1}) p.raxes[f] &= ~(mirror_axes & AX_X);
     for (int f : {F_VOL_FLUX_Y, F_VOL_FLUX_Z, F_MASS_FLUX_Y, F_MASS_FLUX_Z}) p.raxes[f] &= ~(mirror_axes & AX_X);
     return p;
 }

@@ -72,18 +72,6 @@ __host__ __device__ inline void dims_lagrange(const Lay &g, int lw, int planes, 
     gz = nchunks(g.z_max - g.z_min + 2, planes);
 }
 
-// row `p` of an array (uniform) at a lane's byte offset
-template <typename S>
-__device__ inline const S &at(const S *__restrict__ p, unsigned off)
-{
-    return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(p) + off);
-}
-template <typename S>
-__device__ inline S &at(S *__restrict__ p, unsigned off)
-{
-    return *reinterpret_cast<S *>(reinterpret_cast<char *>(p) + off);
-}
-
 // What accelerate uses of one pressure-like field (pressure, viscosity) in one
 // cell plane, for the node (j, k): the area-weighted differences along x in
 // rows k and k-1, along y in column j, and the cells of column j in rows k, k-1

@@ -278,6 +278,20 @@ __device__ inline T next_lane(T x) { return lane_shift<0x130>(x); }
 template <typename T>
 __device__ inline T prev_lane(T x) { return lane_shift<0x138>(x); }
 
+// A row of an array (its address uniform over the wave) at a lane's byte offset:
+// the access takes a scalar address and a 32-bit offset, and no vector address
+// arithmetic.
+template <typename S>
+__device__ inline const S &at(const S *__restrict__ row, unsigned off)
+{
+    return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(row) + off);
+}
+template <typename S>
+__device__ inline S &at(S *__restrict__ row, unsigned off)
+{
+    return *reinterpret_cast<S *>(reinterpret_cast<char *>(row) + off);
+}
+
 constexpr int RED_THREADS = 256;
 
 __device__ inline double wave_min(double v)

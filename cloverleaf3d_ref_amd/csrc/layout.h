@@ -27,8 +27,7 @@ struct Lay {
     // faces whose reflective halo the fused kernels do not read for cell and
     // vertex fields: they read the interior cell or node the halo would
     // mirror instead (bits 1, 2: the x_min and x_max faces; 4, 8: y; 16, 32:
-    // z; 0 where halos are exchanged).  The advection sweeps use the x bits
-    // only.
+    // z; 0 where halos are exchanged).
     int mirror;
 };
 

@@ -327,6 +327,9 @@ __device__ __forceinline__ void mom_tail_body(const Blk &bk, TailSplit ts, Lay g
     const int i0 = DIR == 3 ? idx(g, j, wp, mmin) : idx(g, j, mmin, wp);  // offset at march position mmin
 #define OFF(q) (i0 + ((q) - mmin) * sM)
 
+    constexpr int MA = DIR - 1, WA = DIR == 3 ? 1 : 2;
+    const int sW = DIR == 3 ? g.ld : g.plane, dwc = (cell_m(g, WA, wp) - wp) * sW;  // a mirrored row of density
+    auto dmc = [&](int q) { return (cell_m(g, MA, q) - q) * sM; };                    // a mirrored plane
     const int dxc = cell_xm(g, j) - j;  // a mirrored x face: the interior cell its halo copies
     const int dxm = cell_xm(g, j - 1) - (j - 1);
     const int dxt = tan_xm(g, j) - j, dxtm = tan_xm(g, j - 1) - (j - 1);  // vol_flux_y/z, the sweep's mass flux
@@ -346,15 +349,19 @@ __device__ __forceinline__ void mom_tail_body(const Blk &bk, TailSplit ts, Lay g
         const int i = OFF(q);
         const T a = ok_cell ? (T)mf[i + dxt] : (T)0;  // q <= mmax+3: inside the sweep's face extent
         const T p = (ok_cell && q <= mmax + 2)
-                        ? (T)density1[i + dxc] * mom_post_vol(mode, g, i, V0, vfx, vfy, vfz, dxt)
+                        ? (T)density1[i + dxc + dwc + dmc(q)] * mom_post_vol(mode, g, i, V0, vfx, vfy, vfz, dxt)
                         : (T)0;
         const T am = ok_cm ? (T)mf[i - 1 + dxtm] : (T)0;
         const T pm = (ok_cm && q <= mmax + 2)
-                         ? (T)density1[i - 1 + dxm] * mom_post_vol(mode, g, i - 1, V0, vfx, vfy, vfz, dxtm)
+                         ? (T)density1[i - 1 + dxm + dwc + dmc(q)] * mom_post_vol(mode, g, i - 1, V0, vfx, vfy, vfz, dxtm)
                          : (T)0;
         xchg(a, p, am, pm, F, P);
     };
-    auto vel_at = [&](int c, int q) { return store ? (T)v.in[c][OFF(q)] : (T)0; };
+    auto vel_at = [&](int c, int q) -> T {
+        const int qn = node_m(g, MA, q);
+        const T x = store ? (T)v.in[c][OFF(qn)] : (T)0;
+        return c == MA && qn != q ? -x : x;
+    };
 
     Quad<T> Fa, Pa, Fb, Pb;
     // prologue: nf(m0-2..m0), node masses at m0-1, m0, m0+1, velocities m0-2..m0+1
@@ -392,12 +399,12 @@ __device__ __forceinline__ void mom_tail_body(const Blk &bk, TailSplit ts, Lay g
     // against five) mom_y 2.55 against 2.43 ms and mom_z 2.47 against 2.33.
     for (int m = m0; m <= m1; m++) {
         const Raw<S> rc = load_raw(mode, g, OFF(m + 2), ok_cell, ok_cell && m + 2 <= mmax + 2, mf, vfx, vfy, vfz,
-                                   density1, dxc, dxt, dxt);
+                                   density1, dxc + dwc + dmc(m + 2), dxt, dxt);
         const Raw<S> rcm = load_raw(mode, g, OFF(m + 2) - 1, ok_cm, ok_cm && m + 2 <= mmax + 2, mf, vfx, vfy, vfz,
-                                    density1, dxm, dxtm, dxtm);
+                                    density1, dxm + dwc + dmc(m + 2), dxtm, dxtm);
         T vp2[3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) vp2[c] = store ? (T)v.in[c][OFF(m + 2)] : (T)0;
+        for (int c = 0; c < 3; c++) vp2[c] = vel_at(c, m + 2);
         const T a = (T)rc.a, p = raw_cell_mass(mode, V0, rc, ok_cell && m + 2 <= mmax + 2);
         const T am = (T)rcm.a, pm = raw_cell_mass(mode, V0, rcm, ok_cm && m + 2 <= mmax + 2);
         Quad<T> Fc, Pc;
@@ -424,14 +431,6 @@ __device__ __forceinline__ void mom_tail_body(const Blk &bk, TailSplit ts, Lay g
         Pb = Pc;
     }
 #undef OFF
-}
-
-// A row of an array at a lane's byte offset: with the row's address scalar, the
-// access takes it and a 32-bit offset, and no vector address arithmetic.
-template <typename S>
-__device__ inline S ld(const S *__restrict__ row, unsigned off)
-{
-    return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(row) + off);
 }
 
 // sign-bit mask of x in the high word of its type
@@ -508,7 +507,19 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
     const int jm = min(j - 1, g.x_max + 2);
     unsigned ojm = off(jm), orhom = off(cell_xm(g, jm)), otm = off(tan_xm(g, jm));
     // the wave's row at march position q (elements)
-    auto at = [&](int q) { return (int64_t)(DIR == 3 ? idx(g, g.x_min - 2, wr, q) : idx(g, g.x_min - 2, q, wr)); };
+    const int sM = DIR == 3 ? g.plane : g.ld;
+    const int row0 = DIR == 3 ? idx(g, g.x_min - 2, wr, 0) : idx(g, g.x_min - 2, 0, wr);
+    auto row_at = [&](int q) { return row0 + q * sM; };
+    // on a mirrored face density and the velocities are read at the interior
+    // cell or node their halo copies (the component along the sweep with its
+    // sign flipped): from the row at q, to that one.  The first position past
+    // each face (out of reach where it is not mirrored); q below mmin: prologue.
+    constexpr int MA = DIR - 1, WA = DIR == 3 ? 1 : 2;  // the march's axis and the waves'
+    constexpr int far = 1 << 29;
+    const int dw = (cell_m(g, WA, wr) - wr) * (DIR == 3 ? g.ld : g.plane);
+    const int lo = (g.mirror >> (2 * MA)) & 1 ? mmin : -far, hi = (g.mirror >> (2 * MA)) & 2 ? mmax : far;
+    auto cell_shift = [&](int q, bool pro) { return q > hi ? 2 * (hi - q) + 1 : pro && q < lo ? 2 * (lo - q) - 1 : 0; };
+    auto node_shift = [&](int q, bool pro) { return q > hi + 1 ? 2 * (hi + 1 - q) : pro && q < lo ? 2 * (lo - q) : 0; };
     const int up = DIR == 3 ? g.ld : g.plane;  // to the next row across the sweep
 
     // the values of a plane: the sweep's mass flux, density and the volume
@@ -521,26 +532,27 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
     struct Pl {
         Col c, m;
     };
-    auto load_col = [&](Col &x, int64_t r, int64_t rc, unsigned o, unsigned orh, unsigned otan) {
-        x.a = ld(mf + r, otan);
-        x.rho = ld(density1 + rc, orh);
+    auto load_col = [&](Col &x, int r, int rc, int rr, unsigned o, unsigned orh, unsigned otan) {
+        x.a = at(mf + r, otan);
+        x.rho = at(density1 + rr, orh);
         if constexpr (MODE == 2 || MODE == 4) {
-            x.f[0] = ld(vfx + rc + 1, o);
-            x.f[1] = ld(vfx + rc, o);
+            x.f[0] = at(vfx + rc + 1, o);
+            x.f[1] = at(vfx + rc, o);
         }
         if constexpr (MODE == 2) {
-            x.f[2] = ld(vfy + rc + up, otan);
-            x.f[3] = ld(vfy + rc, otan);
+            x.f[2] = at(vfy + rc + up, otan);
+            x.f[3] = at(vfy + rc, otan);
         }
         if constexpr (MODE == 3) {
-            x.f[0] = ld(vfz + rc + up, otan);
-            x.f[1] = ld(vfz + rc, otan);
+            x.f[0] = at(vfz + rc + up, otan);
+            x.f[1] = at(vfz + rc, otan);
         }
     };
-    auto load = [&](int q, Pl &x) {
-        const int64_t r = at(q), rc = at(min(q, mmax + 2));  // mass fluxes end at mmax+3, cells at mmax+2
-        load_col(x.c, r, rc, oj, orho, ot);
-        if (lane == 0) load_col(x.m, r, rc, ojm, orhom, otm);
+    auto load = [&](int q, int r, Pl &x, bool pro) {  // r: row_at(q)
+        const int qc = min(q, mmax + 2);  // mass fluxes end at mmax+3, cells at mmax+2
+        const int rc = q > mmax + 2 ? r - sM : r, rr = rc + cell_shift(qc, pro) * sM + dw;
+        load_col(x.c, r, rc, rr, oj, orho, ot);
+        if (lane == 0) load_col(x.m, r, rc, rr, ojm, orhom, otm);
     };
     auto cell_mass = [&](const Col &x) -> T {  // mom_post_vol's expressions
         if constexpr (NF == 4) return x.rho * (V0 + x.f[0] - x.f[1] + x.f[2] - x.f[3]);
@@ -562,21 +574,25 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
         F = Quad<T>{a, xbuf[b][0][w][lane], xbuf[b][0][w - 1][lane + 1], xbuf[b][0][w - 1][lane]};
         P = Quad<T>{p, xbuf[b][1][w][lane], xbuf[b][1][w - 1][lane + 1], xbuf[b][1][w - 1][lane]};
     };
-    auto vel_at = [&](int c, int q) { return ld(v.in[c] + at(q), oj); };
+    auto vel_at = [&](int c, int q, int r, bool pro) -> T {
+        const int dq = node_shift(q, pro);
+        const T x = at(v.in[c] + (r + dq * sM), oj);
+        return c == MA ? flip_sign(x, dq ? 0x80000000u : 0u) : x;
+    };
 
     // waves without an owned row only load and publish; the barriers are the
     // same in number: two, then one per position
     if (!row) {
         for (int q = 0; q < 4; q++) {
             Pl x;
-            load(m0 - 2 + q, x);
+            load(m0 - 2 + q, row_at(m0 - 2 + q), x, true);
             publish(q, x);
         }
         __syncthreads();
         __syncthreads();
         for (int m = m0; m <= m1; m++) {
             Pl x;
-            load(m + 2, x);
+            load(m + 2, row_at(m + 2), x, false);
             publish((m - m0) & 1, x);
             __syncthreads();
         }
@@ -593,8 +609,8 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
 #pragma unroll
         for (int q = 0; q < 4; q += 2) {
             Pl x, y;
-            load(m0 - 2 + q, x);
-            load(m0 - 1 + q, y);
+            load(m0 - 2 + q, row_at(m0 - 2 + q), x, true);
+            load(m0 - 1 + q, row_at(m0 - 1 + q), y, true);
             a[q] = x.c.a;
             p[q] = publish(q, x);
             a[q + 1] = y.c.a;
@@ -603,10 +619,10 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            vel[2][c] = vel_at(c, m0 - 2);
-            vel[3][c] = vel_at(c, m0 - 1);
-            vel[0][c] = vel_at(c, m0);
-            vel[1][c] = vel_at(c, m0 + 1);
+            vel[2][c] = vel_at(c, m0 - 2, row_at(m0 - 2), true);
+            vel[3][c] = vel_at(c, m0 - 1, row_at(m0 - 1), true);
+            vel[0][c] = vel_at(c, m0, row_at(m0), true);
+            vel[1][c] = vel_at(c, m0 + 1, row_at(m0 + 1), true);
         }
         __syncthreads();
         gather(0, a[0], p[0], F[0], P[0]);
@@ -641,19 +657,23 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
     // modes 2.15 ms that way, 2.26 with 20 values spilled)
     constexpr bool AHEAD = sizeof(S) == 4 || MODE != 2;
     Pl nx;
-    auto load_ahead = [&](int q, T(&vq)[3]) {
-        load(q, nx);
+    auto load_plane = [&](int q, int r, T(&vq)[3]) {
+        Pl x;  // lanes other than 0 leave its column j-1 unset
+        load(q, r, x, false);
 #pragma unroll
-        for (int c = 0; c < 3; c++) vq[c] = vel_at(c, q);
+        for (int c = 0; c < 3; c++) vq[c] = vel_at(c, q, r, false);
+        return x;
     };
-    if (AHEAD) load_ahead(m0 + 2, vel[2]);
+    int r = row_at(m0);
+    if (AHEAD) nx = load_plane(m0 + 2, r + 2 * sM, vel[2]);
     auto step = [&](auto ic, int m) {
         constexpr int i = decltype(ic)::value, i1 = (i + 1) & 3, i2 = (i + 2) & 3, im = (i + 3) & 3, e = i & 1;
         // keeps the compiler from hoisting array + offset into vector registers
-        asm volatile("" : "+v"(oj), "+v"(orho), "+v"(ot), "+v"(ojm), "+v"(orhom), "+v"(otm));
-        if (!AHEAD) load_ahead(m + 2, vel[i2]);
-        const T a = nx.c.a, p = publish(e, nx);
-        if (AHEAD && m < m1) load_ahead(m + 3, vel[im]);  // vel(m-1) is done with
+        // and from walking a pointer per array
+        asm volatile("" : "+v"(oj), "+v"(orho), "+v"(ot), "+v"(ojm), "+v"(orhom), "+v"(otm), "+s"(r));
+        const Pl x = AHEAD ? nx : load_plane(m + 2, r + 2 * sM, vel[i2]);
+        const T a = x.c.a, p = publish(e, x);
+        if (AHEAD && m < m1) nx = load_plane(m + 3, r + 3 * sM, vel[im]);  // vel(m-1) is done with
         __syncthreads();
         // F[1-e], P[1-e] hold plane m+1
         gather(e, a, p, F[e], P[e]);
@@ -664,16 +684,16 @@ __device__ __forceinline__ void mom_cols_body(const Blk &bk, S (*xbuf)[2][mw_of(
         const bool neg = nf[i] < (T)0;
         const unsigned sgn = neg ? 0x80000000u : 0u;
         const T one_m = (T)1 - sig, two_m = (T)2 - sig, one_p = (T)1 + sig;
-        const int64_t r = at(m);
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             dv[i1][c] = vel[i2][c] - vel[i1][c];
             const T fhi = mom_flux_of<T>(nf[i], neg, sgn, one_m, two_m, one_p, d, rd, geo.r6, vel[i][c], vel[i1][c],
                                          dv[im][c], dv[i][c], dv[i1][c]);  // F(m)
             const T out = quo(vel[i][c] * mq[i] + flo[c] - fhi, mp[i]);
-            if (store) *reinterpret_cast<S *>(reinterpret_cast<char *>(v.out[c] + r) + oj) = out;
+            if (store) at(v.out[c] + r, oj) = out;
             flo[c] = fhi;
         }
+        r += sM;
     };
     for (int m = m0;;) {
         step(std::integral_constant<int, 0>{}, m);
@@ -767,13 +787,16 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mo
 #define OFF(q) (i0 + ((q) - g.z_min) * g.plane)
     // a mirrored x face: the interior cell and node its halos copy, and the
     // sign flip of the x velocity there
-    const int dxc = cell_xm(g, j) - j, dxn = node_xm(g, j) - j, dxt = tan_xm(g, j) - j;
+    const int dxn = node_xm(g, j) - j, dxt = tan_xm(g, j) - j;
+    const int dxc = cell_xm(g, j) - j + (cell_m(g, 1, k) - k) * g.ld;  // and a mirrored row of density
+    auto dmc = [&](int l) { return (cell_m(g, 2, l) - l) * g.plane; };  // and plane
     const bool xneg = node_xsign(g, j);
 
     auto plane = [&](int q, Quad<T> &F, Quad<T> &P, int &b) {
         const int i = OFF(q);
         const T a = ok_face ? (T)mf[i] : (T)0;
-        const T p = ok_cell ? (T)density1[i + dxc] * mom_post_vol(mode, g, i, V0, vfx, vfy, vfz, dxt) : (T)0;
+        const T p =
+            ok_cell ? (T)density1[i + dxc + dmc(q)] * mom_post_vol(mode, g, i, V0, vfx, vfy, vfz, dxt) : (T)0;
         exchange<+1, -1>(xbuf[b], lane, w, a, p, F, P);  // mass flux at j+1, cell mass at j-1
         b ^= 1;
     };
@@ -789,7 +812,7 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mo
     Raw<S> rn{0, 0, 0, 0, 0, 0};
     S vn[3] = {0, 0, 0};
     auto load_plane = [&](int q) {
-        rn = load_raw(mode, g, OFF(q), ok_face, ok_cell, mf, vfx, vfy, vfz, density1, dxc, dxt, 0);
+        rn = load_raw(mode, g, OFF(q), ok_face, ok_cell, mf, vfx, vfy, vfz, density1, dxc + dmc(q), dxt, 0);
 #pragma unroll
         for (int c = 0; c < 3; c++) vn[c] = ok_vert ? v.in[c][OFF(q) + dxn] : (S)0;
     };
