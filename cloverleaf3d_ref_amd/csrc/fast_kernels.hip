@@ -723,7 +723,9 @@ __global__ void __launch_bounds__(RED_THREADS) k_fast_field_summary(Lay g, Geo m
                      const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                      const S *__restrict__ zvel0, double *__restrict__ partial)
 {
-    field_summary_body<S, COMP>(hw_blk(), g, m, nj, nk, ncells, density0, energy0, pressure, xvel0, yvel0, zvel0, partial);
+    // the XCD-contiguous order, as k_field_summary
+    const Blk bk{xcd_block((int)blockIdx.x, (int)gridDim.x), 0, 0, (int)gridDim.x, 1, 1};
+    field_summary_body<S, COMP>(bk, g, m, nj, nk, ncells, density0, energy0, pressure, xvel0, yvel0, zvel0, partial);
 }
 
 template <typename S>
@@ -1149,7 +1151,7 @@ __global__ void __launch_bounds__(RED_THREADS)
 kb_field_summary(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
                  double *__restrict__ partial)
 {
-    DECK_BLOCK(dims_summary(D.g, gx, gy, gz), 0)
+    DECK_BLOCK(dims_summary(D.g, gx, gy, gz), 1)
     const Lay g = D.g;
     const int nj = g.x_max - g.x_min + 1, nk = g.y_max - g.y_min + 1, nl = g.z_max - g.z_min + 1;
     field_summary_body<S, COMP>(bk, g, D.m, nj, nk, nj * nk * nl, CF(F_DENSITY0), CF(F_ENERGY0), CF(F_PRESSURE),

@@ -806,7 +806,13 @@ k_field_summary(Lay g, Lay gv, int nj, int nk, int ncells, const double *__restr
                 const double *__restrict__ yvel0, const double *__restrict__ zvel0, double *__restrict__ partial)
 {
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int c = blockIdx.x * RED_THREADS + threadIdx.x; c < ncells; c += gridDim.x * RED_THREADS) {
+    // The XCD-contiguous order: a cell's rows and planes of nodes are its
+    // neighbours' too, and dealt round-robin the XCDs each fetched them all
+    // (160x96x120 with the final sum 38.9 -> 29.2 us, two cells at a time 27.5;
+    // 200^3 152 -> 123).  The partials stay where they were, so the sums do too.
+    const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
+#pragma unroll 2
+    for (int c = blk * RED_THREADS + threadIdx.x; c < ncells; c += gridDim.x * RED_THREADS) {
         const int j = g.x_min + c % nj;
         const int k = g.y_min + (c / nj) % nk;
         const int l = g.z_min + c / (nj * nk);
@@ -837,7 +843,7 @@ k_field_summary(Lay g, Lay gv, int nj, int nk, int ncells, const double *__restr
     if (threadIdx.x < 5) {
         double b = 0.0;
         for (int w = 0; w < RED_THREADS / 64; w++) b += red[threadIdx.x][w];
-        partial[5 * blockIdx.x + threadIdx.x] = b;
+        partial[5 * blk + threadIdx.x] = b;
     }
 }
 
