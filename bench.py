@@ -50,8 +50,8 @@ TRAFFIC_FILE = ROOT / "profiles" / "traffic_cuboid512_fp64.json"
 ARRAYS_PER_CELL = {
     # per-call kernels (one per reference loop nest)
     "k_ideal_gas": 4, "k_viscosity": 9, "k_calc_dt": 10, "k_revert": 4, "k_accelerate": 13,
-    "k_flux_calc": 12, "k_cell_vols": 5, "k_cell_flux": 6, "k_cell_update": 12, "k_mom_vols": 5,
-    "k_node_flux": 2, "k_node_mass": 5, "k_mom_flux": 4, "k_mom_update": 5, "k_reset_field": 10,
+    "k_flux_calc": 12, "k_cell_vols_flux": 10, "k_cell_update": 12, "k_mom_nodes": 11,
+    "k_mom_vols_flux": 10, "k_mom_flux": 4, "k_mom_update": 5, "k_reset_field": 10,
     "k_field_summary": 7, "k_pdv<1>": 13, "k_pdv<0>": 16,
     # fused kernels (geometry as scalars).  Sweep-dependent ones averaged over
     # the sweeps they run in: cell_x/y/z read 3/2/1 volume fluxes (sweep
@@ -75,10 +75,10 @@ ARRAYS_PER_CELL = {
 
 def kernel_domain_cells(name: str, n: int) -> int:
     """Cells (or nodes) one launch of `name` covers on an n^3 tile."""
-    if name in ("k_cell_vols", "k_mom_vols"):
+    if name in ("k_cell_vols_flux", "k_mom_nodes", "k_mom_vols_flux"):
         return (n + 4) ** 3
-    if name in ("k_accelerate", "k_reset_field", "k_flux_calc", "k_mom_flux", "k_mom_update", "k_node_flux",
-                "k_node_mass", "k_fast_accel_pdv", "k_fast_lagrange", "k_fast_mom_x", "k_fast_mom_y",
+    if name in ("k_accelerate", "k_reset_field", "k_flux_calc", "k_mom_flux", "k_mom_update",
+                "k_fast_accel_pdv", "k_fast_lagrange", "k_fast_mom_x", "k_fast_mom_y",
                 "k_fast_mom_z"):
         return (n + 1) ** 3
     return n ** 3

@@ -31,6 +31,26 @@ static inline dim3 grid_of(const Range &r)
     const int l = (r).l0 + (int)blockIdx.z;                          \
     if (j > (r).j1 || k > (r).k1) return;
 
+// The same with a plane's points dealt to the threads in one line, for ranges a
+// little wider than a multiple of 64 (65 columns of a 61-cell mesh with its halo:
+// half the lanes of 64 x 4 workgroups would be idle)
+static inline dim3 grid_lin(const Range &r)
+{
+    const int n = (r.j1 - r.j0 + 1) * (r.k1 - r.k0 + 1);
+    return dim3((unsigned)((n + BX * BY - 1) / (BX * BY)), 1, (unsigned)(r.l1 - r.l0 + 1));
+}
+
+#define RANGE_THREAD_LIN(r)                                                                          \
+    const unsigned lin_ = blockIdx.x * (BX * BY) + threadIdx.x, wide_ = (unsigned)((r).j1 - (r).j0 + 1); \
+    const int k = (r).k0 + (int)(lin_ / wide_), j = (r).j0 + (int)(lin_ % wide_);                     \
+    const int l = (r).l0 + (int)blockIdx.z;                                                           \
+    if (k > (r).k1) return;
+
+__device__ inline bool in_range(const Range &r, int j, int k, int l)
+{
+    return j >= r.j0 && j <= r.j1 && k >= r.k0 && k <= r.k1 && l >= r.l0 && l <= r.l1;
+}
+
 // Block coordinates of a kernel body: the hardware's for a launch over one
 // tile, or a block of one deck's share of a launch over many decks.
 struct Blk {
@@ -109,6 +129,12 @@ __device__ inline void chunk_range(const Blk &b, int lo, int hi, int &c0, int &c
     do {                                                                                        \
         if ((r).j1 >= (r).j0 && (r).k1 >= (r).k0 && (r).l1 >= (r).l0)                           \
             TIMED_LAUNCH(#kern, st, kern, grid_of(r), dim3(BX, BY, 1), 0, st, __VA_ARGS__);      \
+    } while (0)
+
+#define LAUNCH_LIN(kern, r, st, ...)                                                            \
+    do {                                                                                        \
+        if ((r).j1 >= (r).j0 && (r).k1 >= (r).k0 && (r).l1 >= (r).l0)                           \
+            TIMED_LAUNCH(#kern, st, kern, grid_lin(r), dim3(BX * BY), 0, st, __VA_ARGS__);       \
     } while (0)
 
 // neighbour access relative to the thread's offset i
