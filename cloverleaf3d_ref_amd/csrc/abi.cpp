@@ -48,6 +48,8 @@ struct Ctx {
     double *partial = nullptr;  // reduction partials (device)
     double *scalar = nullptr;   // reduction results (device)
     double *h_scalar = nullptr; // pinned host mirror of `scalar`
+    DtSlot *dt_slot = nullptr;  // pinned: calc_dt's minimum
+    unsigned long long dt_seq = 0;
     Stage stage;                // field uploads and fetches
     std::unordered_map<const void *, Resident> map;
     std::mutex mu;
@@ -85,6 +87,8 @@ void ensure_init()
     hip_check(hipMalloc(&c.partial, sizeof(double) * 5 * kMaxPartials), "hipMalloc partials");
     hip_check(hipMalloc(&c.scalar, sizeof(double) * 8), "hipMalloc scalar");
     hip_check(hipHostMalloc(&c.h_scalar, sizeof(double) * 8, hipHostMallocDefault), "hipHostMalloc");
+    hip_check(hipHostMalloc(&c.dt_slot, sizeof(DtSlot), hipHostMallocCoherent), "hipHostMalloc");
+    c.dt_slot->seq = c.dt_seq = 0;
     noalloc_scratch();  // with the device current
     c.init = true;
 }
@@ -170,6 +174,7 @@ int clover_hip_finalize(void)
     hip_check(hipFree(c.partial), "hipFree");
     hip_check(hipFree(c.scalar), "hipFree");
     hip_check(hipHostFree(c.h_scalar), "hipHostFree");
+    hip_check(hipHostFree(c.dt_slot), "hipHostFree");
     hip_check(hipStreamDestroy(c.stream), "hipStreamDestroy");
     c.init = false;
     CLOVER_API_END
@@ -275,10 +280,9 @@ int clover_hip_calc_dt_kernel(CLOVER_DIMS, double g_small, double g_big, double 
                                       res(xvel0, AC_VERT, g), res(yvel0, AC_VERT, g), res(zvel0, AC_VERT, g),
                                       res(dt_min, AC_VERT, g), C.partial, &nparts, C.stream),
                  "calc_dt");
-    check_launch(launch_min_final(C.partial, nparts, g_big, C.scalar, C.stream), "calc_dt min");
-    hip_check(hipMemcpyAsync(C.h_scalar, C.scalar, sizeof(double), hipMemcpyDeviceToHost, C.stream), "dt D2H");
-    hip_check(hipStreamSynchronize(C.stream), "sync");
-    const double dmin = C.h_scalar[0];
+    check_launch(launch_dt_final(C.partial, nparts, g_big, g_big, g_big, 0.0, C.scalar, C.dt_slot, ++C.dt_seq, C.stream),
+                 "calc_dt min");
+    const double dmin = wait_dt(C.dt_slot, C.dt_seq, C.stream);
     *dt_min_val = dmin;
     // calc_dt_kernel.f90:152-161: jkl_control is the default-real 1.1 and
     // never updated, so the location outputs are constants of the tile.

@@ -675,22 +675,6 @@ static void put_dt(clover_chunk *c, double dt)
 // 64^3 FP64 140 -> 136).
 static bool ahead(const clover_chunk *c) { return c->fast && c->tiles.size() == 1; }
 
-// waits for the dt of step dt_seq, which the stream's kernels are bound to
-// deliver: if the stream ends or fails without it, so does the wait
-static double wait_dt(clover_chunk *c)
-{
-    for (long spins = 0;; spins++) {
-        if (__atomic_load_n(&c->dt_slot->seq, __ATOMIC_ACQUIRE) == c->dt_seq) return c->dt_slot->dtlp;
-        if (spins % 100000 == 99999) {
-            const hipError_t e = hipStreamQuery(c->st);
-            if (e == hipErrorNotReady) continue;
-            hip_check(e, "timestep");
-            if (__atomic_load_n(&c->dt_slot->seq, __ATOMIC_ACQUIRE) == c->dt_seq) return c->dt_slot->dtlp;
-            throw Error(E_HIP, "timestep: the stream ended without a dt");
-        }
-    }
-}
-
 // timestep.f90:93-126 from the tiles' minima.  Returns 1 on a small time step.
 static int take_dt(clover_chunk *c, const double *dtlp, int stride)
 {
@@ -1332,7 +1316,7 @@ static int hydro_step(clover_chunk *c)
         timestep(c);
         const bool gas_fresh = c->gas_fresh, sound_fresh = c->sound_fresh;
         do_step(c);
-        const double dtlp = wait_dt(c);
+        const double dtlp = wait_dt(c->dt_slot, c->dt_seq, c->st);
         if (take_dt(c, &dtlp, 0)) {
             std::copy(f, f + NUM_ARRAYS, t.f);
             c->advect_x = advect_x;

@@ -9,6 +9,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "kernels.h"
 #include "layout.h"
 
 namespace clover {
@@ -32,6 +33,23 @@ inline void hip_check(hipError_t e, const char *what)
     if (e != hipSuccess)
         throw Error(e == hipErrorOutOfMemory ? E_NOMEM : E_HIP,
                     std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// Waits for the dt tagged seq, which a launch_dt_final on the stream is bound to
+// deliver: if the stream ends or fails without it, so does the wait.  Polling
+// pinned memory saves the copy back and the wake-up of a stream synchronisation.
+inline double wait_dt(const DtSlot *slot, unsigned long long seq, hipStream_t st)
+{
+    for (long spins = 0;; spins++) {
+        if (__atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) == seq) return slot->dtlp;
+        if (spins % 100000 == 99999) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            hip_check(e, "calc_dt");
+            if (__atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) == seq) return slot->dtlp;
+            throw Error(E_HIP, "calc_dt: the stream ended without a dt");
+        }
+    }
 }
 
 #define CLOVER_API_BEGIN try {
