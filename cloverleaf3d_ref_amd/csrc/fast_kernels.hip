@@ -102,14 +102,25 @@ __device__ inline QuadS<float> quad_b(const NodePair &n) { return QuadS<float>{{
 // the node velocities of its planes l (ul, vl, wl) and l+1 (uu, vu, wu) as
 // quad_up_raw quads, its density and pressure, the pressures of its six
 // neighbours -> its viscosity q; raises the running maxima of calc_dt's five
-// denominators (mc, mu, mv, mw, mdiv) with the cell's
+// denominators (mc, mu, mv, mw, mdiv) with the cell's.  mc's for a cell without
+// viscosity is ds * c * c of its soundspeed c alone: sqrt and the products round
+// monotonically, so such a cell raises the largest squared soundspeed ms instead,
+// and sound_denominator forms the value once per thread (the sqrt and its
+// surroundings, some 25 instructions per cell in FP64).
+template <typename T>
+__device__ inline T sound_denominator(T mc, T ms, T ds)
+{
+    const T c = sqrt(ms);
+    return tmax(mc, ds * (c * c));
+}
+
 template <typename T>
 __device__ inline T visc_cell(const QuadS<T> &ul, const QuadS<T> &vl, const QuadS<T> &wl, const QuadS<T> &uu,
                               const QuadS<T> &vu, const QuadS<T> &wu, T rho, T p_c, T p_lo, T p_hi, T p_xm, T p_xp,
-                              T p_ym, T p_yp, const Geo &m, T ds, T dx, T dy, T dz, T xa, T ya, T za, T &mc, T &mu,
-                              T &mv, T &mw, T &mdiv)
+                              T p_ym, T p_yp, const Geo &m, T ds, T dx, T dy, T dz, T xa, T ya, T za, T &mc, T &ms,
+                              T &mu, T &mv, T &mw, T &mdiv)
 {
-    const T c = soundspeed_of<T>(rho, p_c);
+    const T c2 = soundspeed2_of<T>(rho, p_c);
 #define U(a, b, c) ((c) ? uu : ul).v[(a) + 2 * (b)]
 #define V(a, b, c) ((c) ? vu : vl).v[(a) + 2 * (b)]
 #define W(a, b, c) ((c) ? wu : wl).v[(a) + 2 * (b)]
@@ -179,11 +190,14 @@ __device__ inline T visc_cell(const QuadS<T> &ul, const QuadS<T> &vl, const Quad
 
     // calc_dt: the denominators of the five candidates (visc_dt_body
     // forms the candidates from their maxima over a thread's cells)
-    T cc = c * c;
-    // in FP64 the divide is skipped where q is zero (adding 2*0/rho
-    // leaves cc as it is); the FP32 reciprocal is cheaper than a branch
-    if (sizeof(T) == 4 || q != (T)0) cc = cc + quo((T)2 * q, rho);
-    mc = tmax(mc, ds * cc);
+    if (q == (T)0 && c2 >= (T)0) {
+        ms = tmax(ms, c2);
+    } else {
+        const T c = sqrt(c2);
+        T cc = c * c;
+        if (q != (T)0) cc = cc + quo((T)2 * q, rho);  // adding 2*0/rho leaves cc as it is
+        mc = tmax(mc, ds * cc);
+    }
     const T du1 = ugradx1 * xa, du2 = ugradx2 * xa;
     mu = tmax(mu, tmax(fabs(du1), fabs(du2)));
     const T dv1 = vgrady1 * ya, dv2 = vgrady2 * ya;
@@ -209,7 +223,7 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
 {
     using T = S;  // arithmetic type of the form
     const int j = g.x_min + bk.x * (int)blockDim.x + (int)threadIdx.x;
-    const int k = g.y_min + bk.y * (int)blockDim.y + (int)threadIdx.y;
+    const int k = g.y_min + bk.y * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
     const bool in = j <= g.x_max && k <= g.y_max && l0 <= l1;  // every thread reaches the reduction
@@ -220,37 +234,52 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
     const T small = (T)g_small;
     double dtmin_thread = 1.0e300;
     if (in) {
-        T mc = 0, mu = 0, mv = 0, mw = 0, mdiv = 0;  // largest dt denominators so far (all are >= 0)
-        int i = idx(g, j, k, l0);
-        QuadS<S> ul = quad_up_raw(xvel0, i, g.ld), vl = quad_up_raw(yvel0, i, g.ld), wl = quad_up_raw(zvel0, i, g.ld);
+        T mc = 0, ms = 0, mu = 0, mv = 0, mw = 0, mdiv = 0;  // largest dt denominators so far (all are >= 0)
+        // the wave's row is scalar; lanes add byte offsets (at)
+        l0 = __builtin_amdgcn_readfirstlane(l0);
+        l1 = __builtin_amdgcn_readfirstlane(l1);
+        int r = __builtin_amdgcn_readfirstlane(idx(g, g.x_min, k, l0));
+        unsigned oj = (unsigned)(j - g.x_min) * (unsigned)sizeof(S);
+        const auto quad = [&](const S *__restrict__ p) {
+            return QuadS<S>{{at(p + r, oj), at(p + r + 1, oj), at(p + r + g.ld, oj), at(p + r + 1 + g.ld, oj)}};
+        };
+        QuadS<S> ul = quad(xvel0), vl = quad(yvel0), wl = quad(zvel0);
         // a mirrored face (Lay::mirror): the neighbour across it is a halo
         // cell, read as the cell itself, which its reflection copies
-        const int oxm = cell_m(g, 0, j - 1) - j, oxp = cell_m(g, 0, j + 1) - j;
+        const int oxm = cell_m(g, 0, j - 1) - (j - 1), oxp = cell_m(g, 0, j + 1) - (j + 1);
+        unsigned om = oj + (unsigned)(oxm * (int)sizeof(S)), op = oj + (unsigned)(oxp * (int)sizeof(S));
         const int oym = (cell_m(g, 1, k - 1) - k) * g.ld, oyp = (cell_m(g, 1, k + 1) - k) * g.ld;
-        T p_lo = pressure[i + (cell_m(g, 2, l0 - 1) - l0) * g.plane], p_c = pressure[i];
+        T p_lo = at(pressure + r + (cell_m(g, 2, l0 - 1) - l0) * g.plane, oj), p_c = at(pressure + r, oj);
         // The cell's soundspeed is not read: it is ideal_gas's of the cell's
         // density and pressure, formed here with the same operations
-        // (soundspeed_of), so it has the same bits.
-        for (int l = l0; l <= l1; l++, i += g.plane) {
+        // (soundspeed2_of), so it has the same bits.
+        for (int l = l0; l <= l1; l++) {
+            asm volatile("" : "+v"(oj), "+v"(om), "+v"(op), "+s"(r));  // no address per array held or walked
             // the upper node plane's velocities and pressure, the cell's
             // density and its x/y pressure neighbours, loaded at the top of
             // the plane: holding the next plane's loads in registers as well
             // took 150 VGPRs in FP64 (three waves per SIMD) against 126 (four)
-            // and measured 1.55 against 1.49 ms at 512^3
-            const QuadS<S> uu = quad_up_raw(xvel0, i + g.plane, g.ld), vu = quad_up_raw(yvel0, i + g.plane, g.ld),
-                           wu = quad_up_raw(zvel0, i + g.plane, g.ld);
-            const T p_hi = pressure[i + (cell_m(g, 2, l + 1) - l) * g.plane];
-            const T rho = density0[i];
-            const T p_xm = pressure[i + oxm], p_xp = pressure[i + oxp];
-            const T p_ym = pressure[i + oym], p_yp = pressure[i + oyp];
-            viscosity[i] = visc_cell<T>(ul, vl, wl, uu, vu, wu, rho, p_c, p_lo, p_hi, p_xm, p_xp, p_ym, p_yp, m, ds,
-                                        dx, dy, dz, xa, ya, za, mc, mu, mv, mw, mdiv);
+            // and measured 1.55 against 1.49 ms at 512^3.  With a scalar row
+            // and no sqrt per cell the batched kernel also runs four waves per
+            // SIMD (145 -> 116 VGPRs; 320^3 as 8 tiles 463 -> 439 us) and the
+            // single tile's issues less (128^3 36.4 -> 35.7 us, 512^3 1.466 ->
+            // 1.453 ms against the 1.24 ms its six arrays take)
+            const int rc = r;
+            r += g.plane;
+            const QuadS<S> uu = quad(xvel0), vu = quad(yvel0), wu = quad(zvel0);
+            const T p_hi = at(pressure + rc + (cell_m(g, 2, l + 1) - l) * g.plane, oj);
+            const T rho = at(density0 + rc, oj);
+            const T p_xm = at(pressure + rc - 1, om), p_xp = at(pressure + rc + 1, op);
+            const T p_ym = at(pressure + rc + oym, oj), p_yp = at(pressure + rc + oyp, oj);
+            at(viscosity + rc, oj) = visc_cell<T>(ul, vl, wl, uu, vu, wu, rho, p_c, p_lo, p_hi, p_xm, p_xp, p_ym, p_yp,
+                                                  m, ds, dx, dy, dz, xa, ya, za, mc, ms, mu, mv, mw, mdiv);
             ul = uu;
             vl = vu;
             wl = wu;
             p_lo = p_c;
             p_c = p_hi;
         }
+        mc = sound_denominator(mc, ms, ds);
         // calc_dt_kernel.f90:127-149 per cell is dt = min(C_c / max(sqrt(ds*cc), g_small),
         // C_u / max(|du1|, |du2|, 1e-5*volume), C_v / .., C_w / .., C_div / max(1e-5*volume, |div|))
         // with constant numerators.  Rounded division by a positive
@@ -307,7 +336,7 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
     double dtmin_thread = 1.0e300;
     if (in) {
         const bool two = j < g.x_max;  // cell j+1 is interior (else the halo cell x_max+1: loaded, not stored)
-        T mc = 0, mu = 0, mv = 0, mw = 0, mdiv = 0;
+        T mc = 0, ms = 0, mu = 0, mv = 0, mw = 0, mdiv = 0;
         int i = idx(g, j, k, l0);  // even: x_min sits on a 32-element boundary
         auto pair = [&](const float *__restrict__ p, int ii) { return *reinterpret_cast<const float2 *>(p + ii); };
         NodePair ul = load_node_pair(xvel0, i, g.ld), vl = load_node_pair(yvel0, i, g.ld),
@@ -325,11 +354,11 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
             const float2 p_ym = pair(pressure, i + oym), p_yp = pair(pressure, i + oyp);
             const T qa = visc_cell<T>(quad_a(ul), quad_a(vl), quad_a(wl), quad_a(uu), quad_a(vu), quad_a(wu), rho.x,
                                       p_c.x, p_lo.x, p_hi.x, p_xm, xp_self ? p_c.x : p_c.y, p_ym.x, p_yp.x, m, ds, dx,
-                                      dy, dz, xa, ya, za, mc, mu, mv, mw, mdiv);
+                                      dy, dz, xa, ya, za, mc, ms, mu, mv, mw, mdiv);
             if (two) {
                 const T qb = visc_cell<T>(quad_b(ul), quad_b(vl), quad_b(wl), quad_b(uu), quad_b(vu), quad_b(wu),
                                           rho.y, p_c.y, p_lo.y, p_hi.y, p_c.x, p_xp2, p_ym.y, p_yp.y, m, ds, dx, dy, dz,
-                                          xa, ya, za, mc, mu, mv, mw, mdiv);
+                                          xa, ya, za, mc, ms, mu, mv, mw, mdiv);
                 *reinterpret_cast<float2 *>(viscosity + i) = make_float2(qa, qb);
             } else {
                 viscosity[i] = qa;
@@ -340,6 +369,7 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
             p_lo = p_c;
             p_c = p_hi;
         }
+        mc = sound_denominator(mc, ms, ds);
         const T dtct = quo((T)dtc_safe * (T)1, tmax(sqrt(mc), small));
         const T dtut = quo((T)dtu_safe * (T)4 * vol, tmax(mu, (T)1.0e-5 * vol));
         const T dtvt = quo((T)dtv_safe * (T)4 * vol, tmax(mv, (T)1.0e-5 * vol));

@@ -220,14 +220,19 @@ __device__ inline T pressure_of(T density, T energy)
 // its pressure (the pressure ideal_gas forms from density and energy); the
 // same operations on the same values as ideal_gas_cell, so the same bits
 template <typename T>
-__device__ inline T soundspeed_of(T density, T pressure)
+__device__ inline T soundspeed2_of(T density, T pressure)  // squared
 {
     const T d = density, p = pressure;
     const T v = quo((T)1, d);
     const T pressurebyenergy = (T)(1.4 - 1.0) * d;
     const T pressurebyvolume = -d * p;
-    const T sound_speed_squared = v * v * (p * pressurebyenergy - pressurebyvolume);
-    return sqrt(sound_speed_squared);
+    return v * v * (p * pressurebyenergy - pressurebyvolume);
+}
+
+template <typename T>
+__device__ inline T soundspeed_of(T density, T pressure)
+{
+    return sqrt(soundspeed2_of(density, pressure));
 }
 
 template <typename S>
