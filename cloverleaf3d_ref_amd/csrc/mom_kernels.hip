@@ -14,7 +14,7 @@
 // runs the same expressions in FP32), and shared with the neighbours that
 // need it:
 //   * lanes of a wavefront lie along x (coalesced rows); neighbours along x
-//     come from lane shuffles;
+//     come from lane shifts (x sweep) or LDS;
 //   * the waves of a workgroup lie along the second axis; a neighbour row is
 //     read from LDS (double-buffered, one barrier per plane).  Wave 0 is the
 //     halo row and stores nothing;
@@ -50,8 +50,8 @@ struct Vel3 {
 };
 
 // post_vol of advec_mom_kernel.f90:95-163 for the sweep `mode`:
-// 1 sweep 1 along x, 2 sweep 1 along z, 3 sweep 2 with advect_x,
-// 4 sweep 2 without, 5 and 6 sweep 3
+// 1 sweep 1 along x (formed in mom_x_body), 2 sweep 1 along z, 3 sweep 2 with
+// advect_x, 4 sweep 2 without, 5 and 6 sweep 3
 template <typename S>
 // (dxt: the offset of the column vol_flux_y and vol_flux_z are read at, on a
 // mirrored x face, launch.h tan_xm)
@@ -61,7 +61,6 @@ __device__ inline S mom_post_vol(int mode, const Lay &g, int i, S V0, const S *_
 #define D(x) (x)
     const int t = i + dxt;
     switch (mode) {
-    case 1: return V0 + D(vfy[t + g.ld]) - D(vfy[t]) + D(vfz[t + g.plane]) - D(vfz[t]);
     case 2: return V0 + D(vfx[i + 1]) - D(vfx[i]) + D(vfy[t + g.ld]) - D(vfy[t]);
     case 3: return V0 + D(vfz[t + g.plane]) - D(vfz[t]);
     case 4: return V0 + D(vfx[i + 1]) - D(vfx[i]);
@@ -108,33 +107,12 @@ __device__ inline T face_sigma(T nf, T mq_lo, T mq_hi)
     return quo(fabs(nf), nf < (T)0 ? mq_hi : mq_lo);
 }
 
-// A value and its neighbours at -1 along the lane axis (or +1, see
-// exchange_x) and -1 along the wave axis.
+// A value and its neighbours: one column along x (-1 in the y and z sweeps; in
+// the x sweep +1 for mass fluxes, -1 for cell masses), one down the wave axis, both.
 template <typename T>
 struct Quad {
     T c, x, w, xw;
 };
-
-// Publishes a and p of every thread of the workgroup and returns each
-// thread's neighbours: a at lane+dxa, p at lane+dxp, both also one wave
-// down.  Lanes and waves without such a neighbour get their own values
-// (used only by threads that store nothing).
-template <int DXA, int DXP, typename T, int W>
-__device__ inline void exchange(T (*buf)[W][64], int lane, int w, T a, T p, Quad<T> &A, Quad<T> &P)
-{
-    buf[0][w][lane] = a;
-    buf[1][w][lane] = p;
-    __syncthreads();
-    const int la = min(max(lane + DXA, 0), 63), lp = min(max(lane + DXP, 0), 63), wd = w > 0 ? w - 1 : 0;
-    A.c = a;
-    A.x = buf[0][w][la];
-    A.w = buf[0][wd][lane];
-    A.xw = buf[0][wd][la];
-    P.c = p;
-    P.x = buf[1][w][lp];
-    P.w = buf[1][wd][lane];
-    P.xw = buf[1][wd][lp];
-}
 
 // The loads of one plane, kept raw so that they can be issued a plane ahead
 // (after the barrier of the plane in hand) and consumed by the next plane:
@@ -159,7 +137,6 @@ __device__ inline Raw<S> load_raw(int mode, const Lay &g, int i, bool ok_a, bool
         r.rho = density1[i + dxc];
         const int t = i + dxt;
         switch (mode) {
-        case 1: r.v0 = vfy[t + g.ld]; r.v1 = vfy[t]; r.v2 = vfz[t + g.plane]; r.v3 = vfz[t]; break;
         case 2: r.v0 = vfx[i + 1]; r.v1 = vfx[i]; r.v2 = vfy[t + g.ld]; r.v3 = vfy[t]; break;
         case 3: r.v0 = vfz[t + g.plane]; r.v1 = vfz[t]; break;
         case 4: r.v0 = vfx[i + 1]; r.v1 = vfx[i]; break;
@@ -176,36 +153,12 @@ __device__ inline S raw_cell_mass(int mode, S V0, const Raw<S> &r, bool ok_p)
     if (!ok_p) return 0;
     S pv;
     switch (mode) {
-    case 1:
     case 2: pv = V0 + r.v0 - r.v1 + r.v2 - r.v3; break;
     case 3:
     case 4: pv = V0 + r.v0 - r.v1; break;
     default: pv = V0; break;
     }
     return r.rho * pv;
-}
-
-// exchange() in two halves, so loads can be issued between them
-template <typename T, int W>
-__device__ inline void publish(T (*buf)[W][64], int lane, int w, T a, T p)
-{
-    buf[0][w][lane] = a;
-    buf[1][w][lane] = p;
-    __syncthreads();
-}
-
-template <int DXA, int DXP, typename T, int W>
-__device__ inline void gather(T (*buf)[W][64], int lane, int w, T a, T p, Quad<T> &A, Quad<T> &P)
-{
-    const int la = min(max(lane + DXA, 0), 63), lp = min(max(lane + DXP, 0), 63), wd = w > 0 ? w - 1 : 0;
-    A.c = a;
-    A.x = buf[0][w][la];
-    A.w = buf[0][wd][lane];
-    A.xw = buf[0][wd][la];
-    P.c = p;
-    P.x = buf[1][w][lp];
-    P.w = buf[1][wd][lane];
-    P.xw = buf[1][wd][lp];
 }
 
 __device__ inline double shfl_d(double x, int src) { return __shfl(x, src, 64); }
@@ -760,105 +713,160 @@ __global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fas
 //   nf(j)  = 0.125*(f(0,-1,0)+f(0,0,0)+f(1,-1,0)+f(1,0,0)+f(0,-1,-1)+f(0,0,-1)+f(1,-1,-1)+f(1,0,-1))
 //   mp(j)  = cells (0,-1,0),(0,0,0),(-1,-1,0),(-1,0,0),(0,-1,-1),(0,0,-1),(-1,-1,-1),(-1,0,-1)
 
-template <typename S>
-__device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
-             const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1,
-             Vel3<S> v)
+//
+// Laid out like mom_cols_body (scalar rows, MODE a template argument, the halo
+// row's wave only loads and publishes); a neighbour along x is a DPP shift, so
+// LDS carries the row below alone, 4 accesses per wave and plane instead of 34,
+// and the VALU issues 239 (FP64) and 125 (FP32) instructions instead of 305 and
+// 190.  The form before against this one, three rounds on one machine: 64^3 FP64
+// 16.2 -> 14.1 us, 131x75x93 24.6 -> 21.1, 256^3 278 -> 256, FP32 101x143x67 16.0
+// -> 15.4; 512^3, at its ten arrays' bandwidth, within the memory's spread.  Of
+// 4, 8 and 16 waves per workgroup: 13.2, 14.1, 17.4 us at 64^3, 21.8, 21.1, 28.3 at
+// 131x75x93.
+template <int MODE, typename S>
+__device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, const S *__restrict__ mf,
+                                           const S *__restrict__ vfy, const S *__restrict__ vfz,
+                                           const S *__restrict__ density1, Vel3<S> v)
 {
+    static_assert(MODE == 1 || MODE == 5, "the x sweep's modes");
     using T = S;  // arithmetic type of the form
     constexpr int MW = mw_of(1);
     __shared__ T xbuf[2][2][MW][64];
-    const int lane = threadIdx.x, w = threadIdx.y;
+    const int lane = (int)threadIdx.x, w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const T d = (T)geo.dx;
     const Recip rd = geo.rx;
     const T V0 = (T)geo.vol;
-    const int j = g.x_min - 2 + bk.x * 60 + lane;
-    const int k = g.y_min - 1 + bk.y * (MW - 1) + w;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max + 1, l0, l1);
     if (l0 > l1) return;  // the whole workgroup: before any barrier
-    // j >= x_min-2 and k >= y_min-1 always.  mass_flux_x ends at x_max+3 /
-    // y_max+2, cells at x_max+2 / y_max+2, vertices at x_max+3 / y_max+3.
-    const bool ok_face = j <= g.x_max + 3 && k <= g.y_max + 2;
-    const bool ok_cell = j <= g.x_max + 2 && k <= g.y_max + 2;
-    const bool ok_vert = j <= g.x_max + 3 && k <= g.y_max + 3;
-    const bool store = lane >= 2 && lane <= 61 && w >= 1 && j <= g.x_max + 1 && k <= g.y_max + 1;
-    const int i0 = idx(g, j, k, g.z_min);
-#define OFF(q) (i0 + ((q) - g.z_min) * g.plane)
-    // a mirrored x face: the interior cell and node its halos copy, and the
-    // sign flip of the x velocity there
-    const int dxn = node_xm(g, j) - j, dxt = tan_xm(g, j) - j;
-    const int dxc = cell_xm(g, j) - j + (cell_m(g, 1, k) - k) * g.ld;  // and a mirrored row of density
-    auto dmc = [&](int l) { return (cell_m(g, 2, l) - l) * g.plane; };  // and plane
-    const bool xneg = node_xsign(g, j);
+    const int j = g.x_min - 2 + bk.x * 60 + lane;
+    const int k = g.y_min - 1 + bk.y * (MW - 1) + w;
+    const bool row = w >= 1 && k <= g.y_max + 1;  // an owned row (uniform)
+    const bool store = lane >= 2 && lane <= 61 && j <= g.x_max + 1;
+    // Lanes and rows outside the arrays read clamped ones, which no stored node
+    // needs: mass_flux_x and the vertices end at x_max+3, cells at x_max+2, and
+    // every row read at y_max+2.  Byte offsets from column x_min-2: faces, nodes,
+    // density and the tangential fluxes on a mirrored x face (launch.h).
+    const int jf = min(j, g.x_max + 3), jc = min(j, g.x_max + 2), kr = min(k, g.y_max + 2);
+    auto off = [&](int col) { return (unsigned)(col - g.x_min + 2) * (unsigned)sizeof(S); };
+    unsigned oj = off(jf), on = off(node_xm(g, jf)), orho = off(cell_xm(g, jc)), ot = off(tan_xm(g, jc));
+    const unsigned sx = node_xsign(g, jf) ? 0x80000000u : 0u;  // the reflection of the x velocity (update_halo_kernel.f90:604-1004)
+    const int dk = (cell_m(g, 1, kr) - kr) * g.ld;  // density's row on a mirrored y face
 
-    auto plane = [&](int q, Quad<T> &F, Quad<T> &P, int &b) {
-        const int i = OFF(q);
-        const T a = ok_face ? (T)mf[i] : (T)0;
-        const T p =
-            ok_cell ? (T)density1[i + dxc + dmc(q)] * mom_post_vol(mode, g, i, V0, vfx, vfy, vfz, dxt) : (T)0;
-        exchange<+1, -1>(xbuf[b], lane, w, a, p, F, P);  // mass flux at j+1, cell mass at j-1
-        b ^= 1;
+    // a plane's values as stored, so that their loads can stay in flight; the
+    // flux through its lower z face is the upper one of the plane before
+    struct Pl {
+        S a, rho, f[MODE == 1 ? 3 : 1];
+    };
+    auto load = [&](int q, int r) {  // r: the wave's row in plane q
+        Pl x;
+        x.a = at(mf + r, oj);
+        x.rho = at(density1 + (r + dk + (cell_m(g, 2, q) - q) * g.plane), orho);
+        if constexpr (MODE == 1) {
+            x.f[0] = at(vfy + r + g.ld, ot);
+            x.f[1] = at(vfy + r, ot);
+            x.f[2] = at(vfz + r + g.plane, ot);
+        }
+        return x;
+    };
+    T zlo = 0;  // MODE 1: vol_flux_z through the lower face of the plane in hand
+    auto publish = [&](int b, const Pl &x) {  // returns the cell mass, post_vol as in advec_mom_kernel.f90:95-163
+        T p;
+        if constexpr (MODE == 1) {
+            p = x.rho * (V0 + x.f[0] - x.f[1] + x.f[2] - zlo);
+            zlo = x.f[2];
+        } else {
+            p = x.rho * V0;
+        }
+        xbuf[b][0][w][lane] = x.a;
+        xbuf[b][1][w][lane] = p;
+        return p;
     };
 
-    int b = 0;
-    Quad<T> Fp, Pp;  // plane l-1
-    plane(l0 - 1, Fp, Pp, b);
-    const int lm = lane > 0 ? lane - 1 : 0, lp = lane < 63 ? lane + 1 : 63, lp2 = lane < 62 ? lane + 2 : 63;
-    // FP64: plane l's loads are issued during plane l-1 (after its barrier);
-    // FP32: each plane's at the top of its step, which measured faster at
-    // 512^3 (1.24 -> 1.20 ms; FP64 2.19 -> 2.29 ms that way)
-    constexpr bool ahead = sizeof(S) == 8;
-    Raw<S> rn{0, 0, 0, 0, 0, 0};
-    S vn[3] = {0, 0, 0};
-    auto load_plane = [&](int q) {
-        rn = load_raw(mode, g, OFF(q), ok_face, ok_cell, mf, vfx, vfy, vfz, density1, dxc + dmc(q), dxt, 0);
-#pragma unroll
-        for (int c = 0; c < 3; c++) vn[c] = ok_vert ? v.in[c][OFF(q) + dxn] : (S)0;
+    int r = idx(g, g.x_min - 2, kr, l0 - 1);
+    if constexpr (MODE == 1) zlo = at(vfz + r, ot);
+    if (!row) {  // loads and publishes only; as many barriers as below
+        publish(1, load(l0 - 1, r));
+        __syncthreads();
+        for (int l = l0; l <= l1; l++) {
+            r += g.plane;
+            publish((l - l0) & 1, load(l, r));
+            __syncthreads();
+        }
+        return;
+    }
+
+    Quad<T> F[2], P[2];
+    auto gather = [&](int b, T a, T p) {
+        const T aw = xbuf[b][0][w - 1][lane], pw = xbuf[b][1][w - 1][lane];
+        F[b] = Quad<T>{a, next_lane(a), aw, next_lane(aw)};
+        P[b] = Quad<T>{p, prev_lane(p), pw, prev_lane(pw)};
     };
-    if (ahead) load_plane(l0);
-    for (int l = l0; l <= l1; l++) {
-        if (!ahead) load_plane(l);
-        const Raw<S> rc = rn;
-        T vc[3];
+    // a plane's loads go out before the barrier of the plane before; in FP32 that
+    // ran 101x143x67 15.6 -> 15.4 us and 512^3 1.04 -> 1.01 ms against loads at the
+    // top of the plane's own step
+    Pl nx;
+    S vn[3];
+    auto load_plane = [&](int q, int rq) {
+        nx = load(q, rq);
 #pragma unroll
-        for (int c = 0; c < 3; c++) vc[c] = (T)vn[c];
-        if (xneg) vc[0] = -vc[0];  // the reflection of the x velocity (update_halo_kernel.f90:604-1004)
-        const T a = (T)rc.a, p = raw_cell_mass(mode, V0, rc, ok_cell);
-        publish(xbuf[b], lane, w, a, p);
-        if (ahead && l < l1) load_plane(l + 1);
-        Quad<T> F, P;
-        gather<+1, -1>(xbuf[b], lane, w, a, p, F, P);  // mass flux at j+1, cell mass at j-1
-        b ^= 1;
+        for (int c = 0; c < 3; c++) vn[c] = at(v.in[c] + rq, on);
+    };
+    {
+        const Pl x = load(l0 - 1, r);
+        r += g.plane;
+        const T p = publish(1, x);
+        load_plane(l0, r);
+        __syncthreads();
+        gather(1, x.a, p);
+    }
+    auto step = [&](auto ic, int l) {
+        constexpr int e = decltype(ic)::value;
+        // keeps array + offset out of vector registers
+        asm volatile("" : "+v"(oj), "+v"(on), "+v"(orho), "+v"(ot), "+s"(r));
+        const Pl x = nx;
+        T v0[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) v0[c] = vn[c];
+        v0[0] = flip_sign(v0[0], sx);
+        const T p = publish(e, x);
+        if (l < l1) load_plane(l + 1, r + g.plane);
+        __syncthreads();
+        gather(e, x.a, p);
         // F.x = f(+1,0), F.w = f(0,-1), F.xw = f(+1,-1); P.x = cell(-1,0), ...
-        const T nf = 0.125 * (F.w + F.c + F.xw + F.x + Fp.w + Fp.c + Fp.xw + Fp.x);
-        const T mp = 0.125 * (P.w + P.c + P.xw + P.x + Pp.w + Pp.c + Pp.xw + Pp.x);
-        const T nf_lo = shfl_d(nf, lm);
-        const T mq = mp - nf_lo + nf;
-        const T mq_hi = shfl_d(mq, lp);
-        const T sig = face_sigma(nf, mq, mq_hi);
-        const int i = OFF(l);
+        const Quad<T> &Fc = F[e], &Fp = F[1 - e], &Pc = P[e], &Pp = P[1 - e];
+        const T nf = (T)0.125 * (Fc.w + Fc.c + Fc.xw + Fc.x + Fp.w + Fp.c + Fp.xw + Fp.x);
+        const T mp = (T)0.125 * (Pc.w + Pc.c + Pc.xw + Pc.x + Pp.w + Pp.c + Pp.xw + Pp.x);
+        const T mq = mp - prev_lane(nf) + nf;
+        const T sig = face_sigma(nf, mq, next_lane(mq));
+        const bool neg = nf < (T)0;
+        const unsigned sgn = neg ? 0x80000000u : 0u;
+        const T one_m = (T)1 - sig, two_m = (T)2 - sig, one_p = (T)1 + sig;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const T v0 = vc[c];
-            const T vm1 = shfl_d(v0, lm), vp1 = shfl_d(v0, lp), vp2 = shfl_d(v0, lp2);
-            const T fhi = mom_face_flux(nf, sig, d, rd, geo.r6, vm1, v0, vp1, vp2);  // face j | j+1
-            const T flo = shfl_d(fhi, lm);                                // face j-1 | j
-            if (store) v.out[c][i] = quo(v0 * mq + flo - fhi, mp);
+            const T vp1 = next_lane(v0[c]), d1 = vp1 - v0[c];
+            const T fhi = mom_flux_of<T>(nf, neg, sgn, one_m, two_m, one_p, d, rd, geo.r6, v0[c], vp1, prev_lane(d1),
+                                         d1, next_lane(d1));  // face j | j+1
+            const T out = quo(v0[c] * mq + prev_lane(fhi) - fhi, mp);
+            if (store) at(v.out[c] + r, oj) = out;
         }
-        Fp = F;
-        Pp = P;
+        r += g.plane;
+    };
+    for (int l = l0;;) {
+        step(std::integral_constant<int, 0>{}, l);
+        if (++l > l1) break;
+        step(std::integral_constant<int, 1>{}, l);
+        if (++l > l1) break;
     }
-#undef OFF
 }
 
-template <typename S>
-__global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1) k_fast_mom_x(const double *__restrict__ dt, int xcd, Lay g, Geo geo, int mode, const S *__restrict__ mf, const S *__restrict__ vfx,
-             const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1,
-             Vel3<S> v)
+template <int MODE, typename S>
+__global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1)
+k_fast_mom_x(const double *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf,
+             const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1, Vel3<S> v)
 {
-    if (*dt < 0.0) return;
-    mom_x_body<S>(hw_blk(xcd), g, geo, mode, mf, vfx, vfy, vfz, density1, v);
+    if (*dt < 0.0) return;  // a small step (launch_dt_final)
+    mom_x_body<MODE, S>(hw_blk(xcd), g, geo, mf, vfy, vfz, density1, v);
 }
 
 // mom_post_vol's mode of a sweep of advection.f90 (x and z in sweeps 1 and 3,
@@ -887,8 +895,9 @@ static hipError_t fast_advec_mom_t(const double *dt, const Lay &g, const Geo &m,
     const dim3 blk(64, MW, 1);
     if (direction == 1) {
         const dim3 grid((nxn + 59) / 60, (nyn + MW - 2) / (MW - 1), nchunks(nzn, sh.planes));
-        TIMED_LAUNCH("k_fast_mom_x", st, k_fast_mom_x<S>, grid, blk, 0, st, dt, sh.xcd, g, m, mode, mass_flux_x, vol_flux_x,
-                     vol_flux_y, vol_flux_z, density1, v);
+        const auto kern = mode == 1 ? k_fast_mom_x<1, S> : k_fast_mom_x<5, S>;
+        TIMED_LAUNCH("k_fast_mom_x", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, mass_flux_x, vol_flux_y, vol_flux_z,
+                     density1, v);
     } else if (direction == 2) {
         const dim3 grid((nxn + 63) / 64, (nzn + MW - 2) / (MW - 1), nchunks(nyn, sh.planes));
         const auto kern = mode == 3 ? k_fast_mom_march<2, 3, S> : k_fast_mom_march<2, 4, S>;
@@ -947,9 +956,9 @@ int batch_blocks_mom(int dir, const Lay &g, int planes)
     return gx * gy * gz;
 }
 
-template <int DIR, int MODE, typename S>  // MODE: 0 for the x sweep, which takes `mode`
+template <int DIR, int MODE, typename S>
 __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
-                                         int mode, int planes, const MomSlots &ms, int hb)
+                                         int planes, const MomSlots &ms, int hb)
 {
     const int d = deck_of(start, nd, hb);
     const DeckDev &D = decks[d];
@@ -968,7 +977,7 @@ __device__ __forceinline__ void mom_tile(const DeckDev *__restrict__ decks, cons
     const S *vfz = static_cast<const S *>(D.f[F_VOL_FLUX_Z]);
     const S *rho = static_cast<const S *>(D.f[ms.rho]);
     if constexpr (DIR == 1)
-        mom_x_body<S>(bk, D.g, D.m, mode, static_cast<const S *>(D.f[F_MASS_FLUX_X]), vfx, vfy, vfz, rho, v);
+        mom_x_body<MODE, S>(bk, D.g, D.m, static_cast<const S *>(D.f[F_MASS_FLUX_X]), vfy, vfz, rho, v);
     else
         mom_march<DIR, MODE, S>(lb, gx, gy, gz, 0, D.g, D.m,
                                 static_cast<const S *>(D.f[DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z]), vfx, vfy, vfz,
@@ -979,13 +988,12 @@ template <int DIR, int MODE, typename S>
 // The FP64 y/z sweeps held to four waves per SIMD (128 VGPRs): at five they
 // spill 18-34 values and the launches of 320^3 as 8 tiles ran 2.00 -> 2.42 ms.
 __global__ void __launch_bounds__(64 * mw_of(DIR), DIR != 1 && sizeof(S) == 8 ? 4 : 1)
-kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int mode, int planes, int xcd,
-       MomSlots ms)
+kb_mom(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd, MomSlots ms)
 {
     int hb, end, step;  // the tiles of this workgroup (persistent when the grid is short)
     tile_walk(start[nd], xcd, hb, end, step);
     for (; hb < end; hb += step) {
-        mom_tile<DIR, MODE, S>(decks, start, nd, mode, planes, ms, hb);
+        mom_tile<DIR, MODE, S>(decks, start, nd, planes, ms, hb);
         __syncthreads();  // the next tile reuses the workgroup's LDS
     }
 }
@@ -999,9 +1007,10 @@ hipError_t batch_advec_mom(Store s, const DeckDev *decks, int nd, const BatchGri
     const dim3 grid(batch_wgs(bg, sh)), blk(64, mw_of(dir));
     const MomSlots ms{sl[F_DENSITY1], {sl[F_XVEL1], sl[F_YVEL1], sl[F_ZVEL1]}, {sl[X_W5], sl[X_W6], sl[X_W7]}};
 #define L(D_, M_, T_)                                                                                        \
-    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, M_, T_>), grid, blk, 0, st, decks, bg.start, nd, mode, sh.planes, sh.xcd, ms)
+    TIMED_LAUNCH("kb_mom", st, (kb_mom<D_, M_, T_>), grid, blk, 0, st, decks, bg.start, nd, sh.planes, sh.xcd, ms)
 #define LM(T_)                                                                                               \
-    if (dir == 1) L(1, 0, T_);                                                                               \
+    if (mode == 1) L(1, 1, T_);                                                                              \
+    else if (mode == 5) L(1, 5, T_);                                                                         \
     else if (mode == 3) L(2, 3, T_);                                                                         \
     else if (mode == 4) L(2, 4, T_);                                                                         \
     else if (mode == 2) L(3, 2, T_);                                                                         \
