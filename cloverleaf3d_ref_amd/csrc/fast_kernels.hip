@@ -14,9 +14,8 @@
 // The stencils here read two neighbouring planes (l and l+1 for cells and
 // faces, l-1 and l for nodes).  Each thread owns one (j, k) column and
 // marches up a chunk of planes, keeping the lower plane's values in
-// registers (or, in accel_pdv, in an LDS ring shared by the workgroup), so
-// every plane is read from memory once per column instead of once per
-// plane that uses it.
+// registers, so every plane is read from memory once per column instead of
+// once per plane that uses it.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -28,9 +27,7 @@
 namespace clover {
 
 // 2x2 corner values of an array around (j, k) in one plane, in the storage
-// type (which is also the arithmetic type of the form):
-//   quad_up:   v[a + 2b] = p(j+a, k+b)           (a, b in {0, 1})
-//   quad_down: v[(a+1) + 2(b+1)] = p(j+a, k+b)   (a, b in {-1, 0})
+// type (which is also the arithmetic type of the form): v[a + 2b] = p(j+a, k+b)
 template <typename S>
 struct QuadS {
     S v[4];
@@ -40,40 +37,6 @@ template <typename S>
 __device__ inline QuadS<S> quad_up_raw(const S *__restrict__ p, int i, int ld)
 {
     return QuadS<S>{{p[i], p[i + 1], p[i + ld], p[i + 1 + ld]}};
-}
-
-template <typename S>
-__device__ inline QuadS<S> quad_down_raw(const S *__restrict__ p, int i, int ld)
-{
-    return QuadS<S>{{p[i - 1 - ld], p[i - ld], p[i - 1], p[i]}};
-}
-
-// A quad_down_raw quad at mirrored faces (Lay::mirror): at the x_min face
-// (xlo) the halo column j-1 takes the values of column j, which its
-// reflection copies, at the x_max face (xhi) column j those of j-1; the
-// same for the rows k-1 and k at the y faces.  The halo values were loaded
-// (in bounds) and are replaced where the quad is used, so the loads keep
-// their constant offsets and stay in flight.
-template <typename S>
-__device__ inline QuadS<S> quad_m(QuadS<S> q, bool xlo, bool xhi, bool ylo, bool yhi)
-{
-    if (xlo) {
-        q.v[0] = q.v[1];
-        q.v[2] = q.v[3];
-    }
-    if (xhi) {
-        q.v[1] = q.v[0];
-        q.v[3] = q.v[2];
-    }
-    if (ylo) {
-        q.v[0] = q.v[2];
-        q.v[1] = q.v[3];
-    }
-    if (yhi) {
-        q.v[2] = q.v[0];
-        q.v[3] = q.v[1];
-    }
-    return q;
 }
 
 // The FP32 forms of visc_dt and the PdV predictor take two cells (j, j+1,
@@ -594,103 +557,6 @@ static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, const double *d
     return hipGetLastError();
 }
 
-// accelerate_kernel.f90:61-109 at one node: density0, pressure and viscosity
-// of the cells (j-1..j, k-1..k) in planes l (du, pu, qu) and l-1 (dl, pl, ql),
-// the node's level-0 velocity (u0, v0, w0) -> its level-1 velocity
-template <typename S>
-__device__ inline void accel_node(const QuadS<S> &du, const QuadS<S> &pu, const QuadS<S> &qu, const QuadS<S> &dl,
-                                  const QuadS<S> &pl, const QuadS<S> &ql, S u0, S v0, S w0, S vol, S xa, S ya, S za,
-                                  S tdt, S &u1, S &v1, S &w1)
-{
-    using T = S;
-    // (a, b, c) in {-1, 0}^3; c = 0 is plane l, c = -1 plane l-1
-#define RV(a, b, c) (((c) ? dl : du).v[((a) + 1) + 2 * ((b) + 1)] * vol)
-#define P(a, b, c) ((c) ? pl : pu).v[((a) + 1) + 2 * ((b) + 1)]
-#define Q(a, b, c) ((c) ? ql : qu).v[((a) + 1) + 2 * ((b) + 1)]
-    const T nodal_mass = (RV(-1, -1, 0) + RV(0, -1, 0) + RV(0, 0, 0) + RV(-1, 0, 0) + RV(-1, -1, -1) +
-                          RV(0, -1, -1) + RV(0, 0, -1) + RV(-1, 0, -1)) *
-                         (T)0.125;
-    const T stepbymass_s = quo((T)0.25 * tdt, nodal_mass);
-    const T xvel1_s = u0 - stepbymass_s * (xa * (P(0, 0, 0) - P(-1, 0, 0)) +
-                                                      xa * (P(0, -1, 0) - P(-1, -1, 0)) +
-                                                      xa * (P(0, 0, -1) - P(-1, 0, -1)) +
-                                                      xa * (P(0, -1, -1) - P(-1, -1, -1)));
-    const T yvel1_s = v0 - stepbymass_s * (ya * (P(0, 0, 0) - P(0, -1, 0)) +
-                                                      ya * (P(-1, 0, 0) - P(-1, -1, 0)) +
-                                                      ya * (P(0, 0, -1) - P(0, -1, -1)) +
-                                                      ya * (P(-1, 0, -1) - P(-1, -1, -1)));
-    const T zvel1_s = w0 - stepbymass_s * (za * (P(0, 0, 0) - P(0, 0, -1)) +
-                                                      za * (P(0, -1, 0) - P(0, -1, -1)) +
-                                                      za * (P(-1, 0, 0) - P(-1, 0, -1)) +
-                                                      za * (P(-1, -1, 0) - P(-1, -1, -1)));
-    u1 = xvel1_s - stepbymass_s * (xa * (Q(0, 0, 0) - Q(-1, 0, 0)) + xa * (Q(0, -1, 0) - Q(-1, -1, 0)) +
-                                         xa * (Q(0, 0, -1) - Q(-1, 0, -1)) + xa * (Q(0, -1, -1) - Q(-1, -1, -1)));
-    v1 = yvel1_s - stepbymass_s * (ya * (Q(0, 0, 0) - Q(0, -1, 0)) + ya * (Q(-1, 0, 0) - Q(-1, -1, 0)) +
-                                         ya * (Q(0, 0, -1) - Q(0, -1, -1)) + ya * (Q(-1, 0, -1) - Q(-1, -1, -1)));
-    w1 = zvel1_s - stepbymass_s * (za * (Q(0, 0, 0) - Q(0, 0, -1)) + za * (Q(0, -1, 0) - Q(0, -1, -1)) +
-                                         za * (Q(-1, 0, 0) - Q(-1, 0, -1)) + za * (Q(-1, -1, 0) - Q(-1, -1, -1)));
-#undef RV
-#undef P
-#undef Q
-}
-
-// PdV corrector (PdV_kernel.f90:126-164) and flux_calc (flux_calc_kernel.f90:
-// 56-90) at plane l of column (j, k), offset i.  at(c, a, b, p) is the
-// velocity component c (0-2 level 0 x/y/z, 3-5 level 1 x/y/z) of node
-// (j+a, k+b) in node plane l+p; plane l+1 is read only when lin
-// (l <= z_max).  The cell's level-0 state is (d0, e0v, p0, q0).
-template <typename S, typename NodeAt>
-__device__ inline void corrector_plane(int i, bool jin, bool kin, bool lin, const NodeAt &at, S d0, S e0v, S p0,
-                                       S q0, S xa, S ya, S za, S vol, S tdt, S c0, S *__restrict__ density1,
-                                       S *__restrict__ energy1, S *__restrict__ vol_flux_x,
-                                       S *__restrict__ vol_flux_y, S *__restrict__ vol_flux_z)
-{
-    using T = S;
-#define U0(a, b, c) at(0, a, b, c)
-#define V0(a, b, c) at(1, a, b, c)
-#define W0(a, b, c) at(2, a, b, c)
-#define U1(a, b, c) at(3, a, b, c)
-#define V1(a, b, c) at(4, a, b, c)
-#define W1(a, b, c) at(5, a, b, c)
-    T sl = 0, sb = 0;
-    if (kin && lin) {
-        sl = U0(0, 0, 0) + U0(0, 1, 0) + U0(0, 0, 1) + U0(0, 1, 1) + U1(0, 0, 0) + U1(0, 1, 0) + U1(0, 0, 1) + U1(0, 1, 1);
-        vol_flux_x[i] = c0 * xa * sl;
-    }
-    if (jin && lin) {
-        sb = V0(0, 0, 0) + V0(1, 0, 0) + V0(0, 0, 1) + V0(1, 0, 1) + V1(0, 0, 0) + V1(1, 0, 0) + V1(0, 0, 1) + V1(1, 0, 1);
-        vol_flux_y[i] = c0 * ya * sb;
-    }
-    if (jin && kin)
-        vol_flux_z[i] = c0 * za *
-                        (W0(0, 0, 0) + W0(1, 0, 0) + W0(1, 0, 0) + W0(1, 1, 0) + W1(0, 0, 0) + W1(1, 0, 0) + W1(0, 1, 0) +
-                         W1(1, 1, 0));
-    if (jin && kin && lin) {
-        const T sr = U0(1, 0, 0) + U0(1, 1, 0) + U0(1, 0, 1) + U0(1, 1, 1) + U1(1, 0, 0) + U1(1, 1, 0) + U1(1, 0, 1) + U1(1, 1, 1);
-        const T stp = V0(0, 1, 0) + V0(1, 1, 0) + V0(0, 1, 1) + V0(1, 1, 1) + V1(0, 1, 0) + V1(1, 1, 0) + V1(0, 1, 1) + V1(1, 1, 1);
-        const T sk = W0(0, 0, 0) + W0(1, 0, 0) + W0(0, 1, 0) + W0(1, 1, 0) + W1(0, 0, 0) + W1(1, 0, 0) + W1(0, 1, 0) + W1(1, 1, 0);
-        const T sf = W0(0, 0, 1) + W0(1, 0, 1) + W0(0, 1, 1) + W0(1, 1, 1) + W1(0, 0, 1) + W1(1, 0, 1) + W1(0, 1, 1) + W1(1, 1, 1);
-        const T left_flux = (xa * sl) * (T)0.125 * tdt;
-        const T right_flux = (xa * sr) * (T)0.125 * tdt;
-        const T bottom_flux = (ya * sb) * (T)0.125 * tdt;
-        const T top_flux = (ya * stp) * (T)0.125 * tdt;
-        const T back_flux = (za * sk) * (T)0.125 * tdt;
-        const T front_flux = (za * sf) * (T)0.125 * tdt;
-        const T total_flux = right_flux - left_flux + top_flux - bottom_flux + front_flux - back_flux;
-        const T vol_change_s = quo(vol, vol + total_flux);
-        const T recip_volume = (T)1 / vol;
-        const T energy_change = (quo(p0, d0) + quo_sparse(q0, d0)) * total_flux * recip_volume;
-        energy1[i] = e0v - energy_change;
-        density1[i] = d0 * vol_change_s;
-    }
-#undef U0
-#undef V0
-#undef W0
-#undef U1
-#undef V1
-#undef W1
-}
-
 // ---------------------------------------------------------------------------
 // field_summary_kernel.f90:51-78 with the scalar cell volume; same
 // reduction tree as the per-call kernel.
@@ -806,183 +672,6 @@ static hipError_t fast_ideal_gas_t(const Lay &g, const S *density, const S *ener
 }
 
 // ---------------------------------------------------------------------------
-// accelerate (accelerate_kernel.f90:61-109), then the PdV corrector and
-// flux_calc on its results (PdV.f90 + flux_calc.f90 follow accelerate in
-// hydro.f90:56-60), in one z-march: the level-1 velocities are stored once
-// and handed to the corrector on chip instead of being read back.
-//
-// A workgroup is 64 lanes (x) by AW waves (y); lane 63 and wave AW-1 are a
-// halo column and row, so workgroups step by 63 and AW-1.  At node plane lp
-// every thread forms the level-1 velocity of its node (accel_node, as the
-// accelerate kernel does; owners store it) from its cells' quads (read from
-// memory one plane ahead) and its own level-0 velocity.  Both velocity
-// levels of the plane go to LDS, into a ring of two planes with two
-// barriers per plane, and the owners then run the corrector and fluxes of
-// plane lp-1 (corrector_plane) reading the node quads of planes lp-1 and lp
-// from the ring; the plane below is read back rather than held in
-// registers.  Each chunk also forms the level-1 velocity of the plane above
-// it, which the next chunk stores.
-// 12 waves: in FP64 the kernel takes 144 VGPRs, three waves per SIMD, so
-// one 12-wave workgroup per CU keeps 12 waves in flight where 8-wave ones
-// kept 8 (4.14 -> 4.05 ms FP64, 2.26 -> 2.23 ms FP32 at 512^3); 10 waves
-// were slower in FP32.  The FP32 kernel is held to 80 VGPRs (six waves per
-// SIMD, two workgroups per CU, one value spilled) instead of 81 (five, one
-// workgroup): 2.15 -> 2.05 ms at 512^3.  16 waves (FP64 held to 128 VGPRs,
-// four waves per SIMD, seven values spilled) ran slower: 4.04 -> 4.55 ms
-// FP64, 2.39 -> 2.55 ms FP32.
-constexpr int AW = 12;
-
-template <typename S>
-__device__ __forceinline__ void accel_pdv_body(const Blk &bk, Lay g, Geo m, double dt,
-                                               const S *__restrict__ density0, S *__restrict__ density1,
-                                               const S *__restrict__ energy0, S *__restrict__ energy1,
-                                               const S *__restrict__ pressure, const S *__restrict__ viscosity,
-                                               const S *__restrict__ xvel0, S *__restrict__ xvel1,
-                                               const S *__restrict__ yvel0, S *__restrict__ yvel1,
-                                               const S *__restrict__ zvel0, S *__restrict__ zvel1,
-                                               S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y,
-                                               S *__restrict__ vol_flux_z)
-{
-    using T = S;  // arithmetic type of the form
-    // node velocities (level 0 x/y/z, level 1 x/y/z) of two node planes.
-    // Slot s is written at plane t (before the first barrier of t) and read
-    // at planes t and t+1 (between their two barriers); it is written again
-    // at t+2, past the second barrier of t+1, which every thread reaches
-    // only after its reads of t+1.  Two planes rather than three measured
-    // faster (8-wave workgroups at 512^3: 4.29 -> 4.16 ms FP64, 2.29 ->
-    // 2.24 ms FP32).
-    __shared__ S nb[2][6][AW][64];
-    const int lane = (int)threadIdx.x, w = (int)threadIdx.y;
-    const int j = g.x_min + bk.x * 63 + lane;
-    const int k = g.y_min + bk.y * (AW - 1) + w;
-    int l0, l1;
-    chunk_range(bk, g.z_min, g.z_max + 1, l0, l1);
-    if (l0 > l1) return;  // the whole workgroup, before any barrier
-    const bool node = j <= g.x_max + 1 && k <= g.y_max + 1;  // j >= x_min, k >= y_min always
-    const bool own = node && lane < 63 && w < AW - 1;
-    const bool jin = j <= g.x_max, kin = k <= g.y_max;
-    const T xa = (T)m.xa, ya = (T)m.ya, za = (T)m.za, vol = (T)m.vol, tdt = (T)dt;
-    const T c0 = (T)0.125 * tdt;
-    const int ln = min(lane + 1, 63), wn = min(w + 1, AW - 1);
-    int i = idx(g, j, k, l0);
-    // accelerate's cells of the plane below the node plane
-    QuadS<S> dlo{}, plo{}, qlo{};
-    // the next plane's loads, issued one plane ahead of their use: its cells
-    // (accelerate), the node's level-0 velocity and the cell's energy0
-    QuadS<S> dn{}, pn{}, qn{};
-    S u0n = 0, v0n = 0, w0n = 0, e0n = 0;
-    // mirrored faces: the node's cells j-1 (x_min face) or j (x_max face),
-    // k-1 or k (y faces) and the planes below z_min or above z_max are halo
-    // cells, read as the interior cells they mirror
-    const bool mlo = cell_m(g, 0, j - 1) != j - 1, mhi = cell_m(g, 0, j) != j;
-    const bool ylo = cell_m(g, 1, k - 1) != k - 1, yhi = cell_m(g, 1, k) != k;
-    auto load = [&](int ii, int lp) {
-        dn = quad_down_raw(density0, ii, g.ld);
-        pn = quad_down_raw(pressure, ii, g.ld);
-        qn = quad_down_raw(viscosity, ii, g.ld);
-        u0n = xvel0[ii];
-        v0n = yvel0[ii];
-        w0n = zvel0[ii];
-        e0n = (lp <= g.z_max && jin && kin) ? energy0[ii] : (S)0;
-    };
-    if (node) {
-        dlo = quad_m(quad_down_raw(density0, i - g.plane, g.ld), mlo, mhi, ylo, yhi);
-        plo = quad_m(quad_down_raw(pressure, i - g.plane, g.ld), mlo, mhi, ylo, yhi);
-        qlo = quad_m(quad_down_raw(viscosity, i - g.plane, g.ld), mlo, mhi, ylo, yhi);
-        load(i, l0);
-    }
-    T e0p = 0;  // energy0 of the cell below
-    const int lend = min(l1 + 1, g.z_max + 1);
-    int s = 0, sp = 1;  // ring slots of the node plane in hand and the one below
-    for (int lp = l0; lp <= lend; lp++, i += g.plane) {
-        QuadS<S> dhi = quad_m(dn, mlo, mhi, ylo, yhi), phi = quad_m(pn, mlo, mhi, ylo, yhi),
-                 qhi = quad_m(qn, mlo, mhi, ylo, yhi);
-        // mirrored z faces: the cell plane below z_min is read as plane
-        // z_min, the one above z_max as plane z_max
-        if (cell_m(g, 2, lp - 1) != lp - 1) {
-            dlo = dhi;
-            plo = phi;
-            qlo = qhi;
-        }
-        if (cell_m(g, 2, lp) != lp) {
-            dhi = dlo;
-            phi = plo;
-            qhi = qlo;
-        }
-        const S u0 = u0n, v0 = v0n, w0 = w0n;
-        const T e0q = (T)e0n;
-        // the next plane's loads go out before this plane's work, so they
-        // have the whole iteration to arrive
-        if (node && lp < lend) load(i + g.plane, lp + 1);
-        S u1 = 0, v1 = 0, w1 = 0;
-        if (node) {
-            accel_node<S>(dhi, phi, qhi, dlo, plo, qlo, u0, v0, w0, vol, xa, ya, za, tdt, u1, v1, w1);
-            if (own && lp <= l1) {
-                xvel1[i] = u1;
-                yvel1[i] = v1;
-                zvel1[i] = w1;
-            }
-        }
-        nb[s][0][w][lane] = u0;
-        nb[s][1][w][lane] = v0;
-        nb[s][2][w][lane] = w0;
-        nb[s][3][w][lane] = u1;
-        nb[s][4][w][lane] = v1;
-        nb[s][5][w][lane] = w1;
-        __syncthreads();
-        const S(*lo)[AW][64] = nb[sp];
-        const S(*up)[AW][64] = nb[s];
-        if (own && lp > l0) {  // plane lp-1, nodes of planes lp-1 and lp; its cell is the (j, k) corner
-            const auto at = [&](int c, int a, int bb, int pl) { return (pl ? up : lo)[c][bb ? wn : w][a ? ln : lane]; };
-            corrector_plane<S>(i - g.plane, jin, kin, true, at, dlo.v[3], e0p, plo.v[3], qlo.v[3], xa, ya, za, vol,
-                               tdt, c0, density1, energy1, vol_flux_x, vol_flux_y, vol_flux_z);
-        }
-        // the top z faces (plane z_max+1) use only their own node plane
-        if (own && lp == lend && l1 == g.z_max + 1) {
-            const auto at = [&](int c, int a, int bb, int) { return up[c][bb ? wn : w][a ? ln : lane]; };
-            corrector_plane<S>(i, jin, kin, false, at, (T)0, (T)0, (T)0, (T)0, xa, ya, za, vol, tdt, c0, density1,
-                               energy1, vol_flux_x, vol_flux_y, vol_flux_z);
-        }
-        dlo = dhi;
-        plo = phi;
-        qlo = qhi;
-        e0p = e0q;
-        sp = s;
-        s ^= 1;
-        __syncthreads();  // the reads of slot sp's plane end before plane lp+1 rewrites it
-    }
-}
-
-template <typename S>
-__global__ void __launch_bounds__(64 * AW, sizeof(S) == 4 ? 6 : 1)
-    k_fast_accel_pdv(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
-                     const S *__restrict__ energy0, S *__restrict__ energy1, const S *__restrict__ pressure,
-                     const S *__restrict__ viscosity, const S *__restrict__ xvel0, S *__restrict__ xvel1,
-                     const S *__restrict__ yvel0, S *__restrict__ yvel1, const S *__restrict__ zvel0,
-                     S *__restrict__ zvel1, S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y,
-                     S *__restrict__ vol_flux_z)
-{
-    const double dt = *dtp;
-    if (dt < 0.0) return;
-    accel_pdv_body<S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, pressure, viscosity, xvel0, xvel1,
-                      yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
-}
-
-template <typename S>
-static hipError_t fast_accel_pdv_t(const Lay &g, const Geo &m, const double *dt, const S *density0, S *density1,
-                                   const S *energy0, S *energy1, const S *pressure, const S *viscosity,
-                                   const S *xvel0, S *xvel1, const S *yvel0, S *yvel1, const S *zvel0, S *zvel1,
-                                   S *vol_flux_x, S *vol_flux_y, S *vol_flux_z, const Shape &sh, hipStream_t st)
-{
-    const int nx = g.x_max - g.x_min + 2, ny = g.y_max - g.y_min + 2, nz = g.z_max - g.z_min + 2;  // nodes
-    const dim3 grid((nx + 62) / 63, (ny + AW - 2) / (AW - 1), nchunks(nz, sh.planes));
-    TIMED_LAUNCH("k_fast_accel_pdv", st, k_fast_accel_pdv<S>, grid, dim3(64, AW, 1), 0, st, sh.xcd, g, m, dt,
-                 density0, density1, energy0, energy1, pressure, viscosity, xvel0, xvel1, yvel0, yvel1, zvel0, zvel1,
-                 vol_flux_x, vol_flux_y, vol_flux_z);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // storage dispatch
 #define CP(T, p) static_cast<const T *>(p)
 #define MP(T, p) static_cast<T *>(p)
@@ -1020,21 +709,6 @@ hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const do
 #undef CALL
 }
 
-hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
-                                 void *density1, const void *energy0, void *energy1, const void *pressure,
-                                 const void *viscosity, const void *xvel0, void *xvel1, const void *yvel0,
-                                 void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,
-                                 void *vol_flux_z, const Shape &sh, hipStream_t st)
-{
-#define CALL(T)                                                                                                 \
-    fast_accel_pdv_t<T>(g, m, dt, CP(T, density0), MP(T, density1), CP(T, energy0), MP(T, energy1),             \
-                        CP(T, pressure), CP(T, viscosity), CP(T, xvel0), MP(T, xvel1), CP(T, yvel0),             \
-                        MP(T, yvel1), CP(T, zvel0), MP(T, zvel1), MP(T, vol_flux_x), MP(T, vol_flux_y),          \
-                        MP(T, vol_flux_z), sh, st)
-    return s == ST_F32 ? CALL(float) : CALL(double);
-#undef CALL
-}
-
 hipError_t launch_fast_field_summary(Store s, const Lay &g, const Geo &m, const void *density0, const void *energy0,
                                      const void *pressure, const void *xvel0, const void *yvel0, const void *zvel0,
                                      double *partial, int *nparts, hipStream_t st)
@@ -1064,13 +738,6 @@ __host__ __device__ inline void dims_cells(const Lay &g, int planes, int cpt, in
     gx = (g.x_max - g.x_min + cpt * BX) / (cpt * BX);
     gy = (g.y_max - g.y_min + BY) / BY;
     gz = nchunks(g.z_max - g.z_min + 1, planes);
-}
-
-__host__ __device__ inline void dims_accel_pdv(const Lay &g, int planes, int &gx, int &gy, int &gz)
-{
-    gx = (g.x_max - g.x_min + 2 + 62) / 63;
-    gy = (g.y_max - g.y_min + 2 + AW - 2) / (AW - 1);
-    gz = nchunks(g.z_max - g.z_min + 2, planes);
 }
 
 __host__ __device__ inline int summary_blocks(const Lay &g)
@@ -1155,21 +822,6 @@ kb_pdv_predict(const DeckDev *__restrict__ decks, const int *__restrict__ start,
     }
 }
 
-template <typename S>
-// held to six waves per SIMD in FP32 like k_fast_accel_pdv (80 VGPRs, no spill here)
-__global__ void __launch_bounds__(64 * AW, sizeof(S) == 4 ? 6 : 1)
-kb_accel_pdv(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd)
-{
-    FOR_TILES(xcd)
-    {
-        DECK_TILE(t_, dims_accel_pdv(D.g, planes, gx, gy, gz))
-        accel_pdv_body<S>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), MF(F_DENSITY1), CF(F_ENERGY0), MF(F_ENERGY1),
-                          CF(F_PRESSURE), CF(F_VISCOSITY), CF(F_XVEL0), MF(F_XVEL1), CF(F_YVEL0), MF(F_YVEL1),
-                          CF(F_ZVEL0), MF(F_ZVEL1), MF(F_VOL_FLUX_X), MF(F_VOL_FLUX_Y), MF(F_VOL_FLUX_Z));
-        __syncthreads();
-    }
-}
-
 __host__ __device__ inline void dims_summary(const Lay &g, int &gx, int &gy, int &gz)
 {
     gx = summary_blocks(g);
@@ -1204,7 +856,7 @@ int batch_blocks(BatchKernel k, const Lay &g, int planes, Store s)
     case BK_IDEAL_GAS: dims_ideal(g, gx, gy, gz); break;
     case BK_VISC_DT:
     case BK_PDV_PREDICT: dims_cells(g, planes, s == ST_F32 ? 2 : 1, gx, gy, gz); break;
-    case BK_ACCEL_PDV: dims_accel_pdv(g, planes, gx, gy, gz); break;
+    case BK_ACCEL_PDV:
     case BK_LAGRANGE: return batch_blocks_lagrange(g, planes, s);
     case BK_SUMMARY: dims_summary(g, gx, gy, gz); break;
     case BK_CELL_X: return batch_blocks_cell(1, g, planes);
@@ -1279,7 +931,6 @@ Shapes size_shapes(Store s, const Lay *lays, int n)
     } const marches[] = {
         {SK_VISC_DT, BK_VISC_DT, 16, 5 * cus, 0},
         {SK_PDV_PREDICT, BK_PDV_PREDICT, 8, 5 * cus, 0},
-        {SK_ACCEL_PDV, BK_ACCEL_PDV, f32 ? 8 : 32, f32 ? 2 * cus : cus, far},
         {SK_CELL_Y, BK_CELL_Y, 16, 5 * cus, 0},
         {SK_CELL_Z, BK_CELL_Z, 16, 5 * cus, 0},
         {SK_MOM_X, BK_MOM_X, 8, 5 * cus, far},
@@ -1294,14 +945,16 @@ Shapes size_shapes(Store s, const Lay *lays, int n)
     for (const auto &m : marches)
         sh.k[m.shape] = Shape{size_planes(m.k, s, lays, n, m.slots, m.cap), m.xcd, 64, 0, m.cap};
     // accel_pdv's shape is the Lagrangian march's where that runs: three extra
-    // planes per chunk (two predicted below it, one accelerated above), one
-    // workgroup per CU in FP64, two in FP32.  64^3 FP64 22.5 us at the rule's 4
-    // planes (61.8 at 32), 131 x 75 x 93 41.6 at 12 (10 by the rule; 83.9 at 32),
-    // FP32 101 x 143 x 67 27.2 at 8; 512^3 FP32 2.10 ms at 8, 2.31 at 32.
-    if (lagrange) {
-        const int cap = f32 ? 8 : 32;
-        sh.k[SK_ACCEL_PDV] = Shape{size_planes(BK_LAGRANGE, s, lays, n, f32 ? 2 * cus : cus, cap, 3), far, 64, 0, cap};
-    }
+    // planes per chunk (two predicted below it, one accelerated above; without the
+    // predictor one and one), one workgroup per CU in FP64, two in FP32.  64^3
+    // FP64 22.5 us at the rule's 4 planes (61.8 at 32), 131 x 75 x 93 41.6 at 12
+    // (10 by the rule; 83.9 at 32), FP32 101 x 143 x 67 27.2 at 8; 512^3 FP32 2.10
+    // ms at 8, 2.31 at 32.  Without the predictor, 320^3 as 8 tiles FP64 1.10 ms
+    // at 16, 1.15 at 32, 1.08 at 8; 160^3 as 8 0.194 ms at 8 and 16, 0.185 at 12.
+    const int cap = !lagrange ? 16 : f32 ? 8 : 32;
+    sh.k[SK_ACCEL_PDV] = Shape{size_planes(lagrange ? BK_LAGRANGE : BK_ACCEL_PDV, s, lays, n, f32 ? 2 * cus : cus, cap,
+                                           lagrange ? 3 : 2),
+                               far, 64, 0, cap};
     return sh;
 }
 
@@ -1338,13 +991,6 @@ hipError_t batch_pdv_predict(Store s, const DeckDev *decks, int nd, const BatchG
 {
     if (s == ST_F32) BLAUNCH_SH("kb_pdv_predict", kb_pdv_predict<float>, dim3(BX, BY), decks, bg.start, nd, sh.planes, sh.xcd);
     else BLAUNCH_SH("kb_pdv_predict", kb_pdv_predict<double>, dim3(BX, BY), decks, bg.start, nd, sh.planes, sh.xcd);
-    return hipGetLastError();
-}
-
-hipError_t batch_accel_pdv(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, const Shape &sh, hipStream_t st)
-{
-    if (s == ST_F32) BLAUNCH_SH("kb_accel_pdv", kb_accel_pdv<float>, dim3(64, AW), decks, bg.start, nd, sh.planes, sh.xcd);
-    else BLAUNCH_SH("kb_accel_pdv", kb_accel_pdv<double>, dim3(64, AW), decks, bg.start, nd, sh.planes, sh.xcd);
     return hipGetLastError();
 }
 

@@ -4,8 +4,9 @@
 // (accelerate_kernel.f90:61-109), the PdV corrector (PdV_kernel.f90:126-164)
 // and flux_calc (flux_calc_kernel.f90:56-90), which hydro.f90:52-60 runs one
 // after the other.  Such a tile needs no exchange between them: the predicted
-// pressure's halo is the mirrored interior cell's.  Tiled chunks exchange that
-// pressure between tiles and keep the two kernels of fast_kernels.hip.
+// pressure's halo is the mirrored interior cell's.  Tiled and thin chunks
+// exchange that pressure: they run the predictor of fast_kernels.hip, then this
+// march without its own (k_fast_accel_pdv).
 //
 // Bytes.  Those two read the level-0 state twice and pass the predicted
 // pressure through memory: 7 + 15 arrays per cell.  Here the state is read once
@@ -103,11 +104,20 @@ __device__ inline void accel_by(const AccelTerms<T> &hi, const AccelTerms<T> &lo
     w = w - st * (z0 + z1 + prev_lane(z0) + prev_lane(z1));
 }
 
-template <typename S>
+// PRED: the whole phase, on a lagrange_tile (512^3: see above).  Otherwise accelerate, the
+// corrector and flux_calc of any tile, after its predicted pressure (`pressure`)
+// has been exchanged: the cells around the tile are read from its halo, or where
+// a face is mirrored from the interior.  That form's own kernel before (quads
+// read from memory and selected at mirrored faces, both velocity levels through
+// LDS, 378 VALU instructions per plane against 252) ran 320^3 as 8 tiles FP64
+// 1.31 -> 1.10 ms, FP32 0.584 -> 0.588, 160^3 as 8 227 -> 179 us and 89 -> 86,
+// 512^3 as 4 tiles 4.90 -> 4.43 ms, 48x40x44 as 8 the same (three rounds on one
+// machine).
+template <bool PRED, typename S>
 __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, double dt,
                                               const S *__restrict__ density0, S *__restrict__ density1,
                                               const S *__restrict__ energy0, S *__restrict__ energy1,
-                                              const S *__restrict__ viscosity, const S *__restrict__ xvel0,
+                                              const S *__restrict__ pressure, const S *__restrict__ viscosity, const S *__restrict__ xvel0,
                                               S *__restrict__ xvel1, const S *__restrict__ yvel0,
                                               S *__restrict__ yvel1, const S *__restrict__ zvel0,
                                               S *__restrict__ zvel1, S *__restrict__ vol_flux_x,
@@ -130,8 +140,9 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
     const bool crow = march && k <= g.y_max;                            // and of cells
     const int wu = min(w + 1, LW - 1);
     // rows of cb that hold the cells of rows k-1 and k: across a mirrored y
-    // face the halo row is the interior one
-    const int r1 = k <= g.y_min ? w : w - 1, r0 = k > g.y_max ? w - 1 : w;
+    // face the halo row is the interior one, which without the predictor was
+    // loaded there
+    const int r1 = PRED && k <= g.y_min ? w : w - 1, r0 = PRED && k > g.y_max ? w - 1 : w;
     const bool xedge = bk.x == 0 || bk.x == bk.gx - 1;  // the block may hold halo columns
     const T xa = (T)m.xa, ya = (T)m.ya, za = (T)m.za, vol = (T)m.vol, tdt = (T)dt;
     // the fluxes' factors 0.125 and 0.5 are powers of two: scaling dt by them
@@ -141,34 +152,40 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
     const T cx = c0 * xa, cy = c0 * ya, cz = c0 * za;
     const T recip_volume = (T)1 / vol;
     const int lend = min(l1 + 1, g.z_max + 1);  // last node plane accelerated
-    const int clast = min(lend, g.z_max);       // last cell plane predicted
-    // first cell plane predicted: l0-1 (the plane below z_min is mirrored)
-    const int lp0 = l0 > g.z_min ? l0 - 1 : l0;
+    // last and first cell plane predicted (the planes past mirrored z faces are
+    // not), or loaded
+    const int clast = PRED ? min(lend, g.z_max) : lend;
+    const int lp0 = !PRED || l0 > g.z_min ? l0 - 1 : l0;
     // lanes outside the mesh read the nearest column and row inside it: nodes
-    // to x_max+1, cells (mirrored halo cells among them) to x_max
-    const int jn = min(max(j, g.x_min), g.x_max + 1), jc = min(max(j, g.x_min), g.x_max);
-    const int kn = min(max(k, g.y_min), g.y_max + 1), kc = min(max(k, g.y_min), g.y_max);
+    // to x_max+1, cells (mirrored halo cells among them) to x_max; without the
+    // predictor cells are read one into the halo where that is not mirrored
+    const int jn = min(max(j, g.x_min), g.x_max + 1);
+    const int kn = min(max(k, g.y_min), g.y_max + 1);
+    const int jc = PRED ? min(max(j, g.x_min), g.x_max) : cell_m(g, 0, min(j, g.x_max + 1));
+    const int kc = PRED ? min(max(k, g.y_min), g.y_max) : cell_m(g, 1, min(k, g.y_max + 1));
     const int kn2 = min(k + LW, g.y_max + 1);  // wave 0: the row above the last wave's
-    unsigned on = (unsigned)(jn - g.x_min) * (unsigned)sizeof(S);
-    unsigned oc = (unsigned)(jc - g.x_min) * (unsigned)sizeof(S);
+    const int xb = PRED ? g.x_min : g.x_min - 1;  // rows are addressed from here
+    unsigned on = (unsigned)(jn - xb) * (unsigned)sizeof(S);
+    unsigned oc = (unsigned)(jc - xb) * (unsigned)sizeof(S);
 
-    S un, vn, wn, u2n = 0, v2n = 0, w2n = 0, dn, en, qn;  // the next planes' loads
+    S un, vn, wn, u2n = 0, v2n = 0, w2n = 0, dn, en, pn = 0, qn;  // the next planes' loads
     auto load_nodes = [&](int l) {
-        const int64_t r = idx(g, g.x_min, kn, l);
+        const int64_t r = idx(g, xb, kn, l);
         un = at(xvel0 + r, on);
         vn = at(yvel0 + r, on);
         wn = at(zvel0 + r, on);
         if (w == 0) {
-            const int64_t r2 = idx(g, g.x_min, kn2, l);
+            const int64_t r2 = idx(g, xb, kn2, l);
             u2n = at(xvel0 + r2, on);
             v2n = at(yvel0 + r2, on);
             w2n = at(zvel0 + r2, on);
         }
     };
     auto load_cells = [&](int l) {
-        const int64_t r = idx(g, g.x_min, kc, l);
+        const int64_t r = idx(g, xb, kc, PRED ? l : cell_m(g, 2, l));
         dn = at(density0 + r, oc);
         en = at(energy0 + r, oc);
+        if constexpr (!PRED) pn = at(pressure + r, oc);
         qn = at(viscosity + r, oc);
     };
     auto put_nodes = [&](int s) {
@@ -203,8 +220,9 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
         return (za * (s4 + wa + wan + wb + wbn)) * cp;  // the predictor's flux: each node twice
     };
     // PdV predictor and ideal_gas of a cell plane of parity p, between the
-    // node planes of parity p (below) and 1-p
-    auto predict = [&](auto par, T d0, T e0, T q0) {
+    // node planes of parity p (below) and 1-p; without PRED the level-0 sums
+    // alone, and pp is the predicted pressure
+    auto predict = [&](auto par, T d0, T e0, T pp, T q0) {
         constexpr int p = decltype(par)::value;
         auto &C = cell[p];
         const T ua = n0[p][0][w][lane], ub = n0[p][0][w + 1][lane];
@@ -216,23 +234,29 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
         C.sl = ua + ub + uc + ud;
         C.sb = va + van + vc + vcn;
         C.st = vb + vbn + vd + vdn;
-        const T left_flux = (xa * (C.sl + ua + ub + uc + ud)) * cp;
-        const T right_flux = next_lane(left_flux);
-        const T bottom_flux = (ya * (C.sb + va + van + vc + vcn)) * cp;
-        const T top_flux = (ya * (C.st + vb + vbn + vd + vdn)) * cp;
-        const T front_flux = z_face(wa, wb, sz[1 - p], qz[1 - p]);
-        const T total_flux = right_flux - left_flux + top_flux - bottom_flux + front_flux - zp;
-        zp = front_flux;
-        const T p0 = pressure_of<T>(d0, e0);
-        const T vol_change_s = quo(vol, vol + total_flux);
-        const T qd = quo_sparse(q0, d0);
-        const T energy_change = (quo(p0, d0) + qd) * total_flux * recip_volume;
-        const T e1 = e0 - energy_change;
-        const T d1 = d0 * vol_change_s;
-        T pp = (T)(1.4 - 1.0) * d1 * e1;
-        if (xedge) {  // mirrored halo columns take their neighbour's (density and viscosity were loaded there)
-            const T lo = next_lane(pp), hi = prev_lane(pp);
-            pp = j < g.x_min ? lo : j > g.x_max ? hi : pp;
+        T qd;
+        if constexpr (!PRED) {
+            z_face(wa, wb, sz[1 - p], qz[1 - p]);
+            qd = quo_sparse(q0, d0);
+        } else {
+            const T left_flux = (xa * (C.sl + ua + ub + uc + ud)) * cp;
+            const T right_flux = next_lane(left_flux);
+            const T bottom_flux = (ya * (C.sb + va + van + vc + vcn)) * cp;
+            const T top_flux = (ya * (C.st + vb + vbn + vd + vdn)) * cp;
+            const T front_flux = z_face(wa, wb, sz[1 - p], qz[1 - p]);
+            const T total_flux = right_flux - left_flux + top_flux - bottom_flux + front_flux - zp;
+            zp = front_flux;
+            const T p0 = pressure_of<T>(d0, e0);
+            const T vol_change_s = quo(vol, vol + total_flux);
+            qd = quo_sparse(q0, d0);
+            const T energy_change = (quo(p0, d0) + qd) * total_flux * recip_volume;
+            const T e1 = e0 - energy_change;
+            const T d1 = d0 * vol_change_s;
+            pp = (T)(1.4 - 1.0) * d1 * e1;
+            if (xedge) {  // mirrored halo columns take their neighbour's (density and viscosity were loaded there)
+                const T lo = next_lane(pp), hi = prev_lane(pp);
+                pp = j < g.x_min ? lo : j > g.x_max ? hi : pp;
+            }
         }
         C.a = quo(pp, d0) + qd;
         C.d = d0;
@@ -251,11 +275,11 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
         // ---- X
         T u = n0[s][0][w][lane], v = n0[s][1][w][lane], ww = n0[s][2][w][lane];
         put_nodes(s);
-        const T d0 = dn, e0 = en, q0 = qn;
-        if (lp + 3 <= clast + 1) load_nodes(lp + 3);
+        const T d0 = dn, e0 = en, p0 = pn, q0 = qn;
+        if (lp + 3 <= clast + PRED) load_nodes(lp + 3);
         if (lp + 2 <= clast) load_cells(lp + 2);
         if (w >= 1) {
-            if (lp <= g.z_max) {
+            if (!PRED || lp <= g.z_max) {
                 pt[s] = accel_terms<T>(cb[1][r0][lane], cb[1][r1][lane], xa, ya);
                 qt[s] = accel_terms<T>(cb[2][r0][lane], cb[2][r1][lane], xa, ya);
                 m0[s] = cb[0][r0][lane] * vol;
@@ -263,7 +287,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
             } else {  // the plane above z_max mirrors z_max
                 pt[s] = pt[1 - s], qt[s] = qt[1 - s], m0[s] = m0[1 - s], m1[s] = m1[1 - s];
             }
-            if (lp == g.z_min)  // the plane below z_min mirrors z_min
+            if (PRED && lp == g.z_min)  // the plane below z_min mirrors z_min
                 pt[1 - s] = pt[s], qt[1 - s] = qt[s], m0[1 - s] = m0[s], m1[1 - s] = m1[s];
             if (lp >= l0) {
                 const T nodal_mass = (prev_lane(m1[s]) + m1[s] + m0[s] + prev_lane(m0[s]) + prev_lane(m1[1 - s]) +
@@ -276,7 +300,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
                 n1[s][1][w][lane] = v;
                 n1[s][2][w][lane] = ww;
                 if (march && lp <= l1 && cols) {
-                    const int64_t r = idx(g, g.x_min, k, lp);
+                    const int64_t r = idx(g, xb, k, lp);
                     at(xvel1 + r, on) = u;
                     at(yvel1 + r, on) = v;
                     at(zvel1 + r, on) = ww;
@@ -290,7 +314,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
             const T wan = next_lane(wa), wbn = next_lane(wb);
             const T zflux = (za * (sz[s] + wa + wan + wb + wbn)) * c0;
             if (crow && lp <= l1 && ccols)
-                at(vol_flux_z + (int64_t)idx(g, g.x_min, k, lp), oc) = cz * (qz[s] + wa + wan + wb + wbn);
+                at(vol_flux_z + (int64_t)idx(g, xb, k, lp), oc) = cz * (qz[s] + wa + wan + wb + wbn);
             if (lp > l0) {  // cell plane lp-1
                 const auto &C = cell[1 - s];
                 const T ua = n1[1 - s][0][w][lane], ub = n1[1 - s][0][wu][lane];
@@ -308,7 +332,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
                 const T energy_change = C.a * total_flux * recip_volume;
                 const T e1 = C.e - energy_change;
                 const T d1 = C.d * quo(vol, vol + total_flux);
-                const int64_t r = idx(g, g.x_min, k, lp - 1);
+                const int64_t r = idx(g, xb, k, lp - 1);
                 if (crow && cols) at(vol_flux_x + r, on) = cx * sl;
                 if (ccols) at(vol_flux_y + r, oc) = cy * sb;
                 if (crow && ccols) {
@@ -318,7 +342,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
             }
             zc = zflux;
         }
-        if (lp + 1 <= clast) predict(std::integral_constant<int, 1 - s>{}, d0, e0, q0);
+        if (lp + 1 <= clast) predict(std::integral_constant<int, 1 - s>{}, d0, e0, p0, q0);
         __syncthreads();
     };
 
@@ -327,12 +351,12 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
     load_nodes(lp0 + 1);
     load_cells(lp0);
     put_nodes(1);
-    const T d0 = dn, e0 = en, q0 = qn;
-    if (lp0 + 2 <= clast + 1) load_nodes(lp0 + 2);
+    const T d0 = dn, e0 = en, p0 = pn, q0 = qn;
+    if (lp0 + 2 <= clast + PRED) load_nodes(lp0 + 2);
     if (lp0 + 1 <= clast) load_cells(lp0 + 1);
     __syncthreads();
     zp = z_face(n0[0][2][w][lane], n0[0][2][w + 1][lane], sz[0], qz[0]);
-    predict(std::integral_constant<int, 0>{}, d0, e0, q0);
+    predict(std::integral_constant<int, 0>{}, d0, e0, p0, q0);
     __syncthreads();
     for (int lp = lp0;; lp++) {
         plane(std::integral_constant<int, 0>{}, lp);
@@ -352,8 +376,23 @@ __global__ void __launch_bounds__(64 * lw_of<S>())
 {
     const double dt = *dtp;
     if (dt < 0.0) return;
-    lagrange_body<S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, viscosity, xvel0, xvel1, yvel0,
-                     yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
+    lagrange_body<true, S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, nullptr, viscosity, xvel0,
+                           xvel1, yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
+}
+
+template <typename S>
+__global__ void __launch_bounds__(64 * lw_of<S>())
+    k_fast_accel_pdv(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
+                     const S *__restrict__ energy0, S *__restrict__ energy1, const S *__restrict__ pressure,
+                     const S *__restrict__ viscosity, const S *__restrict__ xvel0, S *__restrict__ xvel1,
+                     const S *__restrict__ yvel0, S *__restrict__ yvel1, const S *__restrict__ zvel0,
+                     S *__restrict__ zvel1, S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y,
+                     S *__restrict__ vol_flux_z)
+{
+    const double dt = *dtp;
+    if (dt < 0.0) return;
+    lagrange_body<false, S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, pressure, viscosity, xvel0,
+                            xvel1, yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
 }
 
 hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0, void *density1,
@@ -381,6 +420,32 @@ hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const doubl
     return hipGetLastError();
 }
 
+hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
+                                 void *density1, const void *energy0, void *energy1, const void *pressure,
+                                 const void *viscosity, const void *xvel0, void *xvel1, const void *yvel0,
+                                 void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,
+                                 void *vol_flux_z, const Shape &sh, hipStream_t st)
+{
+    int gx, gy, gz;
+    dims_lagrange(g, s == ST_F32 ? lw_of<float>() : lw_of<double>(), sh.planes, gx, gy, gz);
+#define CP(p) static_cast<const T *>(p)
+#define MP(p) static_cast<T *>(p)
+#define CALL(T_)                                                                                              \
+    do {                                                                                                      \
+        using T = T_;                                                                                         \
+        TIMED_LAUNCH("k_fast_accel_pdv", st, k_fast_accel_pdv<T>, dim3(gx, gy, gz), dim3(64, lw_of<T>()), 0, st, sh.xcd, g, m, \
+                     dt, CP(density0), MP(density1), CP(energy0), MP(energy1), CP(pressure), CP(viscosity), CP(xvel0),  \
+                     MP(xvel1), CP(yvel0), MP(yvel1), CP(zvel0), MP(zvel1), MP(vol_flux_x), MP(vol_flux_y),   \
+                     MP(vol_flux_z));                                                                         \
+    } while (0)
+    if (s == ST_F32) CALL(float);
+    else CALL(double);
+#undef CALL
+#undef CP
+#undef MP
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Batched over many decks (batch.h)
 int batch_blocks_lagrange(const Lay &g, int planes, Store s)
@@ -390,9 +455,9 @@ int batch_blocks_lagrange(const Lay &g, int planes, Store s)
     return gx * gy * gz;
 }
 
-template <typename S>
-__global__ void __launch_bounds__(64 * lw_of<S>())
-kb_lagrange(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd)
+template <bool PRED, typename S>
+__device__ __forceinline__ void lagrange_tiles(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd,
+                                               int planes, int xcd)
 {
     int hb, end, step;  // the tiles of this workgroup (persistent when the grid is short)
     tile_walk(start[nd], xcd, hb, end, step);
@@ -405,13 +470,27 @@ kb_lagrange(const DeckDev *__restrict__ decks, const int *__restrict__ start, in
         const Blk bk{lb % gx, (lb / gx) % gy, lb / (gx * gy), gx, gy, gz};
 #define CF(id) static_cast<const S *>(D.f[id])
 #define MF(id) static_cast<S *>(D.f[id])
-        lagrange_body<S>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), MF(F_DENSITY1), CF(F_ENERGY0), MF(F_ENERGY1),
-                         CF(F_VISCOSITY), CF(F_XVEL0), MF(F_XVEL1), CF(F_YVEL0), MF(F_YVEL1), CF(F_ZVEL0),
-                         MF(F_ZVEL1), MF(F_VOL_FLUX_X), MF(F_VOL_FLUX_Y), MF(F_VOL_FLUX_Z));
+        lagrange_body<PRED, S>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), MF(F_DENSITY1), CF(F_ENERGY0), MF(F_ENERGY1),
+                               CF(F_PRESSURE), CF(F_VISCOSITY), CF(F_XVEL0), MF(F_XVEL1), CF(F_YVEL0), MF(F_YVEL1),
+                               CF(F_ZVEL0), MF(F_ZVEL1), MF(F_VOL_FLUX_X), MF(F_VOL_FLUX_Y), MF(F_VOL_FLUX_Z));
 #undef CF
 #undef MF
         __syncthreads();  // the next tile reuses the workgroup's LDS
     }
+}
+
+template <typename S>
+__global__ void __launch_bounds__(64 * lw_of<S>())
+kb_lagrange(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd)
+{
+    lagrange_tiles<true, S>(decks, start, nd, planes, xcd);
+}
+
+template <typename S>
+__global__ void __launch_bounds__(64 * lw_of<S>())
+kb_accel_pdv(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd)
+{
+    lagrange_tiles<false, S>(decks, start, nd, planes, xcd);
 }
 
 hipError_t batch_lagrange(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, const Shape &sh, hipStream_t st)
@@ -422,6 +501,17 @@ hipError_t batch_lagrange(Store s, const DeckDev *decks, int nd, const BatchGrid
         TIMED_LAUNCH("kb_lagrange", st, kb_lagrange<float>, grid, blk, 0, st, decks, bg.start, nd, sh.planes, sh.xcd);
     else
         TIMED_LAUNCH("kb_lagrange", st, kb_lagrange<double>, grid, blk, 0, st, decks, bg.start, nd, sh.planes, sh.xcd);
+    return hipGetLastError();
+}
+
+hipError_t batch_accel_pdv(Store s, const DeckDev *decks, int nd, const BatchGrid &bg, const Shape &sh, hipStream_t st)
+{
+    if (bg.total == 0) return hipSuccess;
+    const dim3 grid(batch_wgs(bg, sh)), blk(64, s == ST_F32 ? lw_of<float>() : lw_of<double>());
+    if (s == ST_F32)
+        TIMED_LAUNCH("kb_accel_pdv", st, kb_accel_pdv<float>, grid, blk, 0, st, decks, bg.start, nd, sh.planes, sh.xcd);
+    else
+        TIMED_LAUNCH("kb_accel_pdv", st, kb_accel_pdv<double>, grid, blk, 0, st, decks, bg.start, nd, sh.planes, sh.xcd);
     return hipGetLastError();
 }
 
