@@ -23,6 +23,8 @@
 // mass and energy update in FP64.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "batch.h"
 #include "fast.h"
 #include "launch.h"
@@ -172,6 +174,23 @@ __global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const double *__rest
                    p_out);
 }
 
+// the order of the y and z marches' positions (launch.h linear_sweep); along z the
+// lanes' 32-bit byte offsets span the array
+template <int DIR>
+__host__ __device__ inline bool linear_cell(const Lay &g)
+{
+    return linear_sweep(g.x_max - g.x_min + 1) &&
+           (DIR == 3 || (long long)g.plane * (g.z_max - g.z_min + 6) < (1LL << 29));
+}
+
+template <int DIR>
+__host__ __device__ inline void dims_march(const Lay &g, int planes, int &gx, int &gy, int &gz)
+{
+    const int nx = g.x_max - g.x_min + 1, ny = g.y_max - g.y_min + 1, nz = g.z_max - g.z_min + 1;
+    dims_rows(linear_cell<DIR>(g), nx, DIR == 3 ? ny : nz + 2, 64, CROWS, gx, gy);
+    gz = nchunks(DIR == 3 ? nz + 2 : ny + 2, planes);
+}
+
 // ---------------------------------------------------------------------------
 // y and z sweeps: lanes along x (interior j), threadIdx.y along the cross
 // axis, march along the sweep axis over faces [smin, smax+2] in chunks.
@@ -180,14 +199,16 @@ __global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const double *__rest
 // 3-6.  Row addresses are scalar (the wave's cross row and the face), a
 // lane adds a byte offset; density and energy across a mirrored face are read
 // at the interior cell.
-template <int DIR, int MODE, typename S>
+template <bool LIN, int DIR, int MODE, typename S>
 __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
-    const int j = g.x_min + (int)(bk.x * 64 + threadIdx.x);
-    const int cr = (DIR == 3 ? g.y_min : g.z_min) + bk.y * CROWS + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    int pos, row0;
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row0);
+    const int crmin = DIR == 3 ? g.y_min : g.z_min;
+    const int j = g.x_min + pos, cr = crmin + row0;
     const int crmax = DIR == 3 ? g.y_max : g.z_max + 2;  // last cross position with faces
     if (j > g.x_max || cr > crmax) return;                 // no cross-lane traffic in this kernel
     const bool cross_in = DIR == 3 || cr <= g.z_max;       // updates only on interior cells
@@ -198,12 +219,18 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
     int f0, f1;
     chunk_range(bk, smin, smax + 2, f0, f1);
     if (f0 > f1) return;
-    unsigned oj = (unsigned)(j - g.x_min) * (unsigned)sizeof(S);
-    auto row = [&](int q) { return (int64_t)(DIR == 3 ? idx(g, g.x_min, cr, q) : idx(g, g.x_min, q, cr)); };
+    // the scalar rows' cross positions, of faces and of cells, and the lane's
+    // byte offsets from them: the wave's own, or the first where lanes lie in
+    // several rows
     const int crc = DIR == 3 ? cr : cell_m(g, 2, cr);
+    const int cb = LIN ? crmin : cr, cbc = LIN ? crmin : crc;
+    const int sC = DIR == 3 ? g.ld : g.plane;
+    unsigned oj = (unsigned)(pos + (LIN ? row0 * sC : 0)) * (unsigned)sizeof(S);
+    unsigned ojc = LIN ? (unsigned)(pos + (crc - crmin) * sC) * (unsigned)sizeof(S) : 0;
+    auto row = [&](int q) { return (int64_t)(DIR == 3 ? idx(g, g.x_min, cb, q) : idx(g, g.x_min, q, cb)); };
     auto cell = [&](const S *__restrict__ p, int q) -> S {  // density or energy
         const int qc = cell_m(g, DIR - 1, q);
-        return at(p + (int64_t)(DIR == 3 ? idx(g, g.x_min, crc, qc) : idx(g, g.x_min, qc, crc)), oj);
+        return at(p + (int64_t)(DIR == 3 ? idx(g, g.x_min, cbc, qc) : idx(g, g.x_min, qc, cbc)), LIN ? ojc : oj);
     };
     // pre_vol's volume fluxes of the cell at q, raw (converted where used, so
     // that a face's loads can be issued a step ahead of their use)
@@ -259,6 +286,7 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
     }
     for (int f = f0; f <= f1; f++) {
         asm volatile("" : "+v"(oj));  // no array + offset hoisted into vector registers
+        if constexpr (LIN) asm volatile("" : "+v"(ojc));
         const T vf = vf_n;
         const double pv_0 = pre_of(pr_n);
         const T r_p1 = f + 1 <= smax + 2 ? r_n : r_0, e_p1 = f + 1 <= smax + 2 ? e_n : e_0;
@@ -299,14 +327,14 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
     }
 }
 
-template <int DIR, int MODE, typename S>
+template <bool LIN, int DIR, int MODE, typename S>
 __global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
     if (*dt < 0.0) return;
-    cell_march_body<DIR, MODE, S>(hw_blk(xcd), g, m, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
+    cell_march_body<LIN, DIR, MODE, S>(hw_blk(xcd), g, m, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
                                   p_out);
 }
 
@@ -324,12 +352,22 @@ static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m
         TIMED_LAUNCH("k_fast_cell_x", st, k_fast_cell_x<S>, grid, blk, 0, st, dt, sh.xcd, g, m, mode, vol_flux_x, vol_flux_y,
                      vol_flux_z, density1, energy1, mass_flux_x, rho_out, e_out, p_out, rows);
     } else if (dir == 2) {
-        const dim3 grid((nx + 63) / 64, (nz + 2 + CROWS - 1) / CROWS, nchunks(ny + 2, sh.planes));
-        const auto kern = mode == 3 ? k_fast_cell_march<2, 3, S> : k_fast_cell_march<2, 4, S>;
+        int gx, gy, gz;
+        dims_march<2>(g, sh.planes, gx, gy, gz);
+        const dim3 grid(gx, gy, gz);
+        const auto kern = linear_cell<2>(g)
+                              ? mode == 3 ? k_fast_cell_march<true, 2, 3, S> : k_fast_cell_march<true, 2, 4, S>
+                          : mode == 3 ? k_fast_cell_march<false, 2, 3, S>
+                                      : k_fast_cell_march<false, 2, 4, S>;
         TIMED_LAUNCH("k_fast_cell_y", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_y, rho_out, e_out, p_out);
     } else {
-        const dim3 grid((nx + 63) / 64, (ny + CROWS - 1) / CROWS, nchunks(nz + 2, sh.planes));
-        const auto kern = mode == 5 ? k_fast_cell_march<3, 5, S> : k_fast_cell_march<3, 6, S>;
+        int gx, gy, gz;
+        dims_march<3>(g, sh.planes, gx, gy, gz);
+        const dim3 grid(gx, gy, gz);
+        const auto kern = linear_cell<3>(g)
+                              ? mode == 5 ? k_fast_cell_march<true, 3, 5, S> : k_fast_cell_march<true, 3, 6, S>
+                          : mode == 5 ? k_fast_cell_march<false, 3, 5, S>
+                                      : k_fast_cell_march<false, 3, 6, S>;
         TIMED_LAUNCH("k_fast_cell_z", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_z, rho_out, e_out, p_out);
     }
     return hipGetLastError();
@@ -371,9 +409,9 @@ __host__ __device__ inline void dims_cell(int dir, const Lay &g, int planes, int
         const int rows = cell_x_rows(planes);
         gx = (nx + 2 + 59) / 60; gy = ((ny * nz + rows - 1) / rows + CROWS - 1) / CROWS; gz = 1;
     } else if (dir == 2) {
-        gx = (nx + 63) / 64; gy = (nz + 2 + CROWS - 1) / CROWS; gz = nchunks(ny + 2, planes);
+        dims_march<2>(g, planes, gx, gy, gz);
     } else {
-        gx = (nx + 63) / 64; gy = (ny + CROWS - 1) / CROWS; gz = nchunks(nz + 2, planes);
+        dims_march<3>(g, planes, gx, gy, gz);
     }
 }
 
@@ -400,13 +438,19 @@ kb_cell(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd
         const Blk bk{lb % gx, (lb / gx) % gy, lb / (gx * gy), gx, gy, gz};
 #define CF(id) static_cast<const S *>(D.f[id])
 #define MF(id) static_cast<S *>(D.f[id])
-        if constexpr (DIR == 1)
+        if constexpr (DIR == 1) {
             cell_x_body<S>(bk, D.g, D.m, mode, cell_x_rows(planes), CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z), CF(cs.rho),
                            CF(cs.e), MF(F_MASS_FLUX_X), MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
-        else
-            cell_march_body<DIR, MODE, S>(bk, D.g, D.m, CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z),
-                                    CF(cs.rho), CF(cs.e), MF(DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z),
-                                    MF(cs.rho_out), MF(cs.e_out), gas ? MF(F_PRESSURE) : nullptr);
+        } else {
+            auto body = [&](auto lin) {
+                cell_march_body<decltype(lin)::value, DIR, MODE, S>(
+                    bk, D.g, D.m, CF(F_VOL_FLUX_X), CF(F_VOL_FLUX_Y), CF(F_VOL_FLUX_Z), CF(cs.rho), CF(cs.e),
+                    MF(DIR == 2 ? F_MASS_FLUX_Y : F_MASS_FLUX_Z), MF(cs.rho_out), MF(cs.e_out),
+                    gas ? MF(F_PRESSURE) : nullptr);
+            };
+            if (linear_cell<DIR>(D.g)) body(std::true_type{});
+            else body(std::false_type{});
+        }
 #undef CF
 #undef MF
         __syncthreads();  // the next tile reuses the workgroup's LDS

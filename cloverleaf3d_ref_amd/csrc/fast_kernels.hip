@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "batch.h"
 #include "fast.h"
@@ -178,15 +179,16 @@ __device__ inline T visc_cell(const QuadS<T> &ul, const QuadS<T> &vl, const Quad
 // (the halo exchange of viscosity between the two in timestep.f90:80-84
 // does not touch interior cells).  Each workgroup leaves one partial of the
 // dt minimum, which is FP64 in both forms.
-template <typename S>
+template <bool LIN, typename S>
 __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double dtc_safe, double dtu_safe, double dtv_safe, double dtw_safe, double dtdiv_safe,
                double g_small, const S *__restrict__ density0, const S *__restrict__ pressure,
                S *__restrict__ viscosity, const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                const S *__restrict__ zvel0, double *__restrict__ partial)
 {
     using T = S;  // arithmetic type of the form
-    const int j = g.x_min + bk.x * (int)blockDim.x + (int)threadIdx.x;
-    const int k = g.y_min + bk.y * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    int pos, row;
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row);
+    const int j = g.x_min + pos, k = g.y_min + row;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
     const bool in = j <= g.x_max && k <= g.y_max && l0 <= l1;  // every thread reaches the reduction
@@ -198,11 +200,12 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
     double dtmin_thread = 1.0e300;
     if (in) {
         T mc = 0, ms = 0, mu = 0, mv = 0, mw = 0, mdiv = 0;  // largest dt denominators so far (all are >= 0)
-        // the wave's row is scalar; lanes add byte offsets (at)
+        // the wave's row (LIN: the plane's row below the first) is scalar; lanes
+        // add byte offsets (at)
         l0 = __builtin_amdgcn_readfirstlane(l0);
         l1 = __builtin_amdgcn_readfirstlane(l1);
-        int r = __builtin_amdgcn_readfirstlane(idx(g, g.x_min, k, l0));
-        unsigned oj = (unsigned)(j - g.x_min) * (unsigned)sizeof(S);
+        int r = __builtin_amdgcn_readfirstlane(idx(g, g.x_min, LIN ? g.y_min - 1 : k, l0));
+        unsigned oj = (unsigned)(LIN ? pos + (row + 1) * g.ld : j - g.x_min) * (unsigned)sizeof(S);
         const auto quad = [&](const S *__restrict__ p) {
             return QuadS<S>{{at(p + r, oj), at(p + r + 1, oj), at(p + r + g.ld, oj), at(p + r + 1 + g.ld, oj)}};
         };
@@ -211,13 +214,16 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
         // cell, read as the cell itself, which its reflection copies
         const int oxm = cell_m(g, 0, j - 1) - (j - 1), oxp = cell_m(g, 0, j + 1) - (j + 1);
         unsigned om = oj + (unsigned)(oxm * (int)sizeof(S)), op = oj + (unsigned)(oxp * (int)sizeof(S));
-        const int oym = (cell_m(g, 1, k - 1) - k) * g.ld, oyp = (cell_m(g, 1, k + 1) - k) * g.ld;
+        const int dym = (cell_m(g, 1, k - 1) - k) * g.ld, dyp = (cell_m(g, 1, k + 1) - k) * g.ld;
+        unsigned oym = LIN ? oj + (unsigned)(dym * (int)sizeof(S)) : 0;
+        unsigned oyp = LIN ? oj + (unsigned)(dyp * (int)sizeof(S)) : 0;
         T p_lo = at(pressure + r + (cell_m(g, 2, l0 - 1) - l0) * g.plane, oj), p_c = at(pressure + r, oj);
         // The cell's soundspeed is not read: it is ideal_gas's of the cell's
         // density and pressure, formed here with the same operations
         // (soundspeed2_of), so it has the same bits.
         for (int l = l0; l <= l1; l++) {
             asm volatile("" : "+v"(oj), "+v"(om), "+v"(op), "+s"(r));  // no address per array held or walked
+            if constexpr (LIN) asm volatile("" : "+v"(oym), "+v"(oyp));
             // the upper node plane's velocities and pressure, the cell's
             // density and its x/y pressure neighbours, loaded at the top of
             // the plane: holding the next plane's loads in registers as well
@@ -233,7 +239,8 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
             const T p_hi = at(pressure + rc + (cell_m(g, 2, l + 1) - l) * g.plane, oj);
             const T rho = at(density0 + rc, oj);
             const T p_xm = at(pressure + rc - 1, om), p_xp = at(pressure + rc + 1, op);
-            const T p_ym = at(pressure + rc + oym, oj), p_yp = at(pressure + rc + oyp, oj);
+            const T p_ym = LIN ? at(pressure + rc, oym) : at(pressure + rc + dym, oj);
+            const T p_yp = LIN ? at(pressure + rc, oyp) : at(pressure + rc + dyp, oj);
             at(viscosity + rc, oj) = visc_cell<T>(ul, vl, wl, uu, vu, wu, rho, p_c, p_lo, p_hi, p_xm, p_xp, p_ym, p_yp,
                                                   m, ds, dx, dy, dz, xa, ya, za, mc, ms, mu, mv, mw, mdiv);
             ul = uu;
@@ -278,6 +285,7 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
 // VGPRs against 88; at 512^3: 827 -> 743 us, three rounds on one machine,
 // same bits.  The batched kernel (kb_visc_dt) uses it too: 640^3 as 8
 // tiles 1.68 -> 1.59 ms (the 512-deck ensemble: unchanged).
+template <bool LIN>
 __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, double dtc_safe, double dtu_safe,
                                                   double dtv_safe, double dtw_safe, double dtdiv_safe, double g_small,
                                                   const float *__restrict__ density0,
@@ -286,8 +294,10 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
                                                   const float *__restrict__ zvel0, double *__restrict__ partial)
 {
     using T = float;
-    const int j = g.x_min + 2 * (bk.x * (int)blockDim.x + (int)threadIdx.x);
-    const int k = g.y_min + bk.y * (int)blockDim.y + (int)threadIdx.y;
+    int pos, row;
+    const int np = (g.x_max - g.x_min + 2) / 2;
+    place_rows<LIN>(bk, np, pos, row);
+    const int j = g.x_min + 2 * pos, k = g.y_min + row;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
     const bool in = j <= g.x_max && k <= g.y_max && l0 <= l1;  // every thread reaches the reduction
@@ -353,17 +363,17 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
     }
 }
 
-template <typename S>
+template <bool LIN, typename S>
 __global__ void __launch_bounds__(kMaxBlock) k_fast_visc_dt(int xcd, Lay g, Geo m, double dtc_safe, double dtu_safe, double dtv_safe, double dtw_safe, double dtdiv_safe,
                double g_small, const S *__restrict__ density0, const S *__restrict__ pressure,
                S *__restrict__ viscosity, const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                const S *__restrict__ zvel0, double *__restrict__ partial)
 {
     if constexpr (sizeof(S) == 4)
-        visc_dt_pair_body(hw_blk(xcd), g, m, dtc_safe, dtu_safe, dtv_safe, dtw_safe, dtdiv_safe, g_small, density0,
+        visc_dt_pair_body<LIN>(hw_blk(xcd), g, m, dtc_safe, dtu_safe, dtv_safe, dtw_safe, dtdiv_safe, g_small, density0,
                           pressure, viscosity, xvel0, yvel0, zvel0, partial);
     else
-        visc_dt_body<S>(hw_blk(xcd), g, m, dtc_safe, dtu_safe, dtv_safe, dtw_safe, dtdiv_safe, g_small, density0,
+        visc_dt_body<LIN, S>(hw_blk(xcd), g, m, dtc_safe, dtu_safe, dtv_safe, dtw_safe, dtdiv_safe, g_small, density0,
                         pressure, viscosity, xvel0, yvel0, zvel0, partial);
 }
 
@@ -377,12 +387,15 @@ static hipError_t fast_visc_dt_t(const Lay &g, const Geo &m, double dtc_safe, do
     const int nx = g.x_max - g.x_min + 1, ny = g.y_max - g.y_min + 1, nz = g.z_max - g.z_min + 1;
     const dim3 blk = block_of(sh);
     const int cpt = sizeof(S) == 4 ? 2 : 1;  // cells per thread along x
-    const int bx = (nx + cpt * (int)blk.x - 1) / (cpt * (int)blk.x), by = (ny + (int)blk.y - 1) / (int)blk.y;
+    const int np = (nx + cpt - 1) / cpt;
+    int bx, by;
+    dims_rows(linear_cells(np), np, ny, (int)blk.x, (int)blk.y, bx, by);
     if (bx * by > kMaxDtPartials) return hipErrorInvalidValue;  // caller keeps tiles within the partial buffer
     int gz = nchunks(nz, sh.planes);
     if (bx * by * gz > kMaxDtPartials) gz = kMaxDtPartials / (bx * by);
     *nparts = bx * by * gz;
-    TIMED_LAUNCH("k_fast_visc_dt", st, k_fast_visc_dt<S>, dim3(bx, by, gz), blk, 0, st, sh.xcd, g, m, dtc_safe,
+    const auto kern = linear_cells(np) ? k_fast_visc_dt<true, S> : k_fast_visc_dt<false, S>;
+    TIMED_LAUNCH("k_fast_visc_dt", st, kern, dim3(bx, by, gz), blk, 0, st, sh.xcd, g, m, dtc_safe,
                  dtu_safe, dtv_safe, dtw_safe, dtdiv_safe, g_small, density0, pressure, viscosity, xvel0, yvel0,
                  zvel0, partial);
     return hipGetLastError();
@@ -432,14 +445,15 @@ __device__ inline T predict_pressure(const QuadS<T> &ul, const QuadS<T> &vl, con
     return (T)(1.4 - 1.0) * d1 * e1;
 }
 
-template <typename S>
+template <bool LIN, typename S>
 __device__ __forceinline__ void pdv_predict_body(const Blk &bk, Lay g, Geo m, double dt, const S *__restrict__ density0, const S *__restrict__ energy0,
                    S *__restrict__ pressure, const S *__restrict__ viscosity,
                    const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                    const S *__restrict__ zvel0)
 {
-    const int j = g.x_min + bk.x * (int)blockDim.x + (int)threadIdx.x;
-    const int k = g.y_min + bk.y * (int)blockDim.y + (int)threadIdx.y;
+    int pos, row;
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row);
+    const int j = g.x_min + pos, k = g.y_min + row;
     if (j > g.x_max || k > g.y_max) return;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
@@ -480,6 +494,7 @@ __device__ __forceinline__ void pdv_predict_body(const Blk &bk, Lay g, Geo m, do
 // 512^3: 834 -> 750 us, three rounds on one machine, same bits.  The batched
 // kernel (kb_pdv_predict) uses it too: 640^3 as 8 tiles 1.66 -> 1.53 ms.
 
+template <bool LIN>
 __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo m, double dt,
                                                       const float *__restrict__ density0,
                                                       const float *__restrict__ energy0, float *__restrict__ pressure,
@@ -487,8 +502,10 @@ __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo 
                                                       const float *__restrict__ xvel0, const float *__restrict__ yvel0,
                                                       const float *__restrict__ zvel0)
 {
-    const int j = g.x_min + 2 * (bk.x * (int)blockDim.x + (int)threadIdx.x);
-    const int k = g.y_min + bk.y * (int)blockDim.y + (int)threadIdx.y;
+    int pos, row;
+    const int np = (g.x_max - g.x_min + 2) / 2;
+    place_rows<LIN>(bk, np, pos, row);
+    const int j = g.x_min + 2 * pos, k = g.y_min + row;
     if (j > g.x_max || k > g.y_max) return;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
@@ -529,7 +546,7 @@ __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo 
     }
 }
 
-template <typename S>
+template <bool LIN, typename S>
 __global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, const S *__restrict__ energy0,
                    S *__restrict__ pressure, const S *__restrict__ viscosity,
                    const S *__restrict__ xvel0, const S *__restrict__ yvel0,
@@ -538,9 +555,9 @@ __global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, 
     const double dt = *dtp;
     if (dt < 0.0) return;
     if constexpr (sizeof(S) == 4)
-        pdv_predict_pair_body(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
+        pdv_predict_pair_body<LIN>(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
     else
-        pdv_predict_body<S>(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
+        pdv_predict_body<LIN, S>(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
 }
 
 template <typename S>
@@ -551,8 +568,12 @@ static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, const double *d
     const int nx = g.x_max - g.x_min + 1, ny = g.y_max - g.y_min + 1, nz = g.z_max - g.z_min + 1;
     const dim3 blk = block_of(sh);
     const int cpt = sizeof(S) == 4 ? 2 : 1;  // cells per thread along x
-    const dim3 grid((nx + cpt * blk.x - 1) / (cpt * blk.x), (ny + blk.y - 1) / blk.y, nchunks(nz, sh.planes));
-    TIMED_LAUNCH("k_fast_pdv_predict", st, k_fast_pdv_predict<S>, grid, blk, 0, st, sh.xcd, g, m, dt, density0,
+    const int np = (nx + cpt - 1) / cpt;
+    int gx, gy;
+    dims_rows(linear_cells(np), np, ny, (int)blk.x, (int)blk.y, gx, gy);
+    const dim3 grid(gx, gy, nchunks(nz, sh.planes));
+    const auto kern = linear_cells(np) ? k_fast_pdv_predict<true, S> : k_fast_pdv_predict<false, S>;
+    TIMED_LAUNCH("k_fast_pdv_predict", st, kern, grid, blk, 0, st, sh.xcd, g, m, dt, density0,
                  energy0, pressure, viscosity, xvel0, yvel0, zvel0);
     return hipGetLastError();
 }
@@ -732,11 +753,13 @@ __host__ __device__ inline void dims_ideal(const Lay &g, int &gx, int &gy, int &
     gz = g.z_max - g.z_min + 1;
 }
 
-// cpt: cells per thread along x (2 in the FP32 visc_dt and predictor)
+// threads of a row; cpt: cells per thread along x (2 in the FP32 visc_dt and predictor)
+__host__ __device__ inline int cell_positions(const Lay &g, int cpt) { return (g.x_max - g.x_min + cpt) / cpt; }
+
 __host__ __device__ inline void dims_cells(const Lay &g, int planes, int cpt, int &gx, int &gy, int &gz)
 {
-    gx = (g.x_max - g.x_min + cpt * BX) / (cpt * BX);
-    gy = (g.y_max - g.y_min + BY) / BY;
+    const int np = cell_positions(g, cpt);
+    dims_rows(linear_cells(np), np, g.y_max - g.y_min + 1, BX, BY, gx, gy);
     gz = nchunks(g.z_max - g.z_min + 1, planes);
 }
 
@@ -784,7 +807,7 @@ kb_ideal_gas(const DeckDev *__restrict__ decks, const int *__restrict__ start, i
     ideal_gas_body<S>(bk, g, r, CF(F_DENSITY0), CF(F_ENERGY0), MF(F_PRESSURE), MF(F_SOUNDSPEED));
 }
 
-// three waves per SIMD in FP64 (168 VGPRs), which the compiler would miss by one register
+// at least three waves per SIMD (both orders in one kernel: 120 VGPRs FP32, 123 FP64, four)
 template <typename S>
 __global__ void __launch_bounds__(BX *BY) __attribute__((amdgpu_waves_per_eu(3)))
 kb_visc_dt(const DeckDev *__restrict__ decks, const int *__restrict__ start, int nd, int planes, int xcd,
@@ -793,14 +816,19 @@ kb_visc_dt(const DeckDev *__restrict__ decks, const int *__restrict__ start, int
     FOR_TILES(xcd)
     {
         DECK_TILE(t_, dims_cells(D.g, planes, sizeof(S) == 4 ? 2 : 1, gx, gy, gz))
-        if constexpr (sizeof(S) == 4)
-            visc_dt_pair_body(bk, D.g, D.m, D.dtc_safe, D.dtu_safe, D.dtv_safe, D.dtw_safe, D.dtdiv_safe, g_small,
-                              CF(F_DENSITY0), CF(F_PRESSURE), MF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0),
-                              CF(F_ZVEL0), partial + start[d]);
-        else
-            visc_dt_body<S>(bk, D.g, D.m, D.dtc_safe, D.dtu_safe, D.dtv_safe, D.dtw_safe, D.dtdiv_safe, g_small,
-                            CF(F_DENSITY0), CF(F_PRESSURE), MF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0), CF(F_ZVEL0),
-                            partial + start[d]);
+        auto body = [&](auto lin) {
+            constexpr bool LIN = decltype(lin)::value;
+            if constexpr (sizeof(S) == 4)
+                visc_dt_pair_body<LIN>(bk, D.g, D.m, D.dtc_safe, D.dtu_safe, D.dtv_safe, D.dtw_safe, D.dtdiv_safe,
+                                       g_small, CF(F_DENSITY0), CF(F_PRESSURE), MF(F_VISCOSITY), CF(F_XVEL0),
+                                       CF(F_YVEL0), CF(F_ZVEL0), partial + start[d]);
+            else
+                visc_dt_body<LIN, S>(bk, D.g, D.m, D.dtc_safe, D.dtu_safe, D.dtv_safe, D.dtw_safe, D.dtdiv_safe,
+                                     g_small, CF(F_DENSITY0), CF(F_PRESSURE), MF(F_VISCOSITY), CF(F_XVEL0),
+                                     CF(F_YVEL0), CF(F_ZVEL0), partial + start[d]);
+        };
+        if (linear_cells(cell_positions(D.g, sizeof(S) == 4 ? 2 : 1))) body(std::true_type{});
+        else body(std::false_type{});
         __syncthreads();
     }
 }
@@ -812,12 +840,17 @@ kb_pdv_predict(const DeckDev *__restrict__ decks, const int *__restrict__ start,
     FOR_TILES(xcd)
     {
         DECK_TILE(t_, dims_cells(D.g, planes, sizeof(S) == 4 ? 2 : 1, gx, gy, gz))
-        if constexpr (sizeof(S) == 4)
-            pdv_predict_pair_body(bk, D.g, D.m, D.dt, CF(F_DENSITY0), CF(F_ENERGY0), MF(F_PRESSURE),
-                                  CF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0), CF(F_ZVEL0));
-        else
-            pdv_predict_body<S>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), CF(F_ENERGY0), MF(F_PRESSURE),
-                                CF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0), CF(F_ZVEL0));
+        auto body = [&](auto lin) {
+            constexpr bool LIN = decltype(lin)::value;
+            if constexpr (sizeof(S) == 4)
+                pdv_predict_pair_body<LIN>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), CF(F_ENERGY0), MF(F_PRESSURE),
+                                           CF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0), CF(F_ZVEL0));
+            else
+                pdv_predict_body<LIN, S>(bk, D.g, D.m, D.dt, CF(F_DENSITY0), CF(F_ENERGY0), MF(F_PRESSURE),
+                                         CF(F_VISCOSITY), CF(F_XVEL0), CF(F_YVEL0), CF(F_ZVEL0));
+        };
+        if (linear_cells(cell_positions(D.g, sizeof(S) == 4 ? 2 : 1))) body(std::true_type{});
+        else body(std::false_type{});
         __syncthreads();
     }
 }

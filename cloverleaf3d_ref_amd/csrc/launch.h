@@ -309,6 +309,41 @@ __device__ inline T next_lane(T x) { return lane_shift<0x130>(x); }
 template <typename T>
 __device__ inline T prev_lane(T x) { return lane_shift<0x138>(x); }
 
+// Marches whose lanes exchange nothing (visc_dt, the PdV predictor, the y and z
+// cell sweeps) take their positions, np to a row, either in tiles of 64 along x or,
+// where that leaves too many lanes without one, one after the other
+// through the plane's rows (LIN: lanes of a wave in several rows, so row offsets
+// are the lane's).
+// Lines, by what both orders measured.  visc_dt (and the predictor): one in eight.
+// FP64 72^3 19.6 -> 13.7 us, 131x75x93 23.7 -> 21.5, 160^3 77 -> 65, 96^3 22.7 ->
+// 21.5, 110^3 (lanes 86 % in use) the same; FP32 101x143x67 14.8 -> 13.8.  The
+// cell sweeps, whose rows are used once: two in five.  72^3 13.7 -> 12.4 us, but
+// 131x75x93 17.2 -> 17.9 and 110^3 20.3 -> 22.4.
+__host__ __device__ inline bool linear_cells(int np) { return ((np + 63) / 64 * 64 - np) * 8 > (np + 63) / 64 * 64; }
+__host__ __device__ inline bool linear_sweep(int np) { return ((np + 63) / 64 * 64 - np) * 5 > (np + 63) / 64 * 64 * 2; }
+
+// workgroups for rows of np positions: gx x gy tiles of bx x by, or gx of bx * by positions
+__host__ __device__ inline void dims_rows(bool lin, int np, int rows, int bx, int by, int &gx, int &gy)
+{
+    gx = lin ? (np * rows + bx * by - 1) / (bx * by) : (np + bx - 1) / bx;
+    gy = lin ? 1 : (rows + by - 1) / by;
+}
+
+// the thread's position and row (uniform over the wave without LIN); they may
+// lie outside the mesh
+template <bool LIN>
+__device__ inline void place_rows(const Blk &bk, int np, int &pos, int &row)
+{
+    if constexpr (LIN) {
+        const int c = (bk.x * (int)blockDim.y + (int)threadIdx.y) * (int)blockDim.x + (int)threadIdx.x;
+        row = c / np;
+        pos = c - row * np;
+    } else {
+        pos = bk.x * (int)blockDim.x + (int)threadIdx.x;
+        row = bk.y * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    }
+}
+
 // A row of an array (its address uniform over the wave) at a lane's byte offset:
 // the access takes a scalar address and a 32-bit offset, and no vector address
 // arithmetic.
