@@ -327,7 +327,7 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
     }
 }
 
-template <bool LIN, int DIR, int MODE, typename S>
+template <int DIR, int MODE, typename S, bool LIN>
 __global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
@@ -355,19 +355,19 @@ static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m
         int gx, gy, gz;
         dims_march<2>(g, sh.planes, gx, gy, gz);
         const dim3 grid(gx, gy, gz);
-        const auto kern = linear_cell<2>(g)
-                              ? mode == 3 ? k_fast_cell_march<true, 2, 3, S> : k_fast_cell_march<true, 2, 4, S>
-                          : mode == 3 ? k_fast_cell_march<false, 2, 3, S>
-                                      : k_fast_cell_march<false, 2, 4, S>;
+        const bool lin = linear_cell<2>(g);
+        const auto kern = mode == 3 ? lin ? k_fast_cell_march<2, 3, S, true> : k_fast_cell_march<2, 3, S, false>
+                          : lin     ? k_fast_cell_march<2, 4, S, true>
+                                    : k_fast_cell_march<2, 4, S, false>;
         TIMED_LAUNCH("k_fast_cell_y", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_y, rho_out, e_out, p_out);
     } else {
         int gx, gy, gz;
         dims_march<3>(g, sh.planes, gx, gy, gz);
         const dim3 grid(gx, gy, gz);
-        const auto kern = linear_cell<3>(g)
-                              ? mode == 5 ? k_fast_cell_march<true, 3, 5, S> : k_fast_cell_march<true, 3, 6, S>
-                          : mode == 5 ? k_fast_cell_march<false, 3, 5, S>
-                                      : k_fast_cell_march<false, 3, 6, S>;
+        const bool lin = linear_cell<3>(g);
+        const auto kern = mode == 5 ? lin ? k_fast_cell_march<3, 5, S, true> : k_fast_cell_march<3, 5, S, false>
+                          : lin     ? k_fast_cell_march<3, 6, S, true>
+                                    : k_fast_cell_march<3, 6, S, false>;
         TIMED_LAUNCH("k_fast_cell_z", st, kern, grid, blk, 0, st, dt, sh.xcd, g, m, vol_flux_x, vol_flux_y, vol_flux_z, density1, energy1, mass_flux_z, rho_out, e_out, p_out);
     }
     return hipGetLastError();

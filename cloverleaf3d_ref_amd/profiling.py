@@ -72,12 +72,14 @@ def kernel_stats(d: str, elem: str = "") -> List[Tuple[str, int, float, float, f
     """(kernel, calls, total_us, avg_us, percent of the kept rows), largest
     total first; elem keeps only the kernels instantiated for that type
     (and the untyped ones)."""
-    rows = []
+    per: Dict[str, List[float]] = defaultdict(lambda: [0, 0.0])  # a kernel's instances together
     with open(_find(d, "kernel_stats.csv")) as f:
         for r in csv.DictReader(f):
             if _keep(r["Name"], elem):
-                rows.append((_short(r["Name"]), int(r["Calls"]), float(r["TotalDurationNs"]) / 1e3,
-                             float(r["AverageNs"]) / 1e3))
+                k = per[_short(r["Name"])]
+                k[0] += int(r["Calls"])
+                k[1] += float(r["TotalDurationNs"]) / 1e3
+    rows = [(n, c, t, t / c) for n, (c, t) in per.items()]
     total = sum(r[2] for r in rows) or 1.0
     rows = [(n, c, t, a, 100.0 * t / total) for n, c, t, a in rows]
     rows.sort(key=lambda r: -r[2])
