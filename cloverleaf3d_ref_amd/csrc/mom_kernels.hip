@@ -412,7 +412,7 @@ __device__ inline T mom_flux_of(T nf, bool neg, unsigned sgn, T one_m, T two_m, 
     return (donor + one_m * limiter) * nf;
 }
 
-// The 64-column layout of the y and z sweeps.  mom_march_body's expressions
+// The 64-column layout of the y and z sweeps.  mom_tail_body's expressions
 // (MODE: the sweep's post_vol, mom_post_vol), with the work per plane cut to
 // what they need, since at 344 (FP64) and 253 (FP32) VALU instructions per wave
 // and plane the sweeps ran at or near the VALU's rate:
