@@ -206,7 +206,7 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
     int pos, row0;
-    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row0);
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, 0, 0, pos, row0);
     const int crmin = DIR == 3 ? g.y_min : g.z_min;
     const int j = g.x_min + pos, cr = crmin + row0;
     const int crmax = DIR == 3 ? g.y_max : g.z_max + 2;  // last cross position with faces

@@ -186,9 +186,8 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
                const S *__restrict__ zvel0, double *__restrict__ partial)
 {
     using T = S;  // arithmetic type of the form
-    int pos, row;
-    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row);
-    const int j = g.x_min + pos, k = g.y_min + row;
+    int j, k;
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, g.x_min, g.y_min, j, k);
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
     const bool in = j <= g.x_max && k <= g.y_max && l0 <= l1;  // every thread reaches the reduction
@@ -205,7 +204,7 @@ __device__ __forceinline__ void visc_dt_body(const Blk &bk, Lay g, Geo m, double
         l0 = __builtin_amdgcn_readfirstlane(l0);
         l1 = __builtin_amdgcn_readfirstlane(l1);
         int r = __builtin_amdgcn_readfirstlane(idx(g, g.x_min, LIN ? g.y_min - 1 : k, l0));
-        unsigned oj = (unsigned)(LIN ? pos + (row + 1) * g.ld : j - g.x_min) * (unsigned)sizeof(S);
+        unsigned oj = (unsigned)(j - g.x_min + (LIN ? (k - g.y_min + 1) * g.ld : 0)) * (unsigned)sizeof(S);
         const auto quad = [&](const S *__restrict__ p) {
             return QuadS<S>{{at(p + r, oj), at(p + r + 1, oj), at(p + r + g.ld, oj), at(p + r + 1 + g.ld, oj)}};
         };
@@ -294,10 +293,9 @@ __device__ __forceinline__ void visc_dt_pair_body(const Blk &bk, Lay g, Geo m, d
                                                   const float *__restrict__ zvel0, double *__restrict__ partial)
 {
     using T = float;
-    int pos, row;
-    const int np = (g.x_max - g.x_min + 2) / 2;
-    place_rows<LIN>(bk, np, pos, row);
-    const int j = g.x_min + 2 * pos, k = g.y_min + row;
+    int pos, k;
+    place_rows<LIN>(bk, (g.x_max - g.x_min + 2) / 2, 0, g.y_min, pos, k);
+    const int j = g.x_min + 2 * pos;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
     const bool in = j <= g.x_max && k <= g.y_max && l0 <= l1;  // every thread reaches the reduction
@@ -451,9 +449,8 @@ __device__ __forceinline__ void pdv_predict_body(const Blk &bk, Lay g, Geo m, do
                    const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                    const S *__restrict__ zvel0)
 {
-    int pos, row;
-    place_rows<LIN>(bk, g.x_max - g.x_min + 1, pos, row);
-    const int j = g.x_min + pos, k = g.y_min + row;
+    int j, k;
+    place_rows<LIN>(bk, g.x_max - g.x_min + 1, g.x_min, g.y_min, j, k);
     if (j > g.x_max || k > g.y_max) return;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);
@@ -502,10 +499,9 @@ __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo 
                                                       const float *__restrict__ xvel0, const float *__restrict__ yvel0,
                                                       const float *__restrict__ zvel0)
 {
-    int pos, row;
-    const int np = (g.x_max - g.x_min + 2) / 2;
-    place_rows<LIN>(bk, np, pos, row);
-    const int j = g.x_min + 2 * pos, k = g.y_min + row;
+    int pos, k;
+    place_rows<LIN>(bk, (g.x_max - g.x_min + 2) / 2, 0, g.y_min, pos, k);
+    const int j = g.x_min + 2 * pos;
     if (j > g.x_max || k > g.y_max) return;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max, l0, l1);

@@ -329,18 +329,19 @@ __host__ __device__ inline void dims_rows(bool lin, int np, int rows, int bx, in
     gy = lin ? 1 : (rows + by - 1) / by;
 }
 
-// the thread's position and row (uniform over the wave without LIN); they may
-// lie outside the mesh
+// the thread's position and row (uniform over the wave without LIN), counted from
+// pos0 and row0; they may lie outside the mesh
 template <bool LIN>
-__device__ inline void place_rows(const Blk &bk, int np, int &pos, int &row)
+__device__ inline void place_rows(const Blk &bk, int np, int pos0, int row0, int &pos, int &row)
 {
     if constexpr (LIN) {
         const int c = (bk.x * (int)blockDim.y + (int)threadIdx.y) * (int)blockDim.x + (int)threadIdx.x;
-        row = c / np;
-        pos = c - row * np;
+        const int r = c / np;
+        row = row0 + r;
+        pos = pos0 + c - r * np;
     } else {
-        pos = bk.x * (int)blockDim.x + (int)threadIdx.x;
-        row = bk.y * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+        pos = pos0 + bk.x * (int)blockDim.x + (int)threadIdx.x;
+        row = row0 + bk.y * (int)blockDim.y + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     }
 }
 
