@@ -68,7 +68,7 @@ constexpr int lw_of() { return sizeof(S) == 4 ? 8 : 12; }
 
 __host__ __device__ inline void dims_lagrange(const Lay &g, int lw, int planes, int &gx, int &gy, int &gz)
 {
-    gx = (g.x_max - g.x_min + 2 + 60) / 61;
+    gx = (g.x_max - g.x_min + 2 + kLagrangeCols - 1) / kLagrangeCols;
     gy = (g.y_max - g.y_min + 2 + lw - 3) / (lw - 2);
     gz = nchunks(g.z_max - g.z_min + 2, planes);
 }
@@ -129,12 +129,12 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
     __shared__ S n1[2][3][LW][64];      // level-1 nodes
     __shared__ S cb[3][LW][64];         // density, predicted pressure, viscosity of the cells
     const int lane = (int)threadIdx.x, w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int j = g.x_min - 1 + bk.x * 61 + lane;
+    const int j = lagrange_col(g, bk.x, lane);
     const int k = g.y_min - 1 + bk.y * (LW - 2) + w;
     int l0, l1;
     chunk_range(bk, g.z_min, g.z_max + 1, l0, l1);
     if (l0 > l1) return;  // the whole workgroup, before any barrier
-    const bool cols = lane >= 1 && lane <= 61 && j <= g.x_max + 1;      // owned columns of nodes
+    const bool cols = lane >= 1 && lane <= kLagrangeCols && j <= g.x_max + 1;  // owned columns of nodes
     const bool ccols = cols && j <= g.x_max;                            // and of cells
     const bool march = w >= 1 && w <= LW - 2 && k <= g.y_max + 1;       // owned row of nodes (uniform)
     const bool crow = march && k <= g.y_max;                            // and of cells
@@ -143,7 +143,7 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
     // face the halo row is the interior one, which without the predictor was
     // loaded there
     const int r1 = PRED && k <= g.y_min ? w : w - 1, r0 = PRED && k > g.y_max ? w - 1 : w;
-    const bool xedge = bk.x == 0 || bk.x == bk.gx - 1;  // the block may hold halo columns
+    const bool xedge = lagrange_halo_cells(g, bk.x);
     const T xa = (T)m.xa, ya = (T)m.ya, za = (T)m.za, vol = (T)m.vol, tdt = (T)dt;
     // the fluxes' factors 0.125 and 0.5 are powers of two: scaling dt by them
     // instead of the product gives the same bits (short of subnormal products,

@@ -49,6 +49,26 @@ inline Lay make_lay(int x_min, int x_max, int y_min, int y_max, int z_min, int z
     return g;
 }
 
+// The Lagrangian march's columns (lagrange_kernels.hip): lane `lane` of the
+// workgroups at x tile bx is node and cell column lagrange_col, of which lanes
+// 1..kLagrangeCols are the workgroup's own; it uses the cells of lanes 0 to
+// kLagrangeCols + 1.
+constexpr int kLagrangeCols = 61;
+
+__host__ __device__ inline int lagrange_col(const Lay &g, int bx, int lane)
+{
+    return g.x_min - 1 + bx * kLagrangeCols + lane;
+}
+
+// Whether one of those cells lies in the halo, to be taken from its mirror
+// image: by the columns themselves, not by the tile's place in the grid.  On a
+// mesh of kLagrangeCols * m cells the last tile owns the wall's nodes alone, and
+// the tile before it ends on the halo's cell.
+__host__ __device__ inline bool lagrange_halo_cells(const Lay &g, int bx)
+{
+    return bx == 0 || lagrange_col(g, bx, kLagrangeCols + 1) > g.x_max;
+}
+
 // elements to allocate for one 3-D field
 inline int64_t lay_elems(const Lay &g)
 {
