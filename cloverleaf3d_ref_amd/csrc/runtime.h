@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -69,7 +70,8 @@ inline double wait_dt(const DtSlot *slot, unsigned long long seq, hipStream_t st
 // class `cls` on the host, through two pinned buffers that its owner keeps
 // (at most kPieceElems doubles each; allocated on first use, freed by the
 // owner's release()).  Every piece is enqueued on the stream, after what is
-// there.
+// there.  Threads may fetch fields of one owner at the same time: one transfer
+// has the buffers at a time.
 class Stage {
   public:
     Stage() = default;
@@ -93,6 +95,7 @@ class Stage {
     static constexpr int64_t kPieceElems = 512 * 1024;  // 4 MiB
     void reserve(int64_t total);
     void wait(Buf &b);
+    std::mutex mu_;
     Buf buf_[2];
     int64_t elems_ = 0;  // doubles per buffer
     int next_ = 0;       // upload's next buffer

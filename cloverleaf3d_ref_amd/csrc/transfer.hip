@@ -80,6 +80,7 @@ static dim3 pack_grid(int n) { return dim3((unsigned)std::min((n + kPackThreads 
 
 void Stage::download(const Lay &g, int cls, const void *dev, size_t es, double *host, hipStream_t st)
 {
+    std::lock_guard<std::mutex> lock(mu_);
     int ex, ey, ez;
     class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
     const int64_t total = (int64_t)ex * ey * ez;
@@ -111,6 +112,7 @@ void Stage::download(const Lay &g, int cls, const void *dev, size_t es, double *
 
 void Stage::upload(const Lay &g, int cls, const double *host, double *dev, hipStream_t st)
 {
+    std::lock_guard<std::mutex> lock(mu_);
     int ex, ey, ez;
     class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
     const int64_t total = (int64_t)ex * ey * ez;
