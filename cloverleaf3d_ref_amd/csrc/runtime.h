@@ -93,7 +93,7 @@ class Stage {
         bool busy = false;
     };
     static constexpr int64_t kPieceElems = 512 * 1024;  // 4 MiB
-    void reserve(int64_t total);
+    void reserve(int64_t total, hipStream_t st);
     void wait(Buf &b);
     std::mutex mu_;
     Buf buf_[2];

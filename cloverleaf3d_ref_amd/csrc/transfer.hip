@@ -55,12 +55,28 @@ void Stage::release()
     elems_ = 0;
 }
 
-// room for pieces of a field of `total` elements
-void Stage::reserve(int64_t total)
+// The stream's device as the calling thread's current one, as long as this lives
+struct DeviceScope {
+    int before = 0;
+    explicit DeviceScope(hipStream_t st)
+    {
+        int device = 0;
+        hip_check(hipGetDevice(&before), "hipGetDevice");
+        hip_check(hipStreamGetDevice(st, &device), "hipStreamGetDevice");
+        hip_check(hipSetDevice(device), "hipSetDevice");
+    }
+    ~DeviceScope() { (void)hipSetDevice(before); }
+};
+
+// Room for pieces of a field of `total` elements.  The buffers and events are
+// the stream's device's, whichever is current: an event of another one cannot be
+// recorded on it, and a caller may fetch from chunks on several devices.
+void Stage::reserve(int64_t total, hipStream_t st)
 {
     const int64_t want = std::min(total, kPieceElems);
     if (want <= elems_) return;
     release();
+    const DeviceScope device(st);
     for (Buf &b : buf_) {
         hip_check(hipHostMalloc((void **)&b.host, sizeof(double) * (size_t)want, hipHostMallocDefault), "hipHostMalloc");
         hip_check(hipHostGetDevicePointer((void **)&b.dev, b.host, 0), "hipHostGetDevicePointer");
@@ -84,7 +100,7 @@ void Stage::download(const Lay &g, int cls, const void *dev, size_t es, double *
     int ex, ey, ez;
     class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
     const int64_t total = (int64_t)ex * ey * ez;
-    reserve(total);
+    reserve(total, st);
     const int64_t pieces = (total + elems_ - 1) / elems_;
     auto len = [&](int64_t p) { return (int)std::min(elems_, total - p * elems_); };
     auto start = [&](int64_t p) {
@@ -116,7 +132,7 @@ void Stage::upload(const Lay &g, int cls, const double *host, double *dev, hipSt
     int ex, ey, ez;
     class_extents(cls, g.x_max - g.x_min + 1, g.y_max - g.y_min + 1, g.z_max - g.z_min + 1, ex, ey, ez);
     const int64_t total = (int64_t)ex * ey * ez;
-    reserve(total);
+    reserve(total, st);
     const int64_t pieces = (total + elems_ - 1) / elems_;
     for (int64_t p = 0; p < pieces; p++) {
         Buf &b = buf_[next_];
