@@ -280,7 +280,7 @@ int clover_hip_calc_dt_kernel(CLOVER_DIMS, double g_small, double g_big, double 
                                       res(xvel0, AC_VERT, g), res(yvel0, AC_VERT, g), res(zvel0, AC_VERT, g),
                                       res(dt_min, AC_VERT, g), C.partial, &nparts, C.stream),
                  "calc_dt");
-    check_launch(launch_dt_final(C.partial, nparts, g_big, g_big, g_big, 0.0, C.scalar, C.dt_slot, ++C.dt_seq, C.stream),
+    check_launch(launch_dt_final(C.partial, nparts, g_big, g_big, g_big, 0.0, reinterpret_cast<DtDev *>(C.scalar), C.dt_slot, ++C.dt_seq, C.stream),
                  "calc_dt min");
     const double dmin = wait_dt(C.dt_slot, C.dt_seq, C.stream);
     *dt_min_val = dmin;

@@ -164,12 +164,12 @@ __device__ __forceinline__ void cell_x_body(const Blk &bk, Lay g, Geo m, int mod
 }
 
 template <typename S>
-__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const double *__restrict__ dt, int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
+__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_x(const DtDev *__restrict__ dt, int xcd, Lay g, Geo m, int mode, const S *__restrict__ vfx, const S *__restrict__ vfy,
               const S *__restrict__ vfz, const S *__restrict__ density1,
               const S *__restrict__ energy1, S *__restrict__ mass_flux_x, S *__restrict__ rho_out,
               S *__restrict__ e_out, S *__restrict__ p_out, int rows)
 {
-    if (*dt < 0.0) return;  // a small step (launch_dt_final)
+    if (dt->small) return;  // a small step (launch_dt_final)
     cell_x_body<S>(hw_blk(xcd), g, m, mode, rows, vfx, vfy, vfz, density1, energy1, mass_flux_x, rho_out, e_out,
                    p_out);
 }
@@ -328,18 +328,18 @@ __device__ __forceinline__ void cell_march_body(const Blk &bk, Lay g, Geo m, con
 }
 
 template <int DIR, int MODE, typename S, bool LIN>
-__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const double *__restrict__ dt, int xcd, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
+__global__ void __launch_bounds__(64 * CROWS) k_fast_cell_march(const DtDev *__restrict__ dt, int xcd, Lay g, Geo m, const S *__restrict__ vfx, const S *__restrict__ vfy,
                   const S *__restrict__ vfz, const S *__restrict__ density1,
                   const S *__restrict__ energy1, S *__restrict__ mass_flux, S *__restrict__ rho_out,
                   S *__restrict__ e_out, S *__restrict__ p_out)
 {
-    if (*dt < 0.0) return;
+    if (dt->small) return;
     cell_march_body<LIN, DIR, MODE, S>(hw_blk(xcd), g, m, vfx, vfy, vfz, density1, energy1, mass_flux, rho_out, e_out,
                                   p_out);
 }
 
 template <typename S>
-static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m, int mode, int dir, const S *density1,
+static hipError_t fast_advec_cell_t(const DtDev *dt, const Lay &g, const Geo &m, int mode, int dir, const S *density1,
                                     const S *energy1, S *mass_flux_x, const S *vol_flux_x, S *mass_flux_y,
                                     const S *vol_flux_y, S *mass_flux_z, const S *vol_flux_z, S *rho_out, S *e_out,
                                     S *p_out, const Shape &sh, hipStream_t st)
@@ -373,7 +373,7 @@ static hipError_t fast_advec_cell_t(const double *dt, const Lay &g, const Geo &m
     return hipGetLastError();
 }
 
-hipError_t launch_fast_advec_cell(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
+hipError_t launch_fast_advec_cell(Store s, const DtDev *dt, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
                                   const void *density1, const void *energy1, void *mass_flux_x,
                                   const void *vol_flux_x, void *mass_flux_y, const void *vol_flux_y,
                                   void *mass_flux_z, const void *vol_flux_z, void *rho_out, void *e_out,

@@ -659,12 +659,13 @@ static void ideal_gas(clover_chunk *c, bool predict, bool need_sound = false)
 }
 
 // the step's dt on the device (fused kernels: launch_dt_final's, else uploaded)
-static double *dt_dev(clover_chunk *c) { return c->scalar + 6; }
+static DtDev *dt_dev(clover_chunk *c) { return reinterpret_cast<DtDev *>(c->scalar + 6); }
 
 static void put_dt(clover_chunk *c, double dt)
 {
-    c->h_scalar[6] = dt;
-    hip_check(hipMemcpyAsync(dt_dev(c), c->h_scalar + 6, sizeof(double), hipMemcpyHostToDevice, c->st), "dt");
+    DtDev *h = reinterpret_cast<DtDev *>(c->h_scalar + 6);
+    *h = DtDev{dt, 0};
+    hip_check(hipMemcpyAsync(dt_dev(c), h, sizeof(DtDev), hipMemcpyHostToDevice, c->st), "dt");
     hip_check(hipStreamSynchronize(c->st), "sync");
 }
 

@@ -28,6 +28,7 @@
 
 #include <cmath>
 
+#include "kernels.h"
 #include "layout.h"
 
 namespace clover {
@@ -144,18 +145,17 @@ hipError_t launch_fast_visc_dt(Store s, const Lay &g, const Geo &m, double dtc_s
 
 // PdV predictor (PdV_kernel.f90:76-117) followed by ideal_gas on the
 // predicted density/energy (ideal_gas.f90:53-62): writes pressure only.
-hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
+hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0,
                                    const void *energy0, void *pressure, const void *viscosity, const void *xvel0,
                                    const void *yvel0, const void *zvel0, const Shape &sh, hipStream_t st);
 
-// (dt here and below: the step's dt in device memory; where it is negative,
-// launch_dt_final's mark of a small step, a kernel does nothing)
+// (dt here and below: the step's dt in device memory, kernels.h DtDev)
 //
 // accelerate (accelerate_kernel.f90:61-109), then the PdV corrector
 // (PdV_kernel.f90:124-165) and flux_calc (flux_calc_kernel.f90:56-90) on its
 // level-1 velocities, in one z-march: writes xvel1/yvel1/zvel1, density1,
 // energy1 and the three volume fluxes
-hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
+hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0,
                                  void *density1, const void *energy0, void *energy1, const void *pressure,
                                  const void *viscosity, const void *xvel0, void *xvel1, const void *yvel0,
                                  void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,
@@ -167,7 +167,7 @@ hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const doub
 // exchanged within it.  Writes what launch_fast_accel_pdv writes; the predicted
 // pressure is not stored.
 inline bool lagrange_tile(const Lay &g) { return g.mirror == 63; }
-hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0, void *density1,
+hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0, void *density1,
                                 const void *energy0, void *energy1, const void *viscosity, const void *xvel0,
                                 void *xvel1, const void *yvel0, void *yvel1, const void *zvel0, void *zvel1,
                                 void *vol_flux_x, void *vol_flux_y, void *vol_flux_z, const Shape &sh, hipStream_t st);
@@ -177,7 +177,7 @@ hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const doubl
 // range, the new density1/energy1 of interior cells go to rho_out/e_out.
 // On the step's third sweep, pressure/soundspeed (both or neither) also get
 // ideal_gas of the new state: the next step's ideal_gas results.
-hipError_t launch_fast_advec_cell(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
+hipError_t launch_fast_advec_cell(Store s, const DtDev *dt, const Lay &g, const Geo &m, int advect_x, int dir, int sweep_number,
                                   const void *density1, const void *energy1, void *mass_flux_x,
                                   const void *vol_flux_x, void *mass_flux_y, const void *vol_flux_y,
                                   void *mass_flux_z, const void *vol_flux_z, void *rho_out, void *e_out,
@@ -189,7 +189,7 @@ hipError_t launch_fast_advec_cell(Store s, const double *dt, const Lay &g, const
 // velocities go to vel_out[3]: they read their neighbours' old values, so
 // they cannot be updated in place.  Only nodes min..max+1 of vel_out are
 // written.
-hipError_t launch_fast_advec_mom(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int sweep_number,
+hipError_t launch_fast_advec_mom(Store s, const DtDev *dt, const Lay &g, const Geo &m, int advect_x, int sweep_number,
                                  int direction, const void *mass_flux_x, const void *vol_flux_x,
                                  const void *mass_flux_y, const void *vol_flux_y, const void *mass_flux_z,
                                  const void *vol_flux_z, const void *density1, const void *const *vel_in,

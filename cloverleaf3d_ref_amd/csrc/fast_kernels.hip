@@ -543,13 +543,13 @@ __device__ __forceinline__ void pdv_predict_pair_body(const Blk &bk, Lay g, Geo 
 }
 
 template <bool LIN, typename S>
-__global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, const S *__restrict__ energy0,
+__global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, Geo m, const DtDev *__restrict__ dtp, const S *__restrict__ density0, const S *__restrict__ energy0,
                    S *__restrict__ pressure, const S *__restrict__ viscosity,
                    const S *__restrict__ xvel0, const S *__restrict__ yvel0,
                    const S *__restrict__ zvel0)
 {
-    const double dt = *dtp;
-    if (dt < 0.0) return;
+    const double dt = dtp->dt;
+    if (dtp->small) return;
     if constexpr (sizeof(S) == 4)
         pdv_predict_pair_body<LIN>(hw_blk(xcd), g, m, dt, density0, energy0, pressure, viscosity, xvel0, yvel0, zvel0);
     else
@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_fast_pdv_predict(int xcd, Lay g, 
 }
 
 template <typename S>
-static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, const double *dt, const S *density0,
+static hipError_t fast_pdv_predict_t(const Lay &g, const Geo &m, const DtDev *dt, const S *density0,
                                    const S *energy0, S *pressure, const S *viscosity,
                                    const S *xvel0, const S *yvel0, const S *zvel0, const Shape &sh, hipStream_t st)
 {
@@ -715,7 +715,7 @@ hipError_t launch_fast_visc_dt(Store s, const Lay &g, const Geo &m, double dtc_s
 #undef CALL
 }
 
-hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
+hipError_t launch_fast_pdv_predict(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0,
                                    const void *energy0, void *pressure, const void *viscosity, const void *xvel0,
                                    const void *yvel0, const void *zvel0, const Shape &sh, hipStream_t st)
 {

@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(MIN_THREADS) k_min_final(const double *__restr
 
 __global__ void __launch_bounds__(MIN_THREADS) k_dt_final(const double *__restrict__ partial, int n, double g_big,
                                                           double dt_rise, double dtmax, double dtmin,
-                                                          double *__restrict__ dt, DtSlot *host, unsigned long long seq)
+                                                          DtDev *__restrict__ dt, DtSlot *host, unsigned long long seq)
 {
     const double b = min_of_partials(partial, n, g_big);
     if (threadIdx.x) return;
@@ -264,13 +264,13 @@ __global__ void __launch_bounds__(MIN_THREADS) k_dt_final(const double *__restri
     if (b <= m) m = b;
     if (dt_rise < m) m = dt_rise;
     if (dtmax < m) m = dtmax;
-    *dt = m < dtmin ? -1.0 : m;
+    *dt = DtDev{m, m < dtmin};
     host->dtlp = b;
     __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 hipError_t launch_dt_final(const double *partial, int n, double g_big, double dt_rise, double dtmax, double dtmin,
-                           double *dt, DtSlot *host, unsigned long long seq, hipStream_t st)
+                           DtDev *dt, DtSlot *host, unsigned long long seq, hipStream_t st)
 {
     TIMED_LAUNCH("k_dt_final", st, k_dt_final, dim3(1), dim3(MIN_THREADS), 0, st, partial, n, g_big, dt_rise, dtmax,
                  dtmin, dt, host, seq);

@@ -42,12 +42,18 @@ struct DtSlot {
     double dtlp;
     unsigned long long seq;
 };
+// A step's dt on the device.  small: it lies below dtmin, and the step's kernels,
+// which may be enqueued before the host knows, do nothing (no value of dt says
+// so: a deck's bounds may make it negative)
+struct DtDev {
+    double dt;
+    long long small;
+};
 // timestep.f90:86-126 for one tile on the device: the minimum of the partials
 // (seeded with g_big) goes to `host` (tagged seq) and the step's dt, min(dtlp,
-// dt_rise, dtmax), to *dt; -1 there when it lies below dtmin, which the step's
-// first kernel takes as nothing to do
+// dt_rise, dtmax), to *dt
 hipError_t launch_dt_final(const double *partial, int n, double g_big, double dt_rise, double dtmax, double dtmin,
-                           double *dt, DtSlot *host, unsigned long long seq, hipStream_t st);
+                           DtDev *dt, DtSlot *host, unsigned long long seq, hipStream_t st);
 
 hipError_t launch_pdv(int predict, const Lay &g, double dt, const double *xarea, const double *yarea,
                       const double *zarea, const double *volume, const double *density0, double *density1,

@@ -368,34 +368,34 @@ __device__ __forceinline__ void lagrange_body(const Blk &bk, Lay g, Geo m, doubl
 
 template <typename S>
 __global__ void __launch_bounds__(64 * lw_of<S>())
-    k_fast_lagrange(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
+    k_fast_lagrange(int xcd, Lay g, Geo m, const DtDev *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
                     const S *__restrict__ energy0, S *__restrict__ energy1, const S *__restrict__ viscosity,
                     const S *__restrict__ xvel0, S *__restrict__ xvel1, const S *__restrict__ yvel0,
                     S *__restrict__ yvel1, const S *__restrict__ zvel0, S *__restrict__ zvel1,
                     S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y, S *__restrict__ vol_flux_z)
 {
-    const double dt = *dtp;
-    if (dt < 0.0) return;
+    const double dt = dtp->dt;
+    if (dtp->small) return;
     lagrange_body<true, S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, nullptr, viscosity, xvel0,
                            xvel1, yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
 }
 
 template <typename S>
 __global__ void __launch_bounds__(64 * lw_of<S>())
-    k_fast_accel_pdv(int xcd, Lay g, Geo m, const double *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
+    k_fast_accel_pdv(int xcd, Lay g, Geo m, const DtDev *__restrict__ dtp, const S *__restrict__ density0, S *__restrict__ density1,
                      const S *__restrict__ energy0, S *__restrict__ energy1, const S *__restrict__ pressure,
                      const S *__restrict__ viscosity, const S *__restrict__ xvel0, S *__restrict__ xvel1,
                      const S *__restrict__ yvel0, S *__restrict__ yvel1, const S *__restrict__ zvel0,
                      S *__restrict__ zvel1, S *__restrict__ vol_flux_x, S *__restrict__ vol_flux_y,
                      S *__restrict__ vol_flux_z)
 {
-    const double dt = *dtp;
-    if (dt < 0.0) return;
+    const double dt = dtp->dt;
+    if (dtp->small) return;
     lagrange_body<false, S>(hw_blk(xcd), g, m, dt, density0, density1, energy0, energy1, pressure, viscosity, xvel0,
                             xvel1, yvel0, yvel1, zvel0, zvel1, vol_flux_x, vol_flux_y, vol_flux_z);
 }
 
-hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0, void *density1,
+hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0, void *density1,
                                 const void *energy0, void *energy1, const void *viscosity, const void *xvel0,
                                 void *xvel1, const void *yvel0, void *yvel1, const void *zvel0, void *zvel1,
                                 void *vol_flux_x, void *vol_flux_y, void *vol_flux_z, const Shape &sh, hipStream_t st)
@@ -420,7 +420,7 @@ hipError_t launch_fast_lagrange(Store s, const Lay &g, const Geo &m, const doubl
     return hipGetLastError();
 }
 
-hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const double *dt, const void *density0,
+hipError_t launch_fast_accel_pdv(Store s, const Lay &g, const Geo &m, const DtDev *dt, const void *density0,
                                  void *density1, const void *energy0, void *energy1, const void *pressure,
                                  const void *viscosity, const void *xvel0, void *xvel1, const void *yvel0,
                                  void *yvel1, const void *zvel0, void *zvel1, void *vol_flux_x, void *vol_flux_y,

@@ -697,11 +697,11 @@ __device__ __forceinline__ void mom_march(int lin, int gx, int gy, int gz, int x
 }
 
 template <int DIR, int MODE, typename S>
-__global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fast_mom_march(const double *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf, const S *__restrict__ vfx,
+__global__ void __launch_bounds__(64 * mw_of(DIR), sizeof(S) == 8 ? 4 : 1) k_fast_mom_march(const DtDev *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf, const S *__restrict__ vfx,
                  const S *__restrict__ vfy, const S *__restrict__ vfz,
                  const S *__restrict__ density1, Vel3<S> v)
 {
-    if (*dt < 0.0) return;  // a small step (launch_dt_final)
+    if (dt->small) return;  // a small step (launch_dt_final)
     const int gx = (int)gridDim.x, gy = (int)gridDim.y, gz = (int)gridDim.z;
     mom_march<DIR, MODE, S>((int)blockIdx.x + gx * ((int)blockIdx.y + gy * (int)blockIdx.z), gx, gy, gz, xcd, g, geo,
                             mf, vfx, vfy, vfz, density1, v);
@@ -862,10 +862,10 @@ __device__ __forceinline__ void mom_x_body(const Blk &bk, Lay g, Geo geo, const 
 
 template <int MODE, typename S>
 __global__ void __launch_bounds__(64 * mw_of(1), sizeof(S) == 8 ? 6 : 1)
-k_fast_mom_x(const double *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf,
+k_fast_mom_x(const DtDev *__restrict__ dt, int xcd, Lay g, Geo geo, const S *__restrict__ mf,
              const S *__restrict__ vfy, const S *__restrict__ vfz, const S *__restrict__ density1, Vel3<S> v)
 {
-    if (*dt < 0.0) return;  // a small step (launch_dt_final)
+    if (dt->small) return;  // a small step (launch_dt_final)
     mom_x_body<MODE, S>(hw_blk(xcd), g, geo, mf, vfy, vfz, density1, v);
 }
 
@@ -880,7 +880,7 @@ static int mom_mode(int advect_x, int sweep_number, int direction)
 }
 
 template <typename S>
-static hipError_t fast_advec_mom_t(const double *dt, const Lay &g, const Geo &m, int mode, int direction, const S *mass_flux_x,
+static hipError_t fast_advec_mom_t(const DtDev *dt, const Lay &g, const Geo &m, int mode, int direction, const S *mass_flux_x,
                                    const S *vol_flux_x, const S *mass_flux_y, const S *vol_flux_y,
                                    const S *mass_flux_z, const S *vol_flux_z, const S *density1,
                                    const void *const *vel_in, void *const *vel_out, const Shape &sh, hipStream_t st)
@@ -912,7 +912,7 @@ static hipError_t fast_advec_mom_t(const double *dt, const Lay &g, const Geo &m,
     return hipGetLastError();
 }
 
-hipError_t launch_fast_advec_mom(Store s, const double *dt, const Lay &g, const Geo &m, int advect_x, int sweep_number,
+hipError_t launch_fast_advec_mom(Store s, const DtDev *dt, const Lay &g, const Geo &m, int advect_x, int sweep_number,
                                  int direction, const void *mass_flux_x, const void *vol_flux_x,
                                  const void *mass_flux_y, const void *vol_flux_y, const void *mass_flux_z,
                                  const void *vol_flux_z, const void *density1, const void *const *vel_in,
