@@ -99,7 +99,7 @@ def gpu_bench(cells: int, steps: int, warmup: int, summary_frequency: int = 25, 
         t0 = time.perf_counter()
         before, after = c.autotune()
         autotune = dict(seconds=time.perf_counter() - t0, pass_ms_before=before, pass_ms_after=after,
-                        shapes=c.shapes())
+                        shapes=c.launch_shapes())
     L = _lib.lib()
     for _ in range(warmup):
         c.step()
@@ -154,7 +154,7 @@ def ensemble_bench(ndecks: int, steps: int, fp32: bool = False, warmup: int = 2,
         t0 = time.perf_counter()
         before, after = e.autotune()
         autotune = dict(seconds=time.perf_counter() - t0, pass_ms_before=before, pass_ms_after=after,
-                        shapes=e.shapes(), workgroups=e.workgroups())
+                        shapes=e.launch_shapes(), workgroups=e.workgroups())
     e.run(warmup)
     t0 = time.perf_counter()
     e.run(steps)

@@ -190,15 +190,27 @@ class Chunk:
                    "clover_chunk_autotune")
         return before.value, after.value
 
-    def shapes(self) -> Dict[str, Tuple[int, int, int]]:
-        """kernel -> (planes per workgroup, XCD-contiguous block order,
-        workgroup width)"""
+    def launch_shapes(self) -> Dict[str, Tuple[int, int, int]]:
+        """kernel -> the shape in force (planes per workgroup, XCD-contiguous
+        block order, workgroup width), as set_shape takes it"""
         out = {}
         for k, name in enumerate(_lib.SHAPE_KERNELS):
             planes, xcd, bx = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
             _lib.check(self._L.clover_chunk_get_shape(self._h, k, ctypes.byref(planes), ctypes.byref(xcd),
                                                       ctypes.byref(bx)), "clover_chunk_get_shape")
             out[name] = (planes.value, xcd.value, bx.value)
+        return out
+
+    def shapes(self) -> Dict[str, Tuple[int, int, int]]:
+        """launch_shapes, with the kernel's bound in place of the planes where
+        they were chosen from the mesh's size: one name for the choice on any
+        mesh, among the planes the autotuner tries"""
+        out = {}
+        for k, (name, (planes, xcd, bx)) in enumerate(self.launch_shapes().items()):
+            bound = ctypes.c_int()
+            _lib.check(self._L.clover_chunk_get_shape_bound(self._h, k, ctypes.byref(bound)),
+                       "clover_chunk_get_shape_bound")
+            out[name] = (bound.value or planes, xcd, bx)
         return out
 
     def set_shape(self, kernel: str, planes: int, xcd: int, block_x: int = 64) -> None:

@@ -1688,10 +1688,18 @@ int clover_chunk_get_shape(const clover_chunk *c, int kernel, int *planes, int *
     CLOVER_API_BEGIN
     if (!c || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    const Shape &sh = c->shapes.k[kernel];
-    *planes = sh.cap ? sh.cap : sh.planes;
+    *planes = c->shapes.k[kernel].planes;
     *xcd = c->shapes.k[kernel].xcd;
     *block_x = c->shapes.k[kernel].bx;
+    CLOVER_API_END
+}
+
+int clover_chunk_get_shape_bound(const clover_chunk *c, int kernel, int *planes)
+{
+    CLOVER_API_BEGIN
+    if (!c || !planes) throw Error(E_ARG, "null argument");
+    if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
+    *planes = c->shapes.k[kernel].cap;
     CLOVER_API_END
 }
 

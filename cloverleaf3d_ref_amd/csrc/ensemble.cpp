@@ -46,7 +46,8 @@ struct clover_ensemble {
     int advect_x = 1;
     Slots slots;  // where the table holds each array (its own slot between steps)
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // index: advect_x
-    Shapes shapes{};                               // launch shapes (size_shapes, autotuner)
+    Shapes shapes{};                               // launch shapes in force (size, autotuner, set_shape)
+    Shapes size{};                                 // those it started with (size_shapes)
 };
 
 namespace {
@@ -463,7 +464,7 @@ int clover_ensemble_create(const clover_deck *decks, int ndecks, int device, int
         hip_check(hipMemcpy(e->dev, e->host.data(), sizeof(DeckDev) * ndecks, hipMemcpyHostToDevice), "H2D decks");
         std::vector<Lay> lays(ndecks);
         for (int d = 0; d < ndecks; d++) lays[d] = e->host[d].g;
-        e->shapes = size_shapes(e->store, lays.data(), ndecks);
+        e->shapes = e->size = size_shapes(e->store, lays.data(), ndecks);
         prepare_grids(e);
         // calc_dt's partials: room for the visc/dt grid of every shape the
         // autotuner tries and of the one the decks start with (the most
@@ -600,10 +601,18 @@ int clover_ensemble_get_shape(const clover_ensemble *e, int kernel, int *planes,
     CLOVER_API_BEGIN
     if (!e || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    const Shape &sh = e->shapes.k[kernel];
-    *planes = sh.cap ? sh.cap : sh.planes;
+    *planes = e->shapes.k[kernel].planes;
     *xcd = e->shapes.k[kernel].xcd;
     *block_x = e->shapes.k[kernel].bx;
+    CLOVER_API_END
+}
+
+int clover_ensemble_get_shape_bound(const clover_ensemble *e, int kernel, int *planes)
+{
+    CLOVER_API_BEGIN
+    if (!e || !planes) throw Error(E_ARG, "null argument");
+    if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
+    *planes = e->shapes.k[kernel].cap;
     CLOVER_API_END
 }
 
@@ -621,8 +630,9 @@ int clover_ensemble_set_shape(clover_ensemble *e, int kernel, int planes, int xc
     CLOVER_API_BEGIN
     if (!e) throw Error(E_ARG, "null ensemble");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    // calc_dt's partial buffer holds the visc/dt tiles of the fewest planes the tuner tries
-    if (planes < kTunePlanes[0]) throw Error(E_ARG, "planes below the smallest tuned value");
+    // calc_dt's partial buffer holds the visc/dt tiles of the fewest planes the
+    // tuner tries, and of those the ensemble started with
+    if (planes < kTunePlanes[0] && planes != e->size.k[kernel].planes) throw Error(E_ARG, "planes below the smallest tuned value");
     if (xcd != 0 && xcd != 1) throw Error(E_ARG, "xcd must be 0 or 1");
     if (workgroups < 0) throw Error(E_ARG, "workgroups must be >= 0");
     hip_check(hipSetDevice(e->device), "hipSetDevice");

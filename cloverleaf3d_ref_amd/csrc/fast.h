@@ -51,8 +51,8 @@ struct Shape {
     int bx;   // z marches: threads along x per workgroup (64, 128, 256 or 512; see block_of)
     int wgs;  // batched launches: 0 for one workgroup per tile, else this many
               // persistent workgroups walk the tile list (batch.h tile_walk)
-    int cap;  // 0, or the most planes size_shapes allows on any mesh: `planes`
-              // is then what it gave this one
+    int cap;  // 0, or the most planes size_shapes allows this kernel on any mesh:
+              // `planes` is then what it gave this one
 };
 
 // Workgroup of a z march for shape sh: bx threads along x and 256/bx rows

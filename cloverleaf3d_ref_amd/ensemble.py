@@ -101,15 +101,31 @@ class Ensemble:
         return out
 
     def set_shape(self, kernel: str, planes: int, xcd: int, workgroups: int = 0) -> None:
-        """Launch shape of one batched kernel (planes >= 8); never changes a value."""
+        """Launch shape of one batched kernel (planes >= 8, or those it started
+        with); never changes a value."""
         _lib.check(self._L.clover_ensemble_set_shape(self._h, _lib.SHAPE_KERNELS.index(kernel), planes, xcd,
                                                      workgroups), "clover_ensemble_set_shape")
 
+    def _shape(self, k: int) -> Tuple[int, int, int]:
+        planes, xcd, bx = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        _lib.check(self._L.clover_ensemble_get_shape(self._h, k, ctypes.byref(planes), ctypes.byref(xcd),
+                                                     ctypes.byref(bx)), "clover_ensemble_get_shape")
+        return planes.value, xcd.value, bx.value
+
+    def launch_shapes(self) -> Dict[str, Tuple[int, int, int]]:
+        """kernel -> the shape in force (planes per workgroup, XCD-contiguous
+        block order, workgroups), as set_shape takes it"""
+        wgs = self.workgroups()
+        return {name: (*self._shape(k)[:2], wgs[name]) for k, name in enumerate(_lib.SHAPE_KERNELS)}
+
     def shapes(self) -> Dict[str, Tuple[int, int, int]]:
+        """kernel -> (planes per workgroup, XCD-contiguous block order, workgroup
+        width), with the kernel's bound in place of the planes where they were
+        chosen from the decks' sizes, as Chunk.shapes"""
         out = {}
         for k, name in enumerate(_lib.SHAPE_KERNELS):
-            planes, xcd, bx = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-            _lib.check(self._L.clover_ensemble_get_shape(self._h, k, ctypes.byref(planes), ctypes.byref(xcd),
-                                                         ctypes.byref(bx)), "clover_ensemble_get_shape")
-            out[name] = (planes.value, xcd.value, bx.value)
+            (planes, xcd, bx), bound = self._shape(k), ctypes.c_int()
+            _lib.check(self._L.clover_ensemble_get_shape_bound(self._h, k, ctypes.byref(bound)),
+                       "clover_ensemble_get_shape_bound")
+            out[name] = (bound.value or planes, xcd, bx)
         return out

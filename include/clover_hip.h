@@ -290,9 +290,11 @@ int clover_chunk_kernel_times(clover_chunk *c, char *buf, int buflen);
  * of the visc/dt and PdV-predictor z marches (64, 128, 256 or 512 threads
  * along x, with 256/64, 256/128 or 1 rows; the other kernels' workgroups are
  * fixed, block_x 64).
- * A chunk (and an ensemble) starts with shapes chosen from its size: `planes`
- * is then the most positions its workgroups march over, and a mesh with few
- * tiles takes fewer so that they fill the GPU.
+ * A chunk (and an ensemble) starts with shapes chosen from its size: a mesh
+ * with few tiles marches over fewer positions so that they fill the GPU, a
+ * large one over at most the kernel's bound (clover_*_get_shape_bound).
+ * clover_*_get_shape returns the shape in force, and setting it again changes
+ * nothing.
  * A shape changes how the work is split, never a value.  Kernel indices: */
 #define CLOVER_SHAPE_VISC_DT 0
 #define CLOVER_SHAPE_PDV_PREDICT 1
@@ -306,12 +308,15 @@ int clover_chunk_kernel_times(clover_chunk *c, char *buf, int buflen);
 #define CLOVER_SHAPE_COUNT 9
 /* The autotuner: times every shaped kernel with every candidate shape (planes
  * 8, 16, 32, 64, 128 x both block orders x, for the z marches, the four
- * workgroup widths) on this chunk's own arrays and keeps
+ * workgroup widths) and the shape in force on this chunk's own arrays and keeps
  * the fastest.  Candidates write only spare work arrays, so every field
  * keeps its value.  ms_before/ms_after (may be null) get one pass of all
  * shaped kernels with the old and the chosen shapes.  Fused kernels only. */
 int clover_chunk_autotune(clover_chunk *c, double *ms_before, double *ms_after);
 int clover_chunk_get_shape(const clover_chunk *c, int kernel, int *planes, int *xcd, int *block_x);
+/* `planes`: the bound under which the kernel's positions were chosen from the
+ * mesh's size, 0 for a shape that the autotuner or set_shape chose */
+int clover_chunk_get_shape_bound(const clover_chunk *c, int kernel, int *planes);
 int clover_chunk_set_shape(clover_chunk *c, int kernel, int planes, int xcd, int block_x);
 
 /* ------------------------------------------------------------ ensembles */
@@ -347,13 +352,14 @@ long long clover_ensemble_device_bytes(const clover_ensemble *e);
  * are captured again with the chosen shapes on the next run. */
 int clover_ensemble_autotune(clover_ensemble *e, double *ms_before, double *ms_after);
 int clover_ensemble_get_shape(const clover_ensemble *e, int kernel, int *planes, int *xcd, int *block_x);
+int clover_ensemble_get_shape_bound(const clover_ensemble *e, int kernel, int *planes);
 /* Workgroups of a batched kernel's launch: 0 for one per tile (a tile is
  * one workgroup-sized block of one deck), else that many persistent
  * workgroups walk the ensemble's tile list.  No counterpart in the
  * reference (it has one deck); chosen by clover_ensemble_autotune. */
 int clover_ensemble_get_workgroups(const clover_ensemble *e, int kernel, int *workgroups);
 /* Set a batched kernel's launch shape by hand (CLOVER_SHAPE_* kernel, planes
- * >= 8, xcd 0/1, workgroups as above).  Changes how the work is split,
+ * >= 8 or those the ensemble started with, xcd 0/1, workgroups as above).  Changes how the work is split,
  * never a value; captured steps are dropped and captured again. */
 int clover_ensemble_set_shape(clover_ensemble *e, int kernel, int planes, int xcd, int workgroups);
 
