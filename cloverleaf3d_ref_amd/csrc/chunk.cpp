@@ -1179,7 +1179,7 @@ static void autotune(clover_chunk *c, double *before, double *after)
     DeckDev *ttab = nullptr;
     if (c->batched) hip_check(hipMalloc(&ttab, sizeof(DeckDev) * c->tiles.size()), "hipMalloc");
     for (int k = 0; k < SK_COUNT; k++) {
-        if (k == SK_PDV_PREDICT && lagrange_chunk(c)) continue;  // not launched: accel_pdv's shape is the whole phase's
+        if (shape_slot(k, lagrange_chunk(c)) != k) continue;  // the march's, tuned as accel_pdv's
         if (ttab) {
             const std::vector<DeckDev> h = tune_table(c, k);
             hip_check(hipMemcpyAsync(ttab, h.data(), sizeof(DeckDev) * h.size(), hipMemcpyHostToDevice, c->st),
@@ -1688,9 +1688,10 @@ int clover_chunk_get_shape(const clover_chunk *c, int kernel, int *planes, int *
     CLOVER_API_BEGIN
     if (!c || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = c->shapes.k[kernel].planes;
-    *xcd = c->shapes.k[kernel].xcd;
-    *block_x = c->shapes.k[kernel].bx;
+    const Shape &sh = c->shapes.k[shape_slot(kernel, lagrange_chunk(c))];
+    *planes = sh.planes;
+    *xcd = sh.xcd;
+    *block_x = sh.bx;
     CLOVER_API_END
 }
 
@@ -1699,7 +1700,7 @@ int clover_chunk_get_shape_bound(const clover_chunk *c, int kernel, int *planes)
     CLOVER_API_BEGIN
     if (!c || !planes) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = c->shapes.k[kernel].cap;
+    *planes = c->shapes.k[shape_slot(kernel, lagrange_chunk(c))].cap;
     CLOVER_API_END
 }
 
@@ -1712,7 +1713,8 @@ int clover_chunk_set_shape(clover_chunk *c, int kernel, int planes, int xcd, int
     if (block_x != 64 && block_x != 128 && block_x != 256 && block_x != 512)
         throw Error(E_ARG, "block_x must be 64, 128, 256 or 512");
     if (block_x != 64 && !z_march(kernel)) throw Error(E_ARG, "only the z marches take a workgroup width");
-    c->shapes.k[kernel] = Shape{planes, xcd, block_x};
+    const int slot = shape_slot(kernel, lagrange_chunk(c));
+    c->shapes.k[slot] = Shape{planes, xcd, z_march(slot) ? block_x : 64};  // the march's workgroups are fixed
     CLOVER_API_END
 }
 

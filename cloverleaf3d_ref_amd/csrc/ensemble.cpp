@@ -601,9 +601,10 @@ int clover_ensemble_get_shape(const clover_ensemble *e, int kernel, int *planes,
     CLOVER_API_BEGIN
     if (!e || !planes || !xcd || !block_x) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = e->shapes.k[kernel].planes;
-    *xcd = e->shapes.k[kernel].xcd;
-    *block_x = e->shapes.k[kernel].bx;
+    const Shape &sh = e->shapes.k[shape_slot(kernel, true)];
+    *planes = sh.planes;
+    *xcd = sh.xcd;
+    *block_x = sh.bx;
     CLOVER_API_END
 }
 
@@ -612,7 +613,7 @@ int clover_ensemble_get_shape_bound(const clover_ensemble *e, int kernel, int *p
     CLOVER_API_BEGIN
     if (!e || !planes) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *planes = e->shapes.k[kernel].cap;
+    *planes = e->shapes.k[shape_slot(kernel, true)].cap;
     CLOVER_API_END
 }
 
@@ -621,7 +622,7 @@ int clover_ensemble_get_workgroups(const clover_ensemble *e, int kernel, int *wo
     CLOVER_API_BEGIN
     if (!e || !workgroups) throw Error(E_ARG, "null argument");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
-    *workgroups = e->shapes.k[kernel].wgs;
+    *workgroups = e->shapes.k[shape_slot(kernel, true)].wgs;
     CLOVER_API_END
 }
 
@@ -630,14 +631,15 @@ int clover_ensemble_set_shape(clover_ensemble *e, int kernel, int planes, int xc
     CLOVER_API_BEGIN
     if (!e) throw Error(E_ARG, "null ensemble");
     if (kernel < 0 || kernel >= SK_COUNT) throw Error(E_ARG, "kernel out of range");
+    const int slot = shape_slot(kernel, true);
     // calc_dt's partial buffer holds the visc/dt tiles of the fewest planes the
     // tuner tries, and of those the ensemble started with
-    if (planes < kTunePlanes[0] && planes != e->size.k[kernel].planes) throw Error(E_ARG, "planes below the smallest tuned value");
+    if (planes < kTunePlanes[0] && planes != e->size.k[slot].planes) throw Error(E_ARG, "planes below the smallest tuned value");
     if (xcd != 0 && xcd != 1) throw Error(E_ARG, "xcd must be 0 or 1");
     if (workgroups < 0) throw Error(E_ARG, "workgroups must be >= 0");
     hip_check(hipSetDevice(e->device), "hipSetDevice");
     hip_check(hipStreamSynchronize(e->st), "sync");
-    Shape &sh = e->shapes.k[kernel];
+    Shape &sh = e->shapes.k[slot];
     sh.planes = planes;
     sh.xcd = xcd;
     sh.wgs = workgroups;

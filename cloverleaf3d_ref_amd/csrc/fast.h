@@ -72,6 +72,10 @@ constexpr int kTuneCount = sizeof(kTunePlanes) / sizeof(kTunePlanes[0]);
 // (the tuner's candidates give 1, 2 and 4)
 __host__ __device__ inline int cell_x_rows(int planes) { return planes >= 64 ? planes / 32 : 1; }
 
+// The shape of kernel SK_* as a caller names it: where the Lagrangian phase is one
+// march, the predictor's is the march's, kept as accel_pdv's
+inline int shape_slot(int kernel, bool lagrange) { return kernel == SK_PDV_PREDICT && lagrange ? SK_ACCEL_PDV : kernel; }
+
 // The launch shapes of a mesh (or of the tiles or decks one launch covers)
 // before any tuning, chosen from its size (fast_kernels.hip)
 Shapes size_shapes(Store s, const Lay *lays, int n);

@@ -298,7 +298,10 @@ int clover_chunk_kernel_times(clover_chunk *c, char *buf, int buflen);
  * A shape changes how the work is split, never a value.  Kernel indices: */
 #define CLOVER_SHAPE_VISC_DT 0
 #define CLOVER_SHAPE_PDV_PREDICT 1
-#define CLOVER_SHAPE_ACCEL_PDV 2 /* accelerate + PdV corrector + flux_calc */
+#define CLOVER_SHAPE_ACCEL_PDV 2 /* accelerate + PdV corrector + flux_calc; on a
+    single tile at least 3 cells thick, and in an ensemble, one march runs the
+    predictor as well, both indices name its shape, and its workgroup width is
+    fixed (a width set through the predictor's index is not taken) */
 #define CLOVER_SHAPE_CELL_X 3
 #define CLOVER_SHAPE_CELL_Y 4
 #define CLOVER_SHAPE_CELL_Z 5

@@ -53,3 +53,24 @@ def test_ensemble(fp32):
             e.set_shape(name, *shape)
         e.run(2)
         assert (e.summaries(), e.state()) == want
+
+
+def test_predictor_names_the_marchs_shape():
+    """One march runs the predictor and accel_pdv on a single tile and in ensembles: both names are its shape's."""
+    print("[gpu] shapes in force, predictor", flush=True)
+    for owner in (Chunk(parse_deck(cuboid_deck(20, 10, 0))), Ensemble([parse_deck(cuboid_deck(20, 10, 0))])):
+        with owner as x:
+            shapes = x.launch_shapes()
+            assert shapes["pdv_predict"] == shapes["accel_pdv"]
+            x.set_shape("pdv_predict", 24, 1)
+            shapes = x.launch_shapes()
+            assert shapes["pdv_predict"] == shapes["accel_pdv"] and shapes["accel_pdv"][:2] == (24, 1)
+            x.autotune()
+            assert x.launch_shapes()["pdv_predict"] == x.launch_shapes()["accel_pdv"]
+    with Chunk(parse_deck(cuboid_deck(20, 10, 0))) as c:
+        c.set_shape("pdv_predict", 24, 1, 256)  # taken as before, but the march has one width
+        assert c.launch_shapes()["pdv_predict"] == (24, 1, 64)
+    with Chunk(parse_deck(cuboid_deck(20, 10, 0, tiles=2))) as c:  # two kernels
+        c.set_shape("pdv_predict", 24, 1, 256)
+        c.set_shape("accel_pdv", 12, 0)
+        assert c.launch_shapes()["pdv_predict"] == (24, 1, 256) and c.launch_shapes()["accel_pdv"] == (12, 0, 64)
