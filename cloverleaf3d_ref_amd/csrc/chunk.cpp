@@ -697,7 +697,7 @@ static int take_dt(clover_chunk *c, const double *dtlp, int stride)
 }
 
 // timestep.f90:28-128; returns 1 on a small time step.  With ahead() the dt is
-// only enqueued, and the caller takes it (finish_step).
+// only enqueued, and the caller takes it (hydro_step).
 static int timestep(clover_chunk *c)
 {
     int fields[NUM_FIELDS];
@@ -732,12 +732,7 @@ static int timestep(clover_chunk *c)
                                           c->partial + (size_t)ti * kMaxPartials * 5, &nparts[ti % 64],
                                           c->shapes.k[SK_VISC_DT], c->st),
                       "visc_dt");
-            if (ahead(c)) {
-                hip_check(launch_dt_final(c->partial, nparts[0], c->g_big, c->dtold * d.dtrise, d.dtmax, d.dtmin,
-                                          dt_dev(c), c->dt_slot, ++c->dt_seq, c->st),
-                          "calc_dt min");
-                continue;
-            }
+            if (ahead(c)) continue;  // below
             hip_check(launch_min_final(c->partial + (size_t)ti * kMaxPartials * 5, nparts[ti % 64], c->g_big,
                                        c->scalar + 8 * ti, c->st),
                       "calc_dt min");
@@ -749,6 +744,12 @@ static int timestep(clover_chunk *c)
                                        t.f[F_DENSITY0], t.f[F_PRESSURE], t.f[F_VISCOSITY], t.f[F_XVEL0],
                                        t.f[F_YVEL0], t.f[F_ZVEL0], c->st),
                       "viscosity");
+    }
+    if (ahead(c)) {
+        Phase ph(c, P_TIMESTEP);
+        hip_check(launch_dt_final(c->partial, nparts[0], c->g_big, c->dtold * d.dtrise, d.dtmax, d.dtmin, dt_dev(c),
+                                  c->dt_slot, ++c->dt_seq, c->st),
+                  "calc_dt min");
     }
     if (c->fast) {
         fused_halo(c, FH_VISCOSITY);

@@ -265,7 +265,11 @@ int clover_decompose_tiles(int x_cells, int y_cells, int z_cells, int tiles_per_
 int clover_chunk_fetch_field(clover_chunk *c, int t, int field, double *host);
 
 /* Per-phase device time (ms) accumulated with HIP events when profiling is
- * on: the reference profiler's categories (hydro.f90:147-167). */
+ * on: the reference profiler's categories (hydro.f90:147-167).  A fused kernel's
+ * time goes to one of them: calc_dt's cells to viscosity (its minimum and dt to
+ * timestep), flux_calc and the PdV corrector to acceleration and, where one
+ * march runs the whole Lagrangian phase (a single tile at least 3 cells thick),
+ * the predictor too, so that PdV is empty there. */
 int clover_chunk_set_profiling(clover_chunk *c, int on);
 int clover_chunk_profile(const clover_chunk *c, double *ms, int *calls, int n);
 const char *clover_chunk_profile_name(int i);
