@@ -1458,7 +1458,7 @@ int clover_chunk_create_ex(const clover_deck *deck, int device, int flags, clove
             }
         }
         // a launch covers every tile where the stages are batched, else one
-        c->shapes = size_shapes(c->store, lays.data(), c->batched ? T : 1);
+        c->shapes = size_shapes(c->store, lays.data(), c->batched ? T : 1, cu_count(device));
         // start.f90:58-129
         c->time = 0.0;
         c->step = 0;

@@ -308,8 +308,7 @@ void shapes_changed(clover_ensemble *e)
 
 void autotune(clover_ensemble *e, double *before, double *after)
 {
-    int cus = 0;
-    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device), "CU count");
+    const int cus = cu_count(e->device);
     hipEvent_t a = nullptr, b = nullptr;
     hip_check(hipEventCreate(&a), "event");
     hip_check(hipEventCreate(&b), "event");
@@ -464,7 +463,7 @@ int clover_ensemble_create(const clover_deck *decks, int ndecks, int device, int
         hip_check(hipMemcpy(e->dev, e->host.data(), sizeof(DeckDev) * ndecks, hipMemcpyHostToDevice), "H2D decks");
         std::vector<Lay> lays(ndecks);
         for (int d = 0; d < ndecks; d++) lays[d] = e->host[d].g;
-        e->shapes = e->size = size_shapes(e->store, lays.data(), ndecks);
+        e->shapes = e->size = size_shapes(e->store, lays.data(), ndecks, cu_count(device));
         prepare_grids(e);
         // calc_dt's partials: room for the visc/dt grid of every shape the
         // autotuner tries and of the one the decks start with (the most

@@ -77,8 +77,8 @@ __host__ __device__ inline int cell_x_rows(int planes) { return planes >= 64 ? p
 inline int shape_slot(int kernel, bool lagrange) { return kernel == SK_PDV_PREDICT && lagrange ? SK_ACCEL_PDV : kernel; }
 
 // The launch shapes of a mesh (or of the tiles or decks one launch covers)
-// before any tuning, chosen from its size (fast_kernels.hip)
-Shapes size_shapes(Store s, const Lay *lays, int n);
+// before any tuning, chosen from its size and the device's CUs (fast_kernels.hip)
+Shapes size_shapes(Store s, const Lay *lays, int n, int cus);
 
 inline size_t store_bytes(Store s) { return s == ST_F32 ? sizeof(float) : sizeof(double); }
 

@@ -941,9 +941,8 @@ static int size_planes(BatchKernel k, Store s, const Lay *lays, int n, int slots
     return best;
 }
 
-Shapes size_shapes(Store s, const Lay *lays, int n)
+Shapes size_shapes(Store s, const Lay *lays, int n, int cus)
 {
-    constexpr int cus = 256;
     const bool f32 = s == ST_F32;
     long long cells = 0;
     for (int i = 0; i < n; i++) {

@@ -36,6 +36,14 @@ inline void hip_check(hipError_t e, const char *what)
                     std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// CUs of a device: 256 on a whole MI355X, fewer of a partition
+inline int cu_count(int device)
+{
+    int cus = 0;
+    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device), "CU count");
+    return cus;
+}
+
 // Waits for the dt tagged seq, which a launch_dt_final on the stream is bound to
 // deliver: if the stream ends or fails without it, so does the wait.  Polling
 // pinned memory saves the copy back and the wake-up of a stream synchronisation.
