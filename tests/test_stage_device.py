@@ -29,6 +29,8 @@ inline hipError_t hipGetDevice(int *d) { *d = g_device; return hipSuccess; }
 inline hipError_t hipSetDevice(int d) { g_device = d; return hipSuccess; }
 inline hipError_t hipStreamGetDevice(hipStream_t s, int *d) { *d = s->device; return hipSuccess; }
 inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount };
+inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = calloc(n, 1); return hipSuccess; }
 inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
