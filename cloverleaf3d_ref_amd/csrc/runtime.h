@@ -9,6 +9,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 
 #include "kernels.h"
 #include "layout.h"
@@ -47,10 +48,15 @@ inline int cu_count(int device)
 // Waits for the dt tagged seq, which a launch_dt_final on the stream is bound to
 // deliver: if the stream ends or fails without it, so does the wait.  Polling
 // pinned memory saves the copy back and the wake-up of a stream synchronisation.
+// Past the first polls, some 20 us, the core is offered to other threads between
+// them: those of other chunks or processes may need it to get their own work to
+// the GPU.
 inline double wait_dt(const DtSlot *slot, unsigned long long seq, hipStream_t st)
 {
     for (long spins = 0;; spins++) {
         if (__atomic_load_n(&slot->seq, __ATOMIC_ACQUIRE) == seq) return slot->dtlp;
+        if (spins < 1000) __builtin_ia32_pause();
+        else std::this_thread::yield();
         if (spins % 100000 == 99999) {
             const hipError_t e = hipStreamQuery(st);
             if (e == hipErrorNotReady) continue;
