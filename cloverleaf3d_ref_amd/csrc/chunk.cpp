@@ -412,8 +412,7 @@ static int shape_of(int bk)
     switch (bk) {
     case BK_VISC_DT: return SK_VISC_DT;
     case BK_PDV_PREDICT: return SK_PDV_PREDICT;
-    case BK_ACCEL_PDV:
-    case BK_LAGRANGE: return SK_ACCEL_PDV;
+    case BK_ACCEL_PDV: return SK_ACCEL_PDV;
     case BK_CELL_X: return SK_CELL_X;
     case BK_CELL_Y: return SK_CELL_Y;
     case BK_CELL_Z: return SK_CELL_Z;

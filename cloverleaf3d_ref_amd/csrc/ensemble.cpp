@@ -225,6 +225,7 @@ void prepare_grids(clover_ensemble *e)
     // the step's halo updates, for both sweep orders
     for (int ax = 0; ax < 2; ax++)
         for (int which = FH_TIMESTEP; which <= FH_MOM3; which++) {
+            if (which == FH_PRESSURE) continue;  // the Lagrangian march exchanges nothing
             const HaloPlan p = fused_halo_plan(which, ax != 0, AX_ALL);
             halo_grid(e, p.fields, p.raxes, p.depth);
         }
