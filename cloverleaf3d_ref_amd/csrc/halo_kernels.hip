@@ -290,7 +290,11 @@ __global__ void __launch_bounds__(kOnceThreads) k_reflect_once(Lay g, int depth,
 // reflection reads the opposite face's halo.  10 x 2 x 2: 40 launches per
 // step -> 8, the step 218 -> 95 us.
 constexpr int kOrderedThreads = 1024;
-constexpr int kOrderedCells = 16 * kOrderedThreads;  // largest face, layers included: beyond it the launches win
+// Largest face, layers included: beyond it the launches win.  n x n x 2 cells, per
+// step, launches against this (two rounds): 16 140 and 140 us against 104 and 100,
+// 64 158 and 197 against 157, 80 (14450 cells) 150 and 193 against 189, 96 (20402)
+// 154 and 194 against 230, 256 242 against 1030.
+constexpr int kOrderedCells = 16 * kOrderedThreads;
 
 template <typename S>
 __global__ void __launch_bounds__(kOrderedThreads) k_reflect_ordered(Lay g, int depth, OnceSet o)
