@@ -44,7 +44,6 @@ struct clover_ensemble {
     double g_small = 0.0, g_big = 0.0;
     int step = 0;
     int advect_x = 1;
-    Slots slots;  // where the table holds each array (its own slot between steps)
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // index: advect_x
     Shapes shapes{};                               // launch shapes in force (size, autotuner, set_shape)
     Shapes size{};                                 // those it started with (size_shapes)
@@ -132,17 +131,16 @@ void set_fields(int *fields, std::initializer_list<int> ids)
 
 // update_halo for single-tile decks: the reflective boundary of every face
 // (axes null), or reduced to the halos the fused kernels read
-void halo(clover_ensemble *e, const int *fields, int depth, const int *axes = nullptr)
+void halo(clover_ensemble *e, const Slots &sl, const int *fields, int depth, const int *axes = nullptr)
 {
-    hip_check(batch_reflect(e->store, e->dev, e->nd, halo_grid(e, fields, axes, depth), depth, fields, e->slots,
-                            e->st, axes),
+    hip_check(batch_reflect(e->store, e->dev, e->nd, halo_grid(e, fields, axes, depth), depth, fields, sl, e->st, axes),
               "halo");
 }
 
-void halo(clover_ensemble *e, int which)
+void halo(clover_ensemble *e, const Slots &sl, int which)
 {
     const HaloPlan p = fused_halo_plan(which, e->advect_x != 0, AX_ALL);  // driver.h
-    halo(e, p.fields, p.depth, p.raxes);
+    halo(e, sl, p.fields, p.depth, p.raxes);
 }
 
 void ideal_gas(clover_ensemble *e)
@@ -150,70 +148,67 @@ void ideal_gas(clover_ensemble *e)
     hip_check(batch_ideal_gas(e->store, e->dev, e->nd, kgrid(e, BK_IDEAL_GAS), e->st), "ideal_gas");
 }
 
-// arrays exchange roles; settle brings the device table in line
-void swap(clover_ensemble *e, std::initializer_list<std::pair<int, int>> pairs)
+// arrays exchange roles within a step
+void swap(Slots &sl, std::initializer_list<std::pair<int, int>> pairs)
 {
-    for (auto &p : pairs) std::swap(e->slots.s[p.first], e->slots.s[p.second]);
+    for (auto &p : pairs) std::swap(sl.s[p.first], sl.s[p.second]);
 }
 
-void settle(clover_ensemble *e, bool add_time)
-{
-    hip_check(batch_move(e->dev, e->nd, e->slots, add_time, e->st), "slots");
-    e->slots = Slots();
-}
-
-void advec_cell(clover_ensemble *e, int sweep, int dir)
+void advec_cell(clover_ensemble *e, Slots &sl, int sweep, int dir)
 {
     const BatchKernel k = dir == 1 ? BK_CELL_X : dir == 2 ? BK_CELL_Y : BK_CELL_Z;
     // the third sweep also writes ideal_gas of the new state: the next step's
     // (or a summary's) equation of state
     hip_check(batch_advec_cell(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, sweep == 3,
-                               e->slots, shape(e, k), e->st),
+                               sl, shape(e, k), e->st),
               "advec_cell");
-    swap(e, {{F_DENSITY1, X_W1}, {F_ENERGY1, X_W2}});
+    swap(sl, {{F_DENSITY1, X_W1}, {F_ENERGY1, X_W2}});
 }
 
-void advec_mom(clover_ensemble *e, int sweep, int dir)
+void advec_mom(clover_ensemble *e, Slots &sl, int sweep, int dir)
 {
     const BatchKernel k = dir == 1 ? BK_MOM_X : dir == 2 ? BK_MOM_Y : BK_MOM_Z;
-    hip_check(batch_advec_mom(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, e->slots, shape(e, k),
-                              e->st),
+    hip_check(batch_advec_mom(e->store, e->dev, e->nd, kgrid(e, k), e->advect_x, dir, sweep, sl, shape(e, k), e->st),
               "advec_mom");
-    swap(e, {{F_XVEL1, X_W5}, {F_YVEL1, X_W6}, {F_ZVEL1, X_W7}});
+    swap(sl, {{F_XVEL1, X_W5}, {F_YVEL1, X_W6}, {F_ZVEL1, X_W7}});
 }
 
 // hydro.f90:48-68 for every deck, device only
 void enqueue_step(clover_ensemble *e)
 {
+    // where the table holds each array: the step's own, so that one that fails, or
+    // whose capture does, leaves nothing behind on the host
+    Slots sl;
     // timestep.f90:28-128; its ideal_gas results were written by the previous
     // step's third cell sweep (or by the start sequence)
-    halo(e, FH_TIMESTEP);
+    halo(e, sl, FH_TIMESTEP);
     const BatchGrid &vg = kgrid(e, BK_VISC_DT);
     hip_check(batch_visc_dt(e->store, e->dev, e->nd, vg, shape(e, BK_VISC_DT), e->g_small, e->visc_partial, e->st),
               "visc_dt");
     hip_check(batch_deck_dt(e->dev, e->nd, vg.start, e->visc_partial, e->g_big, e->st), "deck dt");
-    halo(e, FH_VISCOSITY);
+    halo(e, sl, FH_VISCOSITY);
     // every deck is one mirrored tile: its Lagrangian phase is one march
     hip_check(batch_lagrange(e->store, e->dev, e->nd, kgrid(e, BK_LAGRANGE), shape(e, BK_LAGRANGE), e->st),
               "PdV predict + accelerate + PdV correct + flux_calc");
     // advection.f90:26-181
     int dir = e->advect_x ? 1 : 3;
-    halo(e, FH_CELL1);
-    advec_cell(e, 1, dir);
-    halo(e, FH_MOM1);
-    advec_mom(e, 1, dir);
-    halo(e, FH_CELL2);
-    advec_cell(e, 2, 2);
-    halo(e, FH_MOM2);
-    advec_mom(e, 2, 2);
+    halo(e, sl, FH_CELL1);
+    advec_cell(e, sl, 1, dir);
+    halo(e, sl, FH_MOM1);
+    advec_mom(e, sl, 1, dir);
+    halo(e, sl, FH_CELL2);
+    advec_cell(e, sl, 2, 2);
+    halo(e, sl, FH_MOM2);
+    advec_mom(e, sl, 2, 2);
     dir = e->advect_x ? 3 : 1;
-    advec_cell(e, 3, dir);
-    halo(e, FH_MOM3);
-    advec_mom(e, 3, dir);
-    // reset_field as an exchange of levels, then time = time + dt
-    swap(e, {{F_DENSITY0, F_DENSITY1}, {F_ENERGY0, F_ENERGY1}, {F_XVEL0, F_XVEL1}, {F_YVEL0, F_YVEL1},
-             {F_ZVEL0, F_ZVEL1}});
-    settle(e, true);
+    advec_cell(e, sl, 3, dir);
+    halo(e, sl, FH_MOM3);
+    advec_mom(e, sl, 3, dir);
+    // reset_field as an exchange of levels, the device table brought in line,
+    // then time = time + dt
+    swap(sl, {{F_DENSITY0, F_DENSITY1}, {F_ENERGY0, F_ENERGY1}, {F_XVEL0, F_XVEL1}, {F_YVEL0, F_YVEL1},
+              {F_ZVEL0, F_ZVEL1}});
+    hip_check(batch_move(e->dev, e->nd, sl, true, e->st), "slots");
 }
 
 // every prefix table a step uses, built before any graph capture (building
@@ -479,7 +474,7 @@ int clover_ensemble_create(const clover_deck *decks, int ndecks, int device, int
         int f[NUM_FIELDS];
         set_fields(f, {F_DENSITY0, F_ENERGY0, F_PRESSURE, F_VISCOSITY, F_DENSITY1, F_ENERGY1, F_XVEL0, F_YVEL0,
                        F_ZVEL0, F_XVEL1, F_YVEL1, F_ZVEL1});
-        halo(e, f, 2);
+        halo(e, Slots(), f, 2);
         hip_check(hipStreamSynchronize(e->st), "sync");
         *out = e;
         return 0;
