@@ -925,8 +925,10 @@ k_field_summary(Lay g, Lay gv, int nj, int nk, int ncells, const double *__restr
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     // The XCD-contiguous order: a cell's rows and planes of nodes are its
     // neighbours' too, and dealt round-robin the XCDs each fetched them all
-    // (160x96x120 with the final sum 38.9 -> 29.2 us, two cells at a time 27.5;
-    // 200^3 152 -> 123).  The partials stay where they were, so the sums do too.
+    // (with the final sum, 160x96x120 39.9 -> 33.2 us, two cells at a time 32.5, on
+    // arrays that are not in the caches; 38.7 -> 28.4 and 27.3 on the same arrays
+    // again, 200^3 152 -> 126 and 123).  The partials stay where they were, so the
+    // sums do too.
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
 #pragma unroll 2
     for (int c = blk * RED_THREADS + threadIdx.x; c < ncells; c += gridDim.x * RED_THREADS) {
